@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void k_diff_weights(DiffOpArgs a, double *W, d
     d.rb = a.q0[j].y;
     return d;
   };
-  for_neighbours<4>(a.nb, s, a.npad, a.cnt[s], load, [&](const J &d) {
+  for_neighbours<1, 4>(a.nb, s, 0, a.npad, a.cnt[s], load, [&](const J &d) {
     double xb = d.pb.x, yb = d.pb.y, zb = d.pb.z;
     if (d.code != kNoImage) image_shift(xb, yb, zb, d.code, a.b);
     double G[6];

@@ -16,6 +16,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/sph_hip.h"
@@ -36,16 +37,16 @@ __global__ void k_prep(Fields, const int64_t *, int, int64_t, Box, Grid, int, do
 template <int DIM, bool EXT>
 __global__ void k_neigh(NeighArgs, const double4 *__restrict__, const float4 *__restrict__, uint32_t *__restrict__,
                         int *__restrict__);
-template <int DIM, int KT, typename PT, typename V4>
+template <int DIM, int KT, typename PT, typename V4, int G>
 __global__ void k_loop2_fab(Loop2Args<V4>);
-template <int DIM, int KT, int GRAD, typename PT>
+template <int DIM, int KT, int GRAD, typename PT, int G>
 __global__ void k_loop1(Loop1Args<double4>);
-template <int DIM, int KT, int GRAD, typename PT>
+template <int DIM, int KT, int GRAD, typename PT, int G>
 __global__ void k_loop1_simple(Loop1Args<double4>, Fields);
 template <typename V4>
 __global__ void k_post1(Fields, PostSel, const uint8_t *, int, int, int, int, double, double, V4 *, V4 *,
                         V4 *, V4 *, V4 *, double4 *, double *, float2 *, long long *, long long *);
-template <int DIM, int KT, typename PT, typename V4, int MODE>
+template <int DIM, int KT, typename PT, typename V4, int MODE, int G>
 __global__ void k_loop2(Loop2Args<V4>);
 __global__ void k_aos_to_soa(const double *, int64_t, int, Fields, int64_t *);
 __global__ void k_step_close(const double *, int, const int *, const long long *, long long *);
@@ -130,6 +131,7 @@ constexpr int kZeroLL = kErrLL + 4;
 constexpr int kFlagSlots = 6 * kStripes;
 constexpr int kStepLL = 9 * kStripes;     // the counters before the sweep regions
 enum { kErrSearch = 0, kErrLoop1 = 1, kErrLoop2 = 2 };
+constexpr int kMaxLanes = 8;  // lanes per particle of a pair loop, at most
 constexpr int kAux = 16;  // auxiliary per-particle arrays permuted with the fields
 
 // statevars slots (0-based), const.f90:14-66
@@ -406,7 +408,7 @@ static int ensure_particles(sph_ctx *c, int64_t n) {
   RCHK(dalloc(&c->cnt, npad));
   size_t v4 = c->opt.precision == 1 ? sizeof(float4) : sizeof(double4);
   for (int k = 0; k < 5; k++) RCHK(dev_alloc(&c->q[k], v4 * npad));
-  c->energy_cap = (npad + kBlock - 1) / kBlock;
+  c->energy_cap = (npad * kMaxLanes + kBlock - 1) / kBlock;
   RCHK(dalloc(&c->energy_part, c->energy_cap));
   // radix-sort scratch for n keys
   size_t bytes = 0;
@@ -919,13 +921,78 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
 }
 
 // ------------------------------------------------------------ step: loops
+// Lanes per particle of the pair loops (1, 4 or 8).  One lane walks a list
+// alone: on a lattice in row order the wave's 64 k-th neighbours lie side by
+// side and every list is as long, and the loop is bound by its arithmetic
+// (loop 1 at 128^3 in FP32 0.452 ms, split over 4 lanes 0.495, over 8 0.566).
+// Where lists differ the wave waits for its longest and its k-th neighbours
+// drift apart; several lanes of one particle read runs of its cell rows
+// instead, and few particles then still fill the chip:
+//   3D, particles that move (hydro, MHD, FLD): 8 (the tube of 1M particles,
+//     MHD in FP32: loop 2 3.44 -> 1.46 ms, with 4 lanes 1.73; sweeps 2.65 ->
+//     1.57 ms);
+//   3D diffusion: 4 (100^3 jittered 0.05: loop 2 0.305 -> 0.247 ms FP32, loop 1
+//     0.458 -> 0.361 FP64), 8 below 40k particles (32^3 0.036 -> 0.018 ms),
+//     but 1 for 700k particles and more whose last lists were even, within
+//     5 % of their mean (100^3 lattice 0.219 against 0.247 ms), and 1 for loop
+//     2 of the 2nw operators from 300k particles on (80^3 0.558 against
+//     0.592 ms);
+//   2D, some 28 neighbours: 8 below 40k particles (64^2: sweeps 0.056 ->
+//     0.025 ms, loop 2 0.029 -> 0.011), 4 below 150k (256^2 0.051 -> 0.041 and
+//     0.032 -> 0.025), then 1 (512^2 0.078 against 0.089, 0.069 against 0.071).
+// FP32: loop 1 keeps its sums in list order on 8 lanes (k_loop1), which pays
+// below 100k particles in 3D diffusion (40^3 0.038 -> 0.031 ms, 64^3 0.072
+// against 0.086) and below 40k in 2D; loop 2 of 2D stays on one lane, since
+// the accelerations of a 2D set at rest are the small remainder of large terms
+// and another order's rounding moves them by 4e-5.
+static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2) {
+  const int64_t n = c->n;
+  const bool mixed = c->opt.precision == 1;
+  if (P.dim == 1 || (mixed && loop2 && P.dim == 2)) return 1;
+  if (P.dim == 3 && P.hydro) return 8;
+  if (mixed && !loop2) return n < (P.dim == 3 ? 100000 : 40000) ? 8 : 1;
+  if (n < 40000) return 8;
+  if (P.dim == 2) return n < 150000 ? 4 : 1;
+  if (loop2 && P.diff && !P.fld && (P.ddw == 403 || P.ddw == 404)) return n < 300000 ? 4 : 1;
+  const bool even =
+      c->stats.n_pairs > 0 && (double)c->last_maxcnt * (double)c->n_real <= 1.05 * (double)c->stats.n_pairs;
+  return n >= 700000 && even ? 1 : 4;
+}
+
+// fn(constant G) for lanes = 1, 4 (where HAS4) or 8 (where HAS8)
+template <bool HAS4, bool HAS8, typename Fn>
+static void with_lanes(int lanes, Fn fn) {
+  if constexpr (HAS8) {
+    if (lanes == 8) return fn(std::integral_constant<int, 8>{});
+  }
+  if constexpr (HAS4) {
+    if (lanes == 4) return fn(std::integral_constant<int, 4>{});
+  }
+  fn(std::integral_constant<int, 1>{});
+}
+
 template <int DIM, int KT>
 static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simple, Fields F) {
-  unsigned G = grid_for(a.n);
   bool mixed = c->opt.precision == 1;
-#define L1(GR, PT)                                                                                   \
-  if (simple) hipLaunchKernelGGL((k_loop1_simple<DIM, KT, GR, PT>), dim3(G), dim3(kBlock), 0, c->stream, a, F); \
-  else hipLaunchKernelGGL((k_loop1<DIM, KT, GR, PT>), dim3(G), dim3(kBlock), 0, c->stream, a)
+  if (simple) {
+    // FP32 sums keep the list order: one lane
+    const unsigned B = grid_for((int64_t)a.n * (mixed ? 1 : 8));
+#define L1S(GR, PT, G) \
+  hipLaunchKernelGGL((k_loop1_simple<DIM, KT, GR, PT, G>), dim3(B), dim3(kBlock), 0, c->stream, a, F)
+    if (mixed) {
+      if (grad == 0) { L1S(0, float, 1); } else if (grad == 1) { L1S(1, float, 1); } else { L1S(2, float, 1); }
+    } else {
+      if (grad == 0) { L1S(0, double, 8); } else if (grad == 1) { L1S(1, double, 8); } else { L1S(2, double, 8); }
+    }
+#undef L1S
+    return;
+  }
+  const int lanes = loop_lanes(c, a.p, false);
+#define L1(GR, PT)                                                                                           \
+  with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1>(lanes, [&](auto l) {                          \
+    constexpr int G = decltype(l)::value;                                                                    \
+    hipLaunchKernelGGL((k_loop1<DIM, KT, GR, PT, G>), dim3(grid_for((int64_t)a.n * G)), dim3(kBlock), 0, c->stream, a); \
+  })
   if (mixed) {
     if (grad == 0) { L1(0, float); } else if (grad == 1) { L1(1, float); } else { L1(2, float); }
   } else {
@@ -1017,41 +1084,40 @@ static void launch_sweeps(sph_ctx *c, const Phys &P, int first, int last) {
   tolerate(mark(c, 10));
 }
 
+template <int DIM, int KT, int MODE, typename PT, typename V4>
+static void launch_loop2_p(sph_ctx *c, int lanes, const Loop2Args<V4> &a) {
+  constexpr bool MANY = DIM == 3 || (DIM == 2 && std::is_same_v<PT, double>);
+  with_lanes<MANY, MANY>(lanes, [&](auto l) {
+    constexpr int G = decltype(l)::value;
+    const dim3 B(grid_for(c->n * G)), T(kBlock);
+    if constexpr (MODE == MODE_FAB) hipLaunchKernelGGL((k_loop2_fab<DIM, KT, PT, V4, G>), B, T, 0, c->stream, a);
+    else hipLaunchKernelGGL((k_loop2<DIM, KT, PT, V4, MODE, G>), B, T, 0, c->stream, a);
+  });
+}
 template <int DIM, int KT, int MODE>
-static void launch_loop2(sph_ctx *c, void *args) {
-  unsigned G = grid_for(c->n);
-  if constexpr (MODE == MODE_FAB) {
-    if (c->opt.precision == 1)
-      hipLaunchKernelGGL((k_loop2_fab<DIM, KT, float, float4>), dim3(G), dim3(kBlock), 0, c->stream,
-                         *(Loop2Args<float4> *)args);
-    else
-      hipLaunchKernelGGL((k_loop2_fab<DIM, KT, double, double4>), dim3(G), dim3(kBlock), 0, c->stream,
-                         *(Loop2Args<double4> *)args);
-  } else if (c->opt.precision == 1) {
-    hipLaunchKernelGGL((k_loop2<DIM, KT, float, float4, MODE>), dim3(G), dim3(kBlock), 0, c->stream,
-                       *(Loop2Args<float4> *)args);
-  } else {
-    hipLaunchKernelGGL((k_loop2<DIM, KT, double, double4, MODE>), dim3(G), dim3(kBlock), 0, c->stream,
-                       *(Loop2Args<double4> *)args);
-  }
+static void launch_loop2(sph_ctx *c, int lanes, void *args) {
+  if (c->opt.precision == 1)
+    launch_loop2_p<DIM, KT, MODE, float, float4>(c, lanes, *(Loop2Args<float4> *)args);
+  else
+    launch_loop2_p<DIM, KT, MODE, double, double4>(c, lanes, *(Loop2Args<double4> *)args);
 }
 template <int DIM, int MODE>
-static void launch_loop2_k(sph_ctx *c, void *args) {
-  if (c->kt == KT_M4) launch_loop2<DIM, KT_M4, MODE>(c, args);
-  else if (c->kt == KT_M6) launch_loop2<DIM, KT_M6, MODE>(c, args);
-  else launch_loop2<DIM, KT_GAUSS, MODE>(c, args);
+static void launch_loop2_k(sph_ctx *c, int lanes, void *args) {
+  if (c->kt == KT_M4) launch_loop2<DIM, KT_M4, MODE>(c, lanes, args);
+  else if (c->kt == KT_M6) launch_loop2<DIM, KT_M6, MODE>(c, lanes, args);
+  else launch_loop2<DIM, KT_GAUSS, MODE>(c, lanes, args);
 }
 template <int MODE>
-static void launch_loop2_d(sph_ctx *c, int dim, void *args) {
-  if (dim == 1) launch_loop2_k<1, MODE>(c, args);
-  else if (dim == 2) launch_loop2_k<2, MODE>(c, args);
-  else launch_loop2_k<3, MODE>(c, args);
+static void launch_loop2_d(sph_ctx *c, int dim, int lanes, void *args) {
+  if (dim == 1) launch_loop2_k<1, MODE>(c, lanes, args);
+  else if (dim == 2) launch_loop2_k<2, MODE>(c, lanes, args);
+  else launch_loop2_k<3, MODE>(c, lanes, args);
 }
 // modes built in 2D and 3D only
 template <int MODE>
-static void launch_loop2_d23(sph_ctx *c, int dim, void *args) {
-  if (dim == 2) launch_loop2_k<2, MODE>(c, args);
-  else launch_loop2_k<3, MODE>(c, args);
+static void launch_loop2_d23(sph_ctx *c, int dim, int lanes, void *args) {
+  if (dim == 2) launch_loop2_k<2, MODE>(c, lanes, args);
+  else launch_loop2_k<3, MODE>(c, lanes, args);
 }
 
 template <typename V4>
@@ -1123,17 +1189,18 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P) {
   // is built for it (2D and 3D: hydro, magnetohydro, hydro with FLD)
   const int terms =
       c->loop2_generic ? -1 : (P.hydro ? 1 : 0) | (P.magneto ? 2 : 0) | (P.diff ? 4 : 0) | (P.fld ? 8 : 0);
-  if (generic && P.dim >= 2 && terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, &a);
-  else if (generic && P.dim >= 2 && terms == kSpecMhd) launch_loop2_d23<MODE_SPEC + kSpecMhd>(c, P.dim, &a);
+  const int lanes = loop_lanes(c, P, true);
+  if (generic && P.dim >= 2 && terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, lanes, &a);
+  else if (generic && P.dim >= 2 && terms == kSpecMhd) launch_loop2_d23<MODE_SPEC + kSpecMhd>(c, P.dim, lanes, &a);
   else if (generic && P.dim >= 2 && terms == kSpecHydroFld)
-    launch_loop2_d23<MODE_SPEC + kSpecHydroFld>(c, P.dim, &a);
-  else if (generic) launch_loop2_d<MODE_GENERIC>(c, P.dim, &a);
-  else if (fab) launch_loop2_d<MODE_FAB>(c, P.dim, &a);
-  else launch_loop2_d<MODE_DIFF>(c, P.dim, &a);
+    launch_loop2_d23<MODE_SPEC + kSpecHydroFld>(c, P.dim, lanes, &a);
+  else if (generic) launch_loop2_d<MODE_GENERIC>(c, P.dim, lanes, &a);
+  else if (fab) launch_loop2_d<MODE_FAB>(c, P.dim, lanes, &a);
+  else launch_loop2_d<MODE_DIFF>(c, P.dim, lanes, &a);
   HIPCHK(mark(c, 6));
   // energy, error bits and h_max in one record of d_stripes, which the
   // caller's copy_record brings back with the step's closing sync
-  hipLaunchKernelGGL(k_step_close, dim3(1), dim3(256), 0, c->stream, c->energy_part, (int)G,
+  hipLaunchKernelGGL(k_step_close, dim3(1), dim3(256), 0, c->stream, c->energy_part, (int)grid_for((int64_t)n * lanes),
                      step_err(c) + kErrLoop2, c->d_stripes + kHmaxLL, c->d_stripes + kCloseRec);
   c->loop2_pending = true;
   return SPH_OK;

@@ -84,28 +84,93 @@ struct ExtGrid {
   float lenf[3];  // box lengths in FP32 (0 on axes that are not imaged)
 };
 
-// Neighbour iteration with batched gathers: entries come 8 per coalesced
-// chunk; for every NB of them `load(entry)` issues all gathers first (slots
+// Sum over the G consecutive lanes that share one particle (G = 1, 2, 4, 8),
+// through DPP moves: lane pairs, pairs of a quad, then the two quads of eight
+// (mirrored, each quad holding one value by then).  Every lane of the group
+// gets the same bits.
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true));
+}
+template <int G, typename T>
+__device__ __forceinline__ void group_sum(T &v) {
+  if constexpr (G >= 2) v += dpp_mov<0xB1>(v);   // quad_perm [1,0,3,2]
+  if constexpr (G >= 4) v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
+  if constexpr (G >= 8) v += dpp_mov<0x141>(v);  // row_half_mirror
+}
+template <int G, typename T, typename... R>
+__device__ __forceinline__ void group_sum(T &v, R &...r) {
+  group_sum<G>(v);
+  if constexpr (sizeof...(R) > 0) group_sum<G>(r...);
+}
+
+// Neighbour iteration with batched gathers, G lanes per particle (G = 1, 4 or
+// 8; lane `sub` of them takes entries sub, sub + G, ...: neighbouring lanes
+// take neighbouring entries, mostly neighbouring particles of one cell row).
+// For every NB entries of a lane `load(entry)` issues all gathers first (slots
 // past the list end reload particle s, always a valid address), then
-// `body(data)` runs on the valid ones.  NB gathers are then in flight at once.
-template <int NB, typename Load, typename Body>
-__device__ __forceinline__ void for_neighbours(const uint32_t *nb, int s, int npad, int nn, Load load, Body body) {
+// `body(data)` runs on the valid ones: NB gathers are in flight at once.
+// With G > 1 the next entries are read while this batch's gathers run.
+template <int G, int NB, typename Load, typename Body>
+__device__ __forceinline__ void for_neighbours(const uint32_t *nb, int s, int sub, int npad, int nn, Load load,
+                                               Body body) {
   const uint32_t self = nb_pack((uint32_t)s, kNoImage);
-  for (int k0 = 0; k0 < nn; k0 += 8) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(nb + nb_slot(k0, s, npad));
-    const uint4 lo = p[0], hi = p[1];
-    const uint32_t e8[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    const int m = min(8, nn - k0);
+  if constexpr (G == 1) {
+    for (int k0 = 0; k0 < nn; k0 += 8) {
+      const uint4 *p = reinterpret_cast<const uint4 *>(nb + nb_slot(k0, s, npad));
+      const uint4 lo = p[0], hi = p[1];
+      const uint32_t e8[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      const int m = min(8, nn - k0);
 #pragma unroll
-    for (int h = 0; h < 8; h += NB) {
-      if (h < m) {
+      for (int h = 0; h < 8; h += NB) {
+        if (h < m) {
+          decltype(load(0u)) jd[NB];
+#pragma unroll
+          for (int u = 0; u < NB; u++) jd[u] = load(h + u < m ? e8[h + u] : self);
+#pragma unroll
+          for (int u = 0; u < NB; u++)
+            if (h + u < m) body(jd[u]);
+        }
+      }
+    }
+  } else {
+    // E entries of a lane per chunk, C chunks read together
+    constexpr int E = 8 / G, C = NB > E ? NB / E : 1, M = E * C;
+    static_assert(M % NB == 0, "a batch divides the entries read together");
+    const uint32_t *p = nb + ((size_t)s * 8 + sub);
+    const size_t stride = (size_t)npad * 8;
+    uint32_t e[M], next[M];
+    auto read = [&](int k0) {
+#pragma unroll
+      for (int c = 0; c < C; c++) {
+        if (k0 + 8 * c < nn) {
+#pragma unroll
+          for (int u = 0; u < E; u++) next[c * E + u] = p[u * G];
+        }
+        p += stride;
+      }
+    };
+    read(0);
+    int rem = nn - sub;  // entry u of chunk c exists while 8 c + u G < rem
+    for (int k0 = 0; k0 < nn; k0 += 8 * C) {
+#pragma unroll
+      for (int u = 0; u < M; u++) e[u] = next[u];
+#pragma unroll
+      for (int h = 0; h < M; h += NB) {
         decltype(load(0u)) jd[NB];
 #pragma unroll
-        for (int u = 0; u < NB; u++) jd[u] = load(h + u < m ? e8[h + u] : self);
+        for (int u = h; u < h + NB; u++) jd[u - h] = load(8 * (u / E) + u % E * G < rem ? e[u] : self);
+        if (h == 0) read(k0 + 8 * C);
 #pragma unroll
-        for (int u = 0; u < NB; u++)
-          if (h + u < m) body(jd[u]);
+        for (int u = h; u < h + NB; u++)
+          if (8 * (u / E) + u % E * G < rem) body(jd[u - h]);
       }
+      rem -= 8 * C;
     }
   }
 }

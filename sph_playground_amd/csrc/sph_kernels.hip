@@ -12,9 +12,12 @@
 //              sector per chunk; a wavefront reads a chunk with two
 //              coalesced 16-byte loads per lane
 //
-// Every kernel maps one particle per lane (64-lane wavefronts, 256 per block)
-// and remaps blockIdx so each XCD works on a contiguous range of the Morton
-// curve (its particles' neighbours then stay in that XCD's L2).  Counters are
+// Every kernel but the pair loops maps one particle per lane (64-lane
+// wavefronts, 256 per block); the pair loops give a particle G = 1, 4 or 8
+// consecutive lanes, which share its list and add their sums at its end (the
+// host's loop_lanes holds the rule).  Every kernel remaps blockIdx so each XCD
+// works on a contiguous range of the particle order (its particles'
+// neighbours then stay in that XCD's L2).  Counters are
 // reduced per block and added to one of 64 stripes, never all to one address.
 #include <hip/hip_runtime.h>
 
@@ -833,15 +836,45 @@ __device__ __forceinline__ void fix_sep(const uint3 &qa, const uint3 &qb, uint32
   r2 = DIM == 3 ? (float)(int)dz * f.scale[2] : 0.f;
 }
 
+// Gathers a lane of loop 1 or k_loop2_fab keeps in flight.  One lane per
+// particle: four (eight measured slower at 128^3 in FP32, 0.55 against 0.51 ms;
+// FP64 two and eight both slower).  Four lanes: four in FP32 (k_loop2_fab at
+// 100^3 jittered 0.247 ms against 0.252 with two), two in FP64 (80^3 0.180
+// against 0.187).  Eight lanes: two (sums split over the lanes, the MHD tube's
+// sweeps 1.48 ms against 1.73 with one; four 1.55).
+template <typename PT>
+constexpr int pair_batch(int g) {
+  return g == 1 ? 4 : (g == 4 && std::is_same_v<PT, float> ? 4 : 2);
+}
+
+// Entries per batch of loop 1's FP32 sums over eight lanes: 16 (the MHD tube's
+// sweeps 1.57 ms; 8: 1.92, 32: 1.69).
+constexpr int kOrd = 16;
+
 // ---------------------------------------------------------------- loop 1
 // One Jacobi sweep of c1advanced (circuit1.f90:114-211) for the particles
 // still active (eps > tol); frozen ones carry their state to the next buffer.
 // GRAD: 0 no grad T, 1 standard (:178-179), 2 the 2nw_sd form (:174-176).
 // PT is the pair arithmetic type; the Newton update is always FP64.
-template <int DIM, int KT, int GRAD, typename PT>
+//
+// FP32 sums are run in list order whatever G is: particles with Omega near 0
+// (a close pair in a random set) divide by it in loop 2, so another order's
+// rounding, 1e-7 of the sum, can move their accelerations by 1e-3, and a
+// particle at the Newton tolerance takes a sweep more or less.  With eight
+// lanes the lanes compute the terms' operands side by side, pass them through
+// LDS, and lane k then runs sum k (one fused multiply-add per entry, at most
+// eight sums): the bits of one lane's loop for 5 % more time than sums split
+// over the lanes (MHD tube of 1M particles, five sweeps: one lane 2.65 ms,
+// split 1.49, in order 1.57).
+template <int DIM, int KT, int GRAD, typename PT, int G>
 __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
-  __shared__ long long lds[4];
+  __shared__ int cnts[8];  // per wave: still active, pairs
   __shared__ int skip;
+  // FP32 sums over eight lanes stay in list order (see below)
+  constexpr bool ORD = G == 8 && std::is_same_v<PT, float>;
+  constexpr int NSUM = GRAD == 0 ? 2 : (GRAD == 1 ? 5 : 8);  // sums, and their operands
+  constexpr int NOPS = GRAD == 0 ? 3 : (GRAD == 1 ? 7 : 8);
+  __shared__ __align__(16) float ord_ops[ORD ? 32 * NOPS * kOrd : 4];
   // while maxval(eps) > tol (circuit1.f90:114), decided here: the first
   // wave reads the previous sweep's still-active stripes (set before this
   // launch began) and the error words, so the whole block agrees
@@ -856,7 +889,7 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
     *a.which = a.sweep & 1;
     a.stripes[2 * kStripes] = 1;
   }
-  int s = gtid();
+  const int t = gtid(), s = t / G, sub = t & (G - 1);
   bool inb = s < a.n;
   // the first sweep starts from the fields themselves (h, den, om, T as the
   // step found them) with every real particle active; later sweeps from the
@@ -870,7 +903,7 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
   // the FP32 path gathers 20 bytes per pair: the 12-byte position record
   // (31-bit fractions) and the FP32 m and T den
   constexpr bool PACK = GRAD == 1 && std::is_same_v<PT, float>;
-  if (inb && !act) {
+  if (inb && !act && sub == 0) {
     a.next[s] = c;
     if constexpr (PACK) a.s1n[s] = a.s1c[s];
     else if constexpr (GRAD == 1) a.trn[s] = a.trc[s];
@@ -881,8 +914,7 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
     const double4 pa = a.pm[s];
     const double ma = pa.w;
     const PT inv_ha = (PT)(1.0 / ha);
-    PT dsum = 0, osum = 0;
-    PT g0 = 0, g1 = 0, g2 = 0, h0x = 0, h0y = 0, h0z = 0;
+    PT sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     bool qbad = !(ha > 0.0);
     nn = a.cnt[s];
     // j side: x, y, z, m, and what grad T needs of the previous sweep (GRAD 1:
@@ -905,9 +937,9 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
       if constexpr (GRAD == 2) d.sb = a.cur[j];
       return d;
     };
-    // four gathers in flight (with particles in row order, eight measured
-    // slower in the FP32 path: 0.55 against 0.51 ms at 128^3)
-    for_neighbours<4>(a.nb, s, a.npad, nn, load, [&](const J &d) {
+    // the terms of one pair: add(k, x, y) adds x y to sum k (0 density, 1
+    // Omega, 2..4 grad T, 5..7 the h_b part of the 2nw_sd grad T)
+    auto terms = [&](const J &d, auto add) {
       PT r0, r1, r2;
       if constexpr (PACK) {
         fix_sep<DIM>(qa, d.pc, d.code, a.ff, r0, r1, r2);
@@ -934,8 +966,8 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
       PT mb;
       if constexpr (PACK) mb = d.sc.x;
       else mb = (PT)d.pb.w;
-      dsum += mb * f;
-      osum += mb * (PT(DIM) * f + q * df);
+      add(0, mb, f);
+      add(1, mb, PT(DIM) * f + q * df);
       if constexpr (GRAD != 0) {
         const double4 sb = d.sb;
         // r = 0 gives NaN here, as 1/|r| times the kernels' derivative (0
@@ -946,7 +978,7 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
           if constexpr (PACK) trb = d.sc.y;
           else trb = (PT)d.tr;
           PT w = mb * (trb - (PT)ta * (PT)rhoa) * df * inv_dr;
-          g0 += w * r0; g1 += w * r1; g2 += w * r2;
+          add(2, w, r0); add(3, w, r1); add(4, w, r2);
         } else {
           PT inv_hb, i_ob_rb2;  // 1/h_b and 1/(om_b rho_b^2)
           if constexpr (std::is_same_v<PT, double>) {
@@ -962,12 +994,81 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
           PT dfb = K::df(qb);
           PT wa = mb * df * inv_dr;
           PT wb = mb * (PT)sb.w * (PT)rhoa * i_ob_rb2 * dfb * inv_dr * ipow<DIM + 1>(inv_hb);
-          g0 += wa * r0; g1 += wa * r1; g2 += wa * r2;
-          h0x += wb * r0; h0y += wb * r1; h0z += wb * r2;
+          add(2, wa, r0); add(3, wa, r1); add(4, wa, r2);
+          add(5, wb, r0); add(6, wb, r1); add(7, wb, r2);
         }
       }
       qbad |= !(q >= PT(0));
-    });
+    };
+    if constexpr (ORD) {
+      // A batch of kOrd entries: their operands into the group's LDS rows
+      // (zeros past the list's end: 0 0 adds nothing), then lane k runs sum
+      // k over them in list order.  A group lies in one wavefront, whose LDS
+      // accesses complete in order: no barrier but the compiler's.
+      constexpr int C = kOrd / 8;
+      float *const row = ord_ops + (threadIdx.x / 8) * (NOPS * kOrd);
+      // operand rows: 0 m_b, 1 and 2 its factors, 3 the weight of grad T,
+      // 4..6 the separation, 7 the weight of the h_b part
+      const int k = sub < NSUM ? sub : 0;
+      const float *const xs = row + (k < 2 ? 0 : (k < 5 ? 3 : 7)) * kOrd;
+      const float *const ys = row + (k < 2 ? 1 + k : (k < 5 ? 2 + k : k - 1)) * kOrd;
+      const uint32_t self = nb_pack((uint32_t)s, kNoImage);
+      const uint32_t *p = a.nb + ((size_t)s * 8 + sub);
+      const size_t stride = (size_t)a.npad * 8;
+      uint32_t e[C];
+      auto read = [&](int k0) {
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+          if (k0 + 8 * c < nn) e[c] = *p;
+          p += stride;
+        }
+      };
+      read(0);
+      float acc = 0.f;
+      for (int k0 = 0; k0 < nn; k0 += kOrd) {
+        J jd[C];
+#pragma unroll
+        for (int c = 0; c < C; c++) jd[c] = load(k0 + 8 * c + sub < nn ? e[c] : self);
+        read(k0 + kOrd);
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+          float ops[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+          if (k0 + 8 * c + sub < nn)
+            terms(jd[c], [&](int q, PT x, PT y) {
+              ops[q < 2 ? 0 : (q < 5 ? 3 : 7)] = x;
+              ops[q < 2 ? 1 + q : (q < 5 ? 2 + q : q - 1)] = y;
+            });
+#pragma unroll
+          for (int o = 0; o < NOPS; o++) row[o * kOrd + 8 * c + sub] = ops[o];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int v = 0; v < kOrd; v += 4) {
+          const float4 x = *reinterpret_cast<const float4 *>(xs + v);
+          const float4 y = *reinterpret_cast<const float4 *>(ys + v);
+          acc = fmaf(x.x, y.x, acc);
+          acc = fmaf(x.y, y.y, acc);
+          acc = fmaf(x.z, y.z, acc);
+          acc = fmaf(x.w, y.w, acc);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      // every sum to lane 0 of the group
+#pragma unroll
+      for (int q = 0; q < NSUM; q++) sum[q] = __shfl(acc, (threadIdx.x & 56) + q, 64);
+    } else {
+      for_neighbours<G, pair_batch<PT>(G)>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
+        terms(d, [&](int q, PT x, PT y) { sum[q] += x * y; });
+      });
+#pragma unroll
+      for (int q = 0; q < NSUM; q++) group_sum<G>(sum[q]);
+    }
+    const PT dsum = sum[0], osum = sum[1], g0 = sum[2], g1 = sum[3], g2 = sum[4], h0x = sum[5], h0y = sum[6],
+             h0z = sum[7];
     const double wcv = a.p.wcv;
     const double ih = 1.0 / ha;
     const double cW = wcv * ipow<DIM>(ih);
@@ -984,11 +1085,8 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
     if (qbad) atomicOr(a.err, EB_Q);
     // h at entry: the first sweep starts from it
     double ep = fabs(hn - ha) / (first ? ha : a.h0[s]);
-    a.eps[s] = ep;
-    still = ep > a.tol;
-    a.next[s] = make_double4(hn, den, osm, ta);
-    if constexpr (PACK) a.s1n[s] = make_float2((float)ma, (float)(ta * den));
-    else if constexpr (GRAD == 1) a.trn[s] = ta * den;
+    still = ep > a.tol && sub == 0;
+    if (sub != 0) nn = 0;  // counted once per particle
     double gx = 0, gy = 0, gz = 0;
     if constexpr (GRAD == 1) {
       double cN = wcv * ipow<DIM + 1>(ih) / rhoa / oma;
@@ -999,21 +1097,32 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
       gy = cA * (double)g1 + wcv * (double)h0y;
       gz = cA * (double)g2 + wcv * (double)h0z;
     }
-    a.dtdx[s] = gx; a.dtdy[s] = gy; a.dtdz[s] = gz;
+    if (sub == 0) {
+      a.eps[s] = ep;
+      a.next[s] = make_double4(hn, den, osm, ta);
+      if constexpr (PACK) a.s1n[s] = make_float2((float)ma, (float)(ta * den));
+      else if constexpr (GRAD == 1) a.trn[s] = ta * den;
+      a.dtdx[s] = gx; a.dtdy[s] = gy; a.dtdz[s] = gz;
+    }
   }
-  long long act_n = block_reduce<R_SUM>(still ? 1 : 0, lds);
-  if (threadIdx.x == 0 && act_n) atomicAdd((unsigned long long *)&a.stripes[stripe()], (unsigned long long)act_n);
-  long long pairs = block_reduce<R_SUM>(nn, lds);
-  if (threadIdx.x == 0 && pairs) atomicAdd((unsigned long long *)&a.stripes[kStripes + stripe()], (unsigned long long)pairs);
+  // still-active particles and evaluated pairs of the block
+  const int act_w = __popcll(__ballot(still)), nn_w = wave_sum(nn);
+  if ((threadIdx.x & 63) == 0) { cnts[threadIdx.x >> 6] = act_w; cnts[4 + (threadIdx.x >> 6)] = nn_w; }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const int *c4 = cnts + 4 * threadIdx.x;
+    const int v = c4[0] + c4[1] + c4[2] + c4[3];
+    if (v) atomicAdd((unsigned long long *)&a.stripes[threadIdx.x * kStripes + stripe()], (unsigned long long)v);
+  }
 }
 
 // c1simple (circuit1.f90:227-305): direct summation, h = hfac (m/rho)^(1/dim),
 // grad T only for 2nw_ds (:282-284) / 2nw_sd (:285-289), om = 1 (:62,301).
-template <int DIM, int KT, int GRAD, typename PT>
+template <int DIM, int KT, int GRAD, typename PT, int G>
 __global__ __launch_bounds__(256) void k_loop1_simple(Loop1Args<double4> a, Fields F) {
-  int s = gtid();
+  const int t = gtid(), s = t / G, sub = t & (G - 1);
   if (s >= a.n) return;
-  F.f[F_OM][s] = 1.0;
+  if (sub == 0) F.f[F_OM][s] = 1.0;
   if (!a.real[s]) return;
   using K = KernelFn<KT, PT>;
   const double4 c = a.cur[s];
@@ -1032,7 +1141,7 @@ __global__ __launch_bounds__(256) void k_loop1_simple(Loop1Args<double4> a, Fiel
     if constexpr (GRAD != 0) d.sb = a.cur[j];
     return d;
   };
-  for_neighbours<4>(a.nb, s, a.npad, nn, load, [&](const J &d) {
+  for_neighbours<G, 2>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
     double xb = d.pb.x, yb = d.pb.y, zb = d.pb.z;
     if (d.code != kNoImage) image_shift(xb, yb, zb, d.code, a.b);
     PT r0 = (PT)(pa.x - xb), r1 = (PT)(pa.y - yb), r2 = (PT)(pa.z - zb);
@@ -1062,6 +1171,10 @@ __global__ __launch_bounds__(256) void k_loop1_simple(Loop1Args<double4> a, Fiel
     qbad |= !(q >= PT(0));
   });
   if (qbad) atomicOr(a.err, EB_Q);
+  group_sum<G>(dsum);
+  if constexpr (GRAD != 0) group_sum<G>(g0, g1, g2);
+  if constexpr (GRAD == 2) group_sum<G>(h0x, h0y, h0z);
+  if (sub != 0) return;
   const double wcv = a.p.wcv, ih = 1.0 / ha;
   double f0 = KernelFn<KT, double>::f(0.0);
   double den = wcv * ipow<DIM>(ih) * (double)dsum + pa.w * (wcv * ipow<DIM>(ih) * f0);
@@ -1197,11 +1310,11 @@ __device__ __forceinline__ void tensor_contract(const Sym3<T> &kt, T rx, T ry, T
 // The FP64 diffusion-mode loop is latency-bound: at 176 VGPRs it runs 2 waves
 // per SIMD, capped to 168 it runs 3 (a few registers spill) and measured 17 %
 // faster; the other variants are fastest uncapped.
-template <int DIM, int KT, typename PT, typename V4, int MODE>
+template <int DIM, int KT, typename PT, typename V4, int MODE, int G>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu((MODE == MODE_DIFF && std::is_same_v<PT, double>) ? 3 : 1)))
 void k_loop2(Loop2Args<V4> a) {
-  int s = gtid();
+  const int t = gtid(), s = t / G, sub = t & (G - 1);
   double e_part = 0.0;
   if (s < a.n && a.real[s]) {
     using K = KernelFn<KT, PT>;
@@ -1256,7 +1369,7 @@ void k_loop2(Loop2Args<V4> a) {
         PT lam = (PT(2) + fr) / (PT(6) + PT(3) * fr + fr * fr);
         PT d = (PT)kLightspeed * lam / kappaa / rhoa;
         kta.xx = kta.yy = kta.zz = d;
-        a.out.f[F_VFLD][s] = (double)(d / ((ta * rhoa) / gn));
+        if (sub == 0) a.out.f[F_VFLD][s] = (double)(d / ((ta * rhoa) / gn));
       } else {
         kta = tensor_of_b<PT>(P, bax, bay, baz);
         ktb_fixed = kta;  // isotropic, or every particle has the same B
@@ -1306,11 +1419,18 @@ void k_loop2(Loop2Args<V4> a) {
       }
       return d;
     };
-    // neighbours whose gathers are in flight together: two for the MHD and
-    // FLD sets (1M-particle MHD shock tube: 5.23 -> 5.08 ms per step, FLD
-    // unchanged; no occupancy lost), one where a second would cost waves
-    constexpr int NBATCH = MODE == MODE_DIFF ? 4 : (SPEC && TM != kSpecHydro ? 2 : 1);
-    for_neighbours<NBATCH>(a.nb, s, a.npad, nn, load, [&](const J &d) {
+    // a lane's neighbours whose gathers are in flight together.  Diffusion
+    // alone: four (FP32 with four lanes per particle: two, loop 2 of n2w at
+    // 100^3 0.381 -> 0.357 ms; FP64 there four, 0.324 -> 0.306 ms at 80^3).
+    // The other sets read up to six records per neighbour: with eight lanes
+    // two in FP32 (MHD tube of 1M particles 1.57 -> 1.46 ms) and one in FP64
+    // (radiation tube of 120k 0.399 -> 0.352 ms), with one lane two for the
+    // MHD and FLD sets, else one
+    constexpr bool F32 = std::is_same_v<PT, float>;
+    constexpr int NBATCH = MODE == MODE_DIFF ? (G == 4 && F32 ? 2 : (G == 8 ? 2 : 4))
+                           : G == 8          ? (F32 ? 2 : 1)
+                           : G == 1 && SPEC && TM != kSpecHydro ? 2 : 1;
+    for_neighbours<G, NBATCH>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
       const uint32_t code = d.code;
       PT rx, ry, rz;
       if constexpr (CELL) {
@@ -1505,18 +1625,21 @@ void k_loop2(Loop2Args<V4> a) {
       }
     });
     if (qbad) atomicOr(a.err, EB_Q);
-    double dh = 0.0;
-    if (P.adden) dh = -DIM * ha_d / (double)rhoa * (double)drho / (double)oma;
-    a.out.f[F_AX][s] = (double)dvx; a.out.f[F_AY][s] = (double)dvy; a.out.f[F_AZ][s] = (double)dvz;
-    a.out.f[F_DH][s] = dh;
-    a.out.f[F_DDT][s] = (double)ddt;
-    a.out.f[F_DBX][s] = (double)dbx; a.out.f[F_DBY][s] = (double)dby; a.out.f[F_DBZ][s] = (double)dbz;
-    a.out.f[F_DU][s] = (double)du;
-    // FP64 energy sum (circuit2.f90:490-492)
-    const double vx = vx_d, vy = vy_d, vz = vz_d, bx = bx_d, by = by_d, bz = bz_d, rh = rho_d;
-    e_part = pa.w * (vx * (double)dvx + vy * (double)dvy + vz * (double)dvz + (double)du +
-                     (bx * (double)dbx + by * (double)dby + bz * (double)dbz) / rh -
-                     0.5 * (bx * bx + by * by + bz * bz) / rh / rh * (double)drho / om_d);
+    group_sum<G>(dvx, dvy, dvz, du, ddt, dbx, dby, dbz, drho);
+    if (sub == 0) {
+      double dh = 0.0;
+      if (P.adden) dh = -DIM * ha_d / (double)rhoa * (double)drho / (double)oma;
+      a.out.f[F_AX][s] = (double)dvx; a.out.f[F_AY][s] = (double)dvy; a.out.f[F_AZ][s] = (double)dvz;
+      a.out.f[F_DH][s] = dh;
+      a.out.f[F_DDT][s] = (double)ddt;
+      a.out.f[F_DBX][s] = (double)dbx; a.out.f[F_DBY][s] = (double)dby; a.out.f[F_DBZ][s] = (double)dbz;
+      a.out.f[F_DU][s] = (double)du;
+      // FP64 energy sum (circuit2.f90:490-492)
+      const double vx = vx_d, vy = vy_d, vz = vz_d, bx = bx_d, by = by_d, bz = bz_d, rh = rho_d;
+      e_part = pa.w * (vx * (double)dvx + vy * (double)dvy + vz * (double)dvz + (double)du +
+                       (bx * (double)dbx + by * (double)dby + bz * (double)dbz) / rh -
+                       0.5 * (bx * bx + by * by + bz * bz) / rh / rh * (double)drho / om_d);
+    }
   }
   __shared__ double red[4];
   double w = wave_sum(e_part);
@@ -1540,9 +1663,9 @@ void k_loop2(Loop2Args<V4> a) {
 // -wcv / (h^(dim+1) rho_a) after the sum, so no pair divides by rho_a; both
 // take 1/|r| from one reciprocal square root (FP64: the hardware estimate
 // refined by two Newton-Raphson steps).
-template <int DIM, int KT, typename PT, typename V4>
+template <int DIM, int KT, typename PT, typename V4, int G>
 __global__ __launch_bounds__(256) void k_loop2_fab(Loop2Args<V4> a) {
-  int s = gtid();
+  const int t = gtid(), s = t / G, sub = t & (G - 1);
   double e_part = 0.0;
   if (s < a.n && a.real[s]) {
     using K = KernelFn<KT, PT>;
@@ -1592,7 +1715,7 @@ __global__ __launch_bounds__(256) void k_loop2_fab(Loop2Args<V4> a) {
       }
       return d;
     };
-    for_neighbours<4>(a.nb, s, a.npad, nn, load, [&](const J &d) {
+    for_neighbours<G, pair_batch<PT>(G)>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
       PT rx, ry, rz;
       if constexpr (F32) {
         fix_sep<DIM>(qa, d.pc, d.code, a.ff, rx, ry, rz);
@@ -1642,30 +1765,33 @@ __global__ __launch_bounds__(256) void k_loop2_fab(Loop2Args<V4> a) {
         ddt = fma(mb_rhob * (trb - tra), dfa * inv_dr * x, ddt);
       }
     });
-    ddt *= -wcv * ihd1 * rcp_pair(rhoa);
     if (qbad) atomicOr(a.err, EB_Q);
-    const PT zero = 0;
-    double dh = 0.0;
-    if (P.adden) dh = -DIM * ha_d / (double)rhoa * (double)zero / (double)oma;
-    a.out.f[F_AX][s] = 0.0; a.out.f[F_AY][s] = 0.0; a.out.f[F_AZ][s] = 0.0;
-    a.out.f[F_DH][s] = dh;
-    a.out.f[F_DDT][s] = (double)ddt;
-    a.out.f[F_DBX][s] = 0.0; a.out.f[F_DBY][s] = 0.0; a.out.f[F_DBZ][s] = 0.0;
-    a.out.f[F_DU][s] = 0.0;
-    // FP64 energy sum (circuit2.f90:490-492) with zero dv, du, dB, drho.
-    // Every velocity exactly 0 (a signed zero among them changes no term
-    // after the + 0 below) or one B for every particle: no per-particle loads
-    double vx = 0.0, vy = 0.0, vz = 0.0, bx, by, bz;
-    if (a.v_nonzero) { vx = Fi[F_VX][s]; vy = Fi[F_VY][s]; vz = Fi[F_VZ][s]; }
-    if (a.b_uniform) {
-      bx = Fi[F_BX][0]; by = Fi[F_BY][0]; bz = Fi[F_BZ][0];
-    } else {
-      bx = Fi[F_BX][s]; by = Fi[F_BY][s]; bz = Fi[F_BZ][s];
+    group_sum<G>(ddt);
+    ddt *= -wcv * ihd1 * rcp_pair(rhoa);
+    if (sub == 0) {
+      const PT zero = 0;
+      double dh = 0.0;
+      if (P.adden) dh = -DIM * ha_d / (double)rhoa * (double)zero / (double)oma;
+      a.out.f[F_AX][s] = 0.0; a.out.f[F_AY][s] = 0.0; a.out.f[F_AZ][s] = 0.0;
+      a.out.f[F_DH][s] = dh;
+      a.out.f[F_DDT][s] = (double)ddt;
+      a.out.f[F_DBX][s] = 0.0; a.out.f[F_DBY][s] = 0.0; a.out.f[F_DBZ][s] = 0.0;
+      a.out.f[F_DU][s] = 0.0;
+      // FP64 energy sum (circuit2.f90:490-492) with zero dv, du, dB, drho.
+      // Every velocity exactly 0 (a signed zero among them changes no term
+      // after the + 0 below) or one B for every particle: no per-particle loads
+      double vx = 0.0, vy = 0.0, vz = 0.0, bx, by, bz;
+      if (a.v_nonzero) { vx = Fi[F_VX][s]; vy = Fi[F_VY][s]; vz = Fi[F_VZ][s]; }
+      if (a.b_uniform) {
+        bx = Fi[F_BX][0]; by = Fi[F_BY][0]; bz = Fi[F_BZ][0];
+      } else {
+        bx = Fi[F_BX][s]; by = Fi[F_BY][s]; bz = Fi[F_BZ][s];
+      }
+      const double rh = rho_d;
+      const double z0 = 0.0;
+      e_part = pa.w * (vx * z0 + vy * z0 + vz * z0 + z0 + (bx * z0 + by * z0 + bz * z0) / rh -
+                       0.5 * (bx * bx + by * by + bz * bz) / rh / rh * z0 / om_d);
     }
-    const double rh = rho_d;
-    const double z0 = 0.0;
-    e_part = pa.w * (vx * z0 + vy * z0 + vz * z0 + z0 + (bx * z0 + by * z0 + bz * z0) / rh -
-                     0.5 * (bx * bx + by * by + bz * bz) / rh / rh * z0 / om_d);
   }
   __shared__ double red[4];
   double w = wave_sum(e_part);
@@ -1981,37 +2107,44 @@ __global__ void k_axpy_copy(double *dst, const double *x, const double *y, doubl
 }
 
 // ------------------------------------------------------------ instantiation
-#define SPH_INST_DK(DIM, KT)                                                                 \
-  template __global__ void k_loop1<DIM, KT, 0, double>(Loop1Args<double4>);                  \
-  template __global__ void k_loop1<DIM, KT, 1, double>(Loop1Args<double4>);                  \
-  template __global__ void k_loop1<DIM, KT, 2, double>(Loop1Args<double4>);                  \
-  template __global__ void k_loop1<DIM, KT, 0, float>(Loop1Args<double4>);                   \
-  template __global__ void k_loop1<DIM, KT, 1, float>(Loop1Args<double4>);                   \
-  template __global__ void k_loop1<DIM, KT, 2, float>(Loop1Args<double4>);                   \
-  template __global__ void k_loop1_simple<DIM, KT, 0, double>(Loop1Args<double4>, Fields);   \
-  template __global__ void k_loop1_simple<DIM, KT, 1, double>(Loop1Args<double4>, Fields);   \
-  template __global__ void k_loop1_simple<DIM, KT, 2, double>(Loop1Args<double4>, Fields);   \
-  template __global__ void k_loop1_simple<DIM, KT, 0, float>(Loop1Args<double4>, Fields);    \
-  template __global__ void k_loop1_simple<DIM, KT, 1, float>(Loop1Args<double4>, Fields);    \
-  template __global__ void k_loop1_simple<DIM, KT, 2, float>(Loop1Args<double4>, Fields);    \
-  template __global__ void k_loop2<DIM, KT, double, double4, MODE_GENERIC>(Loop2Args<double4>); \
-  template __global__ void k_loop2<DIM, KT, float, float4, MODE_GENERIC>(Loop2Args<float4>);    \
-  template __global__ void k_loop2<DIM, KT, double, double4, MODE_DIFF>(Loop2Args<double4>);    \
-  template __global__ void k_loop2<DIM, KT, float, float4, MODE_DIFF>(Loop2Args<float4>);       \
-  template __global__ void k_loop2_fab<DIM, KT, double, double4>(Loop2Args<double4>);         \
-  template __global__ void k_loop2_fab<DIM, KT, float, float4>(Loop2Args<float4>);
-
-SPH_INST_DK(1, 0) SPH_INST_DK(1, 1) SPH_INST_DK(1, 2)
-SPH_INST_DK(2, 0) SPH_INST_DK(2, 1) SPH_INST_DK(2, 2)
-SPH_INST_DK(3, 0) SPH_INST_DK(3, 1) SPH_INST_DK(3, 2)
-
-#define SPH_INST_SPEC1(DIM, KT, M)                                                                    \
-  template __global__ void k_loop2<DIM, KT, double, double4, MODE_SPEC + M>(Loop2Args<double4>); \
-  template __global__ void k_loop2<DIM, KT, float, float4, MODE_SPEC + M>(Loop2Args<float4>);
-#define SPH_INST_SPEC(DIM, KT) \
-  SPH_INST_SPEC1(DIM, KT, kSpecHydro) SPH_INST_SPEC1(DIM, KT, kSpecMhd) SPH_INST_SPEC1(DIM, KT, kSpecHydroFld)
-SPH_INST_SPEC(2, 0) SPH_INST_SPEC(2, 1) SPH_INST_SPEC(2, 2)
-SPH_INST_SPEC(3, 0) SPH_INST_SPEC(3, 1) SPH_INST_SPEC(3, 2)
+// Lanes per particle as loop_lanes asks for them: 1, 4 and 8 in FP64 and in
+// loop 2 of 3D, 1 and 8 in loop 1 of FP32, 1 alone in loop 2 of 2D in FP32 and
+// in 1D.
+#define SPH_INST_L1(DIM, KT, PT, G)                                      \
+  template __global__ void k_loop1<DIM, KT, 0, PT, G>(Loop1Args<double4>); \
+  template __global__ void k_loop1<DIM, KT, 1, PT, G>(Loop1Args<double4>); \
+  template __global__ void k_loop1<DIM, KT, 2, PT, G>(Loop1Args<double4>);
+#define SPH_INST_L1S(DIM, KT, PT, G)                                                     \
+  template __global__ void k_loop1_simple<DIM, KT, 0, PT, G>(Loop1Args<double4>, Fields); \
+  template __global__ void k_loop1_simple<DIM, KT, 1, PT, G>(Loop1Args<double4>, Fields); \
+  template __global__ void k_loop1_simple<DIM, KT, 2, PT, G>(Loop1Args<double4>, Fields);
+#define SPH_INST_L2(DIM, KT, PT, V4, G)                                          \
+  template __global__ void k_loop2<DIM, KT, PT, V4, MODE_GENERIC, G>(Loop2Args<V4>); \
+  template __global__ void k_loop2<DIM, KT, PT, V4, MODE_DIFF, G>(Loop2Args<V4>);    \
+  template __global__ void k_loop2_fab<DIM, KT, PT, V4, G>(Loop2Args<V4>);
+#define SPH_INST_SPEC(DIM, KT, PT, V4, G)                                                   \
+  template __global__ void k_loop2<DIM, KT, PT, V4, MODE_SPEC + kSpecHydro, G>(Loop2Args<V4>); \
+  template __global__ void k_loop2<DIM, KT, PT, V4, MODE_SPEC + kSpecMhd, G>(Loop2Args<V4>);   \
+  template __global__ void k_loop2<DIM, KT, PT, V4, MODE_SPEC + kSpecHydroFld, G>(Loop2Args<V4>);
+#define SPH_INST_1D(KT)                                                                    \
+  SPH_INST_L1(1, KT, double, 1) SPH_INST_L1(1, KT, float, 1)                               \
+  SPH_INST_L1S(1, KT, double, 8) SPH_INST_L1S(1, KT, float, 1)                             \
+  SPH_INST_L2(1, KT, double, double4, 1) SPH_INST_L2(1, KT, float, float4, 1)
+#define SPH_INST_23(DIM, KT)                                                               \
+  SPH_INST_L1(DIM, KT, double, 1) SPH_INST_L1(DIM, KT, double, 4) SPH_INST_L1(DIM, KT, double, 8) \
+  SPH_INST_L1(DIM, KT, float, 1) SPH_INST_L1(DIM, KT, float, 8)                            \
+  SPH_INST_L1S(DIM, KT, double, 8) SPH_INST_L1S(DIM, KT, float, 1)                         \
+  SPH_INST_L2(DIM, KT, double, double4, 1) SPH_INST_L2(DIM, KT, double, double4, 4)        \
+  SPH_INST_L2(DIM, KT, double, double4, 8) SPH_INST_L2(DIM, KT, float, float4, 1)          \
+  SPH_INST_SPEC(DIM, KT, double, double4, 1) SPH_INST_SPEC(DIM, KT, double, double4, 4)    \
+  SPH_INST_SPEC(DIM, KT, double, double4, 8) SPH_INST_SPEC(DIM, KT, float, float4, 1)
+#define SPH_INST_3(KT)                                                                     \
+  SPH_INST_L2(3, KT, float, float4, 4) SPH_INST_L2(3, KT, float, float4, 8)                \
+  SPH_INST_SPEC(3, KT, float, float4, 4) SPH_INST_SPEC(3, KT, float, float4, 8)
+SPH_INST_1D(0) SPH_INST_1D(1) SPH_INST_1D(2)
+SPH_INST_23(2, 0) SPH_INST_23(2, 1) SPH_INST_23(2, 2)
+SPH_INST_23(3, 0) SPH_INST_23(3, 1) SPH_INST_23(3, 2)
+SPH_INST_3(0) SPH_INST_3(1) SPH_INST_3(2)
 
 #define SPH_INST_NEIGH(DIM)                                                                              \
   template __global__ void k_neigh<DIM, true>(NeighArgs, const double4 *__restrict__, const float4 *__restrict__, \
