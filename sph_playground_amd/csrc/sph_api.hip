@@ -142,6 +142,9 @@ enum { S_DIM = 0, S_EQS = 1, S_DDW = 2, S_ICS = 3, S_ADDEN = 4, S_ARTTS = 5, S_C
 
 inline unsigned grid_for(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + kBlock - 1) / kBlock); }
 
+// blocks of the store's transposes: tiles of 64 particles
+inline unsigned tiles_for(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + 63) / 64); }
+
 inline double ord2d(long long v) {
   long long b = v >= 0 ? v : (v ^ 0x7FFFFFFFFFFFFFFFLL);
   double d;
@@ -1425,7 +1428,7 @@ static int load_impl(sph_ctx *c, int64_t n, const double *store, int64_t ld, int
   c->w_valid = false;
   c->fw_steps = 0;
   c->fw_tail = false;
-  hipLaunchKernelGGL(k_aos_to_soa, dim3(grid_for(n)), dim3(kBlock), 0, c->stream, src, ld, (int)n, c->fields(),
+  hipLaunchKernelGGL(k_aos_to_soa, dim3(tiles_for(n)), dim3(kBlock), 0, c->stream, src, ld, (int)n, c->fields(),
                      c->orig[0]);
   HIPCHK(hipStreamSynchronize(c->stream));
   return SPH_OK;
@@ -1443,7 +1446,7 @@ static int save_impl(sph_ctx *c, double *store, int64_t ld, int on_device) {
     dst = c->d_staging;
     if (ld > F_TOTAL) HIPCHK(hipMemcpyAsync(dst, store, bytes, hipMemcpyHostToDevice, c->stream));
   }
-  hipLaunchKernelGGL(k_soa_to_aos, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), c->orig[c->cur],
+  hipLaunchKernelGGL(k_soa_to_aos, dim3(tiles_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), c->orig[c->cur],
                      (int)c->n, dst, ld);
   if (!on_device) HIPCHK(hipMemcpyAsync(store, dst, bytes, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
