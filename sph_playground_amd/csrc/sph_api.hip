@@ -258,7 +258,9 @@ struct sph_ctx {
   // ran flag), one region per sweep of a step, and their pinned mirror: the
   // parts of d_stripes and h_rec from kStepLL on
   long long *d_sweep = nullptr, *h_sweep = nullptr;
-  int sweep_hint = 4;             // sweeps the next step launches before it synchronises
+  int sweep_hint = 4;             // sweeps this step launches before it synchronises
+  int sweep_hints[2] = {4, 4};    // for a step on the last one's results, and for the first on a loaded state
+  int fresh = 1;                  // which of the two this step is
   int sweeps_zeroed = 0;          // k_prep cleared the regions of sweeps 1..this for the next batch
   sph_stats stats{};
   bool have_step = false;
@@ -578,6 +580,7 @@ static hipError_t copy_record(sph_ctx *c, int last_sweep) {
 static int sweep_cap(const sph_ctx *c) { return c->opt.max_sweeps > 0 ? c->opt.max_sweeps : 100; }
 static int first_batch_last(const sph_ctx *c) { return std::min(sweep_cap(c), std::max(1, c->sweep_hint)); }
 constexpr int kWhichInt = 6;        // d_int slot: parity of the last sweep that ran
+constexpr int kGoInt = 7;           // d_int slot: the queued tail runs (k_post1 decides)
 constexpr int kExtTotalInt = 16;    // h_int slot: records of the extended grid
 constexpr int kRedoNeigh = 1000; // internal: the lists overflowed, search again (not an SPH_ERR code)
 
@@ -1124,7 +1127,7 @@ static void launch_loop2_d23(sph_ctx *c, int dim, int lanes, void *args) {
 }
 
 template <typename V4>
-static int run_post_and_loop2(sph_ctx *c, const Phys &P) {
+static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pending) {
   const int n = (int)c->n;
   Fields F = c->fields();
   unsigned G = grid_for(n);
@@ -1164,6 +1167,8 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P) {
   sel.which = P.adden ? c->d_int + kWhichInt : nullptr;
   sel.serr = step_err(c) + kErrSearch;
   sel.err1 = step_err(c) + kErrLoop1;
+  sel.pending = pending;
+  sel.go = c->d_int + kGoInt;
   hipLaunchKernelGGL(k_post1<V4>, dim3(G), dim3(kBlock), 0, c->stream, F, sel, c->real, n, P.adden ? 1 : 0,
                      c->do_eos, c->eos_iso, c1, P.gamma, q0, q1, q2, q3, q4,
                      generic || std::is_same_v<V4, float4> ? nullptr : c->pd,
@@ -1182,6 +1187,7 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P) {
   a.v_nonzero = (fl & 1) ? 1 : 0;
   a.b_uniform = (fl & 2) ? 0 : 1;
   // loop 2's error word and k_post1's h_max stripes: cleared by this step's k_prep
+  a.go = c->d_int + kGoInt;
   a.out = F; a.energy_part = c->energy_part; a.err = step_err(c) + kErrLoop2; a.b = c->box; a.p = P; a.n = n;
   a.npad = (int)c->npad;
   HIPCHK(mark(c, 5));
@@ -1240,10 +1246,12 @@ static Phys call_phys(const sph_ctx *c, const double *state) {
 }
 
 // The tail of a step after loop 1: Newton bookkeeping, EOS and packs
-// (k_post1), loop 2, mti gravity and the closing record's copy.
-static int enqueue_tail(sph_ctx *c, const Phys &P) {
+// (k_post1), loop 2, mti gravity and the closing record's copy.  pending: the
+// still-active stripes of the last sweep queued, when more could follow it.
+static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr) {
   HIPCHK(mark(c, 2));
-  int rc = c->opt.precision == 1 ? run_post_and_loop2<float4>(c, P) : run_post_and_loop2<double4>(c, P);
+  int rc = c->opt.precision == 1 ? run_post_and_loop2<float4>(c, P, pending)
+                                   : run_post_and_loop2<double4>(c, P, pending);
   if (rc == SPH_OK && c->gravity)
     hipLaunchKernelGGL(k_gravity, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), c->real, (int)c->n,
                        c->gravity);
@@ -1273,7 +1281,8 @@ static bool loop2_reads_flags(const Phys &P) {
 // wait after the sweeps.  Lists
 // that overflowed leave loop 1 and k_post1 idle (device-side checks), so the
 // step searches again with room and starts over; a batch that ends with
-// particles still active is followed by more sweeps and the tail again.
+// particles still active leaves its tail idle and is followed by more sweeps
+// and another tail.
 static int run_advanced(sph_ctx *c, const Phys &P) {
   const int maxsw = sweep_cap(c);
   int first = 1, sweeps = 0, bits = 0;
@@ -1308,7 +1317,7 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
       }
       RCHK(fin);
     }
-    const int rc = enqueue_tail(c, P);
+    const int rc = enqueue_tail(c, P, last < maxsw ? c->d_sweep + (size_t)last * kSweepRegion : nullptr);
     // the search's read-back if still pending, error words, the tail's record
     // and the sweep regions: one copy
     HIPCHK(copy_record(c, last));
@@ -1344,9 +1353,9 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
   c->stats.ms_k_loop1 = ms1;
   // one sweep more than this step took: a sweep past convergence exits at
   // once (its launch costs about 16 us at 2M particles), while a step that
-  // needs more sweeps than launched runs its queued tail (EOS, packs,
-  // loop 2) again after them
+  // needs more sweeps than launched waits for one more round trip
   c->sweep_hint = std::min(maxsw, std::max(2, sweeps + 1));
+  c->sweep_hints[c->fresh] = c->sweep_hint;
   const int rc2 = finish_loop2(c);
   const int r1 = map_err(bits);
   return r1 != SPH_OK ? r1 : rc2;
@@ -1359,6 +1368,8 @@ static int run_step(sph_ctx *c, const double *state) {
   c->w_valid = false;
   c->fw_steps = 0;
   c->fw_tail = false;
+  c->fresh = c->derivs_ready ? 0 : 1;
+  c->sweep_hint = c->sweep_hints[c->fresh];
   c->derivs_ready = false;
   Phys P = call_phys(c, state);
   c->stats.ms_k_neigh = c->stats.ms_k_loop1 = c->stats.ms_k_loop2 = 0.0;

@@ -226,12 +226,17 @@ struct Loop1Args {
 };
 
 // Where k_post1 finds loop 1's result: st[*which] of the two sweep buffers
-// (fin0 alone when which is null); nothing is written when the search (serr)
-// or loop 1 (err1) raised an error bit: the step then stops or searches again.
+// (fin0 alone when which is null).  Nothing is written when the search (serr)
+// or loop 1 (err1) raised an error bit (the step then stops or searches again)
+// or when the last sweep queued before the tail left particles active
+// (`pending`, its still-active stripes; null: no matter): more sweeps and
+// another tail follow.  *go tells loop 2 which it was.
 struct PostSel {
   const double4 *fin0, *fin1;
   const int *which;
   const int *serr, *err1;
+  const long long *pending;
+  int *go;
 };
 
 template <typename V4>
@@ -253,6 +258,7 @@ struct Loop2Args {
   int v_nonzero;  // 0: every velocity is exactly 0 (v_ab = 0 for all pairs)
   int b_uniform;  // 1: every particle carries the same B bit for bit (kappa_b = kappa_a)
   Fields out;
+  const int *go;         // 0: k_post1 found nothing to do, neither has this kernel
   double *energy_part;   // one FP64 partial per block
   int *err;
   Box b;
