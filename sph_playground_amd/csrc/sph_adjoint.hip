@@ -14,10 +14,12 @@
 //
 // For one K every pair weight is fixed, so the weights are assembled once per
 // K (k_diff_weights in list order, k_diff_rweights in reverse-list order) and
-// each STS stage is a streaming sparse product with one gather per pair
-// (k_diff_spmv, k_diff_adj_spmv).  The adjoint stages accumulate one
-// coefficient per pair, S_t += lam_a (Zt_b - Zt_a), which k_diff_gcontract
-// contracts with G once per backward pass.
+// each STS stage is a streaming sparse product with one gather per pair and
+// the stage's vector arithmetic at its rows' end (k_batch_stage, k_adj_stage).
+// The adjoint stages leave a record (lam, Zt) per particle, and k_diff_coef
+// adds eight stages' records at a time to one coefficient per pair, S_t +=
+// lam_a (Zt_b - Zt_a), which k_diff_gcontract contracts with G once per
+// backward pass.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -31,6 +33,17 @@ __device__ __forceinline__ int xcd_block_a(int b, int nb) {
   return x * q + (x < r ? x : r) + i;
 }
 __device__ __forceinline__ int gtid_a() { return xcd_block_a(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; }
+
+// The row of this thread in a streaming product.  With rev each XCD runs its
+// range of blocks from the far end: successive stages read the same lists and
+// weights, and one that starts where the last ended finds the part the
+// memory-side cache still holds (a 64^3 operator is 356 MB of the cache's 256).
+__device__ __forceinline__ int stage_row(int rev) {
+  const int b = blockIdx.x, nb = gridDim.x;
+  const int x = b & 7, q = nb >> 3, r = nb & 7;
+  const int i = rev ? q + (x < r ? 1 : 0) - 1 - (b >> 3) : b >> 3;
+  return (x * q + (x < r ? x : r) + i) * blockDim.x + threadIdx.x;
+}
 
 // Basis contractions G_k of the Hessian operator at h_a: K:H = sum_k K_k G_k.
 template <int DIM, int KT>
@@ -84,13 +97,14 @@ __global__ void k_zrho(int n, const double *Y, const double4 *q0, double *Z) {
   if (s < n) Z[s] = Y[s] * q0[s].y;
 }
 
-// pxh = (x, y, z, 1 / h) and the 1 / rho of the frozen geometry.
-__global__ void k_diff_pack(int n, const double4 *pm, const double4 *q0, double4 *pxh, double *irho) {
+// pxh = (x, y, z, 1 / h), rho and 1 / rho of the frozen geometry.
+__global__ void k_diff_pack(int n, const double4 *pm, const double4 *q0, double4 *pxh, double *rho, double *irho) {
   int s = gtid_a();
   if (s < n) {
     const double4 p = pm[s];
     const double4 q = q0[s];
     pxh[s] = make_double4(p.x, p.y, p.z, q.x);
+    rho[s] = q.y;
     irho[s] = 1.0 / q.y;
   }
 }
@@ -169,99 +183,145 @@ __global__ __launch_bounds__(256) void k_diff_rweights(DiffOpArgs a, const doubl
   }
 }
 
+// Entries and weights of a row, eight at a time, the next eight read while
+// fn(entries, weights, valid) works on these: a row's chunks otherwise follow
+// each other at the latency of two loads (64^3 has a single round of blocks).
+template <typename WT, typename Fn>
+__device__ __forceinline__ void over_chunks(const uint32_t *nb, const WT *W, int s, int npad, int nn, Fn fn) {
+  using V = std::conditional_t<std::is_same_v<WT, float>, float4, double4>;
+  uint4 e0{}, e1{};
+  V w0{}, w1{};
+  auto read = [&](int k0) {
+    const size_t base = nb_slot(k0, s, npad);
+    const uint4 *pe = reinterpret_cast<const uint4 *>(nb + base);
+    const V *pw = reinterpret_cast<const V *>(W + base);
+    e0 = pe[0]; e1 = pe[1];
+    w0 = pw[0]; w1 = pw[1];
+  };
+  if (nn > 0) read(0);
+  for (int k0 = 0; k0 < nn; k0 += 8) {
+    const uint32_t e8[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+    const double w8[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+    if (k0 + 8 < nn) read(k0 + 8);
+    fn(e8, w8, min(8, nn - k0));
+  }
+}
+
 // out = A(K) Y from Z = Y rho: out_a = (1 / rho_a) sum_b W_ab (Z_b - Z_a);
 // weights stream in list order, Z_b is the one gather per pair.
 __global__ __launch_bounds__(256) void k_diff_spmv(DiffOpArgs a, const double *W, const double *Z, double *out) {
   int s = gtid_a();
   if (s >= a.n || !a.real[s]) return;
   const double za = Z[s];
-  const int nn = a.cnt[s];
   double acc = 0.0;
-  for (int k0 = 0; k0 < nn; k0 += 8) {
-    const size_t base = nb_slot(k0, s, a.npad);
-    const uint4 *pe = reinterpret_cast<const uint4 *>(a.nb + base);
-    const double4 *pw = reinterpret_cast<const double4 *>(W + base);
-    const uint4 e0 = pe[0], e1 = pe[1];
-    const double4 w0 = pw[0], w1 = pw[1];
-    const uint32_t e8[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
-    const double w8[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-    const int m = min(8, nn - k0);
+  over_chunks(a.nb, W, s, a.npad, a.cnt[s], [&](const uint32_t *e, const double *w, int m) {
     double z8[8];
 #pragma unroll
-    for (int u = 0; u < 8; u++) z8[u] = Z[u < m ? nb_index(e8[u]) : (uint32_t)s];
+    for (int u = 0; u < 8; u++) z8[u] = Z[u < m ? nb_index(e[u]) : (uint32_t)s];
 #pragma unroll
     for (int u = 0; u < 8; u++)
-      if (u < m) acc = fma(w8[u], z8[u] - za, acc);
-  }
+      if (u < m) acc = fma(w[u], z8[u] - za, acc);
+  });
   out[s] = acc / a.q0[s].y;
 }
 
-// One adjoint stage over the reverse lists, for every real s:
-//   out_s = sum_t lam_a R_t - lam_s dW_s              (A^T lam, when out != null)
-//   S_t  += sum_q lam^q_a (Zt^q_s - Zt^q_a)           (gradient coefficients, UPD)
-// with t = (a -> s); lam comes from LZ.p[0], the stages q < NS of the S update
-// from LZ.p[q].  rent, R and S stream in the list layout; the LZ records of
-// the owners are the gathers per entry.  Folding several stages into one S
-// update divides the S traffic of the backward pass.
-template <int NS, int UPD>
-__global__ __launch_bounds__(256) void k_diff_adj_spmv(DiffOpArgs a, const double *R, const double *dW, LZSet LZ,
-                                                       double *S, double *out) {
-  int s = gtid_a();
-  if (s >= a.n || !a.real[s]) return;
-  double zs[NS];
-#pragma unroll
-  for (int q = 0; q < NS; q++) zs[q] = UPD ? LZ.p[q][s].y : 0.0;
-  const double ls = LZ.p[0][s].x;
-  const bool tr = out != nullptr;
+// One adjoint stage (AdjStage, sts_integrator.f90:111-115 transposed): U =
+// A^T L over the reverse lists,
+//   U_s = sum_t L_a R_t - L_s dW_s,  t = (a -> s),
+// and the stage's vector updates.  Bound by memory (12 bytes per pair; 64^3:
+// 72 us, 5.2 TB/s, where product, record and update took three launches and
+// 88 us).
+__global__ __launch_bounds__(256) void k_adj_stage(AdjStage a) {
+  const int s = stage_row(a.rev);
+  if (s >= a.n) return;
+  const double l = a.lam[s];
   double acc = 0.0;
-  const int nr = a.rcnt[s];
-  for (int k0 = 0; k0 < nr; k0 += 8) {
-    const size_t base = nb_slot(k0, s, a.npad);
-    const uint4 *pe = reinterpret_cast<const uint4 *>(a.rent + base);
-    const uint4 e0 = pe[0], e1 = pe[1];
-    const uint32_t e8[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
-    const int m = min(8, nr - k0);
-    uint32_t i8[8];
+  over_chunks(a.rent, a.R, s, a.npad, a.rcnt[s], [&](const uint32_t *e, const double *r, int m) {
+    double l8[8];
 #pragma unroll
-    for (int u = 0; u < 8; u++) i8[u] = u < m ? nb_index(e8[u]) : (uint32_t)s;
-    if (tr) {
-      const double4 *pr = reinterpret_cast<const double4 *>(R + base);
-      const double4 r0 = pr[0], r1 = pr[1];
-      const double r8[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
-      double l8[8];
+    for (int u = 0; u < 8; u++) l8[u] = a.lam[u < m ? nb_index(e[u]) : (uint32_t)s];
 #pragma unroll
-      for (int u = 0; u < 8; u++) l8[u] = LZ.p[0][i8[u]].x;
-#pragma unroll
-      for (int u = 0; u < 8; u++)
-        if (u < m) acc += l8[u] * r8[u];
-    }
-    if constexpr (UPD) {
-      double4 *ps = reinterpret_cast<double4 *>(S + base);
-      double4 s0 = ps[0], s1 = ps[1];
-      double s8[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-#pragma unroll
-      for (int q = 0; q < NS; q++) {
-        double2 g8[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) g8[u] = LZ.p[q][i8[u]];
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-          if (u < m) s8[u] += g8[u].x * (zs[q] - g8[u].y);
-      }
-      ps[0] = make_double4(s8[0], s8[1], s8[2], s8[3]);
-      ps[1] = make_double4(s8[4], s8[5], s8[6], s8[7]);
-    }
+    for (int u = 0; u < 8; u++)
+      if (u < m) acc += l8[u] * r[u];
+  });
+  const double u = acc - l * a.dW[s];
+  double next;
+  if (a.last) {
+    next = (a.A0 ? a.A0[s] + l : 0.0) + a.mh * u;
+  } else {
+    next = a.mu * l + a.mh * u;
+    if (a.lam1) next += a.nu1 * a.lam1[s];
+    a.A0[s] = (a.a0_add ? a.A0[s] : 0.0) + a.c0 * l + a.gh * u;
   }
-  if (tr) out[s] = acc - ls * dW[s];
+  a.out[s] = next;
 }
 
-// LZ = (lam, (wa Ya + wb Yb) rho).
-__global__ void k_adj_lz(int n, const double *lam, const double *Ya, const double *Yb, double wa, double wb,
-                         const double4 *q0, double2 *LZ) {
-  int s = gtid_a();
+// The records of stages [first, count) side by side per particle (with `fill`
+// the rest zero): rec[s][q] = (lam^q, Zt^q).  Written by the stages themselves,
+// 16 bytes of each particle's line at a time, they cost every stage some 12 us
+// at 64^3; this pass takes 23 us per eight stages.
+__global__ __launch_bounds__(256) void k_adj_pack(int n, AdjRecs a, int first, int count, int fill, const double *rho,
+                                                  double2 *rec) {
+  const int t = gtid_a(), s = t / kRecs, q = t % kRecs;
+  if (s >= n || q < first || (q >= count && !fill)) return;
+  double2 r = make_double2(0.0, 0.0);
+  if (q < count) {
+    const double yb = a.Yb[q] ? a.wb[q] * a.Yb[q][s] : 0.0;
+    r = make_double2(a.lam[q][s], (a.wa[q] * a.Ya[q][s] + yb) * rho[s]);
+  }
+  rec[t] = r;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double swap_half(bool high, double low_v, double high_v) {
+  // keep one of the two values and add the partner lane's copy of it
+  return (high ? high_v : low_v) + dpp_mov<CTRL>(high ? low_v : high_v);
+}
+
+// Pair coefficients of the tensor gradient, eight stages at once:
+//   S_t (+)= sum_q lam^q_a (Zt^q_s - Zt^q_a),  t = (a -> s).
+// Four lanes share a particle, each on two stages, so the four read a
+// neighbour's records as one 128-byte line; eight entries' products are then
+// summed over the lanes by halves, which leaves entries 2 l and 2 l + 1 on
+// lane l, and S moves once per eight stages in whole lines.  Bound by the
+// records' lines out of the caches and by S (64^3: 0.26 ms per eight stages, 3.8
+// and 0.6 GB; a lane per particle and four stages at a time took 0.18 ms per
+// four; fewer blocks in flight change nothing).
+__global__ __launch_bounds__(256) void k_diff_coef(const uint32_t *rent, const int *rcnt, const double2 *rec,
+                                                   double *S, int add, int n, int npad) {
+  const int t = gtid_a(), s = t >> 2, l = t & 3;
   if (s >= n) return;
-  const double yb = Yb ? wb * Yb[s] : 0.0;
-  LZ[s] = make_double2(lam[s], (wa * Ya[s] + yb) * q0[s].y);
+  const double2 *own = rec + (size_t)s * kRecs + 2 * l;
+  const double z0 = own[0].y, z1 = own[1].y;
+  const int nr = rcnt[s];
+  uint4 e0{}, e1{};
+  auto read = [&](int k0) {
+    const uint4 *pe = reinterpret_cast<const uint4 *>(rent + nb_slot(k0, s, npad));
+    e0 = pe[0]; e1 = pe[1];
+  };
+  if (nr > 0) read(0);
+  for (int k0 = 0; k0 < nr; k0 += 8) {
+    double2 *ps = reinterpret_cast<double2 *>(S + nb_slot(k0, s, npad)) + l;
+    const uint32_t e8[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+    const int m = min(8, nr - k0);
+    double2 sum = make_double2(0.0, 0.0);
+    if (add) sum = *ps;
+    if (k0 + 8 < nr) read(k0 + 8);
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const uint32_t i = u < m ? nb_index(e8[u]) : (uint32_t)s;
+      const double2 *g = rec + (size_t)i * kRecs + 2 * l;
+      const double2 g0 = g[0], g1 = g[1];
+      v[u] = g0.x * (z0 - g0.y) + g1.x * (z1 - g1.y);
+    }
+    double w[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) w[u] = swap_half<0x4E>((l & 2) != 0, v[u], v[4 + u]);  // quad_perm [2,3,0,1]
+    sum.x += swap_half<0xB1>((l & 1) != 0, w[0], w[2]);                                // quad_perm [1,0,3,2]
+    sum.y += swap_half<0xB1>((l & 1) != 0, w[1], w[3]);
+    *ps = sum;  // slots past the list's end are never read
+  }
 }
 
 // Tensor gradient from the accumulated coefficients over the reverse lists:
@@ -401,13 +461,14 @@ __device__ __forceinline__ double mul_rn(double x, double y) {
   return x * y;
 }
 
-// Batch input: Y_0 in merged order and its Z_0 = Y_0 rho.
+// Super-step input: Y_0 in sorted (merged) order and its Z_0 = Y_0 rho; orig
+// null: T0 is in that order already.
 __global__ void k_batch_in(const double *T0, const int64_t *orig, const double *rho, int n, double *Y0,
                            double *Z0) {
   int s = gtid_a();
   if (s >= n) return;
-  const double y = T0[orig[s]];
-  Y0[s] = y;
+  const double y = T0[orig ? orig[s] : s];
+  if (Y0 != T0) Y0[s] = y;
   Z0[s] = mul_rn(y, rho[s]);
 }
 
@@ -416,45 +477,32 @@ __global__ void k_batch_in(const double *T0, const int64_t *orig, const double *
 //   j=1: DY0 = D;  Y_1 = Y_0 + mhat dt DY0
 //   j>1: Y_j = mu Y_{j-1} + nu Y_{j-2} + (1 - mu - nu) Y_0 + mhat dt D + ghat dt DY0
 // and Z_j = Y_j rho for the next stage's gathers.  The per-row summation
-// is k_diff_spmv's and the combination k_lincomb's (a rounded first product,
-// then explicit fused multiply-adds in the same order), so every problem's
-// result is bitwise the unbatched super-step's.  Y_j may be Y_0's buffer:
-// row s reads only its own Y_0 entry before writing it.
-template <bool FIRST, typename WT>
+// is k_diff_spmv's and the combination a rounded first product, then explicit
+// fused multiply-adds, whatever the instantiation, so every problem's result
+// is bitwise the unbatched super-step's.  Y_j may be Y_0's buffer: row s reads
+// only its own Y_0 entry before writing it.
+// ONE: one prepared problem on its own lists, whose entries carry image codes
+// (sph_diff_forward), with one time step.
+template <bool FIRST, typename WT, bool ONE>
 __global__ __launch_bounds__(512) void k_batch_stage(BatchStage a) {
-  int s = gtid_a();
+  const int s = stage_row(a.rev);
   if (s >= a.n) return;
   const double ya = a.Yjm1[s], rs = a.rho[s];
   const double za = mul_rn(ya, rs);
-  const int nn = a.cnt[s];
   double acc = 0.0;
-  for (int k0 = 0; k0 < nn; k0 += 8) {
-    const size_t base = nb_slot(k0, s, a.npad);
-    const uint4 *pe = reinterpret_cast<const uint4 *>(a.nb + base);
-    const uint4 e0 = pe[0], e1 = pe[1];
-    double w8[8];
-    if constexpr (std::is_same_v<WT, float>) {  // FP32 weights, FP64 products and sums
-      const float4 *pw = reinterpret_cast<const float4 *>(a.W32 + base);
-      const float4 w0 = pw[0], w1 = pw[1];
-      w8[0] = w0.x; w8[1] = w0.y; w8[2] = w0.z; w8[3] = w0.w;
-      w8[4] = w1.x; w8[5] = w1.y; w8[6] = w1.z; w8[7] = w1.w;
-    } else {
-      const double4 *pw = reinterpret_cast<const double4 *>(a.W + base);
-      const double4 w0 = pw[0], w1 = pw[1];
-      w8[0] = w0.x; w8[1] = w0.y; w8[2] = w0.z; w8[3] = w0.w;
-      w8[4] = w1.x; w8[5] = w1.y; w8[6] = w1.z; w8[7] = w1.w;
-    }
-    const uint32_t e8[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
-    const int m = min(8, nn - k0);
+  const WT *W;
+  if constexpr (std::is_same_v<WT, float>) W = a.W32;  // FP32 weights, FP64 products and sums
+  else W = a.W;
+  over_chunks(a.nb, W, s, a.npad, a.cnt[s], [&](const uint32_t *e, const double *w, int m) {
     double z8[8];
 #pragma unroll
-    for (int u = 0; u < 8; u++) z8[u] = a.Zjm1[u < m ? e8[u] : (uint32_t)s];
+    for (int u = 0; u < 8; u++) z8[u] = a.Zjm1[u < m ? (ONE ? nb_index(e[u]) : e[u]) : (uint32_t)s];
 #pragma unroll
     for (int u = 0; u < 8; u++)
-      if (u < m) acc = fma(w8[u], z8[u] - za, acc);
-  }
+      if (u < m) acc = fma(w[u], z8[u] - za, acc);
+  });
   const double D = acc / rs;
-  const double h = a.dt[a.pid[s]];
+  const double h = ONE ? a.h : a.dt[a.pid[s]];
   double v;
   if (FIRST) {
     a.DY0[s] = D;
@@ -478,33 +526,6 @@ __global__ void k_to_sorted(const double *src, const int64_t *orig, int n, doubl
 __global__ void k_from_sorted(const double *src, const int64_t *orig, int n, double *dst) {
   int s = gtid_a();
   if (s < n) dst[orig[s]] = src[s];
-}
-
-// Adjoint of one RKL2 stage's combination (sts_integrator.f90:111-115):
-// L1 += mu Lj + mh U, L2 += nu Lj, L0 += (1 - mu - nu) Lj + gh U (L1 or L2 may
-// be L0; each is updated in turn, as three separate sums would).
-__global__ void k_stage_adj(int n, const double *Lj, const double *U, double mu, double nu, double mh, double gh,
-                            double *L1, double *L2, double *L0) {
-  int s = gtid_a();
-  if (s >= n) return;
-  const double lj = Lj[s], u = U[s];
-  L1[s] = 1.0 * L1[s] + mu * lj + mh * u;
-  L2[s] = 1.0 * L2[s] + nu * lj;
-  L0[s] = 1.0 * L0[s] + (1. - mu - nu) * lj + gh * u;
-}
-
-// y = sum_k c_k x_k over up to 5 vectors (null x_k skipped).
-__global__ void k_lincomb(int n, double *y, double c0, const double *x0, double c1, const double *x1, double c2,
-                          const double *x2, double c3, const double *x3, double c4, const double *x4) {
-  int s = gtid_a();
-  if (s >= n) return;
-  // one rounded product, then one fused multiply-add per further term
-  double v = c0 * x0[s];
-  if (x1) v = fma(c1, x1[s], v);
-  if (x2) v = fma(c2, x2[s], v);
-  if (x3) v = fma(c3, x3[s], v);
-  if (x4) v = fma(c4, x4[s], v);
-  y[s] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -811,10 +832,12 @@ SPH_INST_NL(1, 0) SPH_INST_NL(1, 1) SPH_INST_NL(1, 2)
 SPH_INST_NL(2, 0) SPH_INST_NL(2, 1) SPH_INST_NL(2, 2)
 SPH_INST_NL(3, 0) SPH_INST_NL(3, 1) SPH_INST_NL(3, 2)
 
-template __global__ void k_batch_stage<true, double>(BatchStage);
-template __global__ void k_batch_stage<false, double>(BatchStage);
-template __global__ void k_batch_stage<true, float>(BatchStage);
-template __global__ void k_batch_stage<false, float>(BatchStage);
+template __global__ void k_batch_stage<true, double, false>(BatchStage);
+template __global__ void k_batch_stage<false, double, false>(BatchStage);
+template __global__ void k_batch_stage<true, float, false>(BatchStage);
+template __global__ void k_batch_stage<false, float, false>(BatchStage);
+template __global__ void k_batch_stage<true, double, true>(BatchStage);
+template __global__ void k_batch_stage<false, double, true>(BatchStage);
 
 #define SPH_INST_ADJ(DIM, KT)                                                                  \
   template __global__ void k_diff_weights<DIM, KT>(DiffOpArgs, double *, double *);                 \
@@ -823,12 +846,5 @@ template __global__ void k_batch_stage<false, float>(BatchStage);
 SPH_INST_ADJ(1, 0) SPH_INST_ADJ(1, 1) SPH_INST_ADJ(1, 2)
 SPH_INST_ADJ(2, 0) SPH_INST_ADJ(2, 1) SPH_INST_ADJ(2, 2)
 SPH_INST_ADJ(3, 0) SPH_INST_ADJ(3, 1) SPH_INST_ADJ(3, 2)
-#define SPH_INST_ADJS(NS, UPD) \
-  template __global__ void k_diff_adj_spmv<NS, UPD>(DiffOpArgs, const double *, const double *, LZSet, double *, double *);
-SPH_INST_ADJS(1, 0)
-SPH_INST_ADJS(1, 1)
-SPH_INST_ADJS(2, 1)
-SPH_INST_ADJS(3, 1)
-SPH_INST_ADJS(4, 1)
 
 }  // namespace sph

@@ -75,26 +75,21 @@ __global__ void k_diff_rweights(DiffOpArgs, const double *, double *);
 template <int DIM, int KT>
 __global__ void k_diff_gcontract(DiffOpArgs, const double *, const double *, double *);
 __global__ void k_diff_spmv(DiffOpArgs, const double *, const double *, double *);
-template <int NS, int UPD>
-__global__ void k_diff_adj_spmv(DiffOpArgs, const double *, const double *, LZSet, double *, double *);
-__global__ void k_stage_adj(int, const double *, const double *, double, double, double, double, double *, double *,
-                            double *);
-__global__ void k_adj_lz(int, const double *, const double *, const double *, double, double, const double4 *,
-                         double2 *);
+__global__ void k_adj_stage(AdjStage);
+__global__ void k_adj_pack(int, AdjRecs, int, int, int, const double *, double2 *);
+__global__ void k_diff_coef(const uint32_t *, const int *, const double2 *, double *, int, int, int);
 __global__ void k_gk_accum(const double *, int, double, double, double *);
 __global__ void k_zrho(int, const double *, const double4 *, double *);
-__global__ void k_diff_pack(int, const double4 *, const double4 *, double4 *, double *);
+__global__ void k_diff_pack(int, const double4 *, const double4 *, double4 *, double *, double *);
 __global__ void k_rev_count(const uint8_t *, const uint32_t *, const int *, int, int, int *);
 __global__ void k_rev_chunk(const int *, const uint32_t *, int, int, int *, uint32_t *);
 __global__ void k_pair_enum(const uint8_t *, const uint32_t *, const int *, int, int, const int *, uint32_t *,
                             uint32_t *);
 __global__ void k_to_sorted(const double *, const int64_t *, int, double *);
 __global__ void k_from_sorted(const double *, const int64_t *, int, double *);
-__global__ void k_lincomb(int, double *, double, const double *, double, const double *, double, const double *,
-                          double, const double *, double, const double *);
 __global__ void k_batch_merge(int, int, int64_t, int, const int *, const uint32_t *, const double *, const double4 *,
                               const int64_t *, int, int *, uint32_t *, double *, float *, double *, int64_t *, int *);
-template <bool FIRST, typename WT>
+template <bool FIRST, typename WT, bool ONE>
 __global__ void k_batch_stage(BatchStage);
 __global__ void k_batch_in(const double *, const int64_t *, const double *, int, double *, double *);
 template <int DIM, int KT, int MODE>
@@ -280,8 +275,13 @@ struct sph_ctx {
   double *dW = nullptr, *ddW = nullptr;  // forward pair weights (list layout) and their row sums
   double *dR = nullptr, *dS = nullptr;   // reverse weights and gradient coefficients (reverse order)
   double *dZ = nullptr;
-  double2 *dLZ[4] = {nullptr, nullptr, nullptr, nullptr};  // (lam, Zt) of adjoint stages, a ring
-  int lz_pend = 0;               // stages in the ring whose S update is deferred (buffers 0..lz_pend-1)
+  double *drho = nullptr;        // rho of the frozen geometry
+  double2 *dRec = nullptr;       // (lam, Zt) of kRecs adjoint stages per particle
+  AdjRecs recs{};                // stages not yet added to the pair coefficients
+  int rec_pend = 0;              // their number
+  int rec_packed = 0;            // those whose records are written already
+  bool coef_set = false;         // dS holds a sum (else the next records start it)
+  int stage_rev = 0;             // the direction the next product runs its rows in
   bool fw_tail = false;          // the forward kept its last checkpoint segment's stage states
   int *rcnt = nullptr;           // reverse-list lengths
   int rcap = 0;                  // reverse-list capacity (list layout, multiple of 8)
@@ -1588,7 +1588,7 @@ int sph_ctx_destroy(sph_ctx *c) {
                   c->h0, c->eps, c->pf,
                   c->real, c->nb, c->cnt, c->q[0], c->q[1], c->q[2], c->q[3], c->q[4], c->energy_part,
                   c->d_red, c->d_int, c->d_stripes, c->d_staging, c->roff, c->rtmp, c->rent, c->scan_tmp,
-                  c->dvec, c->gpart, c->ckpt, c->rcnt, c->dpxh, c->dirho, c->dW, c->ddW, c->dR, c->dS, c->dZ, c->dLZ[0], c->dLZ[1], c->dLZ[2], c->dLZ[3],
+                  c->dvec, c->gpart, c->ckpt, c->rcnt, c->dpxh, c->dirho, c->dW, c->ddW, c->dR, c->dS, c->dZ, c->drho, c->dRec,
                   c->gkdev, c->nlF, c->nlU, c->nlUB, c->nlNu, c->nlMu, c->nlD, c->nlDD, c->nlR, c->nlSD,
                   c->ext_count, c->ecs, c->erec, c->ext_tmp};
   for (void *p : ptrs)
@@ -2062,45 +2062,38 @@ static void diff_apply(sph_ctx *c, const double K[6], const double *Y, double *o
   hipLaunchKernelGGL(k_zrho, dim3(G), dim3(kBlock), 0, c->stream, (int)c->n, Y, a.q0, c->dZ);
   hipLaunchKernelGGL(k_diff_spmv, dim3(G), dim3(kBlock), 0, c->stream, a, c->dW, c->dZ, out);
 }
-// One adjoint stage: out = A^T lam, and the stage's gradient coefficients
-// S += lam_a (Zt_b - Zt_a), Zt = (wa Ya + wb Yb) rho (Yb may be null).  S
-// updates are deferred and done four stages at a time (one pass over S per
-// four stages); diff_flush settles the deferred ones.
-static void diff_adj_stage(sph_ctx *c, const double K[6], const double *lam, const double *Ya, const double *Yb,
-                           double wa, double wb, double *out) {
-  ensure_weights(c, K);
-  DiffOpArgs a = diff_args(c, K);
-  const unsigned G = grid_for(c->n);
-  // this stage's record goes first in the set; the deferred ones follow
-  LZSet set{};
-  set.p[0] = c->dLZ[c->lz_pend];
-  for (int q = 0; q < c->lz_pend; q++) set.p[q + 1] = c->dLZ[q];
-  hipLaunchKernelGGL(k_adj_lz, dim3(G), dim3(kBlock), 0, c->stream, (int)c->n, lam, Ya, Yb, wa, wb, a.q0,
-                     c->dLZ[c->lz_pend]);
-  if (c->lz_pend == 3) {
-    hipLaunchKernelGGL((k_diff_adj_spmv<4, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dR, c->ddW, set, c->dS,
-                       out);
-    c->lz_pend = 0;
-  } else {
-    hipLaunchKernelGGL((k_diff_adj_spmv<1, 0>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dR, c->ddW, set, c->dS,
-                       out);
-    c->lz_pend++;
-  }
+// Successive products run their rows in alternating directions (stage_row).
+static int next_rev(sph_ctx *c) { return c->stage_rev ^= 1; }
+
+// The records of the pending stages, before their vectors change (fill: and
+// empty ones behind them).
+static void adj_pack(sph_ctx *c, bool fill) {
+  if (c->rec_packed < (fill ? kRecs : c->rec_pend))
+    hipLaunchKernelGGL(k_adj_pack, dim3(grid_for(c->n * kRecs)), dim3(kBlock), 0, c->stream, (int)c->n, c->recs,
+                       c->rec_packed, c->rec_pend, fill ? 1 : 0, c->drho, c->dRec);
+  c->rec_packed = c->rec_pend;
 }
-static void diff_flush(sph_ctx *c, const double K[6]) {
-  if (c->lz_pend == 0) return;
-  DiffOpArgs a = diff_args(c, K);
-  const unsigned G = grid_for(c->n);
-  LZSet set{};
-  for (int q = 0; q < c->lz_pend; q++) set.p[q] = c->dLZ[q];
-  double *none = nullptr;
-  if (c->lz_pend == 1)
-    hipLaunchKernelGGL((k_diff_adj_spmv<1, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dR, c->ddW, set, c->dS, none);
-  else if (c->lz_pend == 2)
-    hipLaunchKernelGGL((k_diff_adj_spmv<2, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dR, c->ddW, set, c->dS, none);
-  else
-    hipLaunchKernelGGL((k_diff_adj_spmv<3, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dR, c->ddW, set, c->dS, none);
-  c->lz_pend = 0;
+// The pending stages into the pair coefficients.
+static void coef_flush(sph_ctx *c) {
+  if (c->rec_pend == 0) return;
+  adj_pack(c, true);
+  hipLaunchKernelGGL(k_diff_coef, dim3(grid_for(c->n * 4)), dim3(kBlock), 0, c->stream, c->rent, c->rcnt, c->dRec,
+                     c->dS, c->coef_set ? 1 : 0, (int)c->n, (int)c->npad);
+  c->coef_set = true;
+  c->rec_pend = c->rec_packed = 0;
+}
+// A stage's record: lam and Zt = (wa Ya + wb Yb) rho (Yb may be null).  The
+// vectors stay as they are until adj_pack.
+static void adj_record(sph_ctx *c, const double *lam, const double *Ya, const double *Yb, double wa, double wb) {
+  const int q = c->rec_pend++;
+  c->recs.lam[q] = lam; c->recs.Ya[q] = Ya; c->recs.Yb[q] = Yb; c->recs.wa[q] = wa; c->recs.wb[q] = wb;
+  if (c->rec_pend == kRecs) coef_flush(c);
+}
+static AdjStage adj_args(sph_ctx *c) {
+  AdjStage a{};
+  a.rent = c->rent; a.rcnt = c->rcnt; a.R = c->dR; a.dW = c->ddW;
+  a.n = (int)c->n; a.npad = (int)c->npad; a.rev = next_rev(c);
+  return a;
 }
 template <int DIM>
 static void launch_gcontract_d(sph_ctx *c, const DiffOpArgs &a) {
@@ -2114,23 +2107,15 @@ static void launch_gcontract_d(sph_ctx *c, const DiffOpArgs &a) {
                        c->gpart);
 }
 // gk[0..5] += sum over pairs of the accumulated coefficients times G (fixed
-// reduction order), then the coefficients are cleared.
-static int diff_gcontract(sph_ctx *c, const double K[6], double *gk) {
-  diff_flush(c, K);
+// reduction order); the next record starts new coefficients.
+static void diff_gcontract(sph_ctx *c, const double K[6], double *gk) {
+  coef_flush(c);
   DiffOpArgs a = diff_args(c, K);
   if (c->diff_phys.dim == 1) launch_gcontract_d<1>(c, a);
   else if (c->diff_phys.dim == 2) launch_gcontract_d<2>(c, a);
   else launch_gcontract_d<3>(c, a);
   hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)grid_for(c->n), 1.0, 0.0, gk);
-  HIPCHK(hipMemsetAsync(c->dS, 0, sizeof(double) * (size_t)c->npad * c->rcap, c->stream));
-  return SPH_OK;
-}
-
-static void lincomb(sph_ctx *c, double *y, double c0, const double *x0, double c1 = 0, const double *x1 = nullptr,
-                    double c2 = 0, const double *x2 = nullptr, double c3 = 0, const double *x3 = nullptr,
-                    double c4 = 0, const double *x4 = nullptr) {
-  hipLaunchKernelGGL(k_lincomb, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, (int)c->n, y, c0, x0, c1, x1, c2,
-                     x2, c3, x3, c4, x4);
+  c->coef_set = false;
 }
 
 static int ensure_dvec(sph_ctx *c, int nvec) {
@@ -2142,33 +2127,60 @@ static int ensure_dvec(sph_ctx *c, int nvec) {
 }
 static double *dv(sph_ctx *c, int k) { return c->dvec + (size_t)k * c->npad; }
 
-// One RKL2 super-step from Y[0] (sorted); stage states into Y[0..s]; work vector W.
-static void sts_forward_step(sph_ctx *c, const double K[6], int s, double dt, double *const *Y, double *DY0,
-                             double *DYm) {
-  diff_apply(c, K, Y[0], DY0);
-  lincomb(c, Y[1], 1.0, Y[0], sts_mu_hat(1, s) * dt, DY0);
-  for (int j = 2; j <= s; j++) {
-    diff_apply(c, K, Y[j - 1], DYm);
-    double mu = sts_mu(j), nu = sts_nu(j);
-    lincomb(c, Y[j], mu, Y[j - 1], nu, Y[j - 2], 1. - mu - nu, Y[0], sts_mu_hat(j, s) * dt, DYm,
-            sts_gm_hat(j, s) * dt, DY0);
+// Work vectors of the super-steps: rotating stage states, the first stage's
+// rate, Z = Y rho of the last and the next state, the state between steps,
+// what the adjoint's L_0 collects, and the adjoint's L in rotation (those of
+// the pending records, the one before them and the next); then the stage
+// states of a checkpoint segment, s per step.
+constexpr int kLams = kRecs + 2;
+enum { V_STATE = 0, V_DY0 = 3, V_Z = 4, V_Y = 6, V_A0 = 7, V_L = 8, V_SEG = V_L + kLams };
+
+// One RKL2 super-step (sts_integrator.f90:100-123) of s stages from Y[0], whose
+// Z is in the Z vector *z (left at the result's): stage states into Y[1..s]
+// (Y[s] may be Y[0]).  keep_last false: the last stage is not needed.
+static void sts_forward_step(sph_ctx *c, int s, double dt, double *const *Y, int *z, bool keep_last = true) {
+  BatchStage a{};
+  a.cnt = c->cnt; a.nb = c->nb; a.W = c->dW; a.rho = c->drho; a.h = dt; a.Y0 = Y[0]; a.DY0 = dv(c, V_DY0);
+  a.n = (int)c->n; a.npad = (int)c->npad;
+  const dim3 B(grid_for(c->n)), T(kBlock);
+  for (int j = 1; j <= (keep_last ? s : s - 1); j++) {
+    a.Yjm1 = Y[j - 1]; a.Yjm2 = j > 1 ? Y[j - 2] : Y[0]; a.Yj = Y[j];
+    a.Zjm1 = dv(c, V_Z + *z); a.Zj = dv(c, V_Z + (*z ^= 1));
+    a.mhat = sts_mu_hat(j, s);
+    a.rev = next_rev(c);
+    if (j == 1) {
+      hipLaunchKernelGGL((k_batch_stage<true, double, true>), B, T, 0, c->stream, a);
+    } else {
+      a.mu = sts_mu(j); a.nu = sts_nu(j); a.c0 = 1. - a.mu - a.nu; a.ghat = sts_gm_hat(j, s);
+      hipLaunchKernelGGL((k_batch_stage<false, double, true>), B, T, 0, c->stream, a);
+    }
   }
 }
 
-// Adjoint of one super-step: lam[s] given (in L[s]); returns dL/dY0 in L[0];
-// the tensor-gradient coefficients accumulate per pair (dS).
-static int sts_backward_step(sph_ctx *c, const double K[6], int s, double dt, double *const *Y, double *const *L,
-                             double *U) {
-  for (int j = s; j >= 2; j--) {
-    double mh = sts_mu_hat(j, s) * dt, gh = sts_gm_hat(j, s) * dt, mu = sts_mu(j), nu = sts_nu(j);
-    diff_adj_stage(c, K, L[j], Y[j - 1], Y[0], mh, gh, U);
-    hipLaunchKernelGGL(k_stage_adj, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, (int)c->n, L[j], U, mu, nu,
-                       mh, gh, L[j - 1], L[j - 2], L[0]);
+// Adjoint of one super-step with the stage states Y[0..s-1]: L (V_L + *l) holds
+// dL/dY_s on entry and dL/dY_0 on return.  The tensor-gradient coefficients
+// accumulate per pair (dS).
+static void sts_backward_step(sph_ctx *c, int s, double dt, double *const *Y, int *l) {
+  auto L = [&](int k) { return dv(c, V_L + (*l + k + kLams) % kLams); };
+  for (int j = s; j >= 1; j--) {
+    AdjStage a = adj_args(c);
+    a.lam = L(0);
+    a.lam1 = j < s ? L(-1) : nullptr;
+    a.out = L(1);
+    a.A0 = dv(c, V_A0);
+    a.mh = sts_mu_hat(j, s) * dt;
+    if (j > 1) {
+      a.mu = sts_mu(j); a.gh = sts_gm_hat(j, s) * dt;
+      a.c0 = 1. - a.mu - sts_nu(j) + (j == 2 ? sts_nu(j) : 0.);
+      a.nu1 = j < s ? sts_nu(j + 1) : 0.;
+      a.a0_add = j < s;
+    } else {
+      a.last = 1;
+    }
+    hipLaunchKernelGGL(k_adj_stage, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, a);
+    adj_record(c, L(0), Y[j - 1], j > 1 ? Y[0] : nullptr, a.mh, a.gh);
+    *l = (*l + 1) % kLams;
   }
-  double m1 = sts_mu_hat(1, s) * dt;
-  diff_adj_stage(c, K, L[1], Y[0], nullptr, m1, 0.0, U);
-  lincomb(c, L[0], 1.0, L[0], 1.0, L[1], m1, U);
-  return SPH_OK;
 }
 
 extern "C" {
@@ -2211,12 +2223,14 @@ int sph_diff_prepare(sph_ctx *c, const double state[49]) {
   if (op == 0) RCHK(dalloc(&c->dW, (size_t)c->npad * c->nb_cap));
   RCHK(dalloc(&c->ddW, c->npad));
   RCHK(dalloc(&c->dZ, c->npad));
-  for (int q = 0; q < 4; q++) RCHK(dalloc(&c->dLZ[q], c->npad));
-  c->lz_pend = 0;
+  RCHK(dalloc(&c->drho, c->npad));
+  if (op == 0) RCHK(dalloc(&c->dRec, (size_t)c->npad * kRecs));
+  c->rec_pend = c->rec_packed = 0;
+  c->coef_set = false;
   RCHK(dalloc(&c->gkdev, 12));
   c->w_valid = false;
   hipLaunchKernelGGL(k_diff_pack, dim3(G), dim3(kBlock), 0, c->stream, n, c->pm, (const double4 *)c->q[0], c->dpxh,
-                     c->dirho);
+                     c->drho, c->dirho);
   // reverse lists: stable radix sort of the owner-major pairs on the neighbour
   // index, then into the list layout (capacity = longest reverse list)
   int *foff = nullptr;
@@ -2261,7 +2275,6 @@ int sph_diff_prepare(sph_ctx *c, const double state[49]) {
     if ((rc = dalloc(&c->rent, rslots))) break;
     if (op == 0) {
       if ((rc = dalloc(&c->dR, rslots)) || (rc = dalloc(&c->dS, rslots))) break;
-      HIPCHK(hipMemsetAsync(c->dS, 0, sizeof(double) * rslots, c->stream));
     }
     // owner-major enumeration of the pairs, stable sort on the neighbour index
     bytes = c->scan_tmp_bytes;
@@ -2340,10 +2353,16 @@ int sph_diff_apply_adjoint(sph_ctx *c, const double K[6], const double *d_lam, c
     DiffOpArgs a = diff_args(c, K ? K : K0);
     NL_DISPATCH(nl_adjoint_k, c, a, dv(c, 0), dv(c, 1), c->diff_op == 5 ? nullptr : dv(c, 2), dv(c, 3));
   } else {
-    diff_adj_stage(c, K, dv(c, 0), dv(c, 1), nullptr, 1.0, 0.0, dv(c, 3));
-    RCHK(diff_gcontract(c, K, c->gkdev));
-    diff_adj_stage(c, K, dv(c, 0), dv(c, 2), nullptr, 1.0, 0.0, dv(c, 3));
-    RCHK(diff_gcontract(c, K, c->gkdev + 6));
+    ensure_weights(c, K);
+    AdjStage a = adj_args(c);  // A^T lam alone
+    a.lam = dv(c, 0); a.out = dv(c, 3); a.mh = 1.0; a.last = 1;
+    hipLaunchKernelGGL(k_adj_stage, dim3(G), dim3(kBlock), 0, c->stream, a);
+    c->rec_pend = c->rec_packed = 0;
+    c->coef_set = false;
+    for (int k = 0; k < 2; k++) {
+      adj_record(c, dv(c, 0), dv(c, 1 + k), nullptr, 1.0, 0.0);
+      diff_gcontract(c, K, c->gkdev + 6 * k);
+    }
   }
   hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 3), o, n, d_out);
   double g12[12];
@@ -2353,8 +2372,13 @@ int sph_diff_apply_adjoint(sph_ctx *c, const double K[6], const double *d_lam, c
   return SPH_OK;
 }
 
-// Vectors: 0..s stage states, s+1 DY0, s+2 DYm, s+3 U, s+4 .. 2s+4 adjoints L[0..s];
-// segment recompute states after that: every x (s+1).
+// A checkpoint segment's stage states: Y[j] of its step k, the first step's
+// Y[0] being the checkpoint itself.
+static void segment_states(sph_ctx *c, int sg, int k, int s, std::vector<double *> &Y) {
+  for (int j = 0; j < s; j++) Y[j] = dv(c, V_SEG + k * s + j);
+  if (k == 0) Y[0] = c->ckpt + (size_t)sg * c->npad;
+}
+
 int sph_diff_forward(sph_ctx *c, const double K[6], int s, double dt, int nsteps, int every, const double *d_T0,
                      double *d_T) {
   if (!c || !c->diff_ready || !K || !d_T0 || !d_T || s < 2 || nsteps < 1 || every < 1) return SPH_ERR_BAD_ARG;
@@ -2367,31 +2391,32 @@ int sph_diff_forward(sph_ctx *c, const double K[6], int s, double dt, int nsteps
     RCHK(dalloc(&c->ckpt, (size_t)nck * c->npad));
     c->ckpt_cap = (int64_t)nck * c->npad;
   }
-  RCHK(ensure_dvec(c, 2 * s + 5 + every * (s + 1)));
-  std::vector<double *> Y(s + 1), Yk(s + 1);
-  for (int j = 0; j <= s; j++) Y[j] = dv(c, j);
-  // the last checkpoint segment runs in the backward pass's segment buffers,
-  // so the backward pass need not recompute it
-  const int tail0 = ((nsteps + every - 1) / every - 1) * every, base = 2 * s + 5;
-  hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_T0, c->orig[c->cur], n, Y[0]);
+  RCHK(ensure_dvec(c, V_SEG + std::min(every, nsteps) * s));
+  ensure_weights(c, K);
+  // a step's last stage writes where the next step's Y_0 is kept: the next
+  // checkpoint, its place in the last segment (whose stage states the
+  // backward pass then need not recompute), or the state between steps
+  const int last_sg = (nsteps - 1) / every;
+  std::vector<double *> Y(s + 1);
+  double *y0 = c->ckpt;
+  int z = 0;
+  hipLaunchKernelGGL(k_batch_in, dim3(G), dim3(kBlock), 0, c->stream, d_T0, c->orig[c->cur], c->drho, n, y0,
+                     dv(c, V_Z));
   for (int st = 0; st < nsteps; st++) {
-    if (st % every == 0)
-      HIPCHK(hipMemcpyAsync(c->ckpt + (size_t)(st / every) * c->npad, Y[0], sizeof(double) * n,
-                            hipMemcpyDeviceToDevice, c->stream));
-    if (st < tail0) {
-      sts_forward_step(c, K, s, dt, Y.data(), dv(c, s + 1), dv(c, s + 2));
-      HIPCHK(hipMemcpyAsync(Y[0], Y[s], sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-      continue;
+    const int sg = st / every, k = st % every;
+    if (sg == last_sg) {
+      segment_states(c, sg, k, s, Y);
+    } else {
+      for (int j = 1; j < s; j++) Y[j] = dv(c, V_STATE + j % 3);
     }
-    const int k = st - tail0;
-    for (int j = 0; j <= s; j++) Yk[j] = dv(c, base + k * (s + 1) + j);
-    HIPCHK(hipMemcpyAsync(Yk[0], k == 0 ? Y[0] : dv(c, base + (k - 1) * (s + 1) + s), sizeof(double) * n,
-                          hipMemcpyDeviceToDevice, c->stream));
-    sts_forward_step(c, K, s, dt, Yk.data(), dv(c, s + 1), dv(c, s + 2));
-    if (st == nsteps - 1)
-      HIPCHK(hipMemcpyAsync(Y[0], Yk[s], sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+    Y[0] = y0;
+    if (st == nsteps - 1) y0 = dv(c, V_Y);
+    else if (k == every - 1) y0 = c->ckpt + (size_t)(sg + 1) * c->npad;
+    else y0 = sg == last_sg ? dv(c, V_SEG + (k + 1) * s) : dv(c, V_Y);
+    Y[s] = y0;
+    sts_forward_step(c, s, dt, Y.data(), &z);
   }
-  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, Y[0], c->orig[c->cur], n, d_T);
+  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, y0, c->orig[c->cur], n, d_T);
   HIPCHK(hipStreamSynchronize(c->stream));
   c->fw_s = s; c->fw_steps = nsteps; c->fw_every = every; c->fw_dt = dt;
   for (int k = 0; k < 6; k++) c->fw_K[k] = K[k];
@@ -2406,44 +2431,37 @@ int sph_diff_backward(sph_ctx *c, const double *d_gT, double *d_gT0, double gK[6
   const double dt = c->fw_dt;
   const double *K = c->fw_K;
   unsigned G = grid_for(n);
-  std::vector<double *> L(s + 1);
-  for (int j = 0; j <= s; j++) L[j] = dv(c, s + 4 + j);
-  double *U = dv(c, s + 3);
-  const int base = 2 * s + 5;
-  auto seg = [&](int k, int j) { return dv(c, base + k * (s + 1) + j); };
-  HIPCHK(hipMemsetAsync(c->dS, 0, sizeof(double) * (size_t)c->npad * c->rcap, c->stream));
+  ensure_weights(c, K);
   HIPCHK(hipMemsetAsync(c->gkdev, 0, sizeof(double) * 12, c->stream));
-  double *lam = dv(c, s + 1);  // running dL/dT (sorted)
-  hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_gT, c->orig[c->cur], n, lam);
-  int nseg = (nsteps + every - 1) / every;
+  c->rec_pend = c->rec_packed = 0;
+  c->coef_set = false;
+  int l = 0;  // the vector of the running L
+  hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_gT, c->orig[c->cur], n, dv(c, V_L));
+  const int nseg = (nsteps + every - 1) / every;
+  std::vector<double *> Y(s + 1);
   for (int sg = nseg - 1; sg >= 0; sg--) {
-    int st0 = sg * every, st1 = std::min(nsteps, st0 + every);
-    // recompute the segment's stage states from its checkpoint (the last
-    // segment's are still there from the forward pass)
-    const bool have = sg == nseg - 1 && c->fw_tail;
-    if (!have)
-      HIPCHK(hipMemcpyAsync(seg(0, 0), c->ckpt + (size_t)sg * c->npad, sizeof(double) * n, hipMemcpyDeviceToDevice,
-                            c->stream));
-    for (int st = st0; st < st1 && !have; st++) {
-      int k = st - st0;
-      std::vector<double *> Y(s + 1);
-      for (int j = 0; j <= s; j++) Y[j] = seg(k, j);
-      sts_forward_step(c, K, s, dt, Y.data(), dv(c, s + 2), U);
-      if (st + 1 < st1)
-        HIPCHK(hipMemcpyAsync(seg(k + 1, 0), Y[s], sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+    const int steps = std::min(nsteps, (sg + 1) * every) - sg * every;
+    // the segment's stage states from its checkpoint (the last segment's are
+    // still there from the forward pass)
+    if (!(sg == nseg - 1 && c->fw_tail)) {
+      adj_pack(c, false);  // the last segment's stages, before their states go
+      double *ck = c->ckpt + (size_t)sg * c->npad;
+      int z = 0;
+      hipLaunchKernelGGL(k_batch_in, dim3(G), dim3(kBlock), 0, c->stream, ck, (const int64_t *)nullptr, c->drho, n, ck,
+                         dv(c, V_Z));
+      for (int k = 0; k < steps; k++) {
+        segment_states(c, sg, k, s, Y);
+        Y[s] = k + 1 < steps ? dv(c, V_SEG + (k + 1) * s) : nullptr;
+        sts_forward_step(c, s, dt, Y.data(), &z, k + 1 < steps);
+      }
     }
-    for (int st = st1 - 1; st >= st0; st--) {
-      int k = st - st0;
-      std::vector<double *> Y(s + 1);
-      for (int j = 0; j <= s; j++) Y[j] = seg(k, j);
-      HIPCHK(hipMemsetAsync(L[0], 0, sizeof(double) * (size_t)c->npad * s, c->stream));
-      HIPCHK(hipMemcpyAsync(L[s], lam, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-      RCHK(sts_backward_step(c, K, s, dt, Y.data(), L.data(), U));
-      HIPCHK(hipMemcpyAsync(lam, L[0], sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+    for (int k = steps - 1; k >= 0; k--) {
+      segment_states(c, sg, k, s, Y);
+      sts_backward_step(c, s, dt, Y.data(), &l);
     }
   }
-  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, lam, c->orig[c->cur], n, d_gT0);
-  RCHK(diff_gcontract(c, K, c->gkdev));
+  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, V_L + l), c->orig[c->cur], n, d_gT0);
+  diff_gcontract(c, K, c->gkdev);
   c->fw_tail = false;  // segment buffers now hold the first segment
   HIPCHK(hipMemcpyAsync(gK, c->gkdev, sizeof(double) * 6, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -2501,14 +2519,15 @@ void batch_super_step(sph_batch *b, int s, int block) {
   a.Yjm1 = Y0; a.Yjm2 = Y0; a.Zjm1 = Z0; a.Yj = Y(1); a.Zj = Z(1);
   a.mhat = sts_mu_hat(1, s);
   const bool f32 = b->precision == 1;
-  if (f32) hipLaunchKernelGGL((k_batch_stage<true, float>), dim3(G), dim3(block), 0, b->stream, a);
-  else hipLaunchKernelGGL((k_batch_stage<true, double>), dim3(G), dim3(block), 0, b->stream, a);
+  if (f32) hipLaunchKernelGGL((k_batch_stage<true, float, false>), dim3(G), dim3(block), 0, b->stream, a);
+  else hipLaunchKernelGGL((k_batch_stage<true, double, false>), dim3(G), dim3(block), 0, b->stream, a);
   for (int j = 2; j <= s; j++) {
     a.Yjm1 = Y(j - 1); a.Yjm2 = Y(j - 2); a.Zjm1 = Z(j - 1); a.Yj = Y(j); a.Zj = Z(j);
     a.mu = sts_mu(j); a.nu = sts_nu(j); a.c0 = 1. - a.mu - a.nu;
     a.mhat = sts_mu_hat(j, s); a.ghat = sts_gm_hat(j, s);
-    if (f32) hipLaunchKernelGGL((k_batch_stage<false, float>), dim3(G), dim3(block), 0, b->stream, a);
-    else hipLaunchKernelGGL((k_batch_stage<false, double>), dim3(G), dim3(block), 0, b->stream, a);
+    a.rev = (j - 1) & 1;
+    if (f32) hipLaunchKernelGGL((k_batch_stage<false, float, false>), dim3(G), dim3(block), 0, b->stream, a);
+    else hipLaunchKernelGGL((k_batch_stage<false, double, false>), dim3(G), dim3(block), 0, b->stream, a);
   }
 }
 

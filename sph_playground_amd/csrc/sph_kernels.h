@@ -266,12 +266,12 @@ struct Loop2Args {
   int n, npad;
 };
 
-// Up to four adjoint stages' (lam, Zt) records (sph_adjoint.hip).
-// One RKL2 stage over merged problems (k_batch_stage): list-layout operator
-// (cnt, nb, W), densities, each row's problem (pid) and the per-problem time
-// steps; stage states Y_{j-1}, Y_{j-2}, Y_0, Z_{j-1} = Y_{j-1} rho, the
-// stage-1 rate DY0 and the outputs Y_j, Z_j; coefficients mu, nu,
-// 1 - mu - nu, mu_hat, gamma_hat.
+// One RKL2 stage (k_batch_stage) over merged problems, or over one prepared
+// problem's own lists: list-layout operator (cnt, nb, W), densities, each
+// row's problem (pid) and the per-problem time steps (one problem: h); stage
+// states Y_{j-1}, Y_{j-2}, Y_0, Z_{j-1} = Y_{j-1} rho, the stage-1 rate DY0 and
+// the outputs Y_j, Z_j; coefficients mu, nu, 1 - mu - nu, mu_hat, gamma_hat.
+// rev: the rows are taken from the far end (see stage_row).
 struct BatchStage {
   const int *cnt;
   const uint32_t *nb;
@@ -281,12 +281,31 @@ struct BatchStage {
   const double *dt;
   const double *Yjm1, *Yjm2, *Y0, *Zjm1;
   double *DY0, *Yj, *Zj;
-  double mu, nu, c0, mhat, ghat;
-  int n, npad;
+  double mu, nu, c0, mhat, ghat, h;
+  int n, npad, rev;
 };
 
-struct LZSet {
-  const double2 *p[4];
+// One adjoint stage j of a super-step (k_adj_stage): U = A^T L_j over the
+// reverse lists, then
+//   j > 1: L_{j-1} = mu L_j + mh U + nu1 L_{j+1} (L_{j+1} null for j = s),
+//          A0 (+)= c0 L_j + gh U, what L_0 collects (c0 holds nu too for j = 2)
+//   j = 1 (last): L_0 = A0 + L_1 + mh U
+// into `out`.
+struct AdjStage {
+  const uint32_t *rent;
+  const int *rcnt;
+  const double *R, *dW, *lam, *lam1;
+  double *A0, *out;
+  double mu, mh, nu1, c0, gh;
+  int a0_add, last, n, npad, rev;
+};
+// Adjoint stages whose part of the tensor gradient one pass over the pair
+// coefficients takes: stage q's L and Zt = (wa Ya + wb Yb) rho (Yb may be null)
+// become its record.
+constexpr int kRecs = 8;
+struct AdjRecs {
+  const double *lam[kRecs], *Ya[kRecs], *Yb[kRecs];
+  double wa[kRecs], wb[kRecs];
 };
 
 // The differentiable diffusion operator (sph_adjoint.hip).
