@@ -546,11 +546,34 @@ __global__ void k_from_sorted(const double *src, const int64_t *orig, int n, dou
 // adjoint is the transposed Jacobian at a state.  Every adjoint sum is a
 // gather over the reverse lists: no atomics, a fixed order.
 
-// nw(r, h) / r-vector: wcv df(q) / (h^(dim+2) q)
+// These operators are bound by the latency of their gathers (a list entry,
+// then up to five records) and by FP64 divisions: 4 or 8 lanes share a
+// particle (nl_lanes), and 1/|r| is the refined reciprocal square root (a few
+// ulp, as in loop 2).  32^3 with one lane, one entry at a time and IEEE
+// divisions: grad T 97 us, the FLD operator 105, its adjoint 191; now
+// 19, 17 and 33.
+
+// nw(r, h) / r-vector: wcv df(q) / (h^(dim+2) q), from 1/|r|
 template <int DIM, int KT>
-__device__ __forceinline__ double nw_coef(const DiffOpArgs &a, double dr, double inv_h) {
-  const double q = dr * inv_h;
-  return a.wcv * KernelFn<KT, double>::df(q) * ipow<DIM + 2>(inv_h) / q;
+__device__ __forceinline__ double nw_coef(const DiffOpArgs &a, double r2, double inv_dr, double inv_h) {
+  const double q = r2 * inv_dr * inv_h;
+  return a.wcv * KernelFn<KT, double>::df(q) * ipow<DIM + 1>(inv_h) * inv_dr;
+}
+
+// tr H of the Hessian operator at h (hess_basis with K = I)
+template <int DIM, int KT>
+__device__ __forceinline__ double hess_trace(const DiffOpArgs &a, double r2, double inv_dr, double inv_h) {
+  using Kf = KernelFn<KT, double>;
+  const double q = r2 * inv_dr * inv_h, ihd1 = ipow<DIM + 1>(inv_h);
+  if (a.ddw == 401) {
+    double df, ddf;
+    Kf::df_ddf(q, df, ddf);
+    // df / q with 1/q = h / |r|
+    return a.wcv * ihd1 * (inv_h * ddf + (DIM - 1) * df * inv_dr);
+  }
+  // half ((dim + 2) - dim)
+  if (a.ddw == 402) return a.fwc * a.wcv * Kf::f(q) * ihd1 * inv_h;
+  return -2.0 * a.wcv * Kf::df(q) * ihd1 * inv_dr;
 }
 
 __device__ __forceinline__ double3 kmul(const double K[6], double x, double y, double z) {
@@ -558,89 +581,96 @@ __device__ __forceinline__ double3 kmul(const double K[6], double x, double y, d
                       K[4] * x + K[5] * y + K[2] * z);
 }
 
-// Pair loop over s's list: fn(j, rx, ry, rz, dr) with r = x_s - x_j(image).
-template <typename Fn>
-__device__ __forceinline__ void over_list(const DiffOpArgs &a, int s, const double4 &ps, Fn fn) {
-  const int nn = a.cnt[s];
-  for (int k = 0; k < nn; k++) {
-    const uint32_t e = a.nb[nb_slot(k, s, a.npad)];
-    const uint32_t j = nb_index(e);
-    const double4 pb = a.pm[j];
-    double xb = pb.x, yb = pb.y, zb = pb.z;
-    if (nb_code(e) != kNoImage) image_shift(xb, yb, zb, nb_code(e), a.b);
+// Pair loop over s's list, G lanes: fn(j's record, rx, ry, rz, r^2, 1/|r|) with
+// r = x_s - x_j(image); rec(j) gathers what fn reads of j.
+template <int G, typename Rec, typename Fn>
+__device__ __forceinline__ void over_list(const DiffOpArgs &a, int s, int sub, const double4 &ps, Rec rec, Fn fn) {
+  struct J { double4 pb; decltype(rec(0u)) r; uint32_t code; };
+  auto load = [&](uint32_t e) { const uint32_t j = nb_index(e); return J{a.pm[j], rec(j), nb_code(e)}; };
+  for_neighbours<G, 1>(a.nb, s, sub, a.npad, a.cnt[s], load, [&](const J &d) {
+    double xb = d.pb.x, yb = d.pb.y, zb = d.pb.z;
+    if (d.code != kNoImage) image_shift(xb, yb, zb, d.code, a.b);
     const double rx = ps.x - xb, ry = ps.y - yb, rz = ps.z - zb;
-    fn(j, rx, ry, rz, sqrt(rx * rx + ry * ry + rz * rz));
-  }
+    const double r2 = rx * rx + ry * ry + rz * rz;
+    fn(d.r, d.pb.w, rx, ry, rz, r2, rsq_nr(r2));
+  });
 }
 
-// Pair loop over s's reverse list: fn(i, rx, ry, rz, dr) with i the owner
+// Pair loop over s's reverse list, G lanes: fn(i's record, ...) with i the owner
 // (s in i's list) and r = x_i - x_s(image as i sees it).
-template <typename Fn>
-__device__ __forceinline__ void over_rlist(const DiffOpArgs &a, int s, const double4 &ps, Fn fn) {
-  const int nr = a.rcnt[s];
-  for (int k = 0; k < nr; k++) {
-    const uint32_t e = a.rent[nb_slot(k, s, a.npad)];
-    const uint32_t i = nb_index(e);
-    const double4 pi = a.pm[i];
+template <int G, typename Rec, typename Fn>
+__device__ __forceinline__ void over_rlist(const DiffOpArgs &a, int s, int sub, const double4 &ps, Rec rec, Fn fn) {
+  struct J { double4 pi; decltype(rec(0u)) r; uint32_t code; };
+  auto load = [&](uint32_t e) { const uint32_t i = nb_index(e); return J{a.pxh[i], rec(i), nb_code(e)}; };
+  for_neighbours<G, 1>(a.rent, s, sub, a.npad, a.rcnt[s], load, [&](const J &d) {
     double xb = ps.x, yb = ps.y, zb = ps.z;
-    if (nb_code(e) != kNoImage) image_shift(xb, yb, zb, nb_code(e), a.b);
-    const double rx = pi.x - xb, ry = pi.y - yb, rz = pi.z - zb;
-    fn(i, rx, ry, rz, sqrt(rx * rx + ry * ry + rz * rz));
-  }
+    if (d.code != kNoImage) image_shift(xb, yb, zb, d.code, a.b);
+    const double rx = d.pi.x - xb, ry = d.pi.y - yb, rz = d.pi.z - zb;
+    const double r2 = rx * rx + ry * ry + rz * rz;
+    fn(d.r, d.pi.w, rx, ry, rz, r2, rsq_nr(r2));
+  });
 }
 
-// U = G(Y), and with FSUM the geometry sum F_s = sum_b m_b nw(r_sb, h_s).
-template <int DIM, int KT, int MODE>
-__global__ __launch_bounds__(256) void k_nl_grad(DiffOpArgs a, const double *Y, double4 *U, double4 *F) {
-  int s = gtid_a();
+// U = G(Y), and with F the geometry sum F_s = sum_b m_b nw(r_sb, h_s).  With D
+// (FLD) also the conductivity at state Y: D, dD/dR and R per particle.
+template <int DIM, int KT, int MODE, int G>
+__global__ __launch_bounds__(256) void k_nl_grad(DiffOpArgs a, const double *Y, double4 *U, double4 *F, double *D,
+                                                 double *dDdR, double *R) {
+  const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
   const double4 qa = a.q0[s];
   const double inv_ha = qa.x, rhoa = qa.y, oma = qa.z;
   const double ya = Y ? Y[s] : 0.0;
   double ux = 0, uy = 0, uz = 0, fx = 0, fy = 0, fz = 0;
-  over_list(a, s, ps, [&](uint32_t j, double rx, double ry, double rz, double dr) {
-    const double4 qb = a.q0[j];
-    const double mb = a.pm[j].w;
-    const double wa = nw_coef<DIM, KT>(a, dr, inv_ha);
+  struct Rec { double y, rho; double4 q; };
+  auto rec = [&](uint32_t j) {
+    Rec r{};
+    if (Y) {
+      r.y = Y[j];
+      if constexpr (MODE == 1) r.rho = a.rho[j];
+      else r.q = a.q0[j];
+    }
+    return r;
+  };
+  over_list<G>(a, s, sub, ps, rec, [&](const Rec &j, double mb, double rx, double ry, double rz, double r2, double ir) {
+    const double wa = nw_coef<DIM, KT>(a, r2, ir, inv_ha);
     if (F) { fx += mb * wa * rx; fy += mb * wa * ry; fz += mb * wa * rz; }
     if (!Y) return;
     if constexpr (MODE == 1) {
-      const double t = mb * (Y[j] * qb.y - ya * rhoa) * wa;
+      const double t = mb * (j.y * j.rho - ya * rhoa) * wa;
       ux += t * rx; uy += t * ry; uz += t * rz;
     } else {
-      const double wb = nw_coef<DIM, KT>(a, dr, qb.x);
-      const double ca = mb * ya / (oma * rhoa) * wa, cb = mb * Y[j] * rhoa / (qb.z * qb.y * qb.y) * wb;
+      const double wb = nw_coef<DIM, KT>(a, r2, ir, j.q.x);
+      const double ca = mb * ya / (oma * rhoa) * wa, cb = mb * j.y * rhoa / (j.q.z * j.q.y * j.q.y) * wb;
       ux += (ca + cb) * rx; uy += (ca + cb) * ry; uz += (ca + cb) * rz;
     }
   });
-  if (Y) {
-    const double c = MODE == 1 ? 1.0 / (rhoa * oma) : 1.0;
-    U[s] = make_double4(c * ux, c * uy, c * uz, 0.0);
-  }
+  group_sum<G>(ux, uy, uz);
+  if (F) group_sum<G>(fx, fy, fz);
+  if (sub != 0) return;
   if (F) F[s] = make_double4(fx, fy, fz, 0.0);
+  if (!Y) return;
+  const double c = MODE == 1 ? 1.0 / (rhoa * oma) : 1.0;
+  ux *= c; uy *= c; uz *= c;
+  U[s] = make_double4(ux, uy, uz, 0.0);
+  if (D) {
+    const double kap = a.kap[s];
+    const double un = sqrt(ux * ux + uy * uy + uz * uz);
+    const double r = un / (kap * rhoa * ya * rhoa);
+    const double den = 6. + 3. * r + r * r;
+    D[s] = kLightspeed * ((2. + r) / den) / kap / rhoa;
+    dDdR[s] = kLightspeed * (-r * (4. + r) / (den * den)) / kap / rhoa;
+    R[s] = r;
+  }
 }
 
-// FLD conductivity at state Y from U = G(Y): D, dD/dR and R per particle.
-__global__ void k_fld_coef(DiffOpArgs a, const double *Y, const double4 *U, double *D, double *dDdR, double *R) {
-  int s = gtid_a();
-  if (s >= a.n || !a.real[s]) return;
-  const double4 u = U[s];
-  const double rho = a.q0[s].y, kap = a.kap[s];
-  const double un = sqrt(u.x * u.x + u.y * u.y + u.z * u.z);
-  const double r = un / (kap * rho * Y[s] * rho);
-  const double den = 6. + 3. * r + r * r;
-  const double lam = (2. + r) / den;
-  D[s] = kLightspeed * lam / kap / rho;
-  dDdR[s] = kLightspeed * (-r * (4. + r) / (den * den)) / kap / rho;
-  R[s] = r;
-}
-
-// f = A Y for the three operators (OP 3 = 2nw-+, 4 = 2nw+-, 5 = FLD).
-template <int DIM, int KT, int OP>
+// f = A Y for the three operators (OP 3 = 2nw-+, 4 = 2nw+-, 5 = FLD), to the
+// particle's place in the original order.
+template <int DIM, int KT, int OP, int G>
 __global__ __launch_bounds__(256) void k_nl_apply(DiffOpArgs a, const double *Y, const double4 *U, const double *D,
-                                                  double *out) {
-  int s = gtid_a();
+                                                  const int64_t *orig, double *out) {
+  const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
   const double4 qa = a.q0[s];
@@ -648,54 +678,66 @@ __global__ __launch_bounds__(256) void k_nl_apply(DiffOpArgs a, const double *Y,
   double acc = 0.0;
   if constexpr (OP == 5) {
     const double za = Y[s] * rhoa, da = D[s];
-    const double I6[6] = {1, 1, 1, 0, 0, 0};
-    over_list(a, s, ps, [&](uint32_t j, double rx, double ry, double rz, double) {
-      const double4 qb = a.q0[j];
-      double G[6];
-      hess_basis<DIM, KT>(a, rx, ry, rz, inv_ha, G);
-      acc += a.pm[j].w / qb.y * kdot(I6, G) * (0.5 * (da + D[j])) * (Y[j] * qb.y - za);
+    struct Rec { double y, rho, d; };
+    auto rec = [&](uint32_t j) { return Rec{Y[j], a.rho[j], D[j]}; };
+    over_list<G>(a, s, sub, ps, rec, [&](const Rec &j, double mb, double, double, double, double r2, double ir) {
+      acc += mb / j.rho * hess_trace<DIM, KT>(a, r2, ir, inv_ha) * (0.5 * (da + j.d)) * (j.y * j.rho - za);
     });
-    out[s] = acc / rhoa;
+    group_sum<G>(acc);
+    if (sub == 0) out[orig[s]] = acc / rhoa;
   } else {
     const double4 ua = U[s];
     const double3 ka = kmul(a.K, ua.x, ua.y, ua.z);
     const double odda = 1.0 / (oma * rhoa * rhoa);
-    over_list(a, s, ps, [&](uint32_t j, double rx, double ry, double rz, double dr) {
-      const double4 qb = a.q0[j];
-      const double4 ub = U[j];
-      const double3 kb = kmul(a.K, ub.x, ub.y, ub.z);
-      const double mb = a.pm[j].w;
-      const double wa = nw_coef<DIM, KT>(a, dr, inv_ha);
+    struct Rec { double4 q, u; };
+    auto rec = [&](uint32_t j) {
+      Rec r{};
+      if constexpr (OP == 3) r.q = a.q0[j];
+      r.u = U[j];
+      return r;
+    };
+    over_list<G>(a, s, sub, ps, rec, [&](const Rec &j, double mb, double rx, double ry, double rz, double r2, double ir) {
+      const double3 kb = kmul(a.K, j.u.x, j.u.y, j.u.z);
+      const double wa = nw_coef<DIM, KT>(a, r2, ir, inv_ha);
       if constexpr (OP == 3) {
-        const double wb = nw_coef<DIM, KT>(a, dr, qb.x);
-        const double oddb = 1.0 / (qb.z * qb.y * qb.y);
+        const double wb = nw_coef<DIM, KT>(a, r2, ir, j.q.x);
+        const double oddb = 1.0 / (j.q.z * j.q.y * j.q.y);
         acc += mb * ((ka.x * rx + ka.y * ry + ka.z * rz) * wa * odda + (kb.x * rx + kb.y * ry + kb.z * rz) * wb * oddb);
       } else {
         acc += mb * ((kb.x - ka.x) * rx + (kb.y - ka.y) * ry + (kb.z - ka.z) * rz) * wa;
       }
     });
-    out[s] = OP == 3 ? acc : acc * odda;
+    group_sum<G>(acc);
+    if (sub == 0) out[orig[s]] = OP == 3 ? acc : acc * odda;
   }
 }
 
 // 2nw adjoint, the vector nu with <lam, A Y> = sum_s (K U_s) . nu_s:
 //   2nw-+ : nu_s = (lam_s F_s + m_s sum_{a in R(s)} lam_a nw(r_as, h_s)) / (Om_s rho_s^2)
 //   2nw+- : nu_s = m_s sum_{a in R(s)} lam_a nw(r_as, h_a)/(Om_a rho_a^2) - lam_s F_s/(Om_s rho_s^2)
-template <int DIM, int KT, int OP>
+template <int DIM, int KT, int OP, int G>
 __global__ __launch_bounds__(256) void k_nl_nu(DiffOpArgs a, const double *lam, const double4 *F, double4 *nu) {
-  int s = gtid_a();
+  const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
   const double4 qs = a.q0[s];
   const double odds = 1.0 / (qs.z * qs.y * qs.y);
   double rx_ = 0, ry_ = 0, rz_ = 0;
-  over_rlist(a, s, ps, [&](uint32_t i, double rx, double ry, double rz, double dr) {
-    const double4 qi = a.q0[i];
+  struct Rec { double lam; double4 q; };
+  auto rec = [&](uint32_t i) {
+    Rec r{};
+    r.lam = lam[i];
+    if constexpr (OP != 3) r.q = a.q0[i];
+    return r;
+  };
+  over_rlist<G>(a, s, sub, ps, rec, [&](const Rec &i, double inv_hi, double rx, double ry, double rz, double r2, double ir) {
     double c;
-    if constexpr (OP == 3) c = lam[i] * nw_coef<DIM, KT>(a, dr, qs.x);
-    else c = lam[i] / (qi.z * qi.y * qi.y) * nw_coef<DIM, KT>(a, dr, qi.x);
+    if constexpr (OP == 3) c = i.lam * nw_coef<DIM, KT>(a, r2, ir, qs.x);
+    else c = i.lam / (i.q.z * i.q.y * i.q.y) * nw_coef<DIM, KT>(a, r2, ir, inv_hi);
     rx_ += c * rx; ry_ += c * ry; rz_ += c * rz;
   });
+  group_sum<G>(rx_, ry_, rz_);
+  if (sub != 0) return;
   const double4 f = F[s];
   const double ls = lam[s], ms = ps.w;
   if constexpr (OP == 3)
@@ -737,97 +779,96 @@ __global__ __launch_bounds__(256) void k_nl_mu(DiffOpArgs a, const double4 *nu, 
   }
 }
 
-// out (+)= d<mu, G(Y)>/dY:
+// out = base + d<mu, G(Y)>/dY (base null: 0), to the original order:
 //   mode 1: rho_s m_s sum_{a in R(s)} mu_a.nw(r_as, h_a)/(rho_a Om_a) - mu_s.F_s/Om_s
 //   mode 2: mu_s.F_s/(Om_s rho_s) + m_s/(Om_s rho_s^2) sum_{a in R(s)} rho_a mu_a.nw(r_as, h_s)
-template <int DIM, int KT, int MODE>
-__global__ __launch_bounds__(256) void k_nl_gT(DiffOpArgs a, const double4 *mu, const double4 *F, double *out, int add) {
-  int s = gtid_a();
+template <int DIM, int KT, int MODE, int G>
+__global__ __launch_bounds__(256) void k_nl_gT(DiffOpArgs a, const double4 *mu, const double4 *F, const double *base,
+                                               const int64_t *orig, double *out) {
+  const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
   const double4 qs = a.q0[s];
   double acc = 0.0;
-  over_rlist(a, s, ps, [&](uint32_t i, double rx, double ry, double rz, double dr) {
-    const double4 qi = a.q0[i];
-    const double4 m = mu[i];
-    const double dot = m.x * rx + m.y * ry + m.z * rz;
-    if constexpr (MODE == 1) acc += dot * nw_coef<DIM, KT>(a, dr, qi.x) / (qi.y * qi.z);
-    else acc += qi.y * dot * nw_coef<DIM, KT>(a, dr, qs.x);
+  struct Rec { double4 q, m; };
+  auto rec = [&](uint32_t i) { return Rec{a.q0[i], mu[i]}; };
+  over_rlist<G>(a, s, sub, ps, rec, [&](const Rec &i, double, double rx, double ry, double rz, double r2, double ir) {
+    const double dot = i.m.x * rx + i.m.y * ry + i.m.z * rz;
+    if constexpr (MODE == 1) acc += dot * nw_coef<DIM, KT>(a, r2, ir, i.q.x) / (i.q.y * i.q.z);
+    else acc += i.q.y * dot * nw_coef<DIM, KT>(a, r2, ir, qs.x);
   });
+  group_sum<G>(acc);
+  if (sub != 0) return;
   const double4 m = mu[s], f = F[s];
   const double mf = m.x * f.x + m.y * f.y + m.z * f.z;
   double v;
   if constexpr (MODE == 1) v = qs.y * ps.w * acc - mf / qs.z;
   else v = mf / (qs.z * qs.y) + ps.w / (qs.z * qs.y * qs.y) * acc;
-  out[s] = add ? out[s] + v : v;
+  out[orig[s]] = base ? base[s] + v : v;
 }
 
 // FLD adjoint at state Y, the part with the conductivity held:
 //   out_s = m_s sum_{a in R(s)} (lam_a/rho_a) trH_as (D_a + D_s)/2 - lam_s sum_b (m_b/rho_b) trH_sb (D_s + D_b)/2
 // and sD_s = d<lam, f>/dD_s
 //   = ((lam_s/rho_s) sum_b (m_b/rho_b) trH_sb (Z_b - Z_s) + (m_s/rho_s) sum_{a in R(s)} (lam_a/rho_a) trH_as (Z_s - Z_a)) / 2
-// with Z = Y rho and trH at the list owner's h.
-template <int DIM, int KT>
+// with Z = Y rho and trH at the list owner's h; then the conductivity's
+// dependence on the state: p = sD dD/dR, the direct dR/dY = -R / Y into out and
+// v = p dR/dU = p U / (|U| kappa rho^2 Y) (0 where U = 0) for k_nl_gT.
+template <int DIM, int KT, int G>
 __global__ __launch_bounds__(256) void k_fld_adj(DiffOpArgs a, const double *lam, const double *Y, const double *D,
-                                                 double *out, double *sD) {
-  int s = gtid_a();
+                                                 const double *dDdR, const double *R, const double4 *U, double *out,
+                                                 double4 *v) {
+  const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
   const double4 qs = a.q0[s];
-  const double zs = Y[s] * qs.y, ds = D[s], ls = lam[s];
-  const double I6[6] = {1, 1, 1, 0, 0, 0};
+  const double ys = Y[s], zs = ys * qs.y, ds = D[s], ls = lam[s];
   double s1 = 0, s2 = 0, s3 = 0, s4 = 0;
-  over_list(a, s, ps, [&](uint32_t j, double rx, double ry, double rz, double) {
-    const double4 qb = a.q0[j];
-    double G[6];
-    hess_basis<DIM, KT>(a, rx, ry, rz, qs.x, G);
-    const double w = a.pm[j].w / qb.y * kdot(I6, G);
-    s1 += w * (0.5 * (ds + D[j]));
-    s2 += w * (Y[j] * qb.y - zs);
+  struct Rec { double y, rho, d, lam; };
+  auto rec = [&](uint32_t j) { return Rec{Y[j], a.rho[j], D[j], 0.0}; };
+  over_list<G>(a, s, sub, ps, rec, [&](const Rec &j, double mb, double, double, double, double r2, double ir) {
+    const double w = mb / j.rho * hess_trace<DIM, KT>(a, r2, ir, qs.x);
+    s1 += w * (0.5 * (ds + j.d));
+    s2 += w * (j.y * j.rho - zs);
   });
-  over_rlist(a, s, ps, [&](uint32_t i, double rx, double ry, double rz, double) {
-    const double4 qi = a.q0[i];
-    double G[6];
-    hess_basis<DIM, KT>(a, rx, ry, rz, qi.x, G);
-    const double w = lam[i] / qi.y * kdot(I6, G);
-    s3 += w * (0.5 * (D[i] + ds));
-    s4 += w * (zs - Y[i] * qi.y);
+  auto rrec = [&](uint32_t i) { return Rec{Y[i], a.rho[i], D[i], lam[i]}; };
+  over_rlist<G>(a, s, sub, ps, rrec, [&](const Rec &i, double inv_hi, double, double, double, double r2, double ir) {
+    const double w = i.lam / i.rho * hess_trace<DIM, KT>(a, r2, ir, inv_hi);
+    s3 += w * (0.5 * (i.d + ds));
+    s4 += w * (zs - i.y * i.rho);
   });
-  out[s] = ps.w * s3 - ls * s1;
-  sD[s] = 0.5 * (ls / qs.y * s2 + ps.w / qs.y * s4);
-}
-
-// FLD adjoint, the conductivity's dependence on the state: p = sD dD/dR,
-// v = p dR/dU = p U / (|U| kappa rho^2 Y) (0 where U = 0), and the direct
-// dR/dY = -R / Y into out.
-__global__ void k_fld_pv(DiffOpArgs a, const double *sD, const double *dDdR, const double *R, const double4 *U,
-                         const double *Y, double *out, double4 *v) {
-  int s = gtid_a();
-  if (s >= a.n || !a.real[s]) return;
-  const double p = sD[s] * dDdR[s];
+  group_sum<G>(s1, s2, s3, s4);
+  if (sub != 0) return;
+  const double sD = 0.5 * (ls / qs.y * s2 + ps.w / qs.y * s4);
+  const double p = sD * dDdR[s];
   const double4 u = U[s];
   const double un = sqrt(u.x * u.x + u.y * u.y + u.z * u.z);
-  const double rho = a.q0[s].y;
-  const double c = un > 0.0 ? p / (un * a.kap[s] * rho * rho * Y[s]) : 0.0;
+  const double rho = qs.y;
+  const double c = un > 0.0 ? p / (un * a.kap[s] * rho * rho * ys) : 0.0;
   v[s] = make_double4(c * u.x, c * u.y, c * u.z, 0.0);
-  out[s] -= p * R[s] / Y[s];
+  out[s] = ps.w * s3 - ls * s1 - p * R[s] / ys;
 }
 
-#define SPH_INST_NL(DIM, KT)                                                                                    \
-  template __global__ void k_nl_grad<DIM, KT, 1>(DiffOpArgs, const double *, double4 *, double4 *);               \
-  template __global__ void k_nl_grad<DIM, KT, 2>(DiffOpArgs, const double *, double4 *, double4 *);               \
-  template __global__ void k_nl_apply<DIM, KT, 3>(DiffOpArgs, const double *, const double4 *, const double *,    \
-                                                  double *);                                                      \
-  template __global__ void k_nl_apply<DIM, KT, 4>(DiffOpArgs, const double *, const double4 *, const double *,    \
-                                                  double *);                                                      \
-  template __global__ void k_nl_apply<DIM, KT, 5>(DiffOpArgs, const double *, const double4 *, const double *,    \
-                                                  double *);                                                      \
-  template __global__ void k_nl_nu<DIM, KT, 3>(DiffOpArgs, const double *, const double4 *, double4 *);           \
-  template __global__ void k_nl_nu<DIM, KT, 4>(DiffOpArgs, const double *, const double4 *, double4 *);           \
-  template __global__ void k_nl_gT<DIM, KT, 1>(DiffOpArgs, const double4 *, const double4 *, double *, int);      \
-  template __global__ void k_nl_gT<DIM, KT, 2>(DiffOpArgs, const double4 *, const double4 *, double *, int);      \
-  template __global__ void k_fld_adj<DIM, KT>(DiffOpArgs, const double *, const double *, const double *, double *, \
-                                              double *);
+#define SPH_INST_NLG(DIM, KT, G)                                                                              \
+  template __global__ void k_nl_grad<DIM, KT, 1, G>(DiffOpArgs, const double *, double4 *, double4 *, double *, \
+                                                    double *, double *);                                      \
+  template __global__ void k_nl_grad<DIM, KT, 2, G>(DiffOpArgs, const double *, double4 *, double4 *, double *, \
+                                                    double *, double *);                                      \
+  template __global__ void k_nl_apply<DIM, KT, 3, G>(DiffOpArgs, const double *, const double4 *, const double *, \
+                                                     const int64_t *, double *);                              \
+  template __global__ void k_nl_apply<DIM, KT, 4, G>(DiffOpArgs, const double *, const double4 *, const double *, \
+                                                     const int64_t *, double *);                              \
+  template __global__ void k_nl_apply<DIM, KT, 5, G>(DiffOpArgs, const double *, const double4 *, const double *, \
+                                                     const int64_t *, double *);                              \
+  template __global__ void k_nl_nu<DIM, KT, 3, G>(DiffOpArgs, const double *, const double4 *, double4 *);    \
+  template __global__ void k_nl_nu<DIM, KT, 4, G>(DiffOpArgs, const double *, const double4 *, double4 *);    \
+  template __global__ void k_nl_gT<DIM, KT, 1, G>(DiffOpArgs, const double4 *, const double4 *, const double *, \
+                                                  const int64_t *, double *);                                 \
+  template __global__ void k_nl_gT<DIM, KT, 2, G>(DiffOpArgs, const double4 *, const double4 *, const double *, \
+                                                  const int64_t *, double *);                                 \
+  template __global__ void k_fld_adj<DIM, KT, G>(DiffOpArgs, const double *, const double *, const double *,  \
+                                                 const double *, const double *, const double4 *, double *, double4 *);
+#define SPH_INST_NL(DIM, KT) SPH_INST_NLG(DIM, KT, 4) SPH_INST_NLG(DIM, KT, 8)
 SPH_INST_NL(1, 0) SPH_INST_NL(1, 1) SPH_INST_NL(1, 2)
 SPH_INST_NL(2, 0) SPH_INST_NL(2, 1) SPH_INST_NL(2, 2)
 SPH_INST_NL(3, 0) SPH_INST_NL(3, 1) SPH_INST_NL(3, 2)

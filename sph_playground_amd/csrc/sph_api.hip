@@ -92,20 +92,18 @@ __global__ void k_batch_merge(int, int, int64_t, int, const int *, const uint32_
 template <bool FIRST, typename WT, bool ONE>
 __global__ void k_batch_stage(BatchStage);
 __global__ void k_batch_in(const double *, const int64_t *, const double *, int, double *, double *);
-template <int DIM, int KT, int MODE>
-__global__ void k_nl_grad(DiffOpArgs, const double *, double4 *, double4 *);
-__global__ void k_fld_coef(DiffOpArgs, const double *, const double4 *, double *, double *, double *);
-template <int DIM, int KT, int OP>
-__global__ void k_nl_apply(DiffOpArgs, const double *, const double4 *, const double *, double *);
-template <int DIM, int KT, int OP>
+template <int DIM, int KT, int MODE, int G>
+__global__ void k_nl_grad(DiffOpArgs, const double *, double4 *, double4 *, double *, double *, double *);
+template <int DIM, int KT, int OP, int G>
+__global__ void k_nl_apply(DiffOpArgs, const double *, const double4 *, const double *, const int64_t *, double *);
+template <int DIM, int KT, int OP, int G>
 __global__ void k_nl_nu(DiffOpArgs, const double *, const double4 *, double4 *);
 __global__ void k_nl_mu(DiffOpArgs, const double4 *, const double4 *, const double4 *, double4 *, double *);
-template <int DIM, int KT, int MODE>
-__global__ void k_nl_gT(DiffOpArgs, const double4 *, const double4 *, double *, int);
-template <int DIM, int KT>
-__global__ void k_fld_adj(DiffOpArgs, const double *, const double *, const double *, double *, double *);
-__global__ void k_fld_pv(DiffOpArgs, const double *, const double *, const double *, const double4 *, const double *,
-                         double *, double4 *);
+template <int DIM, int KT, int MODE, int G>
+__global__ void k_nl_gT(DiffOpArgs, const double4 *, const double4 *, const double *, const int64_t *, double *);
+template <int DIM, int KT, int G>
+__global__ void k_fld_adj(DiffOpArgs, const double *, const double *, const double *, const double *, const double *,
+                          const double4 *, double *, double4 *);
 }  // namespace sph
 
 namespace {
@@ -301,7 +299,7 @@ struct sph_ctx {
   // 0 = the Hessian operators of the assembled path)
   int diff_op = 0;
   double4 *nlF = nullptr, *nlU = nullptr, *nlUB = nullptr, *nlNu = nullptr, *nlMu = nullptr;
-  double *nlD = nullptr, *nlDD = nullptr, *nlR = nullptr, *nlSD = nullptr;
+  double *nlD = nullptr, *nlDD = nullptr, *nlR = nullptr;
 
   Fields fields() const {
     Fields F;
@@ -1589,7 +1587,7 @@ int sph_ctx_destroy(sph_ctx *c) {
                   c->real, c->nb, c->cnt, c->q[0], c->q[1], c->q[2], c->q[3], c->q[4], c->energy_part,
                   c->d_red, c->d_int, c->d_stripes, c->d_staging, c->roff, c->rtmp, c->rent, c->scan_tmp,
                   c->dvec, c->gpart, c->ckpt, c->rcnt, c->dpxh, c->dirho, c->dW, c->ddW, c->dR, c->dS, c->dZ, c->drho, c->dRec,
-                  c->gkdev, c->nlF, c->nlU, c->nlUB, c->nlNu, c->nlMu, c->nlD, c->nlDD, c->nlR, c->nlSD,
+                  c->gkdev, c->nlF, c->nlU, c->nlUB, c->nlNu, c->nlMu, c->nlD, c->nlDD, c->nlR,
                   c->ext_count, c->ecs, c->erec, c->ext_tmp};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -1970,59 +1968,68 @@ static DiffOpArgs diff_args(sph_ctx *c, const double K[6]) {
   a.wcv = c->diff_phys.wcv; a.fwc = c->diff_phys.fwc; a.ddw = c->diff_phys.ddw;
   a.n = (int)c->n; a.npad = (int)c->npad;
   a.kap = c->fields().f[F_KAPPA];
+  a.rho = c->drho;
   return a;
 }
 
 // ---- operators that read grad T (frozen geometry; see sph_adjoint.hip)
+// Lanes per particle of these operators: 8 below 40k particles, else 4 (as
+// loop 2's rule for FP64 diffusion).
+#define COMMA ,
+#define NL_LAUNCH(KERNEL, ...)                                                                                      \
+  do {                                                                                                              \
+    if (c->n < 40000)                                                                                               \
+      hipLaunchKernelGGL((KERNEL, 8>), dim3(grid_for(c->n * 8)), dim3(kBlock), 0, c->stream, __VA_ARGS__);          \
+    else                                                                                                            \
+      hipLaunchKernelGGL((KERNEL, 4>), dim3(grid_for(c->n * 4)), dim3(kBlock), 0, c->stream, __VA_ARGS__);          \
+  } while (0)
+// U = G(Y) and, for FLD with a state, its conductivity
 template <int DIM, int KT>
 static void nl_grad_k(sph_ctx *c, const DiffOpArgs &a, const double *Y, double4 *U, double4 *F) {
-  const unsigned G = grid_for(c->n);
-  if (c->diff_op == 4) hipLaunchKernelGGL((k_nl_grad<DIM, KT, 2>), dim3(G), dim3(kBlock), 0, c->stream, a, Y, U, F);
-  else hipLaunchKernelGGL((k_nl_grad<DIM, KT, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, Y, U, F);
+  double *D = c->diff_op == 5 && Y ? c->nlD : nullptr;
+  if (c->diff_op == 4) NL_LAUNCH(k_nl_grad<DIM COMMA KT COMMA 2, a, Y, U, F, D, c->nlDD, c->nlR);
+  else NL_LAUNCH(k_nl_grad<DIM COMMA KT COMMA 1, a, Y, U, F, D, c->nlDD, c->nlR);
 }
+// f(Y), Y sorted, into `out` in original order
 template <int DIM, int KT>
 static void nl_apply_k(sph_ctx *c, const DiffOpArgs &a, const double *Y, double *out) {
-  const unsigned G = grid_for(c->n);
+  const int64_t *o = c->orig[c->cur];
   nl_grad_k<DIM, KT>(c, a, Y, c->nlU, nullptr);
-  if (c->diff_op == 5) {
-    hipLaunchKernelGGL(k_fld_coef, dim3(G), dim3(kBlock), 0, c->stream, a, Y, c->nlU, c->nlD, c->nlDD, c->nlR);
-    hipLaunchKernelGGL((k_nl_apply<DIM, KT, 5>), dim3(G), dim3(kBlock), 0, c->stream, a, Y, c->nlU, c->nlD, out);
-  } else if (c->diff_op == 3) {
-    hipLaunchKernelGGL((k_nl_apply<DIM, KT, 3>), dim3(G), dim3(kBlock), 0, c->stream, a, Y, c->nlU, c->nlD, out);
-  } else {
-    hipLaunchKernelGGL((k_nl_apply<DIM, KT, 4>), dim3(G), dim3(kBlock), 0, c->stream, a, Y, c->nlU, c->nlD, out);
-  }
+  if (c->diff_op == 5) NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 5, a, Y, c->nlU, c->nlD, o, out);
+  else if (c->diff_op == 3) NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 3, a, Y, c->nlU, c->nlD, o, out);
+  else NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 4, a, Y, c->nlU, c->nlD, o, out);
 }
-// out = A^T lam (2nw: A linear; FLD: the Jacobian of f at Ya, transposed);
-// for 2nw the tensor gradients lam^T dA/dK Ya -> gkdev[0..5], Yb -> [6..11]
+// out (original order) = A^T lam (2nw: A linear; FLD: the Jacobian of f at Ya,
+// transposed), `work` a sorted vector; for 2nw the tensor gradients lam^T
+// dA/dK Ya -> gkdev[0..5], Yb -> [6..11] (Yb may be Ya)
 template <int DIM, int KT>
 static void nl_adjoint_k(sph_ctx *c, const DiffOpArgs &a, const double *lam, const double *Ya, const double *Yb,
-                         double *out) {
+                         double *work, double *out) {
   const unsigned G = grid_for(c->n);
+  const int64_t *o = c->orig[c->cur];
+  const double *none = nullptr;
+  nl_grad_k<DIM, KT>(c, a, Ya, c->nlU, nullptr);
   if (c->diff_op == 5) {
-    nl_grad_k<DIM, KT>(c, a, Ya, c->nlU, nullptr);
-    hipLaunchKernelGGL(k_fld_coef, dim3(G), dim3(kBlock), 0, c->stream, a, Ya, c->nlU, c->nlD, c->nlDD, c->nlR);
-    hipLaunchKernelGGL((k_fld_adj<DIM, KT>), dim3(G), dim3(kBlock), 0, c->stream, a, lam, Ya, c->nlD, out, c->nlSD);
-    hipLaunchKernelGGL(k_fld_pv, dim3(G), dim3(kBlock), 0, c->stream, a, c->nlSD, c->nlDD, c->nlR, c->nlU, Ya, out,
-                       c->nlMu);
-    hipLaunchKernelGGL((k_nl_gT<DIM, KT, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, c->nlMu, c->nlF, out, 1);
+    NL_LAUNCH(k_fld_adj<DIM COMMA KT, a, lam, Ya, c->nlD, c->nlDD, c->nlR, c->nlU, work, c->nlMu);
+    const double *base = work;
+    NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 1, a, c->nlMu, c->nlF, base, o, out);
     return;
   }
-  nl_grad_k<DIM, KT>(c, a, Ya, c->nlU, nullptr);
-  if (Yb) nl_grad_k<DIM, KT>(c, a, Yb, c->nlUB, nullptr);
-  if (c->diff_op == 3)
-    hipLaunchKernelGGL((k_nl_nu<DIM, KT, 3>), dim3(G), dim3(kBlock), 0, c->stream, a, lam, c->nlF, c->nlNu);
-  else
-    hipLaunchKernelGGL((k_nl_nu<DIM, KT, 4>), dim3(G), dim3(kBlock), 0, c->stream, a, lam, c->nlF, c->nlNu);
-  hipLaunchKernelGGL(k_nl_mu, dim3(G), dim3(kBlock), 0, c->stream, a, c->nlNu, c->nlU, Yb ? c->nlUB : nullptr,
-                     c->nlMu, c->gpart);
+  const double4 *UB = c->nlU;
+  if (Yb != Ya) {
+    nl_grad_k<DIM, KT>(c, a, Yb, c->nlUB, nullptr);
+    UB = c->nlUB;
+  }
+  if (c->diff_op == 3) NL_LAUNCH(k_nl_nu<DIM COMMA KT COMMA 3, a, lam, c->nlF, c->nlNu);
+  else NL_LAUNCH(k_nl_nu<DIM COMMA KT COMMA 4, a, lam, c->nlF, c->nlNu);
+  hipLaunchKernelGGL(k_nl_mu, dim3(G), dim3(kBlock), 0, c->stream, a, c->nlNu, c->nlU, UB, c->nlMu, c->gpart);
   hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)G, 1.0, 0.0, c->gkdev);
   hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)G, 0.0, 1.0, c->gkdev + 6);
-  if (c->diff_op == 4)
-    hipLaunchKernelGGL((k_nl_gT<DIM, KT, 2>), dim3(G), dim3(kBlock), 0, c->stream, a, c->nlMu, c->nlF, out, 0);
-  else
-    hipLaunchKernelGGL((k_nl_gT<DIM, KT, 1>), dim3(G), dim3(kBlock), 0, c->stream, a, c->nlMu, c->nlF, out, 0);
+  if (c->diff_op == 4) NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 2, a, c->nlMu, c->nlF, none, o, out);
+  else NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 1, a, c->nlMu, c->nlF, none, o, out);
 }
+#undef NL_LAUNCH
+#undef COMMA
 #define NL_DISPATCH(FN, ...)                                                                       \
   do {                                                                                            \
     const int d_ = c->diff_phys.dim, k_ = c->kt;                                                  \
@@ -2305,7 +2312,6 @@ int sph_diff_prepare(sph_ctx *c, const double state[49]) {
     RCHK(dalloc(&c->nlD, c->npad));
     RCHK(dalloc(&c->nlDD, c->npad));
     RCHK(dalloc(&c->nlR, c->npad));
-    RCHK(dalloc(&c->nlSD, c->npad));
     const double K0[6] = {0, 0, 0, 0, 0, 0};
     DiffOpArgs a = diff_args(c, K0);
     NL_DISPATCH(nl_grad_k, c, a, nullptr, nullptr, c->nlF);  // F_s = sum_b m_b nw(r_sb, h_s)
@@ -2326,11 +2332,11 @@ int sph_diff_apply(sph_ctx *c, const double K[6], const double *d_T, double *d_o
   if (c->diff_op != 0) {
     const double K0[6] = {0, 0, 0, 0, 0, 0};
     DiffOpArgs a = diff_args(c, K ? K : K0);
-    NL_DISPATCH(nl_apply_k, c, a, dv(c, 0), dv(c, 1));
+    NL_DISPATCH(nl_apply_k, c, a, dv(c, 0), d_out);
   } else {
     diff_apply(c, K, dv(c, 0), dv(c, 1));
+    hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 1), c->orig[c->cur], n, d_out);
   }
-  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 1), c->orig[c->cur], n, d_out);
   HIPCHK(hipStreamSynchronize(c->stream));
   return SPH_OK;
 }
@@ -2346,12 +2352,13 @@ int sph_diff_apply_adjoint(sph_ctx *c, const double K[6], const double *d_lam, c
   const int64_t *o = c->orig[c->cur];
   hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_lam, o, n, dv(c, 0));
   hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_Ya, o, n, dv(c, 1));
-  if (d_Yb) hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_Yb, o, n, dv(c, 2));
+  const bool yb = d_Yb && d_Yb != d_Ya;
+  if (yb) hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_Yb, o, n, dv(c, 2));
   HIPCHK(hipMemsetAsync(c->gkdev, 0, sizeof(double) * 12, c->stream));
   if (c->diff_op != 0) {
     const double K0[6] = {0, 0, 0, 0, 0, 0};
     DiffOpArgs a = diff_args(c, K ? K : K0);
-    NL_DISPATCH(nl_adjoint_k, c, a, dv(c, 0), dv(c, 1), c->diff_op == 5 ? nullptr : dv(c, 2), dv(c, 3));
+    NL_DISPATCH(nl_adjoint_k, c, a, dv(c, 0), dv(c, 1), dv(c, yb ? 2 : 1), dv(c, 3), d_out);
   } else {
     ensure_weights(c, K);
     AdjStage a = adj_args(c);  // A^T lam alone
@@ -2359,16 +2366,16 @@ int sph_diff_apply_adjoint(sph_ctx *c, const double K[6], const double *d_lam, c
     hipLaunchKernelGGL(k_adj_stage, dim3(G), dim3(kBlock), 0, c->stream, a);
     c->rec_pend = c->rec_packed = 0;
     c->coef_set = false;
-    for (int k = 0; k < 2; k++) {
+    for (int k = 0; k < (yb ? 2 : 1); k++) {
       adj_record(c, dv(c, 0), dv(c, 1 + k), nullptr, 1.0, 0.0);
       diff_gcontract(c, K, c->gkdev + 6 * k);
     }
+    hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 3), o, n, d_out);
   }
-  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 3), o, n, d_out);
   double g12[12];
   HIPCHK(hipMemcpyAsync(g12, c->gkdev, sizeof(double) * 12, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
-  for (int k = 0; k < 6; k++) { gA[k] = g12[k]; gB[k] = g12[6 + k]; }
+  for (int k = 0; k < 6; k++) { gA[k] = g12[k]; gB[k] = yb || c->diff_op != 0 ? g12[6 + k] : g12[k]; }
   return SPH_OK;
 }
 

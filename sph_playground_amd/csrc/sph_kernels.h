@@ -322,6 +322,7 @@ struct DiffOpArgs {
   double K[6];         // xx, yy, zz, xy, xz, yz
   double wcv, fwc;
   int ddw, n, npad;
+  const double *rho;   // den alone (sorted)
   const double *kap;   // opacity of the frozen state (sorted), flux-limited diffusion
 };
 
