@@ -17,6 +17,7 @@
 #include <cstring>
 #include <mutex>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/sph_hip.h"
@@ -81,6 +82,8 @@ __global__ void k_diff_coef(const uint32_t *, const int *, const double2 *, doub
 __global__ void k_gk_accum(const double *, int, double, double, double *);
 __global__ void k_zrho(int, const double *, const double4 *, double *);
 __global__ void k_diff_pack(int, const double4 *, const double4 *, double4 *, double *, double *);
+__global__ void k_rev_fill(const uint8_t *, const uint32_t *, const int *, int, int, int, int *, uint32_t *);
+__global__ void k_rev_sort(int, int, const int *, uint32_t *);
 __global__ void k_rev_count(const uint8_t *, const uint32_t *, const int *, int, int, int *);
 __global__ void k_rev_chunk(const int *, const uint32_t *, int, int, int *, uint32_t *);
 __global__ void k_pair_enum(const uint8_t *, const uint32_t *, const int *, int, int, const int *, uint32_t *,
@@ -266,7 +269,6 @@ struct sph_ctx {
   // differentiable diffusion (sph_diff_*)
   bool diff_ready = false;
   Phys diff_phys{};
-  int *roff = nullptr, *rtmp = nullptr;
   uint32_t *rent = nullptr;      // reverse entries (owner, image), list layout, rcnt per particle
   double4 *dpxh = nullptr;       // x, y, z, 1 / h of the frozen geometry
   double *dirho = nullptr;       // 1 / rho of the frozen geometry
@@ -286,10 +288,7 @@ struct sph_ctx {
   bool w_valid = false;          // dW/dR hold the weights of w_K
   double w_K[6] = {0, 0, 0, 0, 0, 0};
   double *gkdev = nullptr;       // 12 tensor-gradient accumulators
-  void *scan_tmp = nullptr;
-  size_t scan_tmp_bytes = 0;
-  double *dvec = nullptr;        // work vectors, diff_nvec x npad
-  int diff_nvec = 0;
+  double *dvec = nullptr;        // work vectors of npad
   double *gpart = nullptr;       // 12 partial sums per block
   double *ckpt = nullptr;        // checkpoints of T, (nsteps / every + 1) x npad
   int64_t ckpt_cap = 0;
@@ -300,6 +299,10 @@ struct sph_ctx {
   int diff_op = 0;
   double4 *nlF = nullptr, *nlU = nullptr, *nlUB = nullptr, *nlNu = nullptr, *nlMu = nullptr;
   double *nlD = nullptr, *nlDD = nullptr, *nlR = nullptr;
+
+  // capacity in bytes of the buffers sph_diff_prepare keeps between calls, by
+  // the address of their pointer
+  std::unordered_map<void *, size_t> kept;
 
   Fields fields() const {
     Fields F;
@@ -333,6 +336,20 @@ static int dev_alloc(void **p, size_t bytes) {
 
 template <typename T>
 static int dalloc(T **p, size_t count) { return dev_alloc((void **)p, count * sizeof(T)); }
+
+// A buffer of the prepared operator, kept from one preparation to the next
+// and made anew only to grow (its contents are then gone): allocating and
+// freeing them took 1 ms of a preparation of 40^3 particles.
+template <typename T>
+static int keep(sph_ctx *c, T **p, size_t count) {
+  size_t &cap = c->kept[(void *)p];
+  const size_t bytes = std::max<size_t>(count * sizeof(T), 16);
+  if (*p && bytes <= cap) return SPH_OK;
+  cap = 0;
+  RCHK(dev_alloc((void **)p, bytes));
+  cap = bytes;
+  return SPH_OK;
+}
 
 // --------------------------------------------------------------- kernel base
 static double knorm(int kt, int dim) {
@@ -1585,7 +1602,7 @@ int sph_ctx_destroy(sph_ctx *c) {
                   c->sort_tmp, c->cstart, c->pm, c->st[0], c->st[1], c->tr[0], c->tr[1], c->s1[0], c->s1[1], c->pfix, c->s2, c->pd, c->trd,
                   c->h0, c->eps, c->pf,
                   c->real, c->nb, c->cnt, c->q[0], c->q[1], c->q[2], c->q[3], c->q[4], c->energy_part,
-                  c->d_red, c->d_int, c->d_stripes, c->d_staging, c->roff, c->rtmp, c->rent, c->scan_tmp,
+                  c->d_red, c->d_int, c->d_stripes, c->d_staging, c->rent,
                   c->dvec, c->gpart, c->ckpt, c->rcnt, c->dpxh, c->dirho, c->dW, c->ddW, c->dR, c->dS, c->dZ, c->drho, c->dRec,
                   c->gkdev, c->nlF, c->nlU, c->nlUB, c->nlNu, c->nlMu, c->nlD, c->nlDD, c->nlR,
                   c->ext_count, c->ecs, c->erec, c->ext_tmp};
@@ -2125,13 +2142,7 @@ static void diff_gcontract(sph_ctx *c, const double K[6], double *gk) {
   c->coef_set = false;
 }
 
-static int ensure_dvec(sph_ctx *c, int nvec) {
-  if (nvec <= c->diff_nvec) return SPH_OK;
-  RCHK(dalloc(&c->dvec, (size_t)nvec * c->npad));
-  HIPCHK(hipMemset(c->dvec, 0, sizeof(double) * nvec * c->npad));
-  c->diff_nvec = nvec;
-  return SPH_OK;
-}
+static int ensure_dvec(sph_ctx *c, int nvec) { return keep(c, &c->dvec, (size_t)nvec * c->npad); }
 static double *dv(sph_ctx *c, int k) { return c->dvec + (size_t)k * c->npad; }
 
 // Work vectors of the super-steps: rotating stage states, the first stage's
@@ -2190,6 +2201,72 @@ static void sts_backward_step(sph_ctx *c, int s, double dt, double *const *Y, in
   }
 }
 
+// Reverse lists of more than kRevSort entries: stable radix sort of the
+// owner-major pairs on the neighbour index, then into the list layout.
+static int reverse_lists_radix(sph_ctx *c, int64_t npairs) {
+  const int n = (int)c->n, npad = (int)c->npad;
+  const unsigned G = grid_for(n);
+  int *foff = nullptr, *roff = nullptr;
+  uint32_t *keys = nullptr, *keys2 = nullptr, *vals = nullptr, *flat = nullptr;
+  void *tmp = nullptr;
+  auto run = [&]() -> int {
+    const size_t np = (size_t)std::max<int64_t>(npairs, 1);
+    RCHK(dalloc(&foff, c->npad + 1));
+    RCHK(dalloc(&roff, c->npad + 1));
+    RCHK(dalloc(&keys, np));
+    RCHK(dalloc(&keys2, np));
+    RCHK(dalloc(&vals, np));
+    RCHK(dalloc(&flat, np));
+    size_t b1 = 0, b2 = 0, b3 = 0;
+    int bits = 1;
+    while (bits < 32 && ((int64_t)1 << bits) < (int64_t)n) bits++;
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, b1, c->rcnt, roff, n + 1, c->stream));
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, b2, c->cnt, foff, n, c->stream));
+    HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, b3, keys, keys2, vals, flat, (int)npairs, 0, bits, c->stream));
+    size_t bytes = std::max(b1, std::max(b2, b3));
+    RCHK(dev_alloc(&tmp, bytes));
+    // how often each particle is someone's neighbour, and where its segment starts
+    HIPCHK(hipMemsetAsync(c->rcnt, 0, sizeof(int) * (c->npad + 1), c->stream));
+    hipLaunchKernelGGL(k_rev_count, dim3(G), dim3(kBlock), 0, c->stream, c->real, c->nb, c->cnt, n, npad, c->rcnt);
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, c->rcnt, roff, n + 1, c->stream));
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp, bytes, c->cnt, foff, n, c->stream));
+    hipLaunchKernelGGL(k_pair_enum, dim3(G), dim3(kBlock), 0, c->stream, c->real, c->nb, c->cnt, n, npad, foff, keys,
+                       vals);
+    if (npairs > 0)
+      HIPCHK(hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys, keys2, vals, flat, (int)npairs, 0, bits, c->stream));
+    hipLaunchKernelGGL(k_rev_chunk, dim3(G), dim3(kBlock), 0, c->stream, roff, flat, n, npad, c->rcnt, c->rent);
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return SPH_OK;
+  };
+  const int rc = run();
+  void *t[] = {foff, roff, keys, keys2, vals, flat, tmp};
+  for (void *q : t)
+    if (q) (void)hipFree(q);
+  return rc;
+}
+
+// The reverse lists (rent, rcnt) of the last search, capacity rcap.
+static int reverse_lists(sph_ctx *c, int64_t npairs) {
+  const int n = (int)c->n, npad = (int)c->npad;
+  // room for an eighth more than the longest forward list, or what is there
+  int cap = (c->last_maxcnt + c->last_maxcnt / 8 + 8) / 8 * 8;
+  for (;;) {
+    RCHK(keep(c, &c->rent, (size_t)npad * cap));
+    HIPCHK(hipMemsetAsync(c->rcnt, 0, sizeof(int) * ((size_t)npad + 1), c->stream));
+    hipLaunchKernelGGL(k_rev_fill, dim3(grid_for(c->n * 8)), dim3(kBlock), 0, c->stream, c->real, c->nb, c->cnt, n,
+                       npad, cap, c->rcnt, c->rent);
+    HIPCHK(hipMemcpyAsync(c->h_int, c->rcnt + npad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(wait_stream(c));
+    const int longest = c->h_int[0];
+    c->rcap = std::max(8, (longest + 7) / 8 * 8);
+    if (longest <= cap) break;
+    cap = c->rcap;
+  }
+  if (c->rcap > kRevSort) return reverse_lists_radix(c, npairs);
+  hipLaunchKernelGGL(k_rev_sort, dim3((unsigned)((n + 3) / 4)), dim3(kBlock), 0, c->stream, n, npad, c->rcnt, c->rent);
+  return SPH_OK;
+}
+
 extern "C" {
 
 int sph_diff_prepare(sph_ctx *c, const double state[49]) {
@@ -2222,96 +2299,37 @@ int sph_diff_prepare(sph_ctx *c, const double state[49]) {
   unsigned G = grid_for(n);
   const int64_t npairs = c->stats.n_pairs;
   if (npairs >= ((int64_t)1 << 31)) return SPH_ERR_UNSUPPORTED;  // 32-bit pair counts
-  RCHK(dalloc(&c->roff, c->npad + 1));
-  RCHK(dalloc(&c->rtmp, c->npad + 1));
-  RCHK(dalloc(&c->rcnt, c->npad));
-  RCHK(dalloc(&c->dpxh, c->npad));
-  RCHK(dalloc(&c->dirho, c->npad));
-  if (op == 0) RCHK(dalloc(&c->dW, (size_t)c->npad * c->nb_cap));
-  RCHK(dalloc(&c->ddW, c->npad));
-  RCHK(dalloc(&c->dZ, c->npad));
-  RCHK(dalloc(&c->drho, c->npad));
-  if (op == 0) RCHK(dalloc(&c->dRec, (size_t)c->npad * kRecs));
+  // rcnt: the reverse-list lengths, then the longest of them
+  RCHK(keep(c, &c->rcnt, c->npad + 1));
+  RCHK(keep(c, &c->dpxh, c->npad));
+  RCHK(keep(c, &c->dirho, c->npad));
+  if (op == 0) RCHK(keep(c, &c->dW, (size_t)c->npad * c->nb_cap));
+  RCHK(keep(c, &c->ddW, c->npad));
+  RCHK(keep(c, &c->dZ, c->npad));
+  RCHK(keep(c, &c->drho, c->npad));
+  if (op == 0) RCHK(keep(c, &c->dRec, (size_t)c->npad * kRecs));
   c->rec_pend = c->rec_packed = 0;
   c->coef_set = false;
-  RCHK(dalloc(&c->gkdev, 12));
+  RCHK(keep(c, &c->gkdev, 12));
+  RCHK(keep(c, &c->gpart, (size_t)G * 12));
   c->w_valid = false;
   hipLaunchKernelGGL(k_diff_pack, dim3(G), dim3(kBlock), 0, c->stream, n, c->pm, (const double4 *)c->q[0], c->dpxh,
                      c->drho, c->dirho);
-  // reverse lists: stable radix sort of the owner-major pairs on the neighbour
-  // index, then into the list layout (capacity = longest reverse list)
-  int *foff = nullptr;
-  uint32_t *keys = nullptr, *keys2 = nullptr, *vals = nullptr, *flat = nullptr;
-  auto release = [&]() {
-    void *t[] = {foff, keys, keys2, vals, flat};
-    for (void *q : t)
-      if (q) (void)hipFree(q);
-  };
-  auto tmp_bytes = [&](size_t need) -> int {
-    if (need > c->scan_tmp_bytes) {
-      RCHK(dev_alloc(&c->scan_tmp, need));
-      c->scan_tmp_bytes = need;
-    }
-    return SPH_OK;
-  };
-  int rc = SPH_OK;
-  do {
-    const size_t np = (size_t)std::max<int64_t>(npairs, 1);
-    if ((rc = dalloc(&foff, c->npad + 1)) || (rc = dalloc(&keys, np)) || (rc = dalloc(&keys2, np)) ||
-        (rc = dalloc(&vals, np)) || (rc = dalloc(&flat, np)))
-      break;
-    // reverse segment offsets: how often each particle is someone's neighbour
-    HIPCHK(hipMemsetAsync(c->rtmp, 0, sizeof(int) * (n + 1), c->stream));
-    hipLaunchKernelGGL(k_rev_count, dim3(G), dim3(kBlock), 0, c->stream, c->real, c->nb, c->cnt, n, (int)c->npad,
-                       c->rtmp);
-    size_t b1 = 0, b2 = 0, b3 = 0;
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, b1, c->rtmp, c->roff, n + 1, c->stream));
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, b2, c->cnt, foff, n, c->stream));
-    HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, b3, keys, keys2, vals, flat, (int)npairs, 0, 32, c->stream));
-    if ((rc = tmp_bytes(std::max(b1, std::max(b2, b3))))) break;
-    size_t bytes = c->scan_tmp_bytes;
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(c->scan_tmp, bytes, c->rtmp, c->roff, n + 1, c->stream));
-    // the longest reverse list sets the capacity of the list-layout arrays
-    std::vector<int> hoff(n + 1);
-    HIPCHK(hipMemcpyAsync(hoff.data(), c->roff, sizeof(int) * (n + 1), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    int rmax = 0;
-    for (int k = 0; k < n; k++) rmax = std::max(rmax, hoff[k + 1] - hoff[k]);
-    c->rcap = std::max(8, (rmax + 7) / 8 * 8);
+  RCHK(reverse_lists(c, npairs));
+  if (op == 0) {
     const size_t rslots = (size_t)c->npad * c->rcap;
-    if ((rc = dalloc(&c->rent, rslots))) break;
-    if (op == 0) {
-      if ((rc = dalloc(&c->dR, rslots)) || (rc = dalloc(&c->dS, rslots))) break;
-    }
-    // owner-major enumeration of the pairs, stable sort on the neighbour index
-    bytes = c->scan_tmp_bytes;
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(c->scan_tmp, bytes, c->cnt, foff, n, c->stream));
-    hipLaunchKernelGGL(k_pair_enum, dim3(G), dim3(kBlock), 0, c->stream, c->real, c->nb, c->cnt, n, (int)c->npad,
-                       foff, keys, vals);
-    int bits = 1;
-    while (bits < 32 && ((int64_t)1 << bits) < (int64_t)n) bits++;
-    bytes = c->scan_tmp_bytes;
-    if (npairs > 0)
-      HIPCHK(hipcub::DeviceRadixSort::SortPairs(c->scan_tmp, bytes, keys, keys2, vals, flat, (int)npairs, 0, bits,
-                                                c->stream));
-    hipLaunchKernelGGL(k_rev_chunk, dim3(G), dim3(kBlock), 0, c->stream, c->roff, flat, n, (int)c->npad, c->rcnt,
-                       c->rent);
-    HIPCHK(hipStreamSynchronize(c->stream));
-  } while (false);
-  release();
-  RCHK(rc);
-  if (c->gpart) (void)hipFree(c->gpart);
-  c->gpart = nullptr;
-  RCHK(dalloc(&c->gpart, (size_t)G * 12));
+    RCHK(keep(c, &c->dR, rslots));
+    RCHK(keep(c, &c->dS, rslots));
+  }
   if (op != 0) {
-    RCHK(dalloc(&c->nlF, c->npad));
-    RCHK(dalloc(&c->nlU, c->npad));
-    RCHK(dalloc(&c->nlUB, c->npad));
-    RCHK(dalloc(&c->nlNu, c->npad));
-    RCHK(dalloc(&c->nlMu, c->npad));
-    RCHK(dalloc(&c->nlD, c->npad));
-    RCHK(dalloc(&c->nlDD, c->npad));
-    RCHK(dalloc(&c->nlR, c->npad));
+    RCHK(keep(c, &c->nlF, c->npad));
+    RCHK(keep(c, &c->nlU, c->npad));
+    RCHK(keep(c, &c->nlUB, c->npad));
+    RCHK(keep(c, &c->nlNu, c->npad));
+    RCHK(keep(c, &c->nlMu, c->npad));
+    RCHK(keep(c, &c->nlD, c->npad));
+    RCHK(keep(c, &c->nlDD, c->npad));
+    RCHK(keep(c, &c->nlR, c->npad));
     const double K0[6] = {0, 0, 0, 0, 0, 0};
     DiffOpArgs a = diff_args(c, K0);
     NL_DISPATCH(nl_grad_k, c, a, nullptr, nullptr, c->nlF);  // F_s = sum_b m_b nw(r_sb, h_s)

@@ -299,6 +299,8 @@ struct AdjStage {
   double mu, mh, nu1, c0, gh;
   int a0_add, last, n, npad, rev;
 };
+// longest reverse list k_rev_sort orders
+constexpr int kRevSort = 512;
 // Adjoint stages whose part of the tensor gradient one pass over the pair
 // coefficients takes: stage q's L and Zt = (wa Ya + wb Yb) rho (Yb may be null)
 // become its record.
