@@ -27,14 +27,17 @@ using namespace sph;
 
 namespace sph {
 // kernels (sph_kernels.hip)
-__global__ void k_wrap_reduce(Fields, const int64_t *, int, int64_t, Box, int, long long *, int *);
-__global__ void k_keys(Fields, int, Grid, uint32_t *, uint32_t *, int *);
+__global__ void k_wrap_reduce(Fields, const int64_t *, int, int64_t, Box, int, long long *);
+__global__ void k_keys(Fields, int, Grid, uint32_t *, uint32_t *, int *, int *, long long *);
+__global__ void k_cell_list(const uint32_t *, const uint32_t *, const int *, int, uint32_t *);
+__global__ void k_move(Fields, Fields, const double *, double *, int, int, const uint32_t *, const int *, const uint32_t *,
+                       int *, const int64_t *, int64_t *, int);
 __global__ void k_check_sorted(const uint32_t *, int, int *);
 __global__ void k_reorder(Fields, Fields, const uint32_t *, const int64_t *, int64_t *, int, int);
 __global__ void k_cell_start(const uint32_t *, int, uint32_t, int *);
 __global__ void k_prep(Fields, const int64_t *, int, int64_t, Box, Grid, int, double4 *, double *, float4 *,
                        uint8_t *, double4 *, double *, uint3 *, FixFrame, float2 *, double *, long long *,
-                       long long *, int, long long *, int, int);
+                       long long *, int, long long *, int, long long *, int);
 template <int DIM, bool EXT>
 __global__ void k_neigh(NeighArgs, const double4 *__restrict__, const float4 *__restrict__, uint32_t *__restrict__,
                         int *__restrict__);
@@ -52,8 +55,8 @@ __global__ void k_loop2(Loop2Args<V4>);
 __global__ void k_aos_to_soa(const double *, int64_t, int, Fields, int64_t *);
 __global__ void k_step_close(const double *, int, const int *, const long long *, long long *);
 __global__ void k_soa_to_aos(Fields, const int64_t *, int, double *, int64_t);
-__global__ void k_ext_count(Grid, ExtGrid, const int *, int, int *);
-__global__ void k_ext_fill(Grid, ExtGrid, const int *, const int *, const float4 *, int, float4 *);
+__global__ void k_ext_count(Grid, ExtGrid, const int *, int, int *, long long *);
+__global__ void k_ext_fill(Grid, ExtGrid, const int *, int *, const float4 *, int, int, float4 *, int *, long long *);
 __global__ void k_neigh_export(const uint32_t *, const int *, const int64_t *, const uint8_t *, int, int,
                                const int64_t *, int32_t *, int8_t *, int64_t);
 __global__ void k_set_i64(int64_t *, int64_t);
@@ -61,8 +64,8 @@ __global__ void k_zero_ll(long long *, int);
 __global__ void k_prerun_check(Fields, int, int *);
 __global__ void k_counts_by_orig(const int *, const int64_t *, const uint8_t *, int, int64_t *);
 __global__ void k_find_orig(const int64_t *, int, int64_t, int *);
-__global__ void k_predict(Fields, int, double, int, double *, int);
-__global__ void k_correct(Fields, int, double, int, const double *, int);
+__global__ void k_predict(Fields, int, DtArgs, double *, int);
+__global__ void k_correct(Fields, int, const double *, const double *, int, const int *, const int *);
 __global__ void k_rad_exchange(Fields, int, double, double, double, double, int *);
 __global__ void k_dt_reduce(Fields, const uint8_t *, int, long long *);
 __global__ void k_gravity(Fields, const uint8_t *, int, int);
@@ -123,8 +126,17 @@ constexpr int kSearchLL = 0;
 constexpr int kCloseRec = 2 * kStripes;
 constexpr int kHmaxLL = 4 * kStripes;
 constexpr int kErrLL = 5 * kStripes;      // ints: 0 search, 1 loop 1, 2 loop 2
-constexpr int kZeroLL = kErrLL + 4;
+constexpr int kExtLL = kErrLL + 4;        // where the extended grid was built: its records
+constexpr int kFullLL = kErrLL + 8;       // and its fullest cell (kFullStripes)
+constexpr int kZeroLL = kFullLL + kFullStripes;
 constexpr int kFlagSlots = 6 * kStripes;
+constexpr int kDtLL = 7 * kStripes;       // the leapfrog pass's time step (not cleared)
+constexpr int kDtBlocks = 256;            // k_dt_reduce's blocks at most
+// particles of the fullest cell up to which a step orders them by counting
+// (k_move): a particle looks through its whole cell there, which stays a few
+// percent of the pass at 256, and is then still a small part of what the
+// search reads for it; beyond, one cell's atomics also follow one another
+constexpr long long kCountedCell = 256;
 constexpr int kStepLL = 9 * kStripes;     // the counters before the sweep regions
 enum { kErrSearch = 0, kErrLoop1 = 1, kErrLoop2 = 2 };
 constexpr int kMaxLanes = 8;  // lanes per particle of a pair loop, at most
@@ -194,7 +206,14 @@ struct sph_ctx {
   void *sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
   int *cstart = nullptr;   // first sorted index of every cell key
+  int *ccount = nullptr;   // particles per cell key while they are counted, else zero
   int64_t ncell_cap = 0;
+  long long fullest = 0;   // particles in the fullest search cell last seen (0: not known)
+  bool red_ready = false;  // d_red holds k_wrap_reduce's start values
+  bool ext_exact = false;  // the next extended grid waits for its size
+  bool ext_built = false;  // this step built one: its counts come with the search's
+  bool correct = false;    // this step's tail ends with the leapfrog corrector
+  long long *d_dtpart = nullptr;  // k_dt_reduce's block partials
   double4 *pm = nullptr, *st[2] = {nullptr, nullptr};
   double *tr[2] = {nullptr, nullptr};  // T den of the loop-1 sweep state st[k]
   // mixed path: position records (31-bit fractions, `ff` their frame),
@@ -454,7 +473,10 @@ static int ensure_nb(sph_ctx *c, int cap) {
 static int ensure_cells(sph_ctx *c, int64_t nkeys) {
   if (nkeys + 1 <= c->ncell_cap) return SPH_OK;
   int64_t cap = std::max<int64_t>(nkeys + 1, 1024);
+  c->ncell_cap = 0;
   RCHK(dalloc(&c->cstart, cap));
+  RCHK(dalloc(&c->ccount, cap));
+  HIPCHK(hipMemsetAsync(c->ccount, 0, sizeof(int) * cap, c->stream));
   c->ncell_cap = cap;
   return SPH_OK;
 }
@@ -534,9 +556,6 @@ static long long stripe_min(const long long *h, int v) {
 #endif
 static const int kNeighRS = SPH_NEIGH_RS;
 
-// d_int slot k_wrap_reduce sets when it moved a particle back into the box
-constexpr int kWrapFlag = 4;
-
 // The mixed path's position-record frame: an imaged axis maps its box length
 // L onto 2^(31-k), k the least with 2^k L beyond any listed separation along
 // it (the stencil's reach), so wrap-around differences of the fractions stay
@@ -607,6 +626,18 @@ static int copied_err(const long long *copy, int base, int word) {
 }
 
 static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
+  bool ext_short = false;
+  if (c->ext_built) {
+    c->ext_built = false;
+    c->fullest = *std::max_element(ll + kFullLL, ll + kFullLL + kFullStripes);
+    c->ext_total = ll[kExtLL];
+    c->stats.ext_records = c->ext_total;
+    ext_short = (size_t)c->ext_total + 8 > c->ext_rec_cap;
+    if (ext_short) {  // records were left out: build it again with room
+      c->ext_version = 0;
+      c->ext_exact = true;
+    }
+  }
   if (c->flags_pending) {  // k_prep's v / B flags of this step
     c->step_flags = 0;
     for (int k = 0; k < kStripes; k++) c->step_flags |= ll[kFlagSlots + k];
@@ -619,6 +650,7 @@ static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
   c->stats.ms_k_neigh = elapsed(c, c->ev[4], c->ev[7]);
   if (bits & EB_TRUNC) return SPH_ERR_NEIGH_TRUNCATED;
   if (!(bits & EB_OVERFLOW)) return SPH_OK;
+  if (ext_short) return kRedoNeigh;  // the lists' lengths are not the real ones
   RCHK(ensure_nb(c, maxcnt + 8));
   return kRedoNeigh;
 }
@@ -637,6 +669,21 @@ static int take_neighbours(sph_ctx *c) {
   return finish_neighbours(c, ll, copied_err(ll, 0, kErrSearch));
 }
 
+// out = exclusive prefix sums of count ints.
+static int prefix_sum(sph_ctx *c, const int *in, int *out, int count) {
+  size_t tb = 0;
+  HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, in, out, count, c->stream));
+  if (tb > c->ext_tmp_bytes) {
+    if (c->ext_tmp) { (void)hipFree(c->ext_tmp); c->ext_tmp = nullptr; }
+    c->ext_tmp_bytes = 0;
+    RCHK(dev_alloc(&c->ext_tmp, tb));
+    c->ext_tmp_bytes = tb;
+  }
+  tb = c->ext_tmp_bytes;
+  HIPCHK(hipcub::DeviceScan::ExclusiveSum(c->ext_tmp, tb, in, out, count, c->stream));
+  return SPH_OK;
+}
+
 // defer: launch the search without waiting for its read-back (a later
 // copy_record brings it); the lists then hold at most nb_cap entries per
 // particle, so what runs on them before take_neighbours stays in bounds.
@@ -646,6 +693,7 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   Fields F = c->fields();
   unsigned G = grid_for(n);
   const long long BIG = 0x7FFFFFFFFFFFFFFFLL, SMALL = -0x7FFFFFFFFFFFFFFFLL - 1;
+  c->ext_built = false;
   // 1. wrap escaped real particles, bounding box, max h (striped reductions).
   //    Positions unchanged since the last pass (so none escaped) and h last
   //    set by the previous step (whose k_post1 reduced h_max): nothing to do.
@@ -654,19 +702,21 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
     for (int a = 0; a < 3; a++) { lo[a] = c->last_lo[a]; hi[a] = c->last_hi[a]; }
     hmax = c->next_hmax;
   } else {
-    long long *init = c->h_ll;
-    for (int v = 0; v < 7; v++)
-      for (int k = 0; k < kStripes; k++) init[v * kStripes + k] = v < 3 ? BIG : SMALL;
-    HIPCHK(hipMemcpyAsync(c->d_red, init, sizeof(long long) * 7 * kStripes, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemsetAsync(c->d_int, 0, sizeof(int) * 8, c->stream));
+    if (!c->red_ready) {  // else the last step's k_prep set the start values
+      long long *init = c->h_ll;
+      for (int k = 0; k < kRedLL; k++) init[k] = k < 3 * kStripes ? BIG : (k < 7 * kStripes ? SMALL : 0);
+      HIPCHK(hipMemcpyAsync(c->d_red, init, sizeof(long long) * kRedLL, hipMemcpyHostToDevice, c->stream));
+      HIPCHK(hipMemsetAsync(c->d_int, 0, sizeof(int) * 8, c->stream));
+    }
+    c->red_ready = false;
     // at most 1024 blocks (four per CU), each striding over the particles
     hipLaunchKernelGGL(k_wrap_reduce, dim3(std::min(G, 1024u)), dim3(kBlock), 0, c->stream, F, c->orig[c->cur], n,
-                       c->n_real, c->box, dim, c->d_red, c->d_int);
+                       c->n_real, c->box, dim, c->d_red);
     long long *red = c->h_ll + 512;
-    HIPCHK(hipMemcpyAsync(red, c->d_red, sizeof(long long) * 7 * kStripes, hipMemcpyDeviceToHost, c->stream));
-    RCHK(read_ints(c, 0, kWrapFlag + 1));
-    if (c->h_int[0] & EB_OUTSIDE) return SPH_ERR_UNSUPPORTED;
-    if (c->h_int[kWrapFlag]) c->pos_version++;  // a particle was wrapped back into the box
+    HIPCHK(hipMemcpyAsync(red, c->d_red, sizeof(long long) * kRedLL, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(wait_stream(c));
+    if (red[7 * kStripes] & EB_OUTSIDE) return SPH_ERR_UNSUPPORTED;
+    if (red[7 * kStripes + 1]) c->pos_version++;  // a particle was wrapped back into the box
     for (int a = 0; a < 3; a++) { lo[a] = ord2d(stripe_min(red, a)); hi[a] = ord2d(stripe_max(red, 3 + a)); }
     hmax = c->n_real > 0 ? ord2d(stripe_max(red, 6)) : 0.0;
     for (int a = 0; a < 3; a++) { c->last_lo[a] = lo[a]; c->last_hi[a] = hi[a]; }
@@ -750,19 +800,40 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   const bool keys_kept = c->keys_version == c->pos_version && c->keys_n == n && c->keys_nkeys == nkeys &&
                          same_grid(g, c->keys_grid);
   if (!keys_kept) {
-    // k_keys clears the order check's flag (no fill of its own)
-    hipLaunchKernelGGL(k_keys, dim3(G), dim3(kBlock), 0, c->stream, F, n, g, c->keys, c->vals, c->d_int + 2);
-    hipLaunchKernelGGL(k_check_sorted, dim3(std::min(G, 256u)), dim3(kBlock), 0, c->stream, c->keys, n,
-                       c->d_int + 2);
-    RCHK(read_ints(c, 2, 1));
-    if (c->h_int[2]) {
+    // Particles that moved since the keys were made are ordered by counting,
+    // without asking the host whether their order broke (it nearly always
+    // did), unless the last fullest cell was crowded; others are checked first
+    // and sorted if they must be.
+    const bool counted = c->keys_version != c->pos_version && c->fullest > 0 && c->fullest <= kCountedCell &&
+                         nkeys < INT32_MAX;
+    hipLaunchKernelGGL(k_keys, dim3(G), dim3(kBlock), 0, c->stream, F, n, g, c->keys, c->vals, c->d_int + 2,
+                       counted ? c->ccount : nullptr, c->d_stripes + kFlagSlots);
+    const int nxt = 1 - c->cur;
+    Fields src = c->fields();
+    Fields dst;
+    for (int f = 0; f < F_TOTAL; f++) dst.f[f] = c->fbuf[nxt] + (size_t)f * c->npad;
+    const double *aux_src = c->aux(0);
+    double *aux_dst = c->fbuf[nxt] + (size_t)F_TOTAL * c->npad;
+    bool moved = counted;
+    if (counted) {
+      const int rs = prefix_sum(c, c->ccount, c->cstart, (int)nkeys + 1);
+      if (rs != SPH_OK) {  // no room for the scan: the counts are not left behind
+        HIPCHK(hipMemsetAsync(c->ccount, 0, sizeof(int) * c->ncell_cap, c->stream));
+        return rs;
+      }
+      hipLaunchKernelGGL(k_cell_list, dim3(G), dim3(kBlock), 0, c->stream, c->keys, c->vals, c->cstart, n, c->vals2);
+      hipLaunchKernelGGL(k_move, dim3(G), dim3(kBlock), 0, c->stream, src, dst, aux_src, aux_dst, c->naux,
+                         (int)c->npad, c->keys, c->cstart, c->vals2, c->ccount, c->orig[c->cur], c->orig[nxt], n);
+    } else {
+      hipLaunchKernelGGL(k_check_sorted, dim3(std::min(G, 256u)), dim3(kBlock), 0, c->stream, c->keys, n,
+                         c->d_int + 2);
+      RCHK(read_ints(c, 2, 1));
+      moved = c->h_int[2] != 0;
+    }
+    if (moved && !counted) {
       size_t bytes = c->sort_tmp_bytes;
       HIPCHK(hipcub::DeviceRadixSort::SortPairs(c->sort_tmp, bytes, c->keys, c->keys2, c->vals, c->vals2, n, 0,
                                                 key_bits, c->stream));
-      int nxt = 1 - c->cur;
-      Fields src = c->fields();
-      Fields dst;
-      for (int f = 0; f < F_TOTAL; f++) dst.f[f] = c->fbuf[nxt] + (size_t)f * c->npad;
       hipLaunchKernelGGL(k_reorder, dim3(G), dim3(kBlock), 0, c->stream, src, dst, c->vals2, c->orig[c->cur],
                          c->orig[nxt], n, (int)F_TOTAL);
       // auxiliary arrays ride along in groups of up to 32
@@ -776,13 +847,16 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
         hipLaunchKernelGGL(k_reorder, dim3(G), dim3(kBlock), 0, c->stream, as, ad, c->vals2, c->orig[c->cur],
                            (int64_t *)nullptr, n, m);
       }
-      c->cur = nxt;
       std::swap(c->keys, c->keys2);
+    }
+    if (moved) {
+      c->cur = nxt;
       F = c->fields();
       c->stats.sorted = 1;
     }
-    hipLaunchKernelGGL(k_cell_start, dim3(grid_for(n + 1)), dim3(kBlock), 0, c->stream, c->keys, n, (uint32_t)nkeys,
-                       c->cstart);
+    if (!counted)
+      hipLaunchKernelGGL(k_cell_start, dim3(grid_for(n + 1)), dim3(kBlock), 0, c->stream, c->keys, n, (uint32_t)nkeys,
+                         c->cstart);
     c->keys_version = c->pos_version;
     c->keys_grid = g;
     c->keys_n = n;
@@ -790,7 +864,8 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   }
   // the v / B flags are computed again only when v or B may have changed
   c->flags_pending = c->flags_version != c->vb_version;
-  if (c->flags_pending) HIPCHK(hipMemsetAsync(c->d_stripes + kFlagSlots, 0, sizeof(long long) * kStripes, c->stream));
+  if (c->flags_pending && keys_kept)  // else k_keys cleared them
+    HIPCHK(hipMemsetAsync(c->d_stripes + kFlagSlots, 0, sizeof(long long) * kStripes, c->stream));
   // rows and cells within r_max (1 + 1e-6) of a cell; imaged axes at most
   // one wrap away
   int rc[3];
@@ -812,7 +887,8 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
                      c->pm, c->h0, c->pf, c->real, defer ? nullptr : c->st[0], c->tr[0], c->pfix, ff, c->s1[0],
                      c->eps,
                      c->flags_pending ? c->d_stripes + kFlagSlots : nullptr, c->d_stripes, kZeroLL,
-                     c->d_sweep + kSweepRegion, zlast * kSweepRegion, pos_kept ? 0 : 1);
+                     c->d_sweep + kSweepRegion, zlast * kSweepRegion, c->d_red, pos_kept ? 0 : 1);
+  c->red_ready = true;
   c->sweeps_zeroed = zlast;
   c->prep_version = c->pos_version;
   c->prep_cur = c->cur;
@@ -848,36 +924,38 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
         RCHK(dev_alloc((void **)&c->ecs, sizeof(int) * ((size_t)E + 1)));
         c->ext_cells_cap = (size_t)E + 1;
       }
-      size_t tb = 0;
-      HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, c->ext_count, c->ecs, E + 1, c->stream));
-      if (tb > c->ext_tmp_bytes) {
-        if (c->ext_tmp) { (void)hipFree(c->ext_tmp); c->ext_tmp = nullptr; }
-        c->ext_tmp_bytes = 0;
-        RCHK(dev_alloc(&c->ext_tmp, tb));
-        c->ext_tmp_bytes = tb;
-      }
       hipLaunchKernelGGL(k_ext_count, dim3(grid_for(E + 1)), dim3(kBlock), 0, c->stream, g, xg, c->cstart, E,
-                         c->ext_count);
-      tb = c->ext_tmp_bytes;
-      HIPCHK(hipcub::DeviceScan::ExclusiveSum(c->ext_tmp, tb, c->ext_count, c->ecs, E + 1, c->stream));
-      HIPCHK(hipMemcpyAsync(c->h_int + kExtTotalInt, c->ecs + E, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-      HIPCHK(wait_stream(c));
-      int64_t total = c->h_int[kExtTotalInt];
+                         c->ext_count, c->d_stripes + kFullLL);
+      RCHK(prefix_sum(c, c->ext_count, c->ecs, E + 1));
+      // With records already held (an eighth more than the last grid's) the
+      // step does not wait for their number: what does not fit is left out, and
+      // the search's error word then has it done again with the exact room.
+      int64_t total = c->ext_total;
+      const bool waits = !defer || c->ext_exact || c->ext_rec_cap == 0 || c->ext_total < 0;
+      c->ext_exact = false;
+      if (waits) {
+        HIPCHK(hipMemcpyAsync(c->h_int + kExtTotalInt, c->ecs + E, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(wait_stream(c));
+        total = c->h_int[kExtTotalInt];
+      }
       // 8 records of padding: the search reads whole batches past a row's
       // end.  The search addresses records with 32-bit byte offsets, so a
       // larger set (over 2^28 records) takes the per-lane traversal.
-      if ((total + 8) * (int64_t)sizeof(float4) > (int64_t)UINT32_MAX) {
+      if (waits && (total + 8) * (int64_t)sizeof(float4) > (int64_t)UINT32_MAX) {
         total = -1;
       } else {
-        if ((size_t)total + 8 > c->ext_rec_cap) {
+        if (waits && (size_t)total + 8 > c->ext_rec_cap) {
           if (c->erec) { (void)hipFree(c->erec); c->erec = nullptr; }
           c->ext_rec_cap = 0;
           const size_t cap = std::min<size_t>((size_t)total + 8 + (size_t)total / 8, UINT32_MAX / sizeof(float4));
           RCHK(dev_alloc((void **)&c->erec, sizeof(float4) * cap));
           c->ext_rec_cap = cap;
         }
-        hipLaunchKernelGGL(k_ext_fill, dim3(grid_for(E)), dim3(kBlock), 0, c->stream, g, xg, c->cstart, c->ecs,
-                           c->pf, E, c->erec);
+        total = std::max<int64_t>(total, 0);
+        hipLaunchKernelGGL(k_ext_fill, dim3(grid_for(E + 1)), dim3(kBlock), 0, c->stream, g, xg, c->cstart, c->ecs,
+                           c->pf, E, (int)(c->ext_rec_cap - 8), c->erec, step_err(c) + kErrSearch,
+                           c->d_stripes + kExtLL);
+        c->ext_built = true;
       }
       c->ext_total = total;
       c->ext_version = c->pos_version;
@@ -1261,7 +1339,7 @@ static Phys call_phys(const sph_ctx *c, const double *state) {
 }
 
 // The tail of a step after loop 1: Newton bookkeeping, EOS and packs
-// (k_post1), loop 2, mti gravity and the closing record's copy.  pending: the
+// (k_post1), loop 2, mti gravity, and in a leapfrog pass the corrector.  pending: the
 // still-active stripes of the last sweep queued, when more could follow it.
 static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr) {
   HIPCHK(mark(c, 2));
@@ -1270,6 +1348,10 @@ static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nu
   if (rc == SPH_OK && c->gravity)
     hipLaunchKernelGGL(k_gravity, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), c->real, (int)c->n,
                        c->gravity);
+  if (rc == SPH_OK && c->correct)
+    hipLaunchKernelGGL(k_correct, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), (int)c->n,
+                       reinterpret_cast<const double *>(c->d_stripes + kDtLL), c->aux(0), (int)c->npad,
+                       c->d_int + kGoInt, step_err(c));
   HIPCHK(mark(c, 3));
   return rc;
 }
@@ -1443,6 +1525,7 @@ static int load_impl(sph_ctx *c, int64_t n, const double *store, int64_t ld, int
     src = c->d_staging;
   }
   c->cur = 0;
+  c->fullest = 0;
   c->pos_version++;
   c->vb_version++;
   c->h_version++;
@@ -1579,6 +1662,7 @@ int sph_ctx_create(const double state[49], int kernel_id, const sph_options *opt
   c->n_fixed = (int64_t)state[S_FIXEDPN];
   if (c->n_real < 0) { delete c; return SPH_ERR_BAD_ARG; }
   if (dev_alloc((void **)&c->d_red, 16 * kStripes * sizeof(long long)) != SPH_OK ||
+      dev_alloc((void **)&c->d_dtpart, 8 * kDtBlocks * sizeof(long long)) != SPH_OK ||
       dev_alloc((void **)&c->d_int, 256 * sizeof(int)) != SPH_OK ||
       dev_alloc((void **)&c->d_stripes, kRecLL * sizeof(long long)) != SPH_OK ||
       hipHostMalloc((void **)&c->h_int, 256 * sizeof(int)) != hipSuccess ||
@@ -1599,7 +1683,7 @@ int sph_ctx_destroy(sph_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void *ptrs[] = {c->fbuf[0], c->fbuf[1], c->orig[0], c->orig[1], c->keys, c->keys2, c->vals, c->vals2,
-                  c->sort_tmp, c->cstart, c->pm, c->st[0], c->st[1], c->tr[0], c->tr[1], c->s1[0], c->s1[1], c->pfix, c->s2, c->pd, c->trd,
+                  c->sort_tmp, c->cstart, c->ccount, c->d_dtpart, c->pm, c->st[0], c->st[1], c->tr[0], c->tr[1], c->s1[0], c->s1[1], c->pfix, c->s2, c->pd, c->trd,
                   c->h0, c->eps, c->pf,
                   c->real, c->nb, c->cnt, c->q[0], c->q[1], c->q[2], c->q[3], c->q[4], c->energy_part,
                   c->d_red, c->d_int, c->d_stripes, c->d_staging, c->rent,
@@ -1782,34 +1866,6 @@ int sph_neighbours_device_noalloc(sph_ctx *c, int64_t *d_off, int32_t *d_j, int8
   return (cap_pairs > 0 && total > cap_pairs) ? SPH_ERR_BAD_ARG : SPH_OK;
 }
 
-// timestep.calc, timestep.f90:40-166 (hydro, MHD, diffusion and FLD limits)
-static int calc_dt(sph_ctx *c, const Phys &P, double *dt) {
-  const long long BIG = 0x7FFFFFFFFFFFFFFFLL, SMALL = -0x7FFFFFFFFFFFFFFFLL - 1;
-  const bool is_min[8] = {true, false, true, true, false, false, true, false};
-  long long *init = c->h_ll;
-  for (int v = 0; v < 8; v++)
-    for (int k = 0; k < kStripes; k++) init[v * kStripes + k] = is_min[v] ? BIG : SMALL;
-  HIPCHK(hipMemcpyAsync(c->d_red, init, sizeof(long long) * 8 * kStripes, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_dt_reduce, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), c->real, (int)c->n,
-                     c->d_red);
-  long long *r = c->h_ll + 512;
-  HIPCHK(hipMemcpyAsync(r, c->d_red, sizeof(long long) * 8 * kStripes, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  double v[8];
-  for (int k = 0; k < 8; k++) v[k] = ord2d(is_min[k] ? stripe_min(r, k) : stripe_max(r, k));
-  double minh = v[0], maxc = v[1], minden = v[2], minc = v[3], maxkappa = v[4], maxb = v[5];
-  double minkappa = v[6], maxlambda = v[7];
-  double cnhydro, cnd2;
-  cn_of(c->kt, P.ddw, &cnhydro, &cnd2);
-  double d = HUGE_VAL;
-  if (P.hydro) d = std::min(d, cnhydro * minh / maxc);
-  if (P.magneto) d = std::min(d, .1 * minh / maxc / maxb);
-  if (P.diff) d = std::min(d, cnd2 * minden * minc * minh * minh / maxkappa);
-  if (P.fld) d = std::min(d, cnd2 * minh * minh * minden * minkappa / kLightspeed / maxlambda);
-  *dt = d;
-  return SPH_OK;
-}
-
 // checkVarsReady (preruncheck.f90:13-60) on the resident store; *what gets
 // the failed test: 32 mu0 <= 0 with MHD, 64 isotropic conductivity <= 0,
 // else the per-particle bits of k_prerun_check.
@@ -1852,25 +1908,35 @@ int sph_leapfrog(sph_ctx *c, const double state[49], double dtcap, double *dt_us
     RCHK(prerun_check(c, state, &what));
     RCHK(run_step(c, state));
   }
-  double dt;
-  RCHK(calc_dt(c, P, &dt));
-  dt = std::min(dt, dtcap);
-  if (dt_used) *dt_used = dt;
+  // the time step, the predictor, the iterate and the corrector are queued
+  // one behind the other: the host learns the step with the iterate's record
+  const unsigned G = grid_for(c->n);
+  DtArgs d{};
+  d.part = c->d_dtpart;
+  d.nblk = (int)std::min(G, (unsigned)kDtBlocks);
+  d.hydro = P.hydro; d.magneto = P.magneto; d.diff = P.diff; d.fld = P.fld;
+  cn_of(c->kt, P.ddw, &d.cnhydro, &d.cnd2);
+  d.cap = dtcap;
+  d.out = reinterpret_cast<double *>(c->d_stripes + kDtLL);
+  hipLaunchKernelGGL(k_dt_reduce, dim3((unsigned)d.nblk), dim3(kBlock), 0, c->stream, c->fields(), c->real, (int)c->n,
+                     c->d_dtpart);
   c->naux = 9;
-  hipLaunchKernelGGL(k_predict, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), (int)c->n, dt, 1,
-                     c->aux(0), (int)c->npad);
+  hipLaunchKernelGGL(k_predict, dim3(G), dim3(kBlock), 0, c->stream, c->fields(), (int)c->n, d, c->aux(0),
+                     (int)c->npad);
   c->pos_version++;
   c->vb_version++;
   c->h_version++;
-  int rc = run_step(c, state);
-  if (rc == SPH_OK)
-    hipLaunchKernelGGL(k_correct, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), (int)c->n, dt, 1,
-                       c->aux(0), (int)c->npad);
+  c->correct = true;
+  const int rc = run_step(c, state);
+  c->correct = false;
   c->pos_version++;
   c->vb_version++;
   c->h_version++;
   c->naux = 0;
-  HIPCHK(hipStreamSynchronize(c->stream));
+  if (rc != SPH_OK)  // the record may not hold the time step
+    HIPCHK(hipMemcpyAsync(c->h_rec + kDtLL, c->d_stripes + kDtLL, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(wait_stream(c));
+  if (dt_used) memcpy(dt_used, c->h_rec + kDtLL, sizeof(double));
   return rc;
 }
 

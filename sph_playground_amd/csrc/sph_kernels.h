@@ -38,6 +38,22 @@ __host__ __device__ inline size_t nb_slot(int k, int s, int npad) {
 }
 
 constexpr int kStripes = 64;
+constexpr int kFullStripes = 32;  // k_ext_count's
+// k_wrap_reduce's slots: seven striped reductions, error bits, wrapped flag
+constexpr int kRedLL = 7 * kStripes + 2;
+
+// The time step of a leapfrog pass: k_dt_reduce's block partials (8 ordered
+// int64 each), the terms in force, the CFL numbers, the caller's cap, and where
+// the result is kept.
+struct DtArgs {
+  const long long *part;
+  int nblk;
+  int hydro, magneto, diff, fld;
+  double cnhydro, cnd2, cap;
+  double *out;
+  // which of the eight values are minima (0 h, 2 density, 3 sound speed, 6 opacity)
+  __host__ __device__ static constexpr bool is_min(int k) { return k == 0 || k == 2 || k == 3 || k == 6; }
+};
 
 // Loop-2 kernel variants.  MODE_GENERIC: every term under run-time flags.
 // MODE_DIFF: diffusion with a Hessian operator (fab/fw/n2w) and no

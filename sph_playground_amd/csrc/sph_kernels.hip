@@ -42,6 +42,10 @@ __device__ __forceinline__ long long d2ord(double v) {
   return b >= 0 ? b : (b ^ 0x7FFFFFFFFFFFFFFFLL);
 }
 
+__device__ __forceinline__ double ord2d_dev(long long v) {
+  return __longlong_as_double(v >= 0 ? v : (v ^ 0x7FFFFFFFFFFFFFFFLL));
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -154,8 +158,10 @@ __device__ __forceinline__ void cell_of(const Grid &g, double x, double y, doubl
 // reflectRealParticlesPeriodically (BC.f90:102-194) for real particles, then
 // the bounding box of all particles and the largest h of the real ones.
 // red[v * kStripes + stripe]: v = 0..2 min, 3..5 max (ordered int64), 6 max h.
+// red[7 kStripes] collects error bits, red[7 kStripes + 1] whether a particle
+// was wrapped.
 __global__ __launch_bounds__(256) void k_wrap_reduce(Fields F, const int64_t *orig, int n, int64_t n_real, Box b,
-                                                     int dim, long long *red, int *err) {
+                                                     int dim, long long *red) {
   __shared__ long long lds7[7 * 4];  // per-wave partials of the 256-thread block
   long long mn[3], mx[3], hm;
   const long long BIG = 0x7FFFFFFFFFFFFFFFLL, SMALL = -0x7FFFFFFFFFFFFFFFLL - 1;
@@ -190,8 +196,9 @@ __global__ __launch_bounds__(256) void k_wrap_reduce(Fields F, const int64_t *or
       hm = o > hm ? o : hm;
     }
   }
-  if (outside) atomicOr(err, EB_OUTSIDE);
-  if (wrapped) atomicOr(err + 4, 1);  // positions changed: cell keys must be recomputed
+  if (outside) atomicOr((unsigned long long *)&red[7 * kStripes], (unsigned long long)EB_OUTSIDE);
+  // positions changed: cell keys must be recomputed
+  if (wrapped) atomicOr((unsigned long long *)&red[7 * kStripes + 1], 1ull);
   // the seven block reductions in one pass: per wave, then one barrier, then
   // thread v combines value v over the block's waves
   long long w7[7] = {wave_min(mn[0]), wave_min(mn[1]), wave_min(mn[2]), wave_max(mx[0]), wave_max(mx[1]),
@@ -212,16 +219,29 @@ __global__ __launch_bounds__(256) void k_wrap_reduce(Fields F, const int64_t *or
   }
 }
 
-// sorted_flag: the order check's flag, cleared here for k_check_sorted
-// (which follows on the stream)
-__global__ void k_keys(Fields F, int n, Grid g, uint32_t *keys, uint32_t *vals, int *sorted_flag) {
+// Cell keys.  sorted_flag: the order check's flag, cleared here for
+// k_check_sorted (which follows on the stream), and vals the identity for the
+// sort.  With `count` (zero beforehand) the particles of each key are counted
+// and vals takes the count a particle met: its place in the cell for
+// k_cell_list, in whatever order.
+__global__ void k_keys(Fields F, int n, Grid g, uint32_t *keys, uint32_t *vals, int *sorted_flag, int *count,
+                       long long *flags) {
   int s = gtid();
   if (blockIdx.x == 0 && threadIdx.x == 0) *sorted_flag = 0;
+  // the v / B flags' stripes, for k_prep
+  if (blockIdx.x == 0 && threadIdx.x < kStripes) flags[threadIdx.x] = 0;
   if (s >= n) return;
   int c[3];
   cell_of(g, F.f[F_RX][s], F.f[F_RY][s], F.f[F_RZ][s], c);
-  keys[s] = row_of(g, c[1], c[2]) * (uint32_t)g.nc[0] + (uint32_t)c[0];
-  vals[s] = (uint32_t)s;
+  const uint32_t key = row_of(g, c[1], c[2]) * (uint32_t)g.nc[0] + (uint32_t)c[0];
+  keys[s] = key;
+  vals[s] = count ? (uint32_t)atomicAdd(&count[key], 1) : (uint32_t)s;
+}
+
+// The particles of every cell, in whatever order.
+__global__ void k_cell_list(const uint32_t *keys, const uint32_t *place, const int *cstart, int n, uint32_t *list) {
+  const int s = gtid();
+  if (s < n) list[cstart[keys[s]] + place[s]] = (uint32_t)s;
 }
 
 // Grid-stride over few blocks, one atomic per block that found a break
@@ -253,6 +273,47 @@ __global__ void k_reorder(Fields src, Fields dst, const uint32_t *perm, const in
       if (f0 + k < nf) dst.f[f0 + k][s] = v[k];
   }
   if (orig_dst) orig_dst[s] = orig_src[p];
+}
+
+// Particles straight to their place in the new order: the cell's start plus
+// how many of its particles had a smaller index, which is the order a stable
+// sort by key gives.  One pass over the columns, auxiliary ones included; the
+// counts are cleared for the next step.  A thread takes the particle at its
+// slot of the cells' lists, so a wave reads and writes within the same cells
+// (0.21 ms at 1.1M particles and 41 columns, 4.3 TB/s; threads in the old order
+// scatter their stores over cells, 0.33).  Sorting instead costs, at 301^2
+// particles, eight merge passes (44 us) and two reorders (21) against this
+// (11), the list (3) and a scan (7), and a host round trip (25) to ask first.
+__global__ void k_move(Fields src, Fields dst, const double *aux_src, double *aux_dst, int naux, int npad,
+                       const uint32_t *keys, const int *cstart, const uint32_t *list, int *count,
+                       const int64_t *orig_src, int64_t *orig_dst, int n) {
+  if (gtid() >= n) return;
+  const uint32_t s = list[gtid()];
+  const uint32_t key = keys[s];
+  const int c0 = cstart[key], c1 = cstart[key + 1];
+  int d = c0;
+  for (int q = c0; q < c1; q++) d += list[q] < s;
+  count[key] = 0;
+  constexpr int kGroup = 16;  // loads before their stores (see k_reorder)
+#pragma unroll
+  for (int f0 = 0; f0 < F_TOTAL; f0 += kGroup) {
+    double v[kGroup];
+#pragma unroll
+    for (int k = 0; k < kGroup; k++) v[k] = src.f[f0 + k][s];
+#pragma unroll
+    for (int k = 0; k < kGroup; k++) dst.f[f0 + k][d] = v[k];
+  }
+  const int64_t o = orig_src[s];
+  for (int k0 = 0; k0 < naux; k0 += kGroup) {
+    double v[kGroup];
+#pragma unroll
+    for (int k = 0; k < kGroup; k++)
+      if (k0 + k < naux) v[k] = aux_src[(size_t)(k0 + k) * npad + s];
+#pragma unroll
+    for (int k = 0; k < kGroup; k++)
+      if (k0 + k < naux) aux_dst[(size_t)(k0 + k) * npad + d] = v[k];
+  }
+  orig_dst[d] = o;
 }
 
 // First sorted index of every cell key (cstart[K] = number of particles with
@@ -337,22 +398,31 @@ __device__ __forceinline__ void prep_one(Fields F, const int64_t *orig, int s, i
   pf[s] = make_float4((float)(x - g.lo[0]), (float)(y - g.lo[1]), (float)(z - g.lo[2]), __uint_as_float(code));
 }
 
+// Start value of slot k of k_wrap_reduce's reductions: three minima, four
+// maxima, then its error bits and its wrapped flag.
+__device__ __forceinline__ long long red_start(int k) {
+  const long long BIG = 0x7FFFFFFFFFFFFFFFLL;
+  return k < 3 * kStripes ? BIG : (k < 7 * kStripes ? -BIG - 1 : 0);
+}
+
 // flags: OR of bit 0 = some velocity is non-zero, bit 1 = some B differs from
 // particle 0's (loop 2 skips terms that are exactly zero otherwise; neither
 // changes before loop 2).
 // zero[0, nzero): the step's counters, cleared by the first block before the
 // kernels that count into them run (they all follow k_prep on its stream);
 // zero2[0, nzero2): the counter regions of the step's first Newton sweeps,
-// cleared by the whole grid.
+// cleared by the whole grid.  red: k_wrap_reduce's stripes and its two words,
+// set for its next run.
 __global__ void k_prep(Fields F, const int64_t *orig, int n, int64_t n_real, Box b, Grid g, int dim, double4 *pm,
                        double *h0, float4 *pf, uint8_t *real, double4 *st, double *tr, uint3 *pfix, FixFrame ff,
                        float2 *s1, double *eps, long long *flags, long long *zero, int nzero, long long *zero2,
-                       int nzero2, int pos) {
+                       int nzero2, long long *red, int pos) {
   __shared__ long long lds[4];
   int s = gtid();
   if (blockIdx.x == 0)
     for (int k = threadIdx.x; k < nzero; k += blockDim.x) zero[k] = 0;
   for (int k = s; k < nzero2; k += gridDim.x * blockDim.x) zero2[k] = 0;
+  for (int k = s; k < kRedLL; k += gridDim.x * blockDim.x) red[k] = red_start(k);
   int fl = 0;
   if (s < n) {
     if (flags) {  // null: the caller still holds the flags of unchanged v and B
@@ -1928,27 +1998,48 @@ __device__ __forceinline__ bool ext_source(const Grid &g, const ExtGrid &x, int 
   return ux && uy && uz;
 }
 
-// records per extended cell (count[ncells] = 0 closes the exclusive scan)
-__global__ void k_ext_count(Grid g, ExtGrid x, const int *cstart, int ncells, int *count) {
+// records per extended cell (count[ncells] = 0 closes the exclusive scan), and
+// the fullest cell into fullest[kFullStripes]: one atomic per block that sees
+// a smaller value there (one word for every wave cost 70 us at 81^3)
+__global__ __launch_bounds__(256) void k_ext_count(Grid g, ExtGrid x, const int *cstart, int ncells, int *count,
+                                                   long long *fullest) {
   const int k = gtid();
-  if (k > ncells) return;
-  if (k == ncells) {
-    count[k] = 0;
-    return;
+  int c = 0;
+  if (k < ncells) {
+    int sh[3];
+    uint32_t key;
+    c = ext_source(g, x, k, sh, key) ? cstart[key + 1] - cstart[key] : 0;
   }
-  int sh[3];
-  uint32_t key;
-  count[k] = ext_source(g, x, k, sh, key) ? cstart[key + 1] - cstart[key] : 0;
+  if (k <= ncells) count[k] = c;
+  __shared__ int wmax[4];
+  c = wave_max(c);
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    c = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+    long long *f = fullest + blockIdx.x % kFullStripes;
+    if (c > __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(f, (long long)c);
+  }
 }
 
 // Copy every extended cell's records: the source records with the image
 // shift added to the FP32 coordinates, a NaN x where the reference holds no
 // such image (the band test of createPeriodicBorder, BC.f90:342-355), and the
-// list entry (sorted index << 5 | image code) in the fourth word.
-__global__ void k_ext_fill(Grid g, ExtGrid x, const int *cstart, const int *ecs, const float4 *pf, int ncells,
-                           float4 *erec) {
+// list entry (sorted index << 5 | image code) in the fourth word.  erec holds
+// `cap` records: what does not fit is left out, every cell start is kept within
+// cap, and the search's error word then asks for a search with more room;
+// *total gets the records there are.
+__global__ void k_ext_fill(Grid g, ExtGrid x, const int *cstart, int *ecs, const float4 *pf, int ncells, int cap,
+                           float4 *erec, int *err, long long *total) {
   const int k = gtid();
-  if (k >= ncells) return;
+  if (k > ncells) return;
+  const int o = ecs[k];
+  if (o > cap) ecs[k] = cap;
+  if (k == ncells) {
+    *total = o;
+    if (o > cap) atomicOr(err, EB_OVERFLOW);
+    return;
+  }
   int sh[3];
   uint32_t key;
   if (!ext_source(g, x, k, sh, key)) return;
@@ -1956,7 +2047,7 @@ __global__ void k_ext_fill(Grid g, ExtGrid x, const int *cstart, const int *ecs,
   image_mask(sh[0], sh[1], sh[2], bm, bv);
   const uint32_t code = (uint32_t)((sh[0] + 1) + 3 * (sh[1] + 1) + 9 * (sh[2] + 1));
   const float dx = (float)sh[0] * x.lenf[0], dy = (float)sh[1] * x.lenf[1], dz = (float)sh[2] * x.lenf[2];
-  const int t0 = cstart[key], t1 = cstart[key + 1], o = ecs[k];
+  const int t0 = cstart[key], t1 = min(cstart[key + 1], t0 + max(0, cap - o));
   for (int t = t0; t < t1; t++) {
     float4 q = pf[t];
     const bool there = (__float_as_uint(q.w) & bm) == bv;
@@ -2028,8 +2119,51 @@ __global__ void k_find_orig(const int64_t *orig, int n, int64_t target, int *pos
 // Leapfrog predictor (main.f90:323-342) on rows 1..n of the reference, i.e.
 // real and fixed particles (main.f90:181-184); saves the old derivatives in
 // `sv` (ax, ay, az, du, dh, ddt, dbx, dby, dbz) for the corrector.
-__global__ void k_predict(Fields F, int n, double dt, int do_t, double *sv, int npad) {
+// The time step (timestep.calc, timestep.f90:40-166) is formed here from
+// k_dt_reduce's block partials, by every block alike, and kept in *d.out for
+// the corrector and the host.
+__global__ __launch_bounds__(256) void k_predict(Fields F, int n, DtArgs d, double *sv, int npad) {
 #pragma clang fp contract(off)
+  __shared__ long long red[8][4];
+  __shared__ double dts;
+  const int t = threadIdx.x;
+  long long v[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) v[k] = d.is_min(k) ? 0x7FFFFFFFFFFFFFFFLL : -0x7FFFFFFFFFFFFFFFLL - 1;
+  for (int b = t; b < d.nblk; b += 256) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const long long w = d.part[b * 8 + k];
+      v[k] = d.is_min(k) ? (w < v[k] ? w : v[k]) : (w > v[k] ? w : v[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    v[k] = d.is_min(k) ? wave_min(v[k]) : wave_max(v[k]);
+    if ((t & 63) == 0) red[k][t >> 6] = v[k];
+  }
+  __syncthreads();
+  if (t == 0) {
+    double q[8];
+    for (int k = 0; k < 8; k++) {
+      long long m = red[k][0];
+      for (int w = 1; w < 4; w++) m = d.is_min(k) ? (red[k][w] < m ? red[k][w] : m) : (red[k][w] > m ? red[k][w] : m);
+      q[k] = ord2d_dev(m);
+    }
+    const double minh = q[0], maxc = q[1], minden = q[2], minc = q[3], maxkappa = q[4], maxb = q[5];
+    const double minkappa = q[6], maxlambda = q[7];
+    double dt = HUGE_VAL;
+    auto take = [&](double x) { if (x < dt) dt = x; };
+    if (d.hydro) take(d.cnhydro * minh / maxc);
+    if (d.magneto) take(.1 * minh / maxc / maxb);
+    if (d.diff) take(d.cnd2 * minden * minc * minh * minh / maxkappa);
+    if (d.fld) take(d.cnd2 * minh * minh * minden * minkappa / kLightspeed / maxlambda);
+    take(d.cap);
+    dts = dt;
+    if (blockIdx.x == 0) *d.out = dt;
+  }
+  __syncthreads();
+  const double dt = dts;
   int s = gtid();
   if (s >= n) return;
   const int src[9] = {F_AX, F_AY, F_AZ, F_DU, F_DH, F_DDT, F_DBX, F_DBY, F_DBZ};
@@ -2043,14 +2177,19 @@ __global__ void k_predict(Fields F, int n, double dt, int do_t, double *sv, int 
   }
   F.f[F_U][s] = F.f[F_U][s] + dt * o[3];
   F.f[F_H][s] = F.f[F_H][s] + dt * o[4];
-  if (do_t) F.f[F_T][s] = F.f[F_T][s] + dt * o[5];
+  F.f[F_T][s] = F.f[F_T][s] + dt * o[5];
 }
 
-// Leapfrog corrector (main.f90:348-362), same rows as the predictor.
-__global__ void k_correct(Fields F, int n, double dt, int do_t, const double *sv, int npad) {
+// Leapfrog corrector (main.f90:348-362), same rows as the predictor.  Queued
+// with the step's tail: it has work only where the tail ran (*go) and no error
+// word (err[0..2]) stopped the step.
+__global__ void k_correct(Fields F, int n, const double *dtp, const double *sv, int npad, const int *go,
+                          const int *err) {
 #pragma clang fp contract(off)
+  if (*go == 0 || err[0] != 0 || err[1] != 0 || err[2] != 0) return;
   int s = gtid();
   if (s >= n) return;
+  const double dt = *dtp;
   double o[9];
   for (int k = 0; k < 9; k++) o[k] = sv[(size_t)k * npad + s];
   for (int a = 0; a < 3; a++) {
@@ -2059,40 +2198,40 @@ __global__ void k_correct(Fields F, int n, double dt, int do_t, const double *sv
   }
   F.f[F_U][s] = F.f[F_U][s] + 0.5 * dt * (F.f[F_DU][s] - o[3]);
   F.f[F_H][s] = F.f[F_H][s] + 0.5 * dt * (F.f[F_DH][s] - o[4]);
-  if (do_t) F.f[F_T][s] = F.f[F_T][s] + 0.5 * dt * (F.f[F_DDT][s] - o[5]);
+  F.f[F_T][s] = F.f[F_T][s] + 0.5 * dt * (F.f[F_DDT][s] - o[5]);
 }
 
-// Per-real-particle minima/maxima for timestep.calc (timestep.f90:62-133):
-// red[v * kStripes + stripe] (ordered int64): 0 min h, 1 max c, 2 min den,
+// Per-real-particle minima/maxima for timestep.calc (timestep.f90:62-133), per
+// block into part[block * 8 + v] (ordered int64): 0 min h, 1 max c, 2 min den,
 // 3 min c, 4 max kappa, 5 max of the B components, 6 min kappa,
 // 7 max flux limiter lambda(R), R = |grad T| / (kappa rho^2 T)
-__global__ __launch_bounds__(256) void k_dt_reduce(Fields F, const uint8_t *real, int n, long long *red) {
+__global__ __launch_bounds__(256) void k_dt_reduce(Fields F, const uint8_t *real, int n, long long *part) {
 #pragma clang fp contract(off)
-  __shared__ long long lds[4];
-  int s = gtid();
+  __shared__ long long red[8][4];
   const long long BIG = 0x7FFFFFFFFFFFFFFFLL, SMALL = -0x7FFFFFFFFFFFFFFFLL - 1;
   long long v[8] = {BIG, SMALL, BIG, BIG, SMALL, SMALL, BIG, SMALL};
-  if (s < n && real[s]) {
-    v[0] = d2ord(F.f[F_H][s]);
-    v[1] = d2ord(F.f[F_C][s]);
-    v[2] = d2ord(F.f[F_DEN][s]);
-    v[3] = v[1];
-    double ka = F.f[F_KAPPA][s];
-    v[4] = d2ord(ka);
-    double bm = fmax(fmax(F.f[F_BX][s], F.f[F_BY][s]), F.f[F_BZ][s]);
-    v[5] = d2ord(bm);
-    v[6] = v[4];
-    double gx = F.f[F_DTDX][s], gy = F.f[F_DTDY][s], gz = F.f[F_DTDZ][s], da = F.f[F_DEN][s];
-    double fr = sqrt(gx * gx + gy * gy + gz * gz) / (ka * da * da * F.f[F_T][s]);
-    v[7] = d2ord((2. + fr) / (6. + 3 * fr + fr * fr));
+  for (int s = gtid(); s < n; s += (int)(gridDim.x * blockDim.x)) {
+    if (!real[s]) continue;
+    const double ka = F.f[F_KAPPA][s], c = F.f[F_C][s], da = F.f[F_DEN][s];
+    const double bm = fmax(fmax(F.f[F_BX][s], F.f[F_BY][s]), F.f[F_BZ][s]);
+    const double gx = F.f[F_DTDX][s], gy = F.f[F_DTDY][s], gz = F.f[F_DTDZ][s];
+    const double fr = sqrt(gx * gx + gy * gy + gz * gz) / (ka * da * da * F.f[F_T][s]);
+    const long long w[8] = {d2ord(F.f[F_H][s]), d2ord(c), d2ord(da), d2ord(c), d2ord(ka), d2ord(bm), d2ord(ka),
+                            d2ord((2. + fr) / (6. + 3 * fr + fr * fr))};
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = DtArgs::is_min(k) ? (w[k] < v[k] ? w[k] : v[k]) : (w[k] > v[k] ? w[k] : v[k]);
   }
-  const bool is_min[8] = {true, false, true, true, false, false, true, false};
+#pragma unroll
   for (int k = 0; k < 8; k++) {
-    long long t = is_min[k] ? block_reduce<R_MIN>(v[k], lds) : block_reduce<R_MAX>(v[k], lds);
-    if (threadIdx.x == 0) {
-      if (is_min[k]) atomicMin(&red[k * kStripes + stripe()], t);
-      else atomicMax(&red[k * kStripes + stripe()], t);
-    }
+    v[k] = DtArgs::is_min(k) ? wave_min(v[k]) : wave_max(v[k]);
+    if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = v[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 8) {
+    const int k = threadIdx.x;
+    long long m = red[k][0];
+    for (int w = 1; w < 4; w++) m = DtArgs::is_min(k) ? (red[k][w] < m ? red[k][w] : m) : (red[k][w] > m ? red[k][w] : m);
+    part[blockIdx.x * 8 + k] = m;
   }
 }
 
