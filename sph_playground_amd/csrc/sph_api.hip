@@ -1028,8 +1028,7 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
 // drift apart; several lanes of one particle read runs of its cell rows
 // instead, and few particles then still fill the chip:
 //   3D, particles that move (hydro, MHD, FLD): 8 (the tube of 1M particles,
-//     MHD in FP32: loop 2 3.44 -> 1.46 ms, with 4 lanes 1.73; sweeps 2.65 ->
-//     1.57 ms);
+//     MHD in FP32: loop 2 3.44 -> 1.64 ms; sweeps 2.65 -> 1.57 ms);
 //   3D diffusion: 4 (100^3 jittered 0.05: loop 2 0.305 -> 0.247 ms FP32, loop 1
 //     0.458 -> 0.361 FP64), 8 below 40k particles (32^3 0.036 -> 0.018 ms),
 //     but 1 for 700k particles and more whose last lists were even, within
@@ -1291,7 +1290,10 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
   // is built for it (2D and 3D: hydro, magnetohydro, hydro with FLD)
   const int terms =
       c->loop2_generic ? -1 : (P.hydro ? 1 : 0) | (P.magneto ? 2 : 0) | (P.diff ? 4 : 0) | (P.fld ? 8 : 0);
-  const int lanes = loop_lanes(c, P, true);
+  // FP32 sums of particles that move stay in list order, on eight lanes where
+  // the equation set is fixed (k_loop2), else on one
+  const bool spec = terms == kSpecHydro || terms == kSpecMhd || terms == kSpecHydroFld;
+  const int lanes = P.hydro && !spec && c->opt.precision == 1 ? 1 : loop_lanes(c, P, true);
   if (generic && P.dim >= 2 && terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, lanes, &a);
   else if (generic && P.dim >= 2 && terms == kSpecMhd) launch_loop2_d23<MODE_SPEC + kSpecMhd>(c, P.dim, lanes, &a);
   else if (generic && P.dim >= 2 && terms == kSpecHydroFld)

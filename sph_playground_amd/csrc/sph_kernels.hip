@@ -920,6 +920,48 @@ constexpr int pair_batch(int g) {
 // Entries per batch of loop 1's FP32 sums over eight lanes: 16 (the MHD tube's
 // sweeps 1.57 ms; 8: 1.92, 32: 1.69).
 constexpr int kOrd = 16;
+// The same for loop 2: 8 (MHD tube 1.64 ms; 16, whose rows leave room for
+// fewer waves, 2.2), and the floats between two groups' 17 rows there.
+constexpr int kOrd2 = 8;
+constexpr int kOrdRow2 = 17 * kOrd2 + 4;
+
+// FP32 sums in list order with 8 lanes per particle, in batches of 8 C entries:
+// lane `sub` loads entry 8 c + sub of a batch for each c < C, put(data, c,
+// valid) leaves its terms in LDS (zeros past the list's end: 0 0 adds nothing)
+// and run() adds the batch's terms.  A group lies in one wavefront, whose LDS
+// accesses complete in order: no barrier but the compiler's.
+template <int C, typename Load, typename Put, typename Run>
+__device__ __forceinline__ void for_ordered(const uint32_t *nb, int s, int sub, int npad, int nn, Load load, Put put,
+                                            Run run) {
+  const uint32_t self = nb_pack((uint32_t)s, kNoImage);
+  const uint32_t *p = nb + ((size_t)s * 8 + sub);
+  const size_t stride = (size_t)npad * 8;
+  uint32_t e[C];
+  auto read = [&](int k0) {
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      if (k0 + 8 * c < nn) e[c] = *p;
+      p += stride;
+    }
+  };
+  auto order = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  read(0);
+  for (int k0 = 0; k0 < nn; k0 += 8 * C) {
+    decltype(load(0u)) jd[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) jd[c] = load(k0 + 8 * c + sub < nn ? e[c] : self);
+    read(k0 + 8 * C);
+#pragma unroll
+    for (int c = 0; c < C; c++) put(jd[c], c, k0 + 8 * c + sub < nn);
+    order();
+    run();
+    order();
+  }
+}
 
 // ---------------------------------------------------------------- loop 1
 // One Jacobi sweep of c1advanced (circuit1.f90:114-211) for the particles
@@ -1071,10 +1113,8 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
       qbad |= !(q >= PT(0));
     };
     if constexpr (ORD) {
-      // A batch of kOrd entries: their operands into the group's LDS rows
-      // (zeros past the list's end: 0 0 adds nothing), then lane k runs sum
-      // k over them in list order.  A group lies in one wavefront, whose LDS
-      // accesses complete in order: no barrier but the compiler's.
+      // batches of kOrd entries: their operands into the group's LDS rows, then
+      // lane k runs sum k over them
       constexpr int C = kOrd / 8;
       float *const row = ord_ops + (threadIdx.x / 8) * (NOPS * kOrd);
       // operand rows: 0 m_b, 1 and 2 its factors, 3 the weight of grad T,
@@ -1082,38 +1122,17 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
       const int k = sub < NSUM ? sub : 0;
       const float *const xs = row + (k < 2 ? 0 : (k < 5 ? 3 : 7)) * kOrd;
       const float *const ys = row + (k < 2 ? 1 + k : (k < 5 ? 2 + k : k - 1)) * kOrd;
-      const uint32_t self = nb_pack((uint32_t)s, kNoImage);
-      const uint32_t *p = a.nb + ((size_t)s * 8 + sub);
-      const size_t stride = (size_t)a.npad * 8;
-      uint32_t e[C];
-      auto read = [&](int k0) {
-#pragma unroll
-        for (int c = 0; c < C; c++) {
-          if (k0 + 8 * c < nn) e[c] = *p;
-          p += stride;
-        }
-      };
-      read(0);
       float acc = 0.f;
-      for (int k0 = 0; k0 < nn; k0 += kOrd) {
-        J jd[C];
+      for_ordered<C>(a.nb, s, sub, a.npad, nn, load, [&](const J &d, int c, bool valid) {
+        float ops[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (valid)
+          terms(d, [&](int q, PT x, PT y) {
+            ops[q < 2 ? 0 : (q < 5 ? 3 : 7)] = x;
+            ops[q < 2 ? 1 + q : (q < 5 ? 2 + q : q - 1)] = y;
+          });
 #pragma unroll
-        for (int c = 0; c < C; c++) jd[c] = load(k0 + 8 * c + sub < nn ? e[c] : self);
-        read(k0 + kOrd);
-#pragma unroll
-        for (int c = 0; c < C; c++) {
-          float ops[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-          if (k0 + 8 * c + sub < nn)
-            terms(jd[c], [&](int q, PT x, PT y) {
-              ops[q < 2 ? 0 : (q < 5 ? 3 : 7)] = x;
-              ops[q < 2 ? 1 + q : (q < 5 ? 2 + q : q - 1)] = y;
-            });
-#pragma unroll
-          for (int o = 0; o < NOPS; o++) row[o * kOrd + 8 * c + sub] = ops[o];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int o = 0; o < NOPS; o++) row[o * kOrd + 8 * c + sub] = ops[o];
+      }, [&] {
 #pragma unroll
         for (int v = 0; v < kOrd; v += 4) {
           const float4 x = *reinterpret_cast<const float4 *>(xs + v);
@@ -1123,10 +1142,7 @@ __global__ __launch_bounds__(256) void k_loop1(Loop1Args<double4> a) {
           acc = fmaf(x.z, y.z, acc);
           acc = fmaf(x.w, y.w, acc);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
+      });
       // every sum to lane 0 of the group
 #pragma unroll
       for (int q = 0; q < NSUM; q++) sum[q] = __shfl(acc, (threadIdx.x & 56) + q, 64);
@@ -1393,11 +1409,22 @@ __device__ __forceinline__ void tensor_contract(const Sym3<T> &kt, T rx, T ry, T
 // The FP64 diffusion-mode loop is latency-bound: at 176 VGPRs it runs 2 waves
 // per SIMD, capped to 168 it runs 3 (a few registers spill) and measured 17 %
 // faster; the other variants are fastest uncapped.
+// FP32 with eight lanes and the equation set fixed (particles that move): the
+// sums run in list order through LDS, as in loop 1 and for its reason: where
+// Omega is near 0 a sum's rounding reaches the acceleration and, a pass later,
+// the Newton solve, and one random 1M-particle tube in a few then moves by
+// 2e-3.  MHD tube of 1M particles: one lane 3.44 ms, split sums 1.50, in order
+// 1.64.
 template <int DIM, int KT, typename PT, typename V4, int MODE, int G>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu((MODE == MODE_DIFF && std::is_same_v<PT, double>) ? 3 : 1)))
 void k_loop2(Loop2Args<V4> a) {
   if (*a.go == 0) return;
+  // FP32 sums of particles that move stay in list order (see above)
+  constexpr bool ORD = G == 8 && std::is_same_v<PT, float> && MODE >= MODE_SPEC;
+  // the pair sums; ddt takes dbx's place where only one of them exists
+  enum { L2_VX, L2_VY, L2_VZ, L2_U, L2_BX, L2_BY, L2_BZ, L2_RHO, L2_LAST, L2_T = ORD ? L2_BX : L2_LAST, L2_SUMS = 9 };
+  __shared__ __align__(16) float ord_ops[ORD ? 32 * kOrdRow2 : 4];
   const int t = gtid(), s = t / G, sub = t & (G - 1);
   double e_part = 0.0;
   if (s < a.n && a.real[s]) {
@@ -1463,7 +1490,6 @@ void k_loop2(Loop2Args<V4> a) {
     PT kdax = kta.xx * gax + kta.xy * gay + kta.xz * gaz;
     PT kday = kta.xy * gax + kta.yy * gay + kta.yz * gaz;
     PT kdaz = kta.xz * gax + kta.yz * gay + kta.zz * gaz;
-    PT dvx = 0, dvy = 0, dvz = 0, du = 0, ddt = 0, dbx = 0, dby = 0, dbz = 0, drho = 0;
     bool qbad = !(inv_ha > PT(0));
     const int nn = a.cnt[s];
     // batched: generic mode gathers positions/mass and {1/h, den, om, T};
@@ -1507,14 +1533,15 @@ void k_loop2(Loop2Args<V4> a) {
     // alone: four (FP32 with four lanes per particle: two, loop 2 of n2w at
     // 100^3 0.381 -> 0.357 ms; FP64 there four, 0.324 -> 0.306 ms at 80^3).
     // The other sets read up to six records per neighbour: with eight lanes
-    // two in FP32 (MHD tube of 1M particles 1.57 -> 1.46 ms) and one in FP64
-    // (radiation tube of 120k 0.399 -> 0.352 ms), with one lane two for the
-    // MHD and FLD sets, else one
+    // two in FP32 and one in FP64 (radiation tube of 120k 0.399 -> 0.352 ms),
+    // with one lane two for the MHD and FLD sets, else one
     constexpr bool F32 = std::is_same_v<PT, float>;
     constexpr int NBATCH = MODE == MODE_DIFF ? (G == 4 && F32 ? 2 : (G == 8 ? 2 : 4))
                            : G == 8          ? (F32 ? 2 : 1)
                            : G == 1 && SPEC && TM != kSpecHydro ? 2 : 1;
-    for_neighbours<G, NBATCH>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
+    // the terms of one pair: plus(q, t, x, y) and minus(q, t, x, y) add x y to
+    // sum q and take it off, as its t-th term
+    auto terms = [&](const J &d, auto plus, auto minus) {
       const uint32_t code = d.code;
       PT rx, ry, rz;
       if constexpr (CELL) {
@@ -1581,7 +1608,7 @@ void k_loop2(Loop2Args<V4> a) {
         vabx = vax - (PT)t.x; vaby = vay - (PT)t.y; vabz = vaz - (PT)t.z; pbb = (PT)t.w;
       }
       const PT vnwa = vabx * nwax + vaby * nway + vabz * nwaz;
-      if (P.adden) drho += mb * vnwa;
+      if (P.adden) plus(L2_RHO, 0, mb, vnwa);
       // j-side 1/(rho_b^2 om_b), once per pair where a term divides by it
       // (FP64: a division, so rho_b om_b = 0 still gives inf)
       PT i_rb2_ob = 0;
@@ -1605,22 +1632,22 @@ void k_loop2(Loop2Args<V4> a) {
           qvb = PT(-0.5) * rhob * (cb + PT(2) * fabs(dvr)) * dvr;
         }
         const PT ta_ = qva * i_ra2_oa, tb_ = qvb * i_rb2_ob;
-        dvx -= mb * (ta_ * nwax + tb_ * nwbx);
-        dvy -= mb * (ta_ * nway + tb_ * nwby);
-        dvz -= mb * (ta_ * nwaz + tb_ * nwbz);
+        minus(L2_VX, 0, mb, ta_ * nwax + tb_ * nwbx);
+        minus(L2_VY, 0, mb, ta_ * nway + tb_ * nwby);
+        minus(L2_VZ, 0, mb, ta_ * nwaz + tb_ * nwbz);
         PT qc = 0;
         if (P.au != -1.0) {  // art_termcond, circuit2.f90:520-529
           PT vs = sqrt_pair(div_pair((PT)fabs(pa_ - pbb), PT(0.5) * (rhoa + rhob)));
           qc = (PT)P.au * (vs * (ua - ub) * PT(0.5) * (faba * i_oa_ra + fabb * (rhob * i_rb2_ob)));
         }
-        du += mb * (dvr * qva * faba * i_oa_ra + qc);
+        plus(L2_U, 0, mb, dvr * qva * faba * i_oa_ra + qc);
       }
       if (hydro) {
         const PT ta_ = pa_ * i_ra2_oa, tb_ = pbb * i_rb2_ob;
-        dvx -= mb * (ta_ * nwax + tb_ * nwbx);
-        dvy -= mb * (ta_ * nway + tb_ * nwby);
-        dvz -= mb * (ta_ * nwaz + tb_ * nwbz);
-        du += mb * pa_ * vnwa * i_ra2_oa;
+        minus(L2_VX, 1, mb, ta_ * nwax + tb_ * nwbx);
+        minus(L2_VY, 1, mb, ta_ * nway + tb_ * nwby);
+        minus(L2_VZ, 1, mb, ta_ * nwaz + tb_ * nwbz);
+        plus(L2_U, 1, mb * pa_ * vnwa, i_ra2_oa);
       }
       PT bbx = 0, bby = 0, bbz = 0;
       if (need_q4) {
@@ -1673,19 +1700,19 @@ void k_loop2(Loop2Args<V4> a) {
             contr = half * (PT(DIM + 2) * S - Tr);
           }
           if constexpr (MODE == MODE_DIFF) {
-            ddt += mb_rhob * inv_rhoa * (trb - ta * rhoa) * contr;
+            plus(L2_T, 0, mb_rhob * inv_rhoa * (trb - ta * rhoa), contr);
           }
-          else ddt += div_pair(mb, rhob) * inv_rhoa * (tb * rhob - ta * rhoa) * contr;
+          else plus(L2_T, 0, div_pair(mb, rhob) * inv_rhoa * (tb * rhob - ta * rhoa), contr);
         } else if (GEN) {
           PT kdbx = ktb.xx * gbx + ktb.xy * gby + ktb.xz * gbz;
           PT kdby = ktb.xy * gbx + ktb.yy * gby + ktb.yz * gbz;
           PT kdbz = ktb.xz * gbx + ktb.yz * gby + ktb.zz * gbz;
           if (P.ddw == 403) {
             const PT odda = i_ra2_oa, oddb = i_rb2_ob;
-            ddt += mb * ((kdax * nwax + kday * nway + kdaz * nwaz) * odda +
-                         (kdbx * nwbx + kdby * nwby + kdbz * nwbz) * oddb);
+            plus(L2_T, 0, mb, (kdax * nwax + kday * nway + kdaz * nwaz) * odda +
+                                  (kdbx * nwbx + kdby * nwby + kdbz * nwbz) * oddb);
           } else {
-            ddt += mb * i_ra2_oa * ((kdbx - kdax) * nwax + (kdby - kday) * nway + (kdbz - kdaz) * nwaz);
+            plus(L2_T, 0, mb * i_ra2_oa, (kdbx - kdax) * nwax + (kdby - kday) * nway + (kdbz - kdaz) * nwaz);
           }
         }
       }
@@ -1698,18 +1725,95 @@ void k_loop2(Loop2Args<V4> a) {
         PT mb_x = ((PT(0.5) * b2b - bbx * bbx) * nwbx - bbx * bby * nwby - bbx * bbz * nwbz) * mu0inv;
         PT mb_y = (-bby * bbx * nwbx + (PT(0.5) * b2b - bby * bby) * nwby - bby * bbz * nwbz) * mu0inv;
         PT mb_z = (-bbz * bbx * nwbx - bbz * bby * nwby + (PT(0.5) * b2b - bbz * bbz) * nwbz) * mu0inv;
-        dvx -= mb * (ma_x * i_ra2_oa + mb_x * i_rb2_ob);
-        dvy -= mb * (ma_y * i_ra2_oa + mb_y * i_rb2_ob);
-        dvz -= mb * (ma_z * i_ra2_oa + mb_z * i_rb2_ob);
+        if constexpr (ORD) {  // rounded as the one-lane loop is
+          minus(L2_VX, 2, mb, fmaf(ma_x, i_ra2_oa, mb_x * i_rb2_ob));
+          minus(L2_VY, 2, mb, fmaf(mb_y, i_rb2_ob, ma_y * i_ra2_oa));
+          minus(L2_VZ, 2, mb, fmaf(mb_z, i_rb2_ob, ma_z * i_ra2_oa));
+        } else {
+          minus(L2_VX, 2, mb, ma_x * i_ra2_oa + mb_x * i_rb2_ob);
+          minus(L2_VY, 2, mb, ma_y * i_ra2_oa + mb_y * i_rb2_ob);
+          minus(L2_VZ, 2, mb, ma_z * i_ra2_oa + mb_z * i_rb2_ob);
+        }
         PT bnwa = bax * nwax + bay * nway + baz * nwaz;
         PT f = i_oa_ra * mb;
-        dbx -= f * (vabx * bnwa - bbx * vnwa);
-        dby -= f * (vaby * bnwa - bby * vnwa);
-        dbz -= f * (vabz * bnwa - bbz * vnwa);
+        minus(L2_BX, 0, f, vabx * bnwa - bbx * vnwa);
+        minus(L2_BY, 0, f, vaby * bnwa - bby * vnwa);
+        minus(L2_BZ, 0, f, vabz * bnwa - bbz * vnwa);
       }
-    });
+    };
+    PT sum[L2_SUMS] = {};
+    if constexpr (ORD) {
+      // Batches of kOrd2 entries as in loop 1: the terms' operands into the
+      // group's LDS rows, then lane k runs sum k over them.  Rows: 0 m_b, 1 the
+      // factor x of db and ddt, 2 x of the second term of du (its y is one for
+      // the particle), 3..10 y of the first terms of sums 0..7, 11..13 of the
+      // second terms of dv, 14..16 of its third.
+      constexpr int C = kOrd2 / 8;
+      float *const row = ord_ops + (threadIdx.x / 8) * kOrdRow2;
+      auto at = [&](int r) { return row + r * kOrd2; };
+      const bool dv = sub < 3;
+      const float *const x0 = at(sub >= 4 && sub < 7 ? 1 : 0), *const y0 = at(3 + sub);
+      const float *const x1 = at(sub == 3 ? 2 : 0), *const y1 = at(dv ? 11 + sub : 0);
+      const float *const y2 = at(dv ? 14 + sub : 0);
+      const float second = sub == 3 ? i_ra2_oa : 0.f;
+      float acc = 0.f;
+      for_ordered<C>(a.nb, s, sub, a.npad, nn, load, [&](const J &d, int c, bool valid) {
+        float x[3] = {0.f, 0.f, 0.f}, y[3][8] = {};
+        auto put = [&](int q, int t, PT u, PT v) {
+          if (!(TM & 2) && q == L2_T) {
+            // the one-lane loop adds the rounded product
+            x[1] = 1.f;
+            y[0][q] = u * v;
+            return;
+          }
+          x[t == 1 && q == L2_U ? 2 : (q >= L2_BX && q <= L2_BZ ? 1 : 0)] = u;
+          y[t][q] = v;
+        };
+        if (valid) terms(d, put, put);
+#pragma unroll
+        for (int o = 0; o < 3; o++) at(o)[8 * c + sub] = x[o];
+#pragma unroll
+        for (int q = 0; q < 8; q++) at(3 + q)[8 * c + sub] = y[0][q];
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          at(11 + q)[8 * c + sub] = y[1][q];
+          if (TM & 2) at(14 + q)[8 * c + sub] = y[2][q];
+        }
+      }, [&] {
+#pragma unroll
+        for (int v = 0; v < kOrd2; v += 4) {
+          const float4 u0 = *reinterpret_cast<const float4 *>(x0 + v), w0 = *reinterpret_cast<const float4 *>(y0 + v);
+          const float4 u1 = *reinterpret_cast<const float4 *>(x1 + v), w1 = *reinterpret_cast<const float4 *>(y1 + v);
+          float4 w2{};
+          if (TM & 2) w2 = *reinterpret_cast<const float4 *>(y2 + v);
+          auto step = [&](float u, float w, float u_, float w_, float w__) {
+            acc = fmaf(u, w, acc);
+            acc = fmaf(u_, dv ? w_ : second, acc);
+            if (TM & 2) acc = fmaf(u, dv ? w__ : 0.f, acc);
+          };
+          step(u0.x, w0.x, u1.x, w1.x, w2.x);
+          step(u0.y, w0.y, u1.y, w1.y, w2.y);
+          step(u0.z, w0.z, u1.z, w1.z, w2.z);
+          step(u0.w, w0.w, u1.w, w1.w, w2.w);
+        }
+      });
+      // every sum to lane 0 of the group, dv and db with their sign
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const float v = __shfl(acc, (threadIdx.x & 56) + q, 64);
+        sum[q] = q < 3 || ((TM & 2) && q >= L2_BX && q <= L2_BZ) ? -v : v;
+      }
+    } else {
+      for_neighbours<G, NBATCH>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
+        terms(d, [&](int q, int, PT x, PT y) { sum[q] += x * y; }, [&](int q, int, PT x, PT y) { sum[q] -= x * y; });
+      });
+#pragma unroll
+      for (int q = 0; q < L2_SUMS; q++) group_sum<G>(sum[q]);
+    }
+    const PT dvx = sum[L2_VX], dvy = sum[L2_VY], dvz = sum[L2_VZ], du = sum[L2_U], drho = sum[L2_RHO];
+    const PT ddt = ORD && !diff ? PT(0) : sum[L2_T];
+    const PT dbx = ORD && !magneto ? PT(0) : sum[L2_BX], dby = sum[L2_BY], dbz = sum[L2_BZ];
     if (qbad) atomicOr(a.err, EB_Q);
-    group_sum<G>(dvx, dvy, dvz, du, ddt, dbx, dby, dbz, drho);
     if (sub == 0) {
       double dh = 0.0;
       if (P.adden) dh = -DIM * ha_d / (double)rhoa * (double)drho / (double)oma;

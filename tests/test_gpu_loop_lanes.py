@@ -7,8 +7,9 @@ each side of each line is held to the oracle on jittered particles: FP64
 within 1e-12 of each field's largest value (a sum over the list in another
 order moves it by its rounding, about 1e-15), FP32 pair arithmetic with h, rho
 and Omega within 1e-5 pointwise and the force fields within 1e-4 normwise, the
-bars of the parity and mixed-precision tests.  The FP32 sums of loop 1 run in
-list order on one lane and on eight alike.
+bars of the parity and mixed-precision tests.  The FP32 sums of loop 1, and of
+loop 2 for particles that move, run in list order on one lane and on eight
+alike.
 """
 import numpy as np
 import pytest
@@ -51,6 +52,8 @@ CASES = [
     # particles that move in 3D: 8 lanes at every size
     ("mhd_50000", lambda: P.shock_slab_walls(50000, seed=5, hfac=1.2, equations="magnetohydro", velocity_seed=2),
      dict(neigh_cap=600)),
+    ("hydro3d_5000", lambda: P.shock_slab_walls(5000, seed=6, hfac=1.2, velocity_seed=2), dict(neigh_cap=600)),
+    ("fld_5000", lambda: P.shock_slab_walls(5000, seed=6, hfac=1.2, fld=True, velocity_seed=2), dict(neigh_cap=600)),
     # c1simple
     ("simple_35", lambda: P.diffusion3d(35, ddw="2nw-+", adden="no", kind="square"), {}),
 ]
