@@ -177,6 +177,14 @@ int sph_diff_forward(sph_ctx *ctx, const double K[6], int s, double dt, int nste
 /* Adjoint of the last sph_diff_forward: given dL/dT_final, dL/dT0 and dL/dK
  * (recomputing each checkpoint segment). */
 int sph_diff_backward(sph_ctx *ctx, const double *d_gT, double *d_gT0, double gK[6]);
+/* The same for the operators that read grad T (2nw-+, 2nw+-, flux-limited
+ * diffusion; K may be NULL for the last): super-steps from d_T0 into d_T, with
+ * T before steps 0, every, 2 every, ... into the rows of d_ckpt (n_real each),
+ * and their adjoint from those checkpoints (gK 0 for FLD). */
+int sph_diff_staged_forward(sph_ctx *ctx, const double K[6], int s, double dt, int nsteps, int every,
+                            const double *d_T0, double *d_T, double *d_ckpt);
+int sph_diff_staged_backward(sph_ctx *ctx, const double K[6], int s, double dt, int nsteps, int every,
+                             const double *d_ckpt, const double *d_gT, double *d_gT0, double gK[6]);
 
 /* ---- Batched problems (no reference counterpart: the reference runs one
  * ./execute per problem, e.g. 000_anisopaper_v1_gls_kxx.py:44-118).  Many

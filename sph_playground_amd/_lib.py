@@ -15,7 +15,7 @@ EXPORTS = (
     "sph_get_stats", "sph_error_string", "sph_diff_prepare", "sph_diff_apply", "sph_diff_apply_adjoint",
     "sph_diff_forward", "sph_diff_backward", "sph_rad_exchange", "sph_batch_create", "sph_batch_destroy",
     "sph_batch_sts", "sph_batch_get_info", "sph_batch_offsets", "sph_neighbours_device_noalloc",
-    "sph_prerun_check", "sph_set_timing",
+    "sph_prerun_check", "sph_set_timing", "sph_diff_staged_forward", "sph_diff_staged_backward",
 )
 
 SPH_OK = 0
@@ -95,6 +95,10 @@ def lib():
     L.sph_diff_apply_adjoint.argtypes = [P, D, ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_void_p, D, D]
     L.sph_diff_forward.argtypes = [P, D, ct.c_int, ct.c_double, ct.c_int, ct.c_int, ct.c_void_p, ct.c_void_p]
     L.sph_diff_backward.argtypes = [P, ct.c_void_p, ct.c_void_p, D]
+    L.sph_diff_staged_forward.argtypes = [P, D, ct.c_int, ct.c_double, ct.c_int, ct.c_int, ct.c_void_p, ct.c_void_p,
+                                          ct.c_void_p]
+    L.sph_diff_staged_backward.argtypes = [P, D, ct.c_int, ct.c_double, ct.c_int, ct.c_int, ct.c_void_p, ct.c_void_p,
+                                           ct.c_void_p, D]
     L.sph_neighbours_device_noalloc.argtypes = [P, ct.c_void_p, ct.c_void_p, ct.c_void_p, ct.c_int64,
                                                 ct.POINTER(ct.c_int64)]
     L.sph_prerun_check.argtypes = [P, D, ct.POINTER(ct.c_int)]

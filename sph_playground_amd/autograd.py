@@ -12,15 +12,17 @@ the prepared step frozen; the backward is the hand-written adjoint.
   - Operators that read loop 1's grad T: 2nw-+ and 2nw+- with a global K
     (linear in T and K), and flux-limited diffusion (not linear in T: its
     conductivity follows grad E through the Levermore-Pomraning limiter).
-    Stage by stage here, each stage one ``sph_diff_apply``; the backward
+    ``sph_diff_staged_forward`` / ``sph_diff_staged_backward``; the backward
     recomputes each checkpoint segment's stage states and runs the adjoint
-    recurrence with ``sph_diff_apply_adjoint`` (the transposed operator, or
-    the transposed Jacobian at the stage state, and the tensor gradient).
+    recurrence (the transposed operator, or the transposed Jacobian at the
+    stage state, and the tensor gradient).  A time step per particle runs the
+    same stages here, each one ``sph_diff_apply`` (``_apply_adjoint``).
 
 PyTorch only carries the tensors and the chain rule from K to (kappa_par,
 kappa_perp, theta, phi).
 """
 import ctypes as ct
+from operator import index
 
 import numpy as np
 import torch
@@ -58,6 +60,10 @@ def _tensor6(K):
     if Kh.shape != (6,):
         raise ValueError("K must have 6 components (xx, yy, zz, xy, xz, yz)")
     return Kh
+
+
+def _six(a):
+    return a.ctypes.data_as(ct.POINTER(ct.c_double)) if a is not None else None
 
 
 def _forward(engine, Kh, s, dt, nsteps, every, T0c, out):
@@ -176,21 +182,30 @@ def _super_step_adjoint(engine, Kh, s, dt, Ys, lam, gK):
 
 class DiffusionSTSStaged(torch.autograd.Function):
     """T_final = STS^nsteps(T0; K) for the operators that read grad T (2nw-+,
-    2nw+-, flux-limited diffusion), stage by stage.  K: (6,) for 2nw, None
-    for FLD (its conductivity comes from the state).  Checkpoints of T every
-    ``every`` steps; the backward recomputes one segment's stage states at a
-    time."""
+    2nw+-, flux-limited diffusion).  K: (6,) for 2nw, None for FLD (its
+    conductivity comes from the state).  Checkpoints of T every ``every``
+    steps; the backward recomputes one segment's stage states at a time."""
 
     @staticmethod
     def forward(ctx, T0, K, engine, s, dt, nsteps, every):
-        Y = _vector(engine, T0, "T0").clone()
+        T0c = _vector(engine, T0, "T0")
         Kh = _tensor6(K) if K is not None else None
-        ckpts = []
-        with torch.no_grad():
-            for st in range(nsteps):
-                if st % every == 0:
-                    ckpts.append(Y.clone())
-                Y = _super_step(engine, Kh, s, dt, Y)
+        ctx.native = nsteps >= 1 and every >= 1 and not (isinstance(dt, torch.Tensor) and dt.numel() != 1)
+        if ctx.native:
+            s, dt, nsteps, every = index(s), float(dt), index(nsteps), index(every)
+            Y = torch.empty_like(T0c)
+            ckpts = T0c.new_empty((-(-nsteps // every), engine.n_real))
+            torch.cuda.synchronize()
+            check(lib().sph_diff_staged_forward(engine._h, _six(Kh), s, dt, nsteps, every,
+                                                ct.c_void_p(T0c.data_ptr()), ct.c_void_p(Y.data_ptr()),
+                                                ct.c_void_p(ckpts.data_ptr())), "sph_diff_staged_forward")
+        else:
+            Y, ckpts = T0c.clone(), []
+            with torch.no_grad():
+                for st in range(nsteps):
+                    if st % every == 0:
+                        ckpts.append(Y.clone())
+                    Y = _super_step(engine, Kh, s, dt, Y)
         ctx.engine, ctx.Kh, ctx.args = engine, Kh, (s, dt, nsteps, every)
         ctx.geom = engine._geometry_gen
         ctx.Kdev = K.device if isinstance(K, torch.Tensor) else None
@@ -204,19 +219,29 @@ class DiffusionSTSStaged(torch.autograd.Function):
         if engine._geometry_gen != ctx.geom:
             raise RuntimeError("sts backward: the engine's particles changed since this forward "
                                "(load / step / prepare); its operator no longer exists")
-        lam = _vector(engine, gT, "grad").clone()
+        lam = _vector(engine, gT, "grad")
         gK = np.zeros(6) if Kh is not None else None
-        with torch.no_grad():
-            for seg in range(len(ctx.ckpts) - 1, -1, -1):
-                first = seg * every
-                last = min(first + every, nsteps)
-                states, Y = [], ctx.ckpts[seg]
-                for _ in range(first, last):
-                    keep = []
-                    Y = _super_step(engine, Kh, s, dt, Y, keep)
-                    states.append(keep)
-                for keep in reversed(states):
-                    lam = _super_step_adjoint(engine, Kh, s, dt, keep, lam, gK)
+        if ctx.native:
+            g, lam = lam, torch.empty_like(lam)
+            torch.cuda.synchronize()
+            check(lib().sph_diff_staged_backward(engine._h, _six(Kh), s, dt, nsteps, every,
+                                                 ct.c_void_p(ctx.ckpts.data_ptr()), ct.c_void_p(g.data_ptr()),
+                                                 ct.c_void_p(lam.data_ptr()),
+                                                 _six(gK if gK is not None else np.zeros(6))),
+                  "sph_diff_staged_backward")
+        else:
+            lam = lam.clone()
+            with torch.no_grad():
+                for seg in range(len(ctx.ckpts) - 1, -1, -1):
+                    first = seg * every
+                    last = min(first + every, nsteps)
+                    states, Y = [], ctx.ckpts[seg]
+                    for _ in range(first, last):
+                        keep = []
+                        Y = _super_step(engine, Kh, s, dt, Y, keep)
+                        states.append(keep)
+                    for keep in reversed(states):
+                        lam = _super_step_adjoint(engine, Kh, s, dt, keep, lam, gK)
         gKt = None
         if gK is not None and ctx.Kdev is not None:
             gKt = torch.from_numpy(gK).to(ctx.Kdev)

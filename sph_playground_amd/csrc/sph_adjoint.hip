@@ -722,11 +722,53 @@ __global__ __launch_bounds__(256) void k_nl_grad(DiffOpArgs a, const double *Y, 
   }
 }
 
-// f = A Y for the three operators (OP 3 = 2nw-+, 4 = 2nw+-, 5 = FLD), to the
-// particle's place in the original order.
+// The stages' vector sums are done where f and A^T lam are at hand: as vector
+// operations of their own they were 184 launches of a gradient through 2 FLD
+// super-steps of 4 stages (32^3 particles: 0.41 of 1.74 ms on the device, and
+// a host round trip per stage, 3.68 ms in all).
+__device__ __forceinline__ void nl_stage(const NlStage &o, int s, double f) {
+  if (o.orig) {
+    o.out[o.orig[s]] = f;
+  } else if (o.first) {
+    o.dy0[s] = f;
+    o.out[s] = o.y0[s] + o.cf * f;
+  } else {
+    o.out[s] = o.c1 * o.y1[s] + o.c2 * o.y2[s] + o.c0 * o.y0[s] + o.cf * f + o.cd * o.dy0[s];
+  }
+}
+__device__ __forceinline__ void nl_adj_stage(const NlAdjStage &o, int s, double v) {
+  if (o.orig) {
+    o.out[o.orig[s]] = v;
+    return;
+  }
+  if (o.close) {
+    o.lam[s] = o.l0[s] + v;
+    return;
+  }
+  const double l = o.lam[s], below = o.c2 * l;
+  double lj = o.c1 * l + o.cf * v, l0 = 0.0, ldy0 = 0.0;
+  if (!o.first) {
+    lj += o.pend[s];
+    l0 = o.l0[s];
+    ldy0 = o.ldy0[s];
+  }
+  if (o.last) l0 += below;
+  l0 += o.c0 * l;
+  ldy0 += o.cd * l;
+  if (o.last) {
+    l0 += lj;
+    ldy0 += o.c_1 * lj;
+  }
+  o.lam[s] = lj;
+  o.pend[s] = below;
+  o.l0[s] = l0;
+  o.ldy0[s] = ldy0;
+}
+
+// f = A Y for the three operators (OP 3 = 2nw-+, 4 = 2nw+-, 5 = FLD).
 template <int DIM, int KT, int OP, int G>
 __global__ __launch_bounds__(256) void k_nl_apply(DiffOpArgs a, const double *Y, const double4 *U, const double *D,
-                                                  const int64_t *orig, double *out) {
+                                                  NlStage o) {
   const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
@@ -741,7 +783,7 @@ __global__ __launch_bounds__(256) void k_nl_apply(DiffOpArgs a, const double *Y,
       acc += mb / j.rho * hess_trace<DIM, KT>(a, r2, ir, inv_ha) * (0.5 * (da + j.d)) * (j.y * j.rho - za);
     });
     group_sum<G>(acc);
-    if (sub == 0) out[orig[s]] = acc / rhoa;
+    if (sub == 0) nl_stage(o, s, acc / rhoa);
   } else {
     const double4 ua = U[s];
     const double3 ka = kmul(a.K, ua.x, ua.y, ua.z);
@@ -765,7 +807,7 @@ __global__ __launch_bounds__(256) void k_nl_apply(DiffOpArgs a, const double *Y,
       }
     });
     group_sum<G>(acc);
-    if (sub == 0) out[orig[s]] = OP == 3 ? acc : acc * odda;
+    if (sub == 0) nl_stage(o, s, OP == 3 ? acc : acc * odda);
   }
 }
 
@@ -836,12 +878,12 @@ __global__ __launch_bounds__(256) void k_nl_mu(DiffOpArgs a, const double4 *nu, 
   }
 }
 
-// out = base + d<mu, G(Y)>/dY (base null: 0), to the original order:
+// A^T lam = base + d<mu, G(Y)>/dY (base null: 0):
 //   mode 1: rho_s m_s sum_{a in R(s)} mu_a.nw(r_as, h_a)/(rho_a Om_a) - mu_s.F_s/Om_s
 //   mode 2: mu_s.F_s/(Om_s rho_s) + m_s/(Om_s rho_s^2) sum_{a in R(s)} rho_a mu_a.nw(r_as, h_s)
 template <int DIM, int KT, int MODE, int G>
 __global__ __launch_bounds__(256) void k_nl_gT(DiffOpArgs a, const double4 *mu, const double4 *F, const double *base,
-                                               const int64_t *orig, double *out) {
+                                               NlAdjStage o) {
   const int t = gtid_a(), s = t / G, sub = t & (G - 1);
   if (s >= a.n || !a.real[s]) return;
   const double4 ps = a.pm[s];
@@ -861,7 +903,7 @@ __global__ __launch_bounds__(256) void k_nl_gT(DiffOpArgs a, const double4 *mu, 
   double v;
   if constexpr (MODE == 1) v = qs.y * ps.w * acc - mf / qs.z;
   else v = mf / (qs.z * qs.y) + ps.w / (qs.z * qs.y * qs.y) * acc;
-  out[orig[s]] = base ? base[s] + v : v;
+  nl_adj_stage(o, s, base ? base[s] + v : v);
 }
 
 // FLD adjoint at state Y, the part with the conductivity held:
@@ -912,17 +954,17 @@ __global__ __launch_bounds__(256) void k_fld_adj(DiffOpArgs a, const double *lam
   template __global__ void k_nl_grad<DIM, KT, 2, G>(DiffOpArgs, const double *, double4 *, double4 *, double *, \
                                                     double *, double *);                                      \
   template __global__ void k_nl_apply<DIM, KT, 3, G>(DiffOpArgs, const double *, const double4 *, const double *, \
-                                                     const int64_t *, double *);                              \
+                                                     NlStage);                              \
   template __global__ void k_nl_apply<DIM, KT, 4, G>(DiffOpArgs, const double *, const double4 *, const double *, \
-                                                     const int64_t *, double *);                              \
+                                                     NlStage);                              \
   template __global__ void k_nl_apply<DIM, KT, 5, G>(DiffOpArgs, const double *, const double4 *, const double *, \
-                                                     const int64_t *, double *);                              \
+                                                     NlStage);                              \
   template __global__ void k_nl_nu<DIM, KT, 3, G>(DiffOpArgs, const double *, const double4 *, double4 *);    \
   template __global__ void k_nl_nu<DIM, KT, 4, G>(DiffOpArgs, const double *, const double4 *, double4 *);    \
   template __global__ void k_nl_gT<DIM, KT, 1, G>(DiffOpArgs, const double4 *, const double4 *, const double *, \
-                                                  const int64_t *, double *);                                 \
+                                                  NlAdjStage);                                 \
   template __global__ void k_nl_gT<DIM, KT, 2, G>(DiffOpArgs, const double4 *, const double4 *, const double *, \
-                                                  const int64_t *, double *);                                 \
+                                                  NlAdjStage);                                 \
   template __global__ void k_fld_adj<DIM, KT, G>(DiffOpArgs, const double *, const double *, const double *,  \
                                                  const double *, const double *, const double4 *, double *, double4 *);
 #define SPH_INST_NL(DIM, KT) SPH_INST_NLG(DIM, KT, 4) SPH_INST_NLG(DIM, KT, 8)

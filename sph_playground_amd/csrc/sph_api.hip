@@ -101,12 +101,12 @@ __global__ void k_batch_in(const double *, const int64_t *, const double *, int,
 template <int DIM, int KT, int MODE, int G>
 __global__ void k_nl_grad(DiffOpArgs, const double *, double4 *, double4 *, double *, double *, double *);
 template <int DIM, int KT, int OP, int G>
-__global__ void k_nl_apply(DiffOpArgs, const double *, const double4 *, const double *, const int64_t *, double *);
+__global__ void k_nl_apply(DiffOpArgs, const double *, const double4 *, const double *, NlStage);
 template <int DIM, int KT, int OP, int G>
 __global__ void k_nl_nu(DiffOpArgs, const double *, const double4 *, double4 *);
 __global__ void k_nl_mu(DiffOpArgs, const double4 *, const double4 *, const double4 *, double4 *, double *);
 template <int DIM, int KT, int MODE, int G>
-__global__ void k_nl_gT(DiffOpArgs, const double4 *, const double4 *, const double *, const int64_t *, double *);
+__global__ void k_nl_gT(DiffOpArgs, const double4 *, const double4 *, const double *, NlAdjStage);
 template <int DIM, int KT, int G>
 __global__ void k_fld_adj(DiffOpArgs, const double *, const double *, const double *, const double *, const double *,
                           const double4 *, double *, double4 *);
@@ -2075,43 +2075,42 @@ static void nl_grad_k(sph_ctx *c, const DiffOpArgs &a, const double *Y, double4 
   if (c->diff_op == 4) NL_LAUNCH(k_nl_grad<DIM COMMA KT COMMA 2, a, Y, U, F, D, c->nlDD, c->nlR);
   else NL_LAUNCH(k_nl_grad<DIM COMMA KT COMMA 1, a, Y, U, F, D, c->nlDD, c->nlR);
 }
-// f(Y), Y sorted, into `out` in original order
+// f(Y), Y sorted, to where `o` says
 template <int DIM, int KT>
-static void nl_apply_k(sph_ctx *c, const DiffOpArgs &a, const double *Y, double *out) {
-  const int64_t *o = c->orig[c->cur];
+static void nl_apply_k(sph_ctx *c, const DiffOpArgs &a, const double *Y, const NlStage &o) {
   nl_grad_k<DIM, KT>(c, a, Y, c->nlU, nullptr);
-  if (c->diff_op == 5) NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 5, a, Y, c->nlU, c->nlD, o, out);
-  else if (c->diff_op == 3) NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 3, a, Y, c->nlU, c->nlD, o, out);
-  else NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 4, a, Y, c->nlU, c->nlD, o, out);
+  if (c->diff_op == 5) NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 5, a, Y, c->nlU, c->nlD, o);
+  else if (c->diff_op == 3) NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 3, a, Y, c->nlU, c->nlD, o);
+  else NL_LAUNCH(k_nl_apply<DIM COMMA KT COMMA 4, a, Y, c->nlU, c->nlD, o);
 }
-// out (original order) = A^T lam (2nw: A linear; FLD: the Jacobian of f at Ya,
-// transposed), `work` a sorted vector; for 2nw the tensor gradients lam^T
-// dA/dK Ya -> gkdev[0..5], Yb -> [6..11] (Yb may be Ya)
+// A^T lam (2nw: A linear; FLD: the Jacobian of f at Ya, transposed) to where `o`
+// says, `work` a sorted vector; for 2nw the tensor gradients gw lam^T dA/dK Ya
+// -> gkdev[0..5] and, with Yb (which may be Ya), the same of Yb -> [6..11]
 template <int DIM, int KT>
 static void nl_adjoint_k(sph_ctx *c, const DiffOpArgs &a, const double *lam, const double *Ya, const double *Yb,
-                         double *work, double *out) {
+                         double *work, double gw, const NlAdjStage &o) {
   const unsigned G = grid_for(c->n);
-  const int64_t *o = c->orig[c->cur];
   const double *none = nullptr;
   nl_grad_k<DIM, KT>(c, a, Ya, c->nlU, nullptr);
   if (c->diff_op == 5) {
     NL_LAUNCH(k_fld_adj<DIM COMMA KT, a, lam, Ya, c->nlD, c->nlDD, c->nlR, c->nlU, work, c->nlMu);
     const double *base = work;
-    NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 1, a, c->nlMu, c->nlF, base, o, out);
+    NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 1, a, c->nlMu, c->nlF, base, o);
     return;
   }
-  const double4 *UB = c->nlU;
-  if (Yb != Ya) {
+  const double4 *UB = Yb ? c->nlU : nullptr;
+  if (Yb && Yb != Ya) {
     nl_grad_k<DIM, KT>(c, a, Yb, c->nlUB, nullptr);
     UB = c->nlUB;
   }
   if (c->diff_op == 3) NL_LAUNCH(k_nl_nu<DIM COMMA KT COMMA 3, a, lam, c->nlF, c->nlNu);
   else NL_LAUNCH(k_nl_nu<DIM COMMA KT COMMA 4, a, lam, c->nlF, c->nlNu);
   hipLaunchKernelGGL(k_nl_mu, dim3(G), dim3(kBlock), 0, c->stream, a, c->nlNu, c->nlU, UB, c->nlMu, c->gpart);
-  hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)G, 1.0, 0.0, c->gkdev);
-  hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)G, 0.0, 1.0, c->gkdev + 6);
-  if (c->diff_op == 4) NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 2, a, c->nlMu, c->nlF, none, o, out);
-  else NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 1, a, c->nlMu, c->nlF, none, o, out);
+  hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)G, gw, 0.0, c->gkdev);
+  if (Yb)
+    hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)G, 0.0, gw, c->gkdev + 6);
+  if (c->diff_op == 4) NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 2, a, c->nlMu, c->nlF, none, o);
+  else NL_LAUNCH(k_nl_gT<DIM COMMA KT COMMA 1, a, c->nlMu, c->nlF, none, o);
 }
 #undef NL_LAUNCH
 #undef COMMA
@@ -2418,7 +2417,10 @@ int sph_diff_apply(sph_ctx *c, const double K[6], const double *d_T, double *d_o
   if (c->diff_op != 0) {
     const double K0[6] = {0, 0, 0, 0, 0, 0};
     DiffOpArgs a = diff_args(c, K ? K : K0);
-    NL_DISPATCH(nl_apply_k, c, a, dv(c, 0), d_out);
+    NlStage st{};
+    st.orig = c->orig[c->cur];
+    st.out = d_out;
+    NL_DISPATCH(nl_apply_k, c, a, dv(c, 0), st);
   } else {
     diff_apply(c, K, dv(c, 0), dv(c, 1));
     hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 1), c->orig[c->cur], n, d_out);
@@ -2444,7 +2446,10 @@ int sph_diff_apply_adjoint(sph_ctx *c, const double K[6], const double *d_lam, c
   if (c->diff_op != 0) {
     const double K0[6] = {0, 0, 0, 0, 0, 0};
     DiffOpArgs a = diff_args(c, K ? K : K0);
-    NL_DISPATCH(nl_adjoint_k, c, a, dv(c, 0), dv(c, 1), dv(c, yb ? 2 : 1), dv(c, 3), d_out);
+    NlAdjStage st{};
+    st.orig = o;
+    st.out = d_out;
+    NL_DISPATCH(nl_adjoint_k, c, a, dv(c, 0), dv(c, 1), dv(c, yb ? 2 : 1), dv(c, 3), 1.0, st);
   } else {
     ensure_weights(c, K);
     AdjStage a = adj_args(c);  // A^T lam alone
@@ -2558,6 +2563,125 @@ int sph_diff_backward(sph_ctx *c, const double *d_gT, double *d_gT0, double gK[6
   c->fw_tail = false;  // segment buffers now hold the first segment
   HIPCHK(hipMemcpyAsync(gK, c->gkdev, sizeof(double) * 6, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  return SPH_OK;
+}
+
+// Super-steps of the operators that read grad T.  Work vectors: the adjoint's
+// L, what is pending for the next, L_0 and the first rate's, a scratch vector,
+// the first stage's rate, four states in rotation; then the stage states of a
+// checkpoint segment, s per step.
+enum { W_L = 0, W_PEND, W_L0, W_LDY0, W_WORK, W_DY0, W_STATE, W_SEG = W_STATE + 4 };
+
+// One super-step (sts_integrator.f90:100-123) over Y[0..s]; with a null Y[s]
+// its last stage is left out (the states of a segment's last step).
+static int staged_step(sph_ctx *c, const DiffOpArgs &a, int s, double dt, double *const *Y) {
+  for (int j = 1; j <= s && Y[j]; j++) {
+    double co[4];
+    RCHK(sph_sts_coeffs(j, s, co));
+    NlStage st{};
+    st.out = Y[j];
+    st.y0 = Y[0];
+    st.dy0 = dv(c, W_DY0);
+    st.first = j == 1;
+    st.cf = co[2] * dt;
+    if (j > 1) {
+      st.y1 = Y[j - 1];
+      st.y2 = Y[j - 2];
+      st.c1 = co[0]; st.c2 = co[1]; st.c0 = 1 - co[0] - co[1]; st.cd = co[3] * dt;
+    }
+    NL_DISPATCH(nl_apply_k, c, a, Y[j - 1], st);
+  }
+  return SPH_OK;
+}
+
+// dL/dY_0 of one super-step from dL/dY_s, both in W_L; dL/dK added into gkdev.
+static int staged_step_adjoint(sph_ctx *c, const DiffOpArgs &a, int s, double dt, double *const *Y) {
+  const double *none = nullptr;
+  double co[4];
+  RCHK(sph_sts_coeffs(1, s, co));
+  NlAdjStage st{};
+  st.lam = dv(c, W_L); st.pend = dv(c, W_PEND); st.l0 = dv(c, W_L0); st.ldy0 = dv(c, W_LDY0);
+  st.c_1 = co[2] * dt;
+  for (int j = s; j >= 2; j--) {
+    RCHK(sph_sts_coeffs(j, s, co));
+    st.c1 = co[0]; st.c2 = co[1]; st.c0 = 1 - co[0] - co[1]; st.cf = co[2] * dt; st.cd = co[3] * dt;
+    st.first = j == s;
+    st.last = j == 2;
+    NL_DISPATCH(nl_adjoint_k, c, a, dv(c, W_L), Y[j - 1], none, dv(c, W_WORK), co[2] * dt, st);
+  }
+  st.close = 1;
+  NL_DISPATCH(nl_adjoint_k, c, a, dv(c, W_LDY0), Y[0], none, dv(c, W_WORK), 1.0, st);
+  return SPH_OK;
+}
+
+int sph_diff_staged_forward(sph_ctx *c, const double K[6], int s, double dt, int nsteps, int every, const double *d_T0,
+                            double *d_T, double *d_ckpt) {
+  if (!c || !c->diff_ready || !d_T0 || !d_T || !d_ckpt || s < 2 || nsteps < 1 || every < 1) return SPH_ERR_BAD_ARG;
+  if (c->diff_op == 0) return SPH_ERR_UNSUPPORTED;  // sph_diff_forward
+  if (!K && c->diff_op != 5) return SPH_ERR_BAD_ARG;
+  (void)hipSetDevice(c->device);
+  RCHK(ensure_dvec(c, W_SEG));
+  const int n = (int)c->n;
+  const unsigned G = grid_for(n);
+  const int64_t *o = c->orig[c->cur];
+  const double K0[6] = {0, 0, 0, 0, 0, 0};
+  const DiffOpArgs a = diff_args(c, K ? K : K0);
+  double *ring[4];
+  for (int k = 0; k < 4; k++) ring[k] = dv(c, W_STATE + k);
+  std::vector<double *> Y(s + 1);
+  hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_T0, o, n, ring[0]);
+  for (int st = 0; st < nsteps; st++) {
+    if (st % every == 0)
+      hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, ring[0], o, n,
+                         d_ckpt + (size_t)(st / every) * n);
+    Y[0] = ring[0];
+    for (int j = 1; j <= s; j++) Y[j] = ring[1 + (j - 1) % 3];
+    RCHK(staged_step(c, a, s, dt, Y.data()));
+    std::swap(ring[0], ring[1 + (s - 1) % 3]);
+  }
+  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, ring[0], o, n, d_T);
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return SPH_OK;
+}
+
+int sph_diff_staged_backward(sph_ctx *c, const double K[6], int s, double dt, int nsteps, int every,
+                             const double *d_ckpt, const double *d_gT, double *d_gT0, double gK[6]) {
+  if (!c || !c->diff_ready || !d_ckpt || !d_gT || !d_gT0 || !gK || s < 2 || nsteps < 1 || every < 1)
+    return SPH_ERR_BAD_ARG;
+  if (c->diff_op == 0) return SPH_ERR_UNSUPPORTED;
+  if (!K && c->diff_op != 5) return SPH_ERR_BAD_ARG;
+  (void)hipSetDevice(c->device);
+  RCHK(ensure_dvec(c, W_SEG + std::min(every, nsteps) * s));
+  const int n = (int)c->n;
+  const unsigned G = grid_for(n);
+  const int64_t *o = c->orig[c->cur];
+  const double K0[6] = {0, 0, 0, 0, 0, 0};
+  const DiffOpArgs a = diff_args(c, K ? K : K0);
+  HIPCHK(hipMemsetAsync(c->gkdev, 0, sizeof(double) * 12, c->stream));
+  hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_gT, o, n, dv(c, W_L));
+  std::vector<double *> Y(s + 1);
+  for (int sg = (nsteps - 1) / every; sg >= 0; sg--) {
+    const int steps = std::min(nsteps, (sg + 1) * every) - sg * every;
+    auto states = [&](int k) {
+      for (int j = 0; j < s; j++) Y[j] = dv(c, W_SEG + k * s + j);
+      Y[s] = k + 1 < steps ? dv(c, W_SEG + (k + 1) * s) : nullptr;
+    };
+    hipLaunchKernelGGL(k_to_sorted, dim3(G), dim3(kBlock), 0, c->stream, d_ckpt + (size_t)sg * n, o, n,
+                       dv(c, W_SEG));
+    for (int k = 0; k < steps; k++) {
+      states(k);
+      RCHK(staged_step(c, a, s, dt, Y.data()));
+    }
+    for (int k = steps - 1; k >= 0; k--) {
+      states(k);
+      RCHK(staged_step_adjoint(c, a, s, dt, Y.data()));
+    }
+  }
+  hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, W_L), o, n, d_gT0);
+  double g[6];
+  HIPCHK(hipMemcpyAsync(g, c->gkdev, sizeof(g), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  std::copy(g, g + 6, gK);
   return SPH_OK;
 }
 

@@ -301,6 +301,33 @@ struct BatchStage {
   int n, npad, rev;
 };
 
+// What becomes of a particle's f in k_nl_apply: its place in the original order
+// (orig), or an RKL2 stage in the sorted one,
+//   out = y0 + cf f, f kept in dy0 (the first stage),
+//   out = c1 y1 + c2 y2 + c0 y0 + cf f + cd dy0.
+struct NlStage {
+  const int64_t *orig;
+  double *out;
+  const double *y0, *y1, *y2;
+  double *dy0;
+  double c0, c1, c2, cf, cd;
+  int first;
+};
+
+// What becomes of a particle's (A^T lam) in k_nl_gT: its place in the original
+// order (orig), or the adjoint of a stage j: with l = lam its L_j,
+//   L_{j-1} = pend + c1 l + cf (A^T lam) over l, pend = c2 l (L_{j-2}'s part),
+//   l0 += c0 l, ldy0 += cd l
+// (first: j = s, nothing summed yet; last: j = 2, whose L_1 goes into l0 and
+// ldy0, by c_1, too), or of the first stage (close), lam = l0 + A^T lam.
+struct NlAdjStage {
+  const int64_t *orig;
+  double *out;
+  double *lam, *pend, *l0, *ldy0;
+  double c0, c1, c2, cf, cd, c_1;
+  int first, last, close;
+};
+
 // One adjoint stage j of a super-step (k_adj_stage): U = A^T L_j over the
 // reverse lists, then
 //   j > 1: L_{j-1} = mu L_j + mh U + nu1 L_{j+1} (L_{j+1} null for j = s),
