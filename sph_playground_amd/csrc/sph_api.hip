@@ -52,7 +52,8 @@ __global__ void k_post1(Fields, PostSel, const uint8_t *, int, int, int, int, do
                         V4 *, V4 *, V4 *, double4 *, double *, float2 *, long long *, long long *);
 template <int DIM, int KT, typename PT, typename V4, int MODE, int G>
 __global__ void k_loop2(Loop2Args<V4>);
-__global__ void k_aos_to_soa(const double *, int64_t, int, Fields, int64_t *);
+__global__ void k_aos_to_soa(const double *, int64_t, int, const uint32_t *, Fields, int64_t *);
+__global__ void k_load_cols(const double *, int64_t, int, Fields, int64_t *);
 __global__ void k_step_close(const double *, int, const int *, const long long *, long long *);
 __global__ void k_soa_to_aos(Fields, const int64_t *, int, double *, int64_t);
 __global__ void k_ext_count(Grid, ExtGrid, const int *, int, int *, long long *);
@@ -206,14 +207,15 @@ struct sph_ctx {
   void *sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
   int *cstart = nullptr;   // first sorted index of every cell key
-  int *ccount = nullptr;   // particles per cell key while they are counted, else zero
+  int *ccount = nullptr;   // particles per cell key while they are counted, else zero (behind cstart)
   int64_t ncell_cap = 0;
   long long fullest = 0;   // particles in the fullest search cell last seen (0: not known)
   bool red_ready = false;  // d_red holds k_wrap_reduce's start values
+  bool flags_clear = false;  // the v / B flags' stripes are zero since load_order's k_keys
   bool ext_exact = false;  // the next extended grid waits for its size
   bool ext_built = false;  // this step built one: its counts come with the search's
   bool correct = false;    // this step's tail ends with the leapfrog corrector
-  long long *d_dtpart = nullptr;  // k_dt_reduce's block partials
+  long long *d_dtpart = nullptr;  // k_dt_reduce's block partials (in d_red's allocation)
   double4 *pm = nullptr, *st[2] = {nullptr, nullptr};
   double *tr[2] = {nullptr, nullptr};  // T den of the loop-1 sweep state st[k]
   // mixed path: position records (31-bit fractions, `ff` their frame),
@@ -474,8 +476,8 @@ static int ensure_cells(sph_ctx *c, int64_t nkeys) {
   if (nkeys + 1 <= c->ncell_cap) return SPH_OK;
   int64_t cap = std::max<int64_t>(nkeys + 1, 1024);
   c->ncell_cap = 0;
-  RCHK(dalloc(&c->cstart, cap));
-  RCHK(dalloc(&c->ccount, cap));
+  RCHK(dalloc(&c->cstart, 2 * cap));
+  c->ccount = c->cstart + cap;
   HIPCHK(hipMemsetAsync(c->ccount, 0, sizeof(int) * cap, c->stream));
   c->ncell_cap = cap;
   return SPH_OK;
@@ -684,57 +686,46 @@ static int prefix_sum(sph_ctx *c, const int *in, int *out, int count) {
   return SPH_OK;
 }
 
-// defer: launch the search without waiting for its read-back (a later
-// copy_record brings it); the lists then hold at most nb_cap entries per
-// particle, so what runs on them before take_neighbours stays in bounds.
-static int build_neighbours(sph_ctx *c, bool defer = false) {
-  const int n = (int)c->n;
-  const int dim = c->frozen.dim;
-  Fields F = c->fields();
-  unsigned G = grid_for(n);
+// Escaped real particles wrapped back into the box, the bounding box of all and
+// the largest h of the real ones (F's x, y, z and h in `orig`'s order).
+static int wrap_pass(sph_ctx *c, Fields F, const int64_t *orig, double lo[3], double hi[3], double *hmax,
+                     bool *wrapped) {
   const long long BIG = 0x7FFFFFFFFFFFFFFFLL, SMALL = -0x7FFFFFFFFFFFFFFFLL - 1;
-  c->ext_built = false;
-  // 1. wrap escaped real particles, bounding box, max h (striped reductions).
-  //    Positions unchanged since the last pass (so none escaped) and h last
-  //    set by the previous step (whose k_post1 reduced h_max): nothing to do.
-  double lo[3], hi[3], hmax;
-  if (c->bbox_version == c->pos_version && c->hmax_version == c->h_version && c->n_real > 0) {
-    for (int a = 0; a < 3; a++) { lo[a] = c->last_lo[a]; hi[a] = c->last_hi[a]; }
-    hmax = c->next_hmax;
-  } else {
-    if (!c->red_ready) {  // else the last step's k_prep set the start values
-      long long *init = c->h_ll;
-      for (int k = 0; k < kRedLL; k++) init[k] = k < 3 * kStripes ? BIG : (k < 7 * kStripes ? SMALL : 0);
-      HIPCHK(hipMemcpyAsync(c->d_red, init, sizeof(long long) * kRedLL, hipMemcpyHostToDevice, c->stream));
-      HIPCHK(hipMemsetAsync(c->d_int, 0, sizeof(int) * 8, c->stream));
-    }
-    c->red_ready = false;
-    // at most 1024 blocks (four per CU), each striding over the particles
-    hipLaunchKernelGGL(k_wrap_reduce, dim3(std::min(G, 1024u)), dim3(kBlock), 0, c->stream, F, c->orig[c->cur], n,
-                       c->n_real, c->box, dim, c->d_red);
-    long long *red = c->h_ll + 512;
-    HIPCHK(hipMemcpyAsync(red, c->d_red, sizeof(long long) * kRedLL, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(wait_stream(c));
-    if (red[7 * kStripes] & EB_OUTSIDE) return SPH_ERR_UNSUPPORTED;
-    if (red[7 * kStripes + 1]) c->pos_version++;  // a particle was wrapped back into the box
-    for (int a = 0; a < 3; a++) { lo[a] = ord2d(stripe_min(red, a)); hi[a] = ord2d(stripe_max(red, 3 + a)); }
-    hmax = c->n_real > 0 ? ord2d(stripe_max(red, 6)) : 0.0;
-    for (int a = 0; a < 3; a++) { c->last_lo[a] = lo[a]; c->last_hi[a] = hi[a]; }
-    c->bbox_version = c->pos_version;
+  if (!c->red_ready) {  // else the last step's k_prep set the start values
+    long long *init = c->h_ll;
+    for (int k = 0; k < kRedLL; k++) init[k] = k < 3 * kStripes ? BIG : (k < 7 * kStripes ? SMALL : 0);
+    HIPCHK(hipMemcpyAsync(c->d_red, init, sizeof(long long) * kRedLL, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemsetAsync(c->d_int, 0, sizeof(int) * 8, c->stream));
   }
-  if (!(hmax > 0.0) && c->n_real > 0) return SPH_ERR_Q_NAN_OR_NEG;
+  c->red_ready = false;
+  // at most 1024 blocks (four per CU), each striding over the particles
+  hipLaunchKernelGGL(k_wrap_reduce, dim3(std::min(grid_for(c->n), 1024u)), dim3(kBlock), 0, c->stream, F, orig,
+                     (int)c->n, c->n_real, c->box, c->frozen.dim, c->d_red);
+  long long *red = c->h_ll + 512;
+  HIPCHK(hipMemcpyAsync(red, c->d_red, sizeof(long long) * kRedLL, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(wait_stream(c));
+  if (red[7 * kStripes] & EB_OUTSIDE) return SPH_ERR_UNSUPPORTED;
+  *wrapped = red[7 * kStripes + 1] != 0;
+  for (int a = 0; a < 3; a++) { lo[a] = ord2d(stripe_min(red, a)); hi[a] = ord2d(stripe_max(red, 3 + a)); }
+  *hmax = c->n_real > 0 ? ord2d(stripe_max(red, 6)) : 0.0;
+  return SPH_OK;
+}
+
+// The cell grid: cells at least rmax/RS wide; imaged axes tile
+// [emin, emax] and need 2 RS + 1 cells, else RS drops to 1.  The search
+// reads each (y, z) row as whole ranges along x, so thin rows follow the
+// sphere closely at a few more row ranges, and they order the particles
+// so that adjacent lanes gather adjacent neighbours in the loops.  Cells
+// of a third of the radius measured fastest for the whole step (a half
+// and a quarter were slower in the loops and in the search).
+static Grid search_grid(const sph_ctx *c, const double lo[3], const double hi[3], double hmax, double *rmax_out,
+                        double cs[3], int64_t *nkeys) {
+  const int dim = c->frozen.dim;
   double rmax = c->frozen.krad * hmax * (1.0 + 1e-9);
   if (!(rmax > 0.0)) rmax = 1.0;
-  // 2. cell grid: cells at least rmax/RS wide; imaged axes tile
-  //    [emin, emax] and need 2 RS + 1 cells, else RS drops to 1.  The search
-  //    reads each (y, z) row as whole ranges along x, so thin rows follow the
-  //    sphere closely at a few more row ranges, and they order the particles
-  //    so that adjacent lanes gather adjacent neighbours in the loops.  Cells
-  //    of a third of the radius measured fastest for the whole step (a half
-  //    and a quarter were slower in the loops and in the search).
+  *rmax_out = rmax;
   const int axis_cap = dim == 3 ? 1024 : (dim == 2 ? 32768 : (1 << 30));
   Grid g{};
-  double cs[3];
   int RS = c->opt.cell_div > 0 ? c->opt.cell_div : kNeighRS;
   for (int attempt = 0; attempt < 2; attempt++) {
     g = Grid{};
@@ -789,11 +780,46 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   } else if (dim == 2) {
     nrow = g.nc[1];
   }
-  const int64_t nkeys = nrow * g.nc[0];
+  *nkeys = nrow * g.nc[0];
+  return g;
+}
+
+// The bits a sort by keys below nkeys has to look at.
+static int bits_of(int64_t nkeys) {
+  int b = 1;
+  while (b < 32 && ((int64_t)1 << b) < nkeys) b++;
+  return b;
+}
+
+// defer: launch the search without waiting for its read-back (a later
+// copy_record brings it); the lists then hold at most nb_cap entries per
+// particle, so what runs on them before take_neighbours stays in bounds.
+static int build_neighbours(sph_ctx *c, bool defer = false) {
+  const int n = (int)c->n;
+  const int dim = c->frozen.dim;
+  Fields F = c->fields();
+  unsigned G = grid_for(n);
+  c->ext_built = false;
+  // 1. wrap escaped real particles, bounding box, max h (striped reductions).
+  //    Positions unchanged since the last pass (so none escaped) and h last
+  //    set by the previous step (whose k_post1 reduced h_max): nothing to do.
+  double lo[3], hi[3], hmax;
+  if (c->bbox_version == c->pos_version && c->hmax_version == c->h_version && c->n_real > 0) {
+    for (int a = 0; a < 3; a++) { lo[a] = c->last_lo[a]; hi[a] = c->last_hi[a]; }
+    hmax = c->next_hmax;
+  } else {
+    bool wrapped;
+    RCHK(wrap_pass(c, F, c->orig[c->cur], lo, hi, &hmax, &wrapped));
+    if (wrapped) c->pos_version++;  // keys, records and lists are made anew
+    for (int a = 0; a < 3; a++) { c->last_lo[a] = lo[a]; c->last_hi[a] = hi[a]; }
+    c->bbox_version = c->pos_version;
+  }
+  if (!(hmax > 0.0) && c->n_real > 0) return SPH_ERR_Q_NAN_OR_NEG;
+  double rmax, cs[3];
+  int64_t nkeys;
+  const Grid g = search_grid(c, lo, hi, hmax, &rmax, cs, &nkeys);
   c->grid = g;
   RCHK(ensure_cells(c, nkeys));
-  int key_bits = 1;
-  while (key_bits < 32 && ((int64_t)1 << key_bits) < nkeys) key_bits++;
   // 3. cell keys, sortedness, radix sort + reorder when needed; keys and
   //    cell starts of the same positions on the same grid are still valid
   c->stats.sorted = 0;
@@ -833,7 +859,7 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
     if (moved && !counted) {
       size_t bytes = c->sort_tmp_bytes;
       HIPCHK(hipcub::DeviceRadixSort::SortPairs(c->sort_tmp, bytes, c->keys, c->keys2, c->vals, c->vals2, n, 0,
-                                                key_bits, c->stream));
+                                                bits_of(nkeys), c->stream));
       hipLaunchKernelGGL(k_reorder, dim3(G), dim3(kBlock), 0, c->stream, src, dst, c->vals2, c->orig[c->cur],
                          c->orig[nxt], n, (int)F_TOTAL);
       // auxiliary arrays ride along in groups of up to 32
@@ -864,7 +890,7 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   }
   // the v / B flags are computed again only when v or B may have changed
   c->flags_pending = c->flags_version != c->vb_version;
-  if (c->flags_pending && keys_kept)  // else k_keys cleared them
+  if (c->flags_pending && keys_kept && !c->flags_clear)  // else k_keys cleared them
     HIPCHK(hipMemsetAsync(c->d_stripes + kFlagSlots, 0, sizeof(long long) * kStripes, c->stream));
   // rows and cells within r_max (1 + 1e-6) of a cell; imaged axes at most
   // one wrap away
@@ -889,6 +915,7 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
                      c->flags_pending ? c->d_stripes + kFlagSlots : nullptr, c->d_stripes, kZeroLL,
                      c->d_sweep + kSweepRegion, zlast * kSweepRegion, c->d_red, pos_kept ? 0 : 1);
   c->red_ready = true;
+  c->flags_clear = false;
   c->sweeps_zeroed = zlast;
   c->prep_version = c->pos_version;
   c->prep_cur = c->cur;
@@ -1509,6 +1536,58 @@ static int run_step(sph_ctx *c, const double *state) {
 }
 
 // ----------------------------------------------------------------- loading
+// The order of a new store's rows by cell key, as the first step's sort would
+// make it, so that the fields are read in that order once: *perm gets it, or
+// null where the rows are in order already or cannot be ordered (the step then
+// says why).  A first step after it has bounding box, keys and cell starts, and
+// sorts nothing: the gather of 32 columns over 1.1M random particles was 0.62
+// ms, the rows of 256 bytes are read in any order in 0.15.
+static int load_order(sph_ctx *c, const double *src, int64_t ld, const uint32_t **perm) {
+  const int n = (int)c->n;
+  const unsigned G = grid_for(n);
+  *perm = nullptr;
+  if (c->n_real <= 0) return SPH_OK;
+  Fields F;
+  for (int f = 0; f < F_TOTAL; f++) F.f[f] = c->fbuf[1] + (size_t)f * c->npad;
+  hipLaunchKernelGGL(k_load_cols, dim3(G), dim3(kBlock), 0, c->stream, src, ld, n, F, c->orig[1]);
+  double lo[3], hi[3], hmax, rmax, cs[3];
+  int64_t nkeys;
+  bool wrapped;
+  const int rc = wrap_pass(c, F, c->orig[1], lo, hi, &hmax, &wrapped);
+  if (rc == SPH_ERR_UNSUPPORTED) return SPH_OK;
+  RCHK(rc);
+  bool finite = hmax > 0.0 && std::isfinite(hmax);
+  for (int a = 0; a < 3; a++) finite = finite && std::isfinite(lo[a]) && std::isfinite(hi[a]);
+  if (!finite) return SPH_OK;
+  const Grid g = search_grid(c, lo, hi, hmax, &rmax, cs, &nkeys);
+  const int rk = ensure_cells(c, nkeys);
+  if (rk == SPH_ERR_NOMEM) return SPH_OK;
+  RCHK(rk);
+  hipLaunchKernelGGL(k_keys, dim3(G), dim3(kBlock), 0, c->stream, F, n, g, c->keys, c->vals, c->d_int + 2,
+                     (int *)nullptr, c->d_stripes + kFlagSlots);
+  hipLaunchKernelGGL(k_check_sorted, dim3(std::min(G, 256u)), dim3(kBlock), 0, c->stream, c->keys, n, c->d_int + 2);
+  RCHK(read_ints(c, 2, 1));
+  if (c->h_int[2] != 0) {
+    size_t bytes = c->sort_tmp_bytes;
+    HIPCHK(hipcub::DeviceRadixSort::SortPairs(c->sort_tmp, bytes, c->keys, c->keys2, c->vals, c->vals2, n, 0,
+                                              bits_of(nkeys), c->stream));
+    std::swap(c->keys, c->keys2);
+    *perm = c->vals2;
+  }
+  hipLaunchKernelGGL(k_cell_start, dim3(grid_for(n + 1)), dim3(kBlock), 0, c->stream, c->keys, n, (uint32_t)nkeys,
+                     c->cstart);
+  c->flags_clear = true;
+  if (wrapped) return SPH_OK;  // the step wraps them, and makes the keys of the new positions
+  for (int a = 0; a < 3; a++) { c->last_lo[a] = lo[a]; c->last_hi[a] = hi[a]; }
+  c->next_hmax = hmax;
+  c->bbox_version = c->keys_version = c->pos_version;
+  c->hmax_version = c->h_version;
+  c->keys_grid = g;
+  c->keys_n = n;
+  c->keys_nkeys = nkeys;
+  return SPH_OK;
+}
+
 static int load_impl(sph_ctx *c, int64_t n, const double *store, int64_t ld, int on_device) {
   if (n <= 0 || ld < F_TOTAL || !store) return SPH_ERR_BAD_ARG;
   if (n > ((int64_t)1 << 27) - 1) return SPH_ERR_UNSUPPORTED;
@@ -1539,9 +1618,11 @@ static int load_impl(sph_ctx *c, int64_t n, const double *store, int64_t ld, int
   c->w_valid = false;
   c->fw_steps = 0;
   c->fw_tail = false;
-  hipLaunchKernelGGL(k_aos_to_soa, dim3(tiles_for(n)), dim3(kBlock), 0, c->stream, src, ld, (int)n, c->fields(),
+  const uint32_t *perm;
+  RCHK(load_order(c, src, ld, &perm));
+  hipLaunchKernelGGL(k_aos_to_soa, dim3(tiles_for(n)), dim3(kBlock), 0, c->stream, src, ld, (int)n, perm, c->fields(),
                      c->orig[0]);
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(wait_stream(c));
   return SPH_OK;
 }
 
@@ -1663,8 +1744,7 @@ int sph_ctx_create(const double state[49], int kernel_id, const sph_options *opt
   c->n_real = (int64_t)state[S_REALPN];
   c->n_fixed = (int64_t)state[S_FIXEDPN];
   if (c->n_real < 0) { delete c; return SPH_ERR_BAD_ARG; }
-  if (dev_alloc((void **)&c->d_red, 16 * kStripes * sizeof(long long)) != SPH_OK ||
-      dev_alloc((void **)&c->d_dtpart, 8 * kDtBlocks * sizeof(long long)) != SPH_OK ||
+  if (dev_alloc((void **)&c->d_red, (16 * kStripes + 8 * kDtBlocks) * sizeof(long long)) != SPH_OK ||
       dev_alloc((void **)&c->d_int, 256 * sizeof(int)) != SPH_OK ||
       dev_alloc((void **)&c->d_stripes, kRecLL * sizeof(long long)) != SPH_OK ||
       hipHostMalloc((void **)&c->h_int, 256 * sizeof(int)) != hipSuccess ||
@@ -1673,6 +1753,7 @@ int sph_ctx_create(const double state[49], int kernel_id, const sph_options *opt
     sph_ctx_destroy(c);
     return SPH_ERR_NOMEM;
   }
+  c->d_dtpart = c->d_red + 16 * kStripes;
   c->d_sweep = c->d_stripes + kStepLL;
   c->h_sweep = c->h_rec + kStepLL;
   if (c->opt.max_sweeps > 240) c->opt.max_sweeps = 240;
@@ -1685,7 +1766,7 @@ int sph_ctx_destroy(sph_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void *ptrs[] = {c->fbuf[0], c->fbuf[1], c->orig[0], c->orig[1], c->keys, c->keys2, c->vals, c->vals2,
-                  c->sort_tmp, c->cstart, c->ccount, c->d_dtpart, c->pm, c->st[0], c->st[1], c->tr[0], c->tr[1], c->s1[0], c->s1[1], c->pfix, c->s2, c->pd, c->trd,
+                  c->sort_tmp, c->cstart, c->pm, c->st[0], c->st[1], c->tr[0], c->tr[1], c->s1[0], c->s1[1], c->pfix, c->s2, c->pd, c->trd,
                   c->h0, c->eps, c->pf,
                   c->real, c->nb, c->cnt, c->q[0], c->q[1], c->q[2], c->q[3], c->q[4], c->energy_part,
                   c->d_red, c->d_int, c->d_stripes, c->d_staging, c->rent,

@@ -2033,16 +2033,21 @@ __global__ __launch_bounds__(256) void k_step_close(const double *part, int np, 
 // particles through LDS, so that both sides are whole lines: two rows of 256
 // bytes per wave instruction on the AoS side, 64 particles of a field on the
 // other (a lane per row touched 64 lines per load: 2M particles took 0.48 ms
-// in and 1.16 ms out, now 0.26 and 0.28).  Rows of 33 doubles keep the column
+// in and 1.16 ms out, now 0.20 each).  Rows of 33 doubles keep the column
 // accesses off each other's banks.
+// Loading takes the rows in the order perm (null: as they stand), kept in orig.
 constexpr int kTile = 64;  // kernel launches: one block of 256 threads per tile
-__global__ __launch_bounds__(256) void k_aos_to_soa(const double *aos, int64_t ld, int n, Fields F, int64_t *orig) {
+__global__ __launch_bounds__(256) void k_aos_to_soa(const double *aos, int64_t ld, int n, const uint32_t *perm,
+                                                    Fields F, int64_t *orig) {
   __shared__ double tile[kTile][F_TOTAL + 1];
+  __shared__ int64_t rows[kTile];
   const int s0 = xcd_block(blockIdx.x, gridDim.x) * kTile, m = min(kTile, n - s0), t = threadIdx.x;
+  if (t < m) rows[t] = perm ? perm[s0 + t] : s0 + t;
+  __syncthreads();
 #pragma unroll
   for (int k = 0; k < kTile * F_TOTAL / 256; k++) {
     const int row = k * (256 / F_TOTAL) + t / F_TOTAL, f = t % F_TOTAL;
-    if (row < m) tile[row][f] = aos[(size_t)(s0 + row) * ld + f];
+    if (row < m) tile[row][f] = aos[(size_t)rows[row] * ld + f];
   }
   __syncthreads();
   const int p = t & 63, s = s0 + p, w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -2052,7 +2057,17 @@ __global__ __launch_bounds__(256) void k_aos_to_soa(const double *aos, int64_t l
     const int f = 4 * k + w;
     F.f[f][s] = tile[p][f];
   }
-  if (t < kTile) orig[s] = s;
+  if (t < kTile) orig[s] = rows[t];
+}
+
+// The columns the particles' order depends on, in the store's order.
+__global__ void k_load_cols(const double *aos, int64_t ld, int n, Fields F, int64_t *orig) {
+  const int s = gtid();
+  if (s >= n) return;
+  const double *row = aos + (size_t)s * ld;
+  const int cols[4] = {F_RX, F_RY, F_RZ, F_H};
+  for (int k = 0; k < 4; k++) F.f[cols[k]][s] = row[cols[k]];
+  orig[s] = s;
 }
 
 __global__ __launch_bounds__(256) void k_soa_to_aos(Fields F, const int64_t *orig, int n, double *aos, int64_t ld) {
