@@ -70,9 +70,8 @@ __global__ void k_correct(Fields, int, const double *, const double *, int, cons
 __global__ void k_rad_exchange(Fields, int, double, double, double, double, int *);
 __global__ void k_dt_reduce(Fields, const uint8_t *, int, long long *);
 __global__ void k_gravity(Fields, const uint8_t *, int, int);
-__global__ void k_sts_stage(const double *, const double *, const double *, const double *, const double *, int,
-                            double, double, double, double, double *);
-__global__ void k_axpy_copy(double *, const double *, const double *, double, int);
+__global__ void k_sts_stage(double *, const double *, double *, double *, double *, int, int, double, double, double,
+                            double, const int *, const int *);
 template <int DIM, int KT>
 __global__ void k_diff_weights(DiffOpArgs, double *, double *);
 template <int DIM, int KT>
@@ -215,6 +214,9 @@ struct sph_ctx {
   bool ext_exact = false;  // the next extended grid waits for its size
   bool ext_built = false;  // this step built one: its counts come with the search's
   bool correct = false;    // this step's tail ends with the leapfrog corrector
+  int sts_j = 0;           // or with stage sts_j of sts_s of an RKL2 super-step
+  int sts_s = 0;
+  double sts_dt = 0.0;
   long long *d_dtpart = nullptr;  // k_dt_reduce's block partials (in d_red's allocation)
   double4 *pm = nullptr, *st[2] = {nullptr, nullptr};
   double *tr[2] = {nullptr, nullptr};  // T den of the loop-1 sweep state st[k]
@@ -1368,7 +1370,7 @@ static Phys call_phys(const sph_ctx *c, const double *state) {
 }
 
 // The tail of a step after loop 1: Newton bookkeeping, EOS and packs
-// (k_post1), loop 2, mti gravity, and in a leapfrog pass the corrector.  pending: the
+// (k_post1), loop 2, mti gravity, and a leapfrog pass's corrector or an RKL2 stage.  pending: the
 // still-active stripes of the last sweep queued, when more could follow it.
 static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr) {
   HIPCHK(mark(c, 2));
@@ -1381,6 +1383,14 @@ static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nu
     hipLaunchKernelGGL(k_correct, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), (int)c->n,
                        reinterpret_cast<const double *>(c->d_stripes + kDtLL), c->aux(0), (int)c->npad,
                        c->d_int + kGoInt, step_err(c));
+  if (rc == SPH_OK && c->sts_j > 0) {
+    double co[4];
+    RCHK(sph_sts_coeffs(c->sts_j, c->sts_s, co));
+    Fields F = c->fields();
+    hipLaunchKernelGGL(k_sts_stage, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, F.f[F_T], F.f[F_DDT], c->aux(0),
+                       c->aux(1), c->aux(2), (int)c->n, c->sts_j == 1 ? 1 : 0, co[0], co[1], co[2] * c->sts_dt,
+                       co[3] * c->sts_dt, c->d_int + kGoInt, step_err(c));
+  }
   HIPCHK(mark(c, 3));
   return rc;
 }
@@ -2055,38 +2065,23 @@ int sph_sts_coeffs(int j, int s, double out[4]) {
   return SPH_OK;
 }
 
-// sts_integrate, sts_integrator.f90:87-124: aux arrays 0 Y0, 1 Yjm1, 2 Yjm2,
-// 3 DY0, 4 DYjm1, 5 Yj (permuted with the particles at every re-sort).
+// sts_integrate, sts_integrator.f90:87-124: s steps, each with its stage behind
+// it (k_sts_stage); aux arrays 0 Y_0, 1 dY_0, 2 Y_{j-2} (permuted with the
+// particles at every re-sort).
 int sph_sts(sph_ctx *c, const double state[49], int s, double dt) {
   if (!c || !state || c->n <= 0 || s < 2) return SPH_ERR_BAD_ARG;
   (void)hipSetDevice(c->device);
-  const int n = (int)c->n;
-  unsigned G = grid_for(n);
-  c->naux = 6;
-  auto T = [&]() { return c->fields().f[F_T]; };
-  auto DDT = [&]() { return c->fields().f[F_DDT]; };
-  HIPCHK(hipMemcpyAsync(c->aux(0), T(), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-  int rc = run_step(c, state);
-  if (rc != SPH_OK) { c->naux = 0; return rc; }
-  HIPCHK(hipMemcpyAsync(c->aux(3), DDT(), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->aux(2), c->aux(0), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-  hipLaunchKernelGGL(k_axpy_copy, dim3(G), dim3(kBlock), 0, c->stream, c->aux(1), c->aux(0), c->aux(3),
-                     sts_mu_hat(1, s) * dt, n);
-  for (int j = 2; j <= s; j++) {
-    HIPCHK(hipMemcpyAsync(T(), c->aux(1), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+  c->sts_s = s;
+  c->sts_dt = dt;
+  int rc = SPH_OK;
+  for (int j = 1; j <= s && rc == SPH_OK; j++) {
+    c->naux = j == 1 ? 0 : 3;
+    c->sts_j = j;
     rc = run_step(c, state);
-    if (rc != SPH_OK) { c->naux = 0; return rc; }
-    HIPCHK(hipMemcpyAsync(c->aux(4), DDT(), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-    double mu = sts_mu(j), nu = sts_nu(j);
-    hipLaunchKernelGGL(k_sts_stage, dim3(G), dim3(kBlock), 0, c->stream, c->aux(0), c->aux(1), c->aux(2),
-                       c->aux(3), c->aux(4), n, mu, nu, sts_mu_hat(j, s) * dt, sts_gm_hat(j, s) * dt, c->aux(5));
-    HIPCHK(hipMemcpyAsync(c->aux(2), c->aux(1), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->aux(1), c->aux(5), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
   }
-  HIPCHK(hipMemcpyAsync(T(), c->aux(5), sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  c->sts_j = 0;
   c->naux = 0;
-  return SPH_OK;
+  return rc;
 }
 
 int sph_set_timing(sph_ctx *c, int on) {
