@@ -61,7 +61,7 @@ typedef struct {
   int64_t n_pairs;    /* P = sum_i |N_i| of the last step */
   int64_t loop1_pairs;/* pairs evaluated by loop 1 over all Newton sweeps */
   int sweeps;         /* Newton sweeps of the last step (0 for c1simple) */
-  int sorted;         /* 1 if the last step had to reorder particles */
+  int sorted;         /* 1 if the last step, or the load before it, reordered particles */
   double energy;      /* FP64 energy sum of loop 2 (circuit2.f90:490-492); the
                          reference computes and discards it */
   double ms_neigh, ms_loop1, ms_loop2, ms_total; /* device time of the last step's phases

@@ -210,6 +210,7 @@ struct sph_ctx {
   int64_t ncell_cap = 0;
   long long fullest = 0;   // particles in the fullest search cell last seen (0: not known)
   bool red_ready = false;  // d_red holds k_wrap_reduce's start values
+  bool load_moved = false;   // the load before this step reordered the rows
   bool flags_clear = false;  // the v / B flags' stripes are zero since load_order's k_keys
   bool ext_exact = false;  // the next extended grid waits for its size
   bool ext_built = false;  // this step built one: its counts come with the search's
@@ -824,7 +825,8 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   RCHK(ensure_cells(c, nkeys));
   // 3. cell keys, sortedness, radix sort + reorder when needed; keys and
   //    cell starts of the same positions on the same grid are still valid
-  c->stats.sorted = 0;
+  c->stats.sorted = c->load_moved ? 1 : 0;
+  c->load_moved = false;
   const bool keys_kept = c->keys_version == c->pos_version && c->keys_n == n && c->keys_nkeys == nkeys &&
                          same_grid(g, c->keys_grid);
   if (!keys_kept) {
@@ -1556,6 +1558,7 @@ static int load_order(sph_ctx *c, const double *src, int64_t ld, const uint32_t 
   const int n = (int)c->n;
   const unsigned G = grid_for(n);
   *perm = nullptr;
+  c->load_moved = false;
   if (c->n_real <= 0) return SPH_OK;
   Fields F;
   for (int f = 0; f < F_TOTAL; f++) F.f[f] = c->fbuf[1] + (size_t)f * c->npad;
@@ -1583,6 +1586,7 @@ static int load_order(sph_ctx *c, const double *src, int64_t ld, const uint32_t 
                                               bits_of(nkeys), c->stream));
     std::swap(c->keys, c->keys2);
     *perm = c->vals2;
+    c->load_moved = true;
   }
   hipLaunchKernelGGL(k_cell_start, dim3(grid_for(n + 1)), dim3(kBlock), 0, c->stream, c->keys, n, (uint32_t)nkeys,
                      c->cstart);
