@@ -638,10 +638,10 @@ static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
     c->ext_total = ll[kExtLL];
     c->stats.ext_records = c->ext_total;
     ext_short = (size_t)c->ext_total + 8 > c->ext_rec_cap;
-    if (ext_short) {  // records were left out: build it again with room
-      c->ext_version = 0;
-      c->ext_exact = true;
-    }
+    // the grid is kept only now that it is known to be whole; where records
+    // were left out it is built again with room
+    c->ext_version = ext_short ? 0 : c->pos_version;
+    c->ext_exact = ext_short;
   }
   if (c->flags_pending) {  // k_prep's v / B flags of this step
     c->step_flags = 0;
@@ -989,7 +989,9 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
         c->ext_built = true;
       }
       c->ext_total = total;
-      c->ext_version = c->pos_version;
+      // a grid being filled counts as kept once its size is read back
+      // (finish_neighbours): a step that ends before that leaves none
+      c->ext_version = c->ext_built ? 0 : c->pos_version;
       c->ext_cur = c->cur;
       c->ext_n = n;
       c->ext_grid = g;
