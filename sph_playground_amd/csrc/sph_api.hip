@@ -235,6 +235,7 @@ struct sph_ctx {
   uint32_t *nb = nullptr;
   int nb_cap = 0;
   int last_maxcnt = 0;  // longest neighbour list of the last search
+  int even = -1;        // whether its lists were even (lists_even; -1: none since the load)
   long long step_flags = 0;       // k_prep's v / B flags of this step
   bool loop2_pending = false;     // loop 2's read-back still to be taken
   bool neigh_pending = false;     // the search's read-back still to be taken (loop 1's first sync brings it)
@@ -652,6 +653,7 @@ static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
   c->stats.n_pairs = stripe_sum(ll, 0);
   int maxcnt = (int)stripe_max(ll, 1);
   c->last_maxcnt = maxcnt;
+  c->even = lists_even(maxcnt, c->n_real, c->stats.n_pairs) ? 1 : 0;
   c->stats.ms_k_neigh = elapsed(c, c->ev[4], c->ev[7]);
   if (bits & EB_TRUNC) return SPH_ERR_NEIGH_TRUNCATED;
   if (!(bits & EB_OVERFLOW)) return SPH_OK;
@@ -1053,6 +1055,14 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
 }
 
 // ------------------------------------------------------------ step: loops
+// The equation set of loop 2 where one is fixed at compile time (2D and 3D:
+// hydro, magnetohydro, hydro with FLD), else -1.
+static int loop2_terms(const sph_ctx *c, const Phys &P) {
+  if (c->loop2_generic || P.dim < 2) return -1;
+  const int terms = (P.hydro ? 1 : 0) | (P.magneto ? 2 : 0) | (P.diff ? 4 : 0) | (P.fld ? 8 : 0);
+  return terms == kSpecHydro || terms == kSpecMhd || terms == kSpecHydroFld ? terms : -1;
+}
+
 // Lanes per particle of the pair loops (1, 4 or 8).  One lane walks a list
 // alone: on a lattice in row order the wave's 64 k-th neighbours lie side by
 // side and every list is as long, and the loop is bound by its arithmetic
@@ -1064,8 +1074,8 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
 //     MHD in FP32: loop 2 3.44 -> 1.64 ms; sweeps 2.65 -> 1.57 ms);
 //   3D diffusion: 4 (100^3 jittered 0.05: loop 2 0.305 -> 0.247 ms FP32, loop 1
 //     0.458 -> 0.361 FP64), 8 below 40k particles (32^3 0.036 -> 0.018 ms),
-//     but 1 for 700k particles and more whose last lists were even, within
-//     5 % of their mean (100^3 lattice 0.219 against 0.247 ms), and 1 for loop
+//     but 1 for 700k particles and more whose lists are even, within 5 % of
+//     their mean (100^3 lattice 0.219 against 0.247 ms), and 1 for loop
 //     2 of the 2nw operators from 300k particles on (80^3 0.558 against
 //     0.592 ms);
 //   2D, some 28 neighbours: 8 below 40k particles (64^2: sweeps 0.056 ->
@@ -1075,19 +1085,28 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
 // below 100k particles in 3D diffusion (40^3 0.038 -> 0.031 ms, 64^3 0.072
 // against 0.086) and below 40k in 2D; loop 2 of 2D stays on one lane, since
 // the accelerations of a 2D set at rest are the small remainder of large terms
-// and another order's rounding moves them by 4e-5.
-static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2) {
+// and another order's rounding moves them by 4e-5.  The same for loop 2 of
+// particles that move where the equation set is not fixed (k_loop2).
+// `even` is of the step's own lists wherever it changes how a sum is rounded
+// (run_advanced), so that a step's bits depend on nothing before it.
+static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2, bool even) {
   const int64_t n = c->n;
   const bool mixed = c->opt.precision == 1;
   if (P.dim == 1 || (mixed && loop2 && P.dim == 2)) return 1;
+  if (mixed && loop2 && P.hydro && loop2_terms(c, P) < 0) return 1;
   if (P.dim == 3 && P.hydro) return 8;
   if (mixed && !loop2) return n < (P.dim == 3 ? 100000 : 40000) ? 8 : 1;
   if (n < 40000) return 8;
   if (P.dim == 2) return n < 150000 ? 4 : 1;
   if (loop2 && P.diff && !P.fld && (P.ddw == 403 || P.ddw == 404)) return n < 300000 ? 4 : 1;
-  const bool even =
-      c->stats.n_pairs > 0 && (double)c->last_maxcnt * (double)c->n_real <= 1.05 * (double)c->stats.n_pairs;
   return n >= 700000 && even ? 1 : 4;
+}
+
+// Whether the evenness of the lists decides over lanes whose sums it rounds
+// otherwise: loop 2, and loop 1 in FP64 (in FP32 its order is the list's).
+static bool lanes_follow_lists(const sph_ctx *c, const Phys &P) {
+  auto differ = [&](bool loop2) { return loop_lanes(c, P, loop2, false) != loop_lanes(c, P, loop2, true); };
+  return differ(true) || (c->opt.precision != 1 && differ(false));
 }
 
 // fn(constant G) for lanes = 1, 4 (where HAS4) or 8 (where HAS8)
@@ -1118,7 +1137,7 @@ static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simpl
 #undef L1S
     return;
   }
-  const int lanes = loop_lanes(c, a.p, false);
+  const int lanes = loop_lanes(c, a.p, false, c->even == 1);
 #define L1(GR, PT)                                                                                           \
   with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1>(lanes, [&](auto l) {                          \
     constexpr int G = decltype(l)::value;                                                                    \
@@ -1252,7 +1271,7 @@ static void launch_loop2_d23(sph_ctx *c, int dim, int lanes, void *args) {
 }
 
 template <typename V4>
-static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pending) {
+static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pending, int even) {
   const int n = (int)c->n;
   Fields F = c->fields();
   unsigned G = grid_for(n);
@@ -1293,6 +1312,9 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
   sel.serr = step_err(c) + kErrSearch;
   sel.err1 = step_err(c) + kErrLoop1;
   sel.pending = pending;
+  sel.lists = c->d_stripes + kSearchLL;
+  sel.n_real = c->n_real;
+  sel.even = even;
   sel.go = c->d_int + kGoInt;
   hipLaunchKernelGGL(k_post1<V4>, dim3(G), dim3(kBlock), 0, c->stream, F, sel, c->real, n, P.adden ? 1 : 0,
                      c->do_eos, c->eos_iso, c1, P.gamma, q0, q1, q2, q3, q4,
@@ -1319,18 +1341,11 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
   // fab with one tensor for every pair and no velocity term: the loop
   // without run-time choices
   const bool fab = !generic && P.ddw == 400 && q1 == nullptr && q4 == nullptr;
-  // the generic loop with its equation set fixed at compile time where one
-  // is built for it (2D and 3D: hydro, magnetohydro, hydro with FLD)
-  const int terms =
-      c->loop2_generic ? -1 : (P.hydro ? 1 : 0) | (P.magneto ? 2 : 0) | (P.diff ? 4 : 0) | (P.fld ? 8 : 0);
-  // FP32 sums of particles that move stay in list order, on eight lanes where
-  // the equation set is fixed (k_loop2), else on one
-  const bool spec = terms == kSpecHydro || terms == kSpecMhd || terms == kSpecHydroFld;
-  const int lanes = P.hydro && !spec && c->opt.precision == 1 ? 1 : loop_lanes(c, P, true);
-  if (generic && P.dim >= 2 && terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, lanes, &a);
-  else if (generic && P.dim >= 2 && terms == kSpecMhd) launch_loop2_d23<MODE_SPEC + kSpecMhd>(c, P.dim, lanes, &a);
-  else if (generic && P.dim >= 2 && terms == kSpecHydroFld)
-    launch_loop2_d23<MODE_SPEC + kSpecHydroFld>(c, P.dim, lanes, &a);
+  const int terms = generic ? loop2_terms(c, P) : -1;
+  const int lanes = loop_lanes(c, P, true, c->even == 1);
+  if (terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, lanes, &a);
+  else if (terms == kSpecMhd) launch_loop2_d23<MODE_SPEC + kSpecMhd>(c, P.dim, lanes, &a);
+  else if (terms == kSpecHydroFld) launch_loop2_d23<MODE_SPEC + kSpecHydroFld>(c, P.dim, lanes, &a);
   else if (generic) launch_loop2_d<MODE_GENERIC>(c, P.dim, lanes, &a);
   else if (fab) launch_loop2_d<MODE_FAB>(c, P.dim, lanes, &a);
   else launch_loop2_d<MODE_DIFF>(c, P.dim, lanes, &a);
@@ -1375,11 +1390,13 @@ static Phys call_phys(const sph_ctx *c, const double *state) {
 
 // The tail of a step after loop 1: Newton bookkeeping, EOS and packs
 // (k_post1), loop 2, mti gravity, and a leapfrog pass's corrector or an RKL2 stage.  pending: the
-// still-active stripes of the last sweep queued, when more could follow it.
-static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr) {
+// still-active stripes of the last sweep queued, when more could follow it;
+// even: what the loops' lanes take the lists for, while the step's own are not
+// known (-1: they are, or no matter).
+static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr, int even = -1) {
   HIPCHK(mark(c, 2));
-  int rc = c->opt.precision == 1 ? run_post_and_loop2<float4>(c, P, pending)
-                                   : run_post_and_loop2<double4>(c, P, pending);
+  int rc = c->opt.precision == 1 ? run_post_and_loop2<float4>(c, P, pending, even)
+                                   : run_post_and_loop2<double4>(c, P, pending, even);
   if (rc == SPH_OK && c->gravity)
     hipLaunchKernelGGL(k_gravity, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, c->fields(), c->real, (int)c->n,
                        c->gravity);
@@ -1422,7 +1439,10 @@ static bool loop2_reads_flags(const Phys &P) {
 // that overflowed leave loop 1 and k_post1 idle (device-side checks), so the
 // step searches again with room and starts over; a batch that ends with
 // particles still active leaves its tail idle and is followed by more sweeps
-// and another tail.
+// and another tail.  Where the evenness of the lists decides over the lanes
+// and so over the sums' rounding, the step is queued for lists like the last
+// ones' and done again if its own are not (the tail then stayed idle); the first
+// after a load waits for its own.
 static int run_advanced(sph_ctx *c, const Phys &P) {
   const int maxsw = sweep_cap(c);
   int first = 1, sweeps = 0, bits = 0;
@@ -1442,6 +1462,23 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
     const int rc2 = finish_loop2(c);
     return rc != SPH_OK ? rc : rc2;
   }
+  int even = -1;
+  if (c->neigh_pending && lanes_follow_lists(c, P)) {
+    even = c->even;
+    if (even < 0) {
+      HIPCHK(copy_record(c, 0));
+      HIPCHK(wait_stream(c));
+      const int fin = take_neighbours(c);
+      if (fin == kRedoNeigh) RCHK(build_neighbours(c));
+      else RCHK(fin);
+    }
+  }
+  auto start_over = [&] {
+    first = 1; sweeps = 0; pairs = 0; ms1 = 0.f;
+    even = -1;
+  };
+  // the step's own lists are known: were the loops queued for such?
+  auto other_lists = [&] { return even >= 0 && c->even != even; };
   for (;;) {
     const int last = std::min(maxsw, first + std::max(1, c->sweep_hint) - 1);
     launch_sweeps(c, P, first, last);
@@ -1452,12 +1489,18 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
       const int fin = take_neighbours_now(c);
       if (fin == kRedoNeigh) {
         RCHK(build_neighbours(c));
-        first = 1; sweeps = 0; pairs = 0; ms1 = 0.f;
+        start_over();
         continue;
       }
       RCHK(fin);
+      if (other_lists()) {
+        HIPCHK(hipMemsetAsync(step_err(c) + kErrLoop1, 0, 2 * sizeof(int), c->stream));
+        start_over();
+        continue;
+      }
+      even = -1;
     }
-    const int rc = enqueue_tail(c, P, last < maxsw ? c->d_sweep + (size_t)last * kSweepRegion : nullptr);
+    const int rc = enqueue_tail(c, P, last < maxsw ? c->d_sweep + (size_t)last * kSweepRegion : nullptr, even);
     // the search's read-back if still pending, error words, the tail's record
     // and the sweep regions: one copy
     HIPCHK(copy_record(c, last));
@@ -1469,10 +1512,16 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
       const int fin = take_neighbours_now(c);
       if (fin == kRedoNeigh) {
         RCHK(build_neighbours(c));
-        first = 1; sweeps = 0; pairs = 0; ms1 = 0.f;
+        start_over();
         continue;
       }
       RCHK(fin);
+      if (other_lists()) {
+        HIPCHK(hipMemsetAsync(step_err(c) + kErrLoop1, 0, 2 * sizeof(int), c->stream));
+        start_over();
+        continue;
+      }
+      even = -1;
     }
     for (int it = first; it <= last; it++) {
       const long long *r = c->h_sweep + (size_t)it * kSweepRegion;
@@ -1623,6 +1672,7 @@ static int load_impl(sph_ctx *c, int64_t n, const double *store, int64_t ld, int
   }
   c->cur = 0;
   c->fullest = 0;
+  c->even = -1;
   c->pos_version++;
   c->vb_version++;
   c->h_version++;

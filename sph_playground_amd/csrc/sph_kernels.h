@@ -241,17 +241,27 @@ struct Loop1Args {
   int sweep;
 };
 
+// Even neighbour lists: the longest within 5 % of the mean.
+__host__ __device__ inline bool lists_even(long long longest, long long n_real, long long pairs) {
+  return pairs > 0 && (double)longest * (double)n_real <= 1.05 * (double)pairs;
+}
+
 // Where k_post1 finds loop 1's result: st[*which] of the two sweep buffers
 // (fin0 alone when which is null).  Nothing is written when the search (serr)
 // or loop 1 (err1) raised an error bit (the step then stops or searches again)
 // or when the last sweep queued before the tail left particles active
 // (`pending`, its still-active stripes; null: no matter): more sweeps and
-// another tail follow.  *go tells loop 2 which it was.
+// another tail follow; nor when the lists are not as even as the loops queued
+// with it assume (`even`, -1: no matter; `lists`: the search's pair counts and
+// list lengths).  *go tells loop 2 which it was.
 struct PostSel {
   const double4 *fin0, *fin1;
   const int *which;
   const int *serr, *err1;
   const long long *pending;
+  const long long *lists;
+  long long n_real;
+  int even;
   int *go;
 };
 

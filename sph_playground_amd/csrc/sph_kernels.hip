@@ -1296,8 +1296,14 @@ __global__ __launch_bounds__(256) void k_post1(Fields F, PostSel sel, const uint
   // MHD tube 3.3 ms)
   if (threadIdx.x < 64) {
     const unsigned long long more = __ballot(sel.pending && sel.pending[threadIdx.x] != 0);
+    bool other = false;
+    if (sel.even >= 0) {
+      const long long pairs = wave_sum(sel.lists[threadIdx.x]);
+      const long long longest = wave_max(sel.lists[kStripes + threadIdx.x]);
+      other = lists_even(longest, sel.n_real, pairs) != (sel.even != 0);
+    }
     if (threadIdx.x == 0) {
-      skip = more != 0 || *sel.serr != 0 || *sel.err1 != 0;
+      skip = more != 0 || other || *sel.serr != 0 || *sel.err1 != 0;
       if (blockIdx.x == 0) *sel.go = !skip;
     }
   }
