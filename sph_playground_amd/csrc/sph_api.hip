@@ -1063,27 +1063,47 @@ static int loop2_terms(const sph_ctx *c, const Phys &P) {
   return terms == kSpecHydro || terms == kSpecMhd || terms == kSpecHydroFld ? terms : -1;
 }
 
+// Whether loop 2 runs its general form (k_loop2 with every term, or a fixed
+// equation set): all but diffusion alone with a Hessian operator.
+static bool loop2_general(const Phys &P) {
+  return !(P.diff && !P.hydro && !P.artts && !P.magneto && !P.fld &&
+           (P.ddw == 400 || P.ddw == 401 || P.ddw == 402));
+}
+
 // Lanes per particle of the pair loops (1, 4 or 8).  One lane walks a list
 // alone: on a lattice in row order the wave's 64 k-th neighbours lie side by
-// side and every list is as long, and the loop is bound by its arithmetic
-// (loop 1 at 128^3 in FP32 0.452 ms, split over 4 lanes 0.495, over 8 0.566).
+// side and every list is as long, and the loop is bound by its arithmetic.
 // Where lists differ the wave waits for its longest and its k-th neighbours
 // drift apart; several lanes of one particle read runs of its cell rows
-// instead, and few particles then still fill the chip:
-//   3D, particles that move (hydro, MHD, FLD): 8 (the tube of 1M particles,
-//     MHD in FP32: loop 2 3.44 -> 1.64 ms; sweeps 2.65 -> 1.57 ms);
-//   3D diffusion: 4 (100^3 jittered 0.05: loop 2 0.305 -> 0.247 ms FP32, loop 1
-//     0.458 -> 0.361 FP64), 8 below 40k particles (32^3 0.036 -> 0.018 ms),
-//     but 1 for 700k particles and more whose lists are even, within 5 % of
-//     their mean (100^3 lattice 0.219 against 0.247 ms), and 1 for loop
-//     2 of the 2nw operators from 300k particles on (80^3 0.558 against
-//     0.592 ms);
+// instead, and few particles then still fill the chip.  Measured, one lane
+// against several, loop 2 where nothing else is said (us):
+//   3D below 40k particles: 8 (2nw FP64 at 30^3 108 against 49).
+//   Particles that move (hydro, MHD, FLD): 8 (FP32 MHD tube of 1M 3440 against
+//     1640, sweeps 2650 against 1570; FP64 hydro tube of 300k 1118 against
+//     515), but even lists take 1 where more lanes only add work: in FP32 from
+//     170k particles (lattice, hydro: 56^3 127 and 135, 64^3 154 and 192,
+//     128^3 1207 and 1500; sweeps with grad T 64^3 69 and 92), in FP64 the
+//     sets that are not fixed at compile time from 110k (hydro with diffusion:
+//     46^3 208 and 194, 58^3 338 and 364, 100^3 1522 and 1862).
+//   General form without hydro: 4, even lists 1 from 110k in FP64 (2nw: 48^3
+//     141 and 159, 64^3 272 and 337; FLD 46^3 200 and 179, 64^3 387 and 436) and
+//     from 150k in FP32 (2nw: 52^3 124 and 114, 54^3 127 and 135, 100^3 722 and
+//     823; FLD 58^3 152 and 173; jittered, uneven: 64^3 320 and 222); the 2nw
+//     operators 1 from 300k on also where lists are uneven (FP64 80^3 616 and
+//     661).
+//   fab (and FP64 n2w, fw): 4, even lists 1 from 700k (FP32 lattice 88^3 172
+//     and 174, 100^3 236 and 254; jittered 100^3 330 and 243; FP64 lattice
+//     100^3 366 and 361, 128^3 666 and 731; jittered 128^3 1025 and 741).
+//   n2w and fw in FP32: 4 below 225k, then 1 (60^3 102 and 99, 64^3 104 and 113,
+//     100^3 393 and 431, jittered 387 and 409).
+//   Loop 1 in FP64 without hydro: 4, even lists 1 from 700k (128^3 677 and
+//     723, jittered 1015 and 733).
 //   2D, some 28 neighbours: 8 below 40k particles (64^2: sweeps 0.056 ->
 //     0.025 ms, loop 2 0.029 -> 0.011), 4 below 150k (256^2 0.051 -> 0.041 and
 //     0.032 -> 0.025), then 1 (512^2 0.078 against 0.089, 0.069 against 0.071).
 // FP32: loop 1 keeps its sums in list order on 8 lanes (k_loop1), which pays
-// below 100k particles in 3D diffusion (40^3 0.038 -> 0.031 ms, 64^3 0.072
-// against 0.086) and below 40k in 2D; loop 2 of 2D stays on one lane, since
+// below 100k particles in 3D diffusion (46^3 45.8 against 43, 58^3 58 against
+// 75) and below 40k in 2D; loop 2 of 2D stays on one lane, since
 // the accelerations of a 2D set at rest are the small remainder of large terms
 // and another order's rounding moves them by 4e-5.  The same for loop 2 of
 // particles that move where the equation set is not fixed (k_loop2).
@@ -1093,20 +1113,33 @@ static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2, bool even) {
   const int64_t n = c->n;
   const bool mixed = c->opt.precision == 1;
   if (P.dim == 1 || (mixed && loop2 && P.dim == 2)) return 1;
-  if (mixed && loop2 && P.hydro && loop2_terms(c, P) < 0) return 1;
-  if (P.dim == 3 && P.hydro) return 8;
-  if (mixed && !loop2) return n < (P.dim == 3 ? 100000 : 40000) ? 8 : 1;
+  if (P.dim == 2) {
+    if (n < 40000) return 8;
+    return !mixed && n < 150000 ? 4 : 1;
+  }
+  const bool fixed_set = loop2_terms(c, P) >= 0;
+  if (P.hydro) {
+    if (mixed && loop2 && !fixed_set) return 1;
+    if (mixed) return n >= 170000 && even ? 1 : 8;
+    return loop2 && !fixed_set && n >= 110000 && even ? 1 : 8;
+  }
+  if (mixed && !loop2) return n < 100000 ? 8 : 1;
   if (n < 40000) return 8;
-  if (P.dim == 2) return n < 150000 ? 4 : 1;
-  if (loop2 && P.diff && !P.fld && (P.ddw == 403 || P.ddw == 404)) return n < 300000 ? 4 : 1;
+  if (loop2 && loop2_general(P)) {
+    if (n >= (mixed ? 150000 : 110000) && even) return 1;
+    return P.diff && !P.fld && (P.ddw == 403 || P.ddw == 404) && n >= 300000 ? 1 : 4;
+  }
+  if (mixed && P.ddw != 400) return n < 225000 ? 4 : 1;
   return n >= 700000 && even ? 1 : 4;
 }
 
 // Whether the evenness of the lists decides over lanes whose sums it rounds
-// otherwise: loop 2, and loop 1 in FP64 (in FP32 its order is the list's).
+// otherwise (FP32 sums of loop 1, and of loop 2 of a fixed equation set, are in
+// the list's order on any lanes).
 static bool lanes_follow_lists(const sph_ctx *c, const Phys &P) {
   auto differ = [&](bool loop2) { return loop_lanes(c, P, loop2, false) != loop_lanes(c, P, loop2, true); };
-  return differ(true) || (c->opt.precision != 1 && differ(false));
+  if (c->opt.precision == 1) return loop2_terms(c, P) < 0 && differ(true);
+  return differ(true) || differ(false);
 }
 
 // fn(constant G) for lanes = 1, 4 (where HAS4) or 8 (where HAS8)
@@ -1287,8 +1320,7 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
     memcpy(&c1, c->h_ll + 4, sizeof(double));
   }
   // which j-side packs loop 2 may gather (must match k_loop2)
-  const bool generic = !(P.diff && !P.hydro && !P.artts && !P.magneto && !P.fld &&
-                         (P.ddw == 400 || P.ddw == 401 || P.ddw == 402));
+  const bool generic = loop2_general(P);
   const bool want_v = P.adden || P.artts || P.hydro || P.magneto;
   const bool want_q2 = generic && ((P.diff && P.fld) || P.artts);
   const bool want_q3 = generic && P.diff && (P.fld || P.ddw == 403 || P.ddw == 404);
@@ -1423,8 +1455,7 @@ static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nu
 // them only for a diffusion tensor from B (k_loop2).  Otherwise a step need
 // not wait for the flags before its tail: they come back at its end.
 static bool loop2_reads_flags(const Phys &P) {
-  const bool generic = !(P.diff && !P.hydro && !P.artts && !P.magneto && !P.fld &&
-                         (P.ddw == 400 || P.ddw == 401 || P.ddw == 402));
+  const bool generic = loop2_general(P);
   if (!generic) return true;
   const bool v_always = P.hydro || P.magneto || P.artts;
   const bool tensor_b = P.diff && !P.fld && P.diso == 0;

@@ -1731,7 +1731,7 @@ void k_loop2(Loop2Args<V4> a) {
         PT mb_x = ((PT(0.5) * b2b - bbx * bbx) * nwbx - bbx * bby * nwby - bbx * bbz * nwbz) * mu0inv;
         PT mb_y = (-bby * bbx * nwbx + (PT(0.5) * b2b - bby * bby) * nwby - bby * bbz * nwbz) * mu0inv;
         PT mb_z = (-bbz * bbx * nwbx - bbz * bby * nwby + (PT(0.5) * b2b - bbz * bbz) * nwbz) * mu0inv;
-        if constexpr (ORD) {  // rounded as the one-lane loop is
+        if constexpr (DIM == 3 && F32 && SPEC) {  // rounded alike on one lane and on eight
           minus(L2_VX, 2, mb, fmaf(ma_x, i_ra2_oa, mb_x * i_rb2_ob));
           minus(L2_VY, 2, mb, fmaf(mb_y, i_rb2_ob, ma_y * i_ra2_oa));
           minus(L2_VZ, 2, mb, fmaf(mb_z, i_rb2_ob, ma_z * i_ra2_oa));

@@ -1,0 +1,126 @@
+"""Lanes per particle on each side of the lines that even lists draw, and every
+field of the mixed path at each line.
+
+Lattices whose lists are even at the first step (h at entry 1.03 spacings holds
+whole shells of neighbours) lie on both sides of the sizes from which such lists
+take one lane: FP64 within 1e-12 of each field's largest value (a vector's, over its
+components: by symmetry some of them are rounding alone; a sum in another order
+moves it by its rounding), the bar of the parity tests.
+
+The mixed path is held to the FP64 oracle over the same three sweeps in which no
+particle freezes (tolerance 1e-300), so that grad T and what reads it are taken
+at the same h on both sides: every field loop 1 and loop 2 write, dT/dt, grad T
+and the FLD velocity among them, within 1e-4 of the field's norm (a vector's, over
+its components), the bar of the mixed-precision tests.
+
+The FP32 sums of particles that move run in list order on one lane and on eight:
+a step whose lists the step before found even gives the bits of a first step.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from sph_playground_amd import consts as C
+from sph_playground_amd import problems as P
+from tests.test_gpu_loop_lanes import CASES as LINES
+
+pytestmark = pytest.mark.gpu
+
+SCHEDULE = dict(max_sweeps=3, tol=1e-300)
+FULL = dict(tensor="full", kappa_perp=0.1)
+
+
+def _diffusion(side, ddw):
+    return P.diffusion3d(side, ddw=ddw, b=(1.0, 0.4, 0.3), kind="square", h_scale=1.03)
+
+
+def _moving(side, equations="hydro", fld=False):
+    n = side ** 3
+    box = (0.0, 1.0, 0.0, 1.0, 0.0, 1.0)
+    state, st = P.random_slab3d(n, box=box, hfac=1.0, equations=equations, fld=fld, lattice=(side,) * 3,
+                                velocity_seed=2)
+    pos, dx = P.lattice_positions(3, side, box)
+    x = 2.0 * np.pi * pos[:, 0]
+    st[:, 0:3] = pos
+    for f, v in (("m", 1.0 / n), ("den", 1.0), ("h", 1.03 * dx), ("u", 1.5 + 0.3 * np.sin(x)), ("t", 1.0 + 0.2 * np.cos(x))):
+        st[:, getattr(C, "es_" + f) - 1] = v
+    P._eos_fill(st, 5.0 / 3.0)
+    return state, st
+
+
+EVEN = [
+    # general form: from 110,000 particles in FP64, 150,000 in FP32
+    ("2nw_47", lambda: _diffusion(47, "2nw-+"), FULL, ("fp64",)),
+    ("2nw_48", lambda: _diffusion(48, "2nw-+"), FULL, ("fp64",)),
+    ("2nw_sd_53", lambda: _diffusion(53, "2nw+-"), FULL, ("mixed",)),
+    ("2nw_sd_54", lambda: _diffusion(54, "2nw+-"), FULL, ("mixed",)),
+    # n2w and fw in FP32: from 225,000
+    ("n2w_60", lambda: _diffusion(60, "n2w"), FULL, ("mixed",)),
+    ("fw_61", lambda: _diffusion(61, "fw"), FULL, ("mixed",)),
+]
+
+VECTORS = (("ax", "ay", "az"), ("dbx", "dby", "dbz"), ("dtdx", "dtdy", "dtdz"))
+SCALARS = ("den", "h", "om", "p", "c", "du", "dh", "ddt", "vfld")
+
+
+def _check(state, st, precision, kw):
+    from sph_playground_amd.engine import Engine
+    nr = int(state[C.ec_realpn - 1])
+    okw = {"neigh_cap": kw["neigh_cap"]} if "neigh_cap" in kw else {}
+    if kw.get("tensor") == "full":
+        okw.update(tensor_mode=1, kappa_perp=kw["kappa_perp"])
+    if precision == "mixed" and state[C.ec_adden - 1] == C.YESNO["yes"]:
+        okw.update(SCHEDULE)
+        kw = dict(kw, max_sweeps=SCHEDULE["max_sweeps"], newton_tol=SCHEDULE["tol"])
+    ref = oracle.iterate(state, st, kernel=1, **okw)
+    eng = Engine(state, kernel="m6", precision=precision, **kw)
+    got = st.copy()
+    eng.iterate(got)
+    assert eng.stats()["n_pairs"] == ref["off"][-1] and eng.stats()["sweeps"] == ref["sweeps"]
+    eng.close()
+    ref = ref["store"]
+    norms = {}
+    for group in VECTORS + tuple((f,) for f in SCALARS):
+        k = [getattr(C, "es_" + f) - 1 for f in group]
+        diff = got[:nr, k] - ref[:nr, k]
+        norms[group] = np.linalg.norm(ref[:nr, k])
+        print(group, "%.1e of %.1e" % (np.linalg.norm(diff), norms[group]), flush=True)
+        if precision == "fp64":
+            assert np.abs(diff).max() <= 1e-12 * np.abs(ref[:nr, k]).max(), group
+        else:
+            assert np.linalg.norm(diff) <= 1e-4 * norms[group], group
+    assert norms[VECTORS[0]] > 0.0 or norms[("ddt",)] > 0.0  # loop 2 wrote something
+
+
+@pytest.mark.parametrize("name,make,kw,precision", [(n, m, kw, p) for n, m, kw, ps in EVEN for p in ps],
+                         ids=["%s-%s" % (e[0], p) for e in EVEN for p in e[3]])
+def test_even_lists_on_each_side(gpu, name, make, kw, precision):
+    print("case", name, precision, flush=True)
+    state, st = make()
+    _check(state, st, precision, kw)
+
+
+@pytest.mark.parametrize("name,make,kw", LINES, ids=[c[0] for c in LINES])
+def test_every_field_of_the_mixed_path(gpu, name, make, kw):
+    print("case", name, flush=True)
+    state, st = make()
+    _check(state, st, "mixed", kw)
+
+
+@pytest.mark.parametrize("equations,fld", [("hydro", False), ("magnetohydro", False), ("hydro", True)],
+                         ids=["hydro", "mhd", "fld"])
+def test_even_lists_of_moving_particles_keep_their_bits(gpu, equations, fld):
+    # 56^3 = 175,616 particles; cells of a quarter radius hold one particle
+    # each, so their order is the same however it came about
+    from sph_playground_amd.engine import Engine
+    state, st = _moving(56, equations, fld)
+    eng = Engine(state, kernel="m6", precision="mixed", cell_div=4)
+    eng.load(st)
+    eng.step()
+    first = eng.save()
+    eng.step()
+    second = eng.save()
+    eng.load(first)
+    eng.step()
+    assert np.array_equal(eng.save(), second)
+    eng.close()
