@@ -1158,14 +1158,20 @@ template <int DIM, int KT>
 static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simple, Fields F) {
   bool mixed = c->opt.precision == 1;
   if (simple) {
-    // FP32 sums keep the list order: one lane
-    const unsigned B = grid_for((int64_t)a.n * (mixed ? 1 : 8));
-#define L1S(GR, PT, G) \
-  hipLaunchKernelGGL((k_loop1_simple<DIM, KT, GR, PT, G>), dim3(B), dim3(kBlock), 0, c->stream, a, F)
+    // FP32 sums keep the list order: one lane.  FP64: loop 1's lanes of uneven
+    // lists (1M particles in 1D, us: one lane 32, eight 76; 1000^2 82, 122;
+    // 100^3 lattice 302, four 267, jittered 403, 279)
+    const int lanes = mixed ? 1 : loop_lanes(c, a.p, false, false);
+#define L1S(GR, PT)                                                                                          \
+  with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1 && std::is_same_v<PT, double>>(lanes, [&](auto l) { \
+    constexpr int G = decltype(l)::value;                                                                    \
+    hipLaunchKernelGGL((k_loop1_simple<DIM, KT, GR, PT, G>), dim3(grid_for((int64_t)a.n * G)), dim3(kBlock), 0, \
+                       c->stream, a, F);                                                                     \
+  })
     if (mixed) {
-      if (grad == 0) { L1S(0, float, 1); } else if (grad == 1) { L1S(1, float, 1); } else { L1S(2, float, 1); }
+      if (grad == 0) { L1S(0, float); } else if (grad == 1) { L1S(1, float); } else { L1S(2, float); }
     } else {
-      if (grad == 0) { L1S(0, double, 8); } else if (grad == 1) { L1S(1, double, 8); } else { L1S(2, double, 8); }
+      if (grad == 0) { L1S(0, double); } else if (grad == 1) { L1S(1, double); } else { L1S(2, double); }
     }
 #undef L1S
     return;

@@ -1227,7 +1227,8 @@ __global__ __launch_bounds__(256) void k_loop1_simple(Loop1Args<double4> a, Fiel
     if constexpr (GRAD != 0) d.sb = a.cur[j];
     return d;
   };
-  for_neighbours<G, 2>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
+  // gathers in flight: four on one lane (FP32 100^3 lattice, a step 0.943 ms, with two 0.967)
+  for_neighbours<G, G == 1 ? 4 : 2>(a.nb, s, sub, a.npad, nn, load, [&](const J &d) {
     double xb = d.pb.x, yb = d.pb.y, zb = d.pb.z;
     if (d.code != kNoImage) image_shift(xb, yb, zb, d.code, a.b);
     PT r0 = (PT)(pa.x - xb), r1 = (PT)(pa.y - yb), r2 = (PT)(pa.z - zb);
@@ -2441,12 +2442,13 @@ __global__ void k_sts_stage(double *T, const double *DT, double *y0, double *dy0
   template __global__ void k_loop2<DIM, KT, PT, V4, MODE_SPEC + kSpecHydroFld, G>(Loop2Args<V4>);
 #define SPH_INST_1D(KT)                                                                    \
   SPH_INST_L1(1, KT, double, 1) SPH_INST_L1(1, KT, float, 1)                               \
-  SPH_INST_L1S(1, KT, double, 8) SPH_INST_L1S(1, KT, float, 1)                             \
+  SPH_INST_L1S(1, KT, double, 1) SPH_INST_L1S(1, KT, float, 1)                             \
   SPH_INST_L2(1, KT, double, double4, 1) SPH_INST_L2(1, KT, float, float4, 1)
 #define SPH_INST_23(DIM, KT)                                                               \
   SPH_INST_L1(DIM, KT, double, 1) SPH_INST_L1(DIM, KT, double, 4) SPH_INST_L1(DIM, KT, double, 8) \
   SPH_INST_L1(DIM, KT, float, 1) SPH_INST_L1(DIM, KT, float, 8)                            \
-  SPH_INST_L1S(DIM, KT, double, 8) SPH_INST_L1S(DIM, KT, float, 1)                         \
+  SPH_INST_L1S(DIM, KT, double, 1) SPH_INST_L1S(DIM, KT, double, 4) SPH_INST_L1S(DIM, KT, double, 8) \
+  SPH_INST_L1S(DIM, KT, float, 1)                                                          \
   SPH_INST_L2(DIM, KT, double, double4, 1) SPH_INST_L2(DIM, KT, double, double4, 4)        \
   SPH_INST_L2(DIM, KT, double, double4, 8) SPH_INST_L2(DIM, KT, float, float4, 1)          \
   SPH_INST_SPEC(DIM, KT, double, double4, 1) SPH_INST_SPEC(DIM, KT, double, double4, 4)    \

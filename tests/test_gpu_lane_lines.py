@@ -107,6 +107,25 @@ def test_every_field_of_the_mixed_path(gpu, name, make, kw):
     _check(state, st, "mixed", kw)
 
 
+def _simple1d(n):
+    state, st = P.hydro1d(n)
+    state[C.ec_adden - 1] = C.YESNO["no"]
+    return state, st
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("make", [lambda: _simple1d(1000), lambda: P.hydro2d(199, seed=3, jitter=0.05, adden="no"),
+                                  lambda: P.hydro2d(201, seed=3, jitter=0.05, adden="no"),
+                                  lambda: P.hydro2d(388, seed=3, jitter=0.05, adden="no"),
+                                  lambda: P.diffusion3d(34, ddw="2nw+-", adden="no", kind="square", h_scale=1.03),
+                                  lambda: P.diffusion3d(35, ddw="2nw+-", adden="no", kind="square", h_scale=1.03)],
+                         ids=["1d", "2d_199", "2d_201", "2d_388", "3d_34", "3d_35"])
+def test_direct_summation_on_each_side(gpu, make, precision):
+    # c1simple takes loop 1's lanes of uneven lists in FP64, one in FP32
+    state, st = make()
+    _check(state, st, precision, {})
+
+
 @pytest.mark.parametrize("equations,fld", [("hydro", False), ("magnetohydro", False), ("hydro", True)],
                          ids=["hydro", "mhd", "fld"])
 def test_even_lists_of_moving_particles_keep_their_bits(gpu, equations, fld):
