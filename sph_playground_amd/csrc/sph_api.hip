@@ -1142,16 +1142,17 @@ static bool lanes_follow_lists(const sph_ctx *c, const Phys &P) {
   return differ(true) || differ(false);
 }
 
-// fn(constant G) for lanes = 1, 4 (where HAS4) or 8 (where HAS8)
-template <bool HAS4, bool HAS8, typename Fn>
+// fn(constant G) for lanes = 1 (where HAS1), 4 (HAS4) or 8 (HAS8): the counts
+// loop_lanes can give a kernel
+template <bool HAS1, bool HAS4, bool HAS8, typename Fn>
 static void with_lanes(int lanes, Fn fn) {
   if constexpr (HAS8) {
-    if (lanes == 8) return fn(std::integral_constant<int, 8>{});
+    if (lanes == 8 || !(HAS4 || HAS1)) return fn(std::integral_constant<int, 8>{});
   }
   if constexpr (HAS4) {
-    if (lanes == 4) return fn(std::integral_constant<int, 4>{});
+    if (lanes == 4 || !HAS1) return fn(std::integral_constant<int, 4>{});
   }
-  fn(std::integral_constant<int, 1>{});
+  if constexpr (HAS1) fn(std::integral_constant<int, 1>{});
 }
 
 template <int DIM, int KT>
@@ -1163,7 +1164,8 @@ static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simpl
     // 100^3 lattice 302, four 267, jittered 403, 279)
     const int lanes = mixed ? 1 : loop_lanes(c, a.p, false, false);
 #define L1S(GR, PT)                                                                                          \
-  with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1 && std::is_same_v<PT, double>>(lanes, [&](auto l) { \
+  with_lanes<DIM != 3 || std::is_same_v<PT, float>, DIM != 1 && std::is_same_v<PT, double>,                  \
+             DIM != 1 && std::is_same_v<PT, double>>(lanes, [&](auto l) {                                    \
     constexpr int G = decltype(l)::value;                                                                    \
     hipLaunchKernelGGL((k_loop1_simple<DIM, KT, GR, PT, G>), dim3(grid_for((int64_t)a.n * G)), dim3(kBlock), 0, \
                        c->stream, a, F);                                                                     \
@@ -1178,7 +1180,7 @@ static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simpl
   }
   const int lanes = loop_lanes(c, a.p, false, c->even == 1);
 #define L1(GR, PT)                                                                                           \
-  with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1>(lanes, [&](auto l) {                          \
+  with_lanes<true, DIM != 1 && std::is_same_v<PT, double>, DIM != 1>(lanes, [&](auto l) {                    \
     constexpr int G = decltype(l)::value;                                                                    \
     hipLaunchKernelGGL((k_loop1<DIM, KT, GR, PT, G>), dim3(grid_for((int64_t)a.n * G)), dim3(kBlock), 0, c->stream, a); \
   })
@@ -1275,8 +1277,9 @@ static void launch_sweeps(sph_ctx *c, const Phys &P, int first, int last) {
 
 template <int DIM, int KT, int MODE, typename PT, typename V4>
 static void launch_loop2_p(sph_ctx *c, int lanes, const Loop2Args<V4> &a) {
-  constexpr bool MANY = DIM == 3 || (DIM == 2 && std::is_same_v<PT, double>);
-  with_lanes<MANY, MANY>(lanes, [&](auto l) {
+  constexpr bool F64 = std::is_same_v<PT, double>, MANY = DIM == 3 || (DIM == 2 && F64);
+  constexpr bool MOVING3 = DIM == 3 && MODE >= MODE_SPEC;  // eight lanes, in FP32 also one
+  with_lanes<!(MOVING3 && F64), MANY && !MOVING3, MANY>(lanes, [&](auto l) {
     constexpr int G = decltype(l)::value;
     const dim3 B(grid_for(c->n * G)), T(kBlock);
     if constexpr (MODE == MODE_FAB) hipLaunchKernelGGL((k_loop2_fab<DIM, KT, PT, V4, G>), B, T, 0, c->stream, a);

@@ -2421,9 +2421,10 @@ __global__ void k_sts_stage(double *T, const double *DT, double *y0, double *dy0
 }
 
 // ------------------------------------------------------------ instantiation
-// Lanes per particle as loop_lanes asks for them: 1, 4 and 8 in FP64 and in
-// loop 2 of 3D, 1 and 8 in loop 1 of FP32, 1 alone in loop 2 of 2D in FP32 and
-// in 1D.
+// Lanes per particle as loop_lanes asks for them: 1, 4 and 8 in FP64 (the fixed
+// equation sets in 3D 8 alone, c1simple in 3D 4 and 8) and in loop 2 of 3D in
+// FP32 (the fixed sets 1 and 8), 1 and 8 in loop 1 of FP32, 1 alone in loop 2 of
+// 2D in FP32, in c1simple of FP32 and in 1D.
 #define SPH_INST_L1(DIM, KT, PT, G)                                      \
   template __global__ void k_loop1<DIM, KT, 0, PT, G>(Loop1Args<double4>); \
   template __global__ void k_loop1<DIM, KT, 1, PT, G>(Loop1Args<double4>); \
@@ -2447,18 +2448,19 @@ __global__ void k_sts_stage(double *T, const double *DT, double *y0, double *dy0
 #define SPH_INST_23(DIM, KT)                                                               \
   SPH_INST_L1(DIM, KT, double, 1) SPH_INST_L1(DIM, KT, double, 4) SPH_INST_L1(DIM, KT, double, 8) \
   SPH_INST_L1(DIM, KT, float, 1) SPH_INST_L1(DIM, KT, float, 8)                            \
-  SPH_INST_L1S(DIM, KT, double, 1) SPH_INST_L1S(DIM, KT, double, 4) SPH_INST_L1S(DIM, KT, double, 8) \
-  SPH_INST_L1S(DIM, KT, float, 1)                                                          \
+  SPH_INST_L1S(DIM, KT, double, 4) SPH_INST_L1S(DIM, KT, double, 8) SPH_INST_L1S(DIM, KT, float, 1) \
   SPH_INST_L2(DIM, KT, double, double4, 1) SPH_INST_L2(DIM, KT, double, double4, 4)        \
   SPH_INST_L2(DIM, KT, double, double4, 8) SPH_INST_L2(DIM, KT, float, float4, 1)          \
-  SPH_INST_SPEC(DIM, KT, double, double4, 1) SPH_INST_SPEC(DIM, KT, double, double4, 4)    \
   SPH_INST_SPEC(DIM, KT, double, double4, 8) SPH_INST_SPEC(DIM, KT, float, float4, 1)
+#define SPH_INST_2(KT)                                                                     \
+  SPH_INST_23(2, KT) SPH_INST_L1S(2, KT, double, 1)                                        \
+  SPH_INST_SPEC(2, KT, double, double4, 1) SPH_INST_SPEC(2, KT, double, double4, 4)
 #define SPH_INST_3(KT)                                                                     \
+  SPH_INST_23(3, KT)                                                                       \
   SPH_INST_L2(3, KT, float, float4, 4) SPH_INST_L2(3, KT, float, float4, 8)                \
-  SPH_INST_SPEC(3, KT, float, float4, 4) SPH_INST_SPEC(3, KT, float, float4, 8)
+  SPH_INST_SPEC(3, KT, float, float4, 8)
 SPH_INST_1D(0) SPH_INST_1D(1) SPH_INST_1D(2)
-SPH_INST_23(2, 0) SPH_INST_23(2, 1) SPH_INST_23(2, 2)
-SPH_INST_23(3, 0) SPH_INST_23(3, 1) SPH_INST_23(3, 2)
+SPH_INST_2(0) SPH_INST_2(1) SPH_INST_2(2)
 SPH_INST_3(0) SPH_INST_3(1) SPH_INST_3(2)
 
 #define SPH_INST_NEIGH(DIM)                                                                              \
