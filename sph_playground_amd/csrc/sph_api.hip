@@ -31,7 +31,7 @@ __global__ void k_wrap_reduce(Fields, const int64_t *, int, int64_t, Box, int, l
 __global__ void k_keys(Fields, int, Grid, uint32_t *, uint32_t *, int *, int *, long long *);
 __global__ void k_cell_list(const uint32_t *, const uint32_t *, const int *, int, uint32_t *);
 __global__ void k_move(Fields, Fields, const double *, double *, int, int, const uint32_t *, const int *, const uint32_t *,
-                       int *, const int64_t *, int64_t *, int);
+                       int *, const int64_t *, int64_t *, int, int *);
 __global__ void k_check_sorted(const uint32_t *, int, int *);
 __global__ void k_reorder(Fields, Fields, const uint32_t *, const int64_t *, int64_t *, int, int);
 __global__ void k_cell_start(const uint32_t *, int, uint32_t, int *);
@@ -131,6 +131,7 @@ constexpr int kFullLL = kErrLL + 8;       // and its fullest cell (kFullStripes)
 constexpr int kZeroLL = kFullLL + kFullStripes;
 constexpr int kFlagSlots = 6 * kStripes;
 constexpr int kDtLL = 7 * kStripes;       // the leapfrog pass's time step (not cleared)
+constexpr int kMovedLL = kDtLL + 1;       // an int: the order of the particles broke (cleared by k_keys)
 constexpr int kDtBlocks = 256;            // k_dt_reduce's blocks at most
 // particles of the fullest cell up to which a step orders them by counting
 // (k_move): a particle looks through its whole cell there, which stays a few
@@ -209,6 +210,8 @@ struct sph_ctx {
   int *ccount = nullptr;   // particles per cell key while they are counted, else zero (behind cstart)
   int64_t ncell_cap = 0;
   long long fullest = 0;   // particles in the fullest search cell last seen (0: not known)
+  int breaks = 2;          // how often the particles' moves broke their order lately (see note_order)
+  bool counted = false;    // this step ordered them by counting: whether it had to comes with the search's counts
   bool red_ready = false;  // d_red holds k_wrap_reduce's start values
   bool load_moved = false;   // the load before this step reordered the rows
   bool flags_clear = false;  // the v / B flags' stripes are zero since load_order's k_keys
@@ -631,6 +634,10 @@ static int copied_err(const long long *copy, int base, int word) {
   return reinterpret_cast<const int *>(copy + (kErrLL - base))[word];
 }
 
+// A move of the particles broke their order or left it: `breaks` climbs where
+// more than a third of them did.
+static void note_order(sph_ctx *c, bool broke) { c->breaks = std::clamp(c->breaks + (broke ? 2 : -1), 0, 6); }
+
 static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
   bool ext_short = false;
   if (c->ext_built) {
@@ -643,6 +650,12 @@ static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
     // were left out it is built again with room
     c->ext_version = ext_short ? 0 : c->pos_version;
     c->ext_exact = ext_short;
+  }
+  if (c->counted) {
+    c->counted = false;
+    const bool broke = *reinterpret_cast<const int *>(ll + kMovedLL) != 0;
+    note_order(c, broke);
+    c->stats.sorted = broke ? 1 : 0;
   }
   if (c->flags_pending) {  // k_prep's v / B flags of this step
     c->step_flags = 0;
@@ -804,7 +817,7 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
   const int dim = c->frozen.dim;
   Fields F = c->fields();
   unsigned G = grid_for(n);
-  c->ext_built = false;
+  c->ext_built = c->counted = false;
   // 1. wrap escaped real particles, bounding box, max h (striped reductions).
   //    Positions unchanged since the last pass (so none escaped) and h last
   //    set by the previous step (whose k_post1 reduced h_max): nothing to do.
@@ -833,12 +846,20 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
                          same_grid(g, c->keys_grid);
   if (!keys_kept) {
     // Particles that moved since the keys were made are ordered by counting,
-    // without asking the host whether their order broke (it nearly always
-    // did), unless the last fullest cell was crowded; others are checked first
-    // and sorted if they must be.
-    const bool counted = c->keys_version != c->pos_version && c->fullest > 0 && c->fullest <= kCountedCell &&
+    // without asking the host whether their order broke, unless the last
+    // fullest cell was crowded; others are checked first and sorted if they
+    // must be.  Counting reads and writes every column, which large sets whose
+    // moves mostly leave the order pay for each pass: they are checked too
+    // (diffusion at rest, 128^3 in FP32, a pass 2.23 ms, counted 2.57; 1M
+    // particles in 1D 0.60 and 0.73; at 262k 0.51 and 0.52, at 90k 0.21 and
+    // 0.20; 1000^2 hydro, where the grid's changes break it every other pass,
+    // counted 1.00, checked and sorted 1.14).
+    const bool moves = c->keys_version != c->pos_version;
+    const bool counted = moves && (n < 200000 || c->breaks >= 2) && c->fullest > 0 && c->fullest <= kCountedCell &&
                          nkeys < INT32_MAX;
-    hipLaunchKernelGGL(k_keys, dim3(G), dim3(kBlock), 0, c->stream, F, n, g, c->keys, c->vals, c->d_int + 2,
+    c->counted = counted;
+    int *order_flag = reinterpret_cast<int *>(c->d_stripes + kMovedLL);
+    hipLaunchKernelGGL(k_keys, dim3(G), dim3(kBlock), 0, c->stream, F, n, g, c->keys, c->vals, order_flag,
                        counted ? c->ccount : nullptr, c->d_stripes + kFlagSlots);
     const int nxt = 1 - c->cur;
     Fields src = c->fields();
@@ -855,12 +876,14 @@ static int build_neighbours(sph_ctx *c, bool defer = false) {
       }
       hipLaunchKernelGGL(k_cell_list, dim3(G), dim3(kBlock), 0, c->stream, c->keys, c->vals, c->cstart, n, c->vals2);
       hipLaunchKernelGGL(k_move, dim3(G), dim3(kBlock), 0, c->stream, src, dst, aux_src, aux_dst, c->naux,
-                         (int)c->npad, c->keys, c->cstart, c->vals2, c->ccount, c->orig[c->cur], c->orig[nxt], n);
+                         (int)c->npad, c->keys, c->cstart, c->vals2, c->ccount, c->orig[c->cur], c->orig[nxt], n,
+                         order_flag);
     } else {
-      hipLaunchKernelGGL(k_check_sorted, dim3(std::min(G, 256u)), dim3(kBlock), 0, c->stream, c->keys, n,
-                         c->d_int + 2);
-      RCHK(read_ints(c, 2, 1));
+      hipLaunchKernelGGL(k_check_sorted, dim3(std::min(G, 256u)), dim3(kBlock), 0, c->stream, c->keys, n, order_flag);
+      HIPCHK(hipMemcpyAsync(c->h_int + 2, order_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(wait_stream(c));
       moved = c->h_int[2] != 0;
+      if (moves) note_order(c, moved);
     }
     if (moved && !counted) {
       size_t bytes = c->sort_tmp_bytes;
@@ -1713,6 +1736,7 @@ static int load_impl(sph_ctx *c, int64_t n, const double *store, int64_t ld, int
   c->cur = 0;
   c->fullest = 0;
   c->even = -1;
+  c->breaks = 2;
   c->pos_version++;
   c->vb_version++;
   c->h_version++;

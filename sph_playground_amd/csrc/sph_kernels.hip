@@ -284,36 +284,44 @@ __global__ void k_reorder(Fields src, Fields dst, const uint32_t *perm, const in
 // scatter their stores over cells, 0.33).  Sorting instead costs, at 301^2
 // particles, eight merge passes (44 us) and two reorders (21) against this
 // (11), the list (3) and a scan (7), and a host round trip (25) to ask first.
-__global__ void k_move(Fields src, Fields dst, const double *aux_src, double *aux_dst, int naux, int npad,
-                       const uint32_t *keys, const int *cstart, const uint32_t *list, int *count,
-                       const int64_t *orig_src, int64_t *orig_dst, int n) {
-  if (gtid() >= n) return;
-  const uint32_t s = list[gtid()];
-  const uint32_t key = keys[s];
-  const int c0 = cstart[key], c1 = cstart[key + 1];
-  int d = c0;
-  for (int q = c0; q < c1; q++) d += list[q] < s;
-  count[key] = 0;
-  constexpr int kGroup = 16;  // loads before their stores (see k_reorder)
+// *moved: set where any particle changed its place.
+__global__ __launch_bounds__(256) void k_move(Fields src, Fields dst, const double *aux_src, double *aux_dst, int naux,
+                                              int npad, const uint32_t *keys, const int *cstart, const uint32_t *list,
+                                              int *count, const int64_t *orig_src, int64_t *orig_dst, int n,
+                                              int *moved) {
+  bool changed = false;
+  if (gtid() < n) {
+    const uint32_t s = list[gtid()];
+    const uint32_t key = keys[s];
+    const int c0 = cstart[key], c1 = cstart[key + 1];
+    int d = c0;
+    for (int q = c0; q < c1; q++) d += list[q] < s;
+    changed = d != (int)s;
+    count[key] = 0;
+    constexpr int kGroup = 16;  // loads before their stores (see k_reorder)
 #pragma unroll
-  for (int f0 = 0; f0 < F_TOTAL; f0 += kGroup) {
-    double v[kGroup];
+    for (int f0 = 0; f0 < F_TOTAL; f0 += kGroup) {
+      double v[kGroup];
 #pragma unroll
-    for (int k = 0; k < kGroup; k++) v[k] = src.f[f0 + k][s];
+      for (int k = 0; k < kGroup; k++) v[k] = src.f[f0 + k][s];
 #pragma unroll
-    for (int k = 0; k < kGroup; k++) dst.f[f0 + k][d] = v[k];
+      for (int k = 0; k < kGroup; k++) dst.f[f0 + k][d] = v[k];
+    }
+    const int64_t o = orig_src[s];
+    for (int k0 = 0; k0 < naux; k0 += kGroup) {
+      double v[kGroup];
+#pragma unroll
+      for (int k = 0; k < kGroup; k++)
+        if (k0 + k < naux) v[k] = aux_src[(size_t)(k0 + k) * npad + s];
+#pragma unroll
+      for (int k = 0; k < kGroup; k++)
+        if (k0 + k < naux) aux_dst[(size_t)(k0 + k) * npad + d] = v[k];
+    }
+    orig_dst[d] = o;
   }
-  const int64_t o = orig_src[s];
-  for (int k0 = 0; k0 < naux; k0 += kGroup) {
-    double v[kGroup];
-#pragma unroll
-    for (int k = 0; k < kGroup; k++)
-      if (k0 + k < naux) v[k] = aux_src[(size_t)(k0 + k) * npad + s];
-#pragma unroll
-    for (int k = 0; k < kGroup; k++)
-      if (k0 + k < naux) aux_dst[(size_t)(k0 + k) * npad + d] = v[k];
-  }
-  orig_dst[d] = o;
+  if (__syncthreads_or(changed) && threadIdx.x == 0 &&
+      !__hip_atomic_load(moved, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    __hip_atomic_store(moved, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // First sorted index of every cell key (cstart[K] = number of particles with
