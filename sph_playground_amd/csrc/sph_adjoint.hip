@@ -244,14 +244,14 @@ __global__ __launch_bounds__(256) void k_adj_stage(AdjStage a) {
     for (int u = 0; u < 8; u++)
       if (u < m) acc += l8[u] * r[u];
   });
-  const double u = acc - l * a.dW[s];
+  // each sum in the order its terms come in, one rounding per term
+  const double u = fma(-l, a.dW[s], acc);
   double next;
   if (a.last) {
-    next = (a.A0 ? a.A0[s] + l : 0.0) + a.mh * u;
+    next = fma(a.mh, u, a.A0 ? a.A0[s] + l : 0.0);
   } else {
-    next = a.mu * l + a.mh * u;
-    if (a.lam1) next += a.nu1 * a.lam1[s];
-    a.A0[s] = (a.a0_add ? a.A0[s] : 0.0) + a.c0 * l + a.gh * u;
+    next = fma(a.mh, u, fma(a.mu, l, a.lam1 ? a.nu1 * a.lam1[s] : 0.0));
+    a.A0[s] = fma(a.gh, u, fma(a.c0, l, fma(a.nu0, l, a.a0_add ? a.A0[s] : 0.0)));
   }
   a.out[s] = next;
 }

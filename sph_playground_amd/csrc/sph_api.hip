@@ -2452,7 +2452,8 @@ static void sts_backward_step(sph_ctx *c, int s, double dt, double *const *Y, in
     a.mh = sts_mu_hat(j, s) * dt;
     if (j > 1) {
       a.mu = sts_mu(j); a.gh = sts_gm_hat(j, s) * dt;
-      a.c0 = 1. - a.mu - sts_nu(j) + (j == 2 ? sts_nu(j) : 0.);
+      a.c0 = 1. - a.mu - sts_nu(j);
+      a.nu0 = j == 2 ? sts_nu(j) : 0.;
       a.nu1 = j < s ? sts_nu(j + 1) : 0.;
       a.a0_add = j < s;
     } else {

@@ -341,7 +341,7 @@ struct NlAdjStage {
 // One adjoint stage j of a super-step (k_adj_stage): U = A^T L_j over the
 // reverse lists, then
 //   j > 1: L_{j-1} = mu L_j + mh U + nu1 L_{j+1} (L_{j+1} null for j = s),
-//          A0 (+)= c0 L_j + gh U, what L_0 collects (c0 holds nu too for j = 2)
+//          A0 (+)= nu0 L_j + c0 L_j + gh U, what L_0 collects (nu0: j = 2's nu, else 0)
 //   j = 1 (last): L_0 = A0 + L_1 + mh U
 // into `out`.
 struct AdjStage {
@@ -349,7 +349,7 @@ struct AdjStage {
   const int *rcnt;
   const double *R, *dW, *lam, *lam1;
   double *A0, *out;
-  double mu, mh, nu1, c0, gh;
+  double mu, mh, nu1, nu0, c0, gh;
   int a0_add, last, n, npad, rev;
 };
 // longest reverse list k_rev_sort orders
