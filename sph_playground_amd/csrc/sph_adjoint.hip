@@ -726,7 +726,10 @@ __global__ __launch_bounds__(256) void k_nl_grad(DiffOpArgs a, const double *Y, 
 // operations of their own they were 184 launches of a gradient through 2 FLD
 // super-steps of 4 stages (32^3 particles: 0.41 of 1.74 ms on the device, and
 // a host round trip per stage, 3.68 ms in all).
+// Each product and each sum is rounded by itself, as vector operations round
+// them and a time step per particle still has them.
 __device__ __forceinline__ void nl_stage(const NlStage &o, int s, double f) {
+#pragma clang fp contract(off)
   if (o.orig) {
     o.out[o.orig[s]] = f;
   } else if (o.first) {
@@ -737,6 +740,7 @@ __device__ __forceinline__ void nl_stage(const NlStage &o, int s, double f) {
   }
 }
 __device__ __forceinline__ void nl_adj_stage(const NlAdjStage &o, int s, double v) {
+#pragma clang fp contract(off)
   if (o.orig) {
     o.out[o.orig[s]] = v;
     return;

@@ -3,13 +3,17 @@
 Assembled operators: the adjoint of a super-step is one fused multiply-add per
 term, in the order the terms come in (mu L_j and mu_hat A^T L_j onto what stage
 j + 1 left, nu, 1 - mu - nu and gamma_hat onto L_0's sum), computed here exactly
-and rounded after each term from the transposed operator's own bits.
+and rounded after each term from the transposed operator's own bits.  Operators
+that read grad T: the stages in one call give the bits of the same stages as
+vector operations (a time step per particle takes those), forward, and for
+flux-limited diffusion backward.
 """
 from fractions import Fraction
 
 import numpy as np
 import pytest
 
+from sph_playground_amd import consts as C
 from sph_playground_amd import problems as P
 
 pytestmark = pytest.mark.gpu
@@ -48,4 +52,39 @@ def test_adjoint_super_step_is_its_terms_in_order(gpu, s):
         lam, above, nu_above = low, lam, nu
     want = fma(sts_coeffs(1, s)[2] * dt, transposed(lam), base + lam)
     assert np.array_equal(T0.grad.cpu().numpy(), want)
+    eng.close()
+
+
+def _fld():
+    state, st = P.diffusion2d(12, seed=4, jitter=0.05)
+    state[C.ec_eqs - 1] = C.eeq_manual
+    state[C.ec_eqondiff - 1] = state[C.ec_eqonfluxlim - 1] = 1
+    st[:, C.es_t - 1] += 2.0
+    return state, st
+
+
+@pytest.mark.parametrize("make,backward", [(lambda: P.diffusion2d(12, ddw="2nw-+", seed=4, jitter=0.05), False),
+                                           (lambda: P.diffusion2d(12, ddw="2nw+-", seed=4, jitter=0.05), False),
+                                           (_fld, True)], ids=["2nw-+", "2nw+-", "fld"])
+def test_stages_in_one_call_are_the_vector_operations(gpu, make, backward):
+    import torch
+    from sph_playground_amd import autograd as AG
+    from sph_playground_amd.engine import Engine
+    state, st = make()
+    n, dt = st.shape[0], 1e-5
+    K = None if backward else torch.tensor([1.0, 0.4, 0.1, 0.2, 0.0, 0.0], dtype=torch.float64)
+    eng = Engine(state, kernel="m6")
+    eng.load(st)
+    AG.prepare(eng)
+    g = torch.from_numpy(np.random.default_rng(3).standard_normal(n)).cuda()
+    outs = []
+    for step in (dt, torch.full((n,), dt, dtype=torch.float64, device="cuda")):
+        T0 = torch.from_numpy(st[:, C.es_t - 1].copy()).cuda().requires_grad_(backward)
+        T = AG.sts(T0, K, eng, 4, step, 3, every=2)
+        if backward:
+            T.backward(g)
+        outs.append((T.detach(), T0.grad))
+    assert torch.equal(outs[0][0], outs[1][0])
+    if backward:
+        assert torch.equal(outs[0][1], outs[1][1])
     eng.close()
