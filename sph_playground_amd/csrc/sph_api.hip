@@ -77,7 +77,7 @@ __global__ void k_diff_weights(DiffOpArgs, double *, double *);
 template <int DIM, int KT>
 __global__ void k_diff_rweights(DiffOpArgs, const double *, double *);
 template <int DIM, int KT>
-__global__ void k_diff_gcontract(DiffOpArgs, const double *, const double *, double *);
+__global__ void k_diff_gcontract(DiffOpArgs, const double *, const double *, const double *, const double *, double *);
 __global__ void k_diff_spmv(DiffOpArgs, const double *, const double *, double *);
 __global__ void k_adj_stage(AdjStage);
 __global__ void k_adj_pack(int, AdjRecs, int, int, int, const double *, double2 *);
@@ -2383,26 +2383,32 @@ static AdjStage adj_args(sph_ctx *c) {
   return a;
 }
 template <int DIM>
-static void launch_gcontract_d(sph_ctx *c, const DiffOpArgs &a) {
-  unsigned G = grid_for(c->n);
-  if (c->kt == KT_M4)
-    hipLaunchKernelGGL((k_diff_gcontract<DIM, KT_M4>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dirho, c->dS, c->gpart);
-  else if (c->kt == KT_M6)
-    hipLaunchKernelGGL((k_diff_gcontract<DIM, KT_M6>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dirho, c->dS, c->gpart);
-  else
-    hipLaunchKernelGGL((k_diff_gcontract<DIM, KT_GAUSS>), dim3(G), dim3(kBlock), 0, c->stream, a, c->dirho, c->dS,
-                       c->gpart);
+static void launch_gcontract_d(sph_ctx *c, const DiffOpArgs &a, const double *S, const double *lam) {
+  const dim3 G(grid_for(c->n)), T(kBlock);
+  const double *Z = c->dZ;
+  if (c->kt == KT_M4) hipLaunchKernelGGL((k_diff_gcontract<DIM, KT_M4>), G, T, 0, c->stream, a, c->dirho, S, lam, Z, c->gpart);
+  else if (c->kt == KT_M6) hipLaunchKernelGGL((k_diff_gcontract<DIM, KT_M6>), G, T, 0, c->stream, a, c->dirho, S, lam, Z, c->gpart);
+  else hipLaunchKernelGGL((k_diff_gcontract<DIM, KT_GAUSS>), G, T, 0, c->stream, a, c->dirho, S, lam, Z, c->gpart);
+}
+static void launch_gcontract(sph_ctx *c, const double K[6], const double *S, const double *lam, double *gk) {
+  DiffOpArgs a = diff_args(c, K);
+  if (c->diff_phys.dim == 1) launch_gcontract_d<1>(c, a, S, lam);
+  else if (c->diff_phys.dim == 2) launch_gcontract_d<2>(c, a, S, lam);
+  else launch_gcontract_d<3>(c, a, S, lam);
+  hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)grid_for(c->n), 1.0, 0.0, gk);
 }
 // gk[0..5] += sum over pairs of the accumulated coefficients times G (fixed
 // reduction order); the next record starts new coefficients.
 static void diff_gcontract(sph_ctx *c, const double K[6], double *gk) {
   coef_flush(c);
-  DiffOpArgs a = diff_args(c, K);
-  if (c->diff_phys.dim == 1) launch_gcontract_d<1>(c, a);
-  else if (c->diff_phys.dim == 2) launch_gcontract_d<2>(c, a);
-  else launch_gcontract_d<3>(c, a);
-  hipLaunchKernelGGL(k_gk_accum, dim3(1), dim3(256), 0, c->stream, c->gpart, (int)grid_for(c->n), 1.0, 0.0, gk);
+  launch_gcontract(c, K, c->dS, nullptr, gk);
   c->coef_set = false;
+}
+// The same for one stage: lam^T dA/dK Y.
+static void stage_gcontract(sph_ctx *c, const double K[6], const double *lam, const double *Y, double *gk) {
+  hipLaunchKernelGGL(k_zrho, dim3(grid_for(c->n)), dim3(kBlock), 0, c->stream, (int)c->n, Y, (const double4 *)c->q[0],
+                     c->dZ);
+  launch_gcontract(c, K, nullptr, lam, gk);
 }
 
 static int ensure_dvec(sph_ctx *c, int nvec) { return keep(c, &c->dvec, (size_t)nvec * c->npad); }
@@ -2652,12 +2658,7 @@ int sph_diff_apply_adjoint(sph_ctx *c, const double K[6], const double *d_lam, c
     AdjStage a = adj_args(c);  // A^T lam alone
     a.lam = dv(c, 0); a.out = dv(c, 3); a.mh = 1.0; a.last = 1;
     hipLaunchKernelGGL(k_adj_stage, dim3(G), dim3(kBlock), 0, c->stream, a);
-    c->rec_pend = c->rec_packed = 0;
-    c->coef_set = false;
-    for (int k = 0; k < (yb ? 2 : 1); k++) {
-      adj_record(c, dv(c, 0), dv(c, 1 + k), nullptr, 1.0, 0.0);
-      diff_gcontract(c, K, c->gkdev + 6 * k);
-    }
+    for (int k = 0; k < (yb ? 2 : 1); k++) stage_gcontract(c, K, dv(c, 0), dv(c, 1 + k), c->gkdev + 6 * k);
     hipLaunchKernelGGL(k_from_sorted, dim3(G), dim3(kBlock), 0, c->stream, dv(c, 3), o, n, d_out);
   }
   double g12[12];
