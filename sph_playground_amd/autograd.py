@@ -15,8 +15,9 @@ the prepared step frozen; the backward is the hand-written adjoint.
     ``sph_diff_staged_forward`` / ``sph_diff_staged_backward``; the backward
     recomputes each checkpoint segment's stage states and runs the adjoint
     recurrence (the transposed operator, or the transposed Jacobian at the
-    stage state, and the tensor gradient).  A time step per particle runs the
-    same stages here, each one ``sph_diff_apply`` (``_apply_adjoint``).
+    stage state, and the tensor gradient).  A time step per particle, or an
+    ``every`` that is no integer, runs the same stages here, each one
+    ``sph_diff_apply`` (``_apply_adjoint``).
 
 PyTorch only carries the tensors and the chain rule from K to (kappa_par,
 kappa_perp, theta, phi).
@@ -60,6 +61,14 @@ def _tensor6(K):
     if Kh.shape != (6,):
         raise ValueError("K must have 6 components (xx, yy, zz, xy, xz, yz)")
     return Kh
+
+
+def _whole(v):
+    try:
+        index(v)
+    except TypeError:
+        return False
+    return True
 
 
 def _six(a):
@@ -190,7 +199,8 @@ class DiffusionSTSStaged(torch.autograd.Function):
     def forward(ctx, T0, K, engine, s, dt, nsteps, every):
         T0c = _vector(engine, T0, "T0")
         Kh = _tensor6(K) if K is not None else None
-        ctx.native = nsteps >= 1 and every >= 1 and not (isinstance(dt, torch.Tensor) and dt.numel() != 1)
+        ctx.native = (nsteps >= 1 and every >= 1 and _whole(every)
+                      and not (isinstance(dt, torch.Tensor) and dt.numel() != 1))
         if ctx.native:
             s, dt, nsteps, every = index(s), float(dt), index(nsteps), index(every)
             Y = torch.empty_like(T0c)
