@@ -929,9 +929,9 @@ constexpr int pair_batch(int g) {
 // sweeps 1.57 ms; 8: 1.92, 32: 1.69).
 constexpr int kOrd = 16;
 // The same for loop 2: 8 (MHD tube 1.64 ms; 16, whose rows leave room for
-// fewer waves, 2.2), and the floats between two groups' 17 rows there.
+// fewer waves, 2.2), and the floats between two groups' 18 rows there.
 constexpr int kOrd2 = 8;
-constexpr int kOrdRow2 = 17 * kOrd2 + 4;
+constexpr int kOrdRow2 = 18 * kOrd2 + 4;
 
 // FP32 sums in list order with 8 lanes per particle, in batches of 8 C entries:
 // lane `sub` loads entry 8 c + sub of a batch for each c < C, put(data, c,
@@ -1760,17 +1760,17 @@ void k_loop2(Loop2Args<V4> a) {
     if constexpr (ORD) {
       // Batches of kOrd2 entries as in loop 1: the terms' operands into the
       // group's LDS rows, then lane k runs sum k over them.  Rows: 0 m_b, 1 the
-      // factor x of db and ddt, 2 x of the second term of du (its y is one for
-      // the particle), 3..10 y of the first terms of sums 0..7, 11..13 of the
-      // second terms of dv, 14..16 of its third.
+      // factor x of db and ddt, 2 x of the second term of du, 3..10 y of the
+      // first terms of sums 0..7, 11..14 of the second terms of dv and du, 15..17
+      // of the third of dv.  A lane without a term skips it: times zero, an
+      // infinite factor (Omega 0, rho^2 past FP32) would make its sum NaN.
       constexpr int C = kOrd2 / 8;
       float *const row = ord_ops + (threadIdx.x / 8) * kOrdRow2;
       auto at = [&](int r) { return row + r * kOrd2; };
       const bool dv = sub < 3;
       const float *const x0 = at(sub >= 4 && sub < 7 ? 1 : 0), *const y0 = at(3 + sub);
-      const float *const x1 = at(sub == 3 ? 2 : 0), *const y1 = at(dv ? 11 + sub : 0);
-      const float *const y2 = at(dv ? 14 + sub : 0);
-      const float second = sub == 3 ? i_ra2_oa : 0.f;
+      const float *const x1 = at(sub == 3 ? 2 : 0), *const y1 = at(sub < 4 ? 11 + sub : 0);
+      const float *const y2 = at(dv ? 15 + sub : 0);
       float acc = 0.f;
       for_ordered<C>(a.nb, s, sub, a.npad, nn, load, [&](const J &d, int c, bool valid) {
         float x[3] = {0.f, 0.f, 0.f}, y[3][8] = {};
@@ -1790,10 +1790,10 @@ void k_loop2(Loop2Args<V4> a) {
 #pragma unroll
         for (int q = 0; q < 8; q++) at(3 + q)[8 * c + sub] = y[0][q];
 #pragma unroll
-        for (int q = 0; q < 3; q++) {
-          at(11 + q)[8 * c + sub] = y[1][q];
-          if (TM & 2) at(14 + q)[8 * c + sub] = y[2][q];
-        }
+        for (int q = 0; q < 4; q++) at(11 + q)[8 * c + sub] = y[1][q];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+          if (TM & 2) at(15 + q)[8 * c + sub] = y[2][q];
       }, [&] {
 #pragma unroll
         for (int v = 0; v < kOrd2; v += 4) {
@@ -1803,8 +1803,8 @@ void k_loop2(Loop2Args<V4> a) {
           if (TM & 2) w2 = *reinterpret_cast<const float4 *>(y2 + v);
           auto step = [&](float u, float w, float u_, float w_, float w__) {
             acc = fmaf(u, w, acc);
-            acc = fmaf(u_, dv ? w_ : second, acc);
-            if (TM & 2) acc = fmaf(u, dv ? w__ : 0.f, acc);
+            acc = sub < 4 ? fmaf(u_, w_, acc) : acc;
+            if (TM & 2) acc = dv ? fmaf(u, w__, acc) : acc;
           };
           step(u0.x, w0.x, u1.x, w1.x, w2.x);
           step(u0.y, w0.y, u1.y, w1.y, w2.y);
