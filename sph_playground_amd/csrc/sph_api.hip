@@ -1093,6 +1093,15 @@ static bool loop2_general(const Phys &P) {
            (P.ddw == 400 || P.ddw == 401 || P.ddw == 402));
 }
 
+// Whether loop 2 is k_loop2_fab: fab with one tensor for every pair and no
+// velocity term, by the v and B flags last read.
+static bool loop2_fab(const sph_ctx *c, const Phys &P) {
+  if (loop2_general(P) || P.ddw != 400) return false;
+  const bool reads_v = P.adden && (c->step_flags & 1) != 0;
+  const bool reads_b = P.diso == 0 && (c->step_flags & 2) != 0;
+  return !reads_v && !reads_b;
+}
+
 // Lanes per particle of the pair loops (1, 4 or 8).  One lane walks a list
 // alone: on a lattice in row order the wave's 64 k-th neighbours lie side by
 // side and every list is as long, and the loop is bound by its arithmetic.
@@ -1118,7 +1127,9 @@ static bool loop2_general(const Phys &P) {
 //     and 174, 100^3 236 and 254; jittered 100^3 330 and 243; FP64 lattice
 //     100^3 366 and 361, 128^3 666 and 731; jittered 128^3 1025 and 741).
 //   n2w and fw in FP32: 4 below 225k, then 1 (60^3 102 and 99, 64^3 104 and 113,
-//     100^3 393 and 431, jittered 387 and 409).
+//     100^3 393 and 431, jittered 387 and 409); fab there with velocities or a B
+//     of its own per particle 4, even lists 1 from 225k (with velocities 58^3
+//     131 and 124, 64^3 142 and 160, 80^3 315 and 356; jittered 390 and 346).
 //   Loop 1 in FP64 without hydro: 4, even lists 1 from 700k (128^3 677 and
 //     723, jittered 1015 and 733).
 //   2D, some 28 neighbours: 8 below 40k particles (64^2: sweeps 0.056 ->
@@ -1153,7 +1164,7 @@ static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2, bool even) {
     return P.diff && !P.fld && (P.ddw == 403 || P.ddw == 404) && n >= 300000 ? 1 : 4;
   }
   if (mixed && P.ddw != 400) return n < 225000 ? 4 : 1;
-  return n >= 700000 && even ? 1 : 4;
+  return n >= (mixed && !loop2_fab(c, P) ? 225000 : 700000) && even ? 1 : 4;
 }
 
 // Whether the evenness of the lists decides over lanes whose sums it rounds
@@ -1402,9 +1413,7 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
   a.out = F; a.energy_part = c->energy_part; a.err = step_err(c) + kErrLoop2; a.b = c->box; a.p = P; a.n = n;
   a.npad = (int)c->npad;
   HIPCHK(mark(c, 5));
-  // fab with one tensor for every pair and no velocity term: the loop
-  // without run-time choices
-  const bool fab = !generic && P.ddw == 400 && q1 == nullptr && q4 == nullptr;
+  const bool fab = loop2_fab(c, P);  // the loop without run-time choices
   const int terms = generic ? loop2_terms(c, P) : -1;
   const int lanes = loop_lanes(c, P, true, c->even == 1);
   if (terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, lanes, &a);

@@ -34,6 +34,12 @@ def _diffusion(side, ddw):
     return P.diffusion3d(side, ddw=ddw, b=(1.0, 0.4, 0.3), kind="square", h_scale=1.03)
 
 
+def _varied(side):
+    state, st = _diffusion(side, "fab")
+    st[:, C.es_bx - 1] += 0.3 * np.sin(2.0 * np.pi * st[:, 1])
+    return state, st
+
+
 def _moving(side, equations="hydro", fld=False):
     n = side ** 3
     box = (0.0, 1.0, 0.0, 1.0, 0.0, 1.0)
@@ -57,6 +63,9 @@ EVEN = [
     # n2w and fw in FP32: from 225,000
     ("n2w_60", lambda: _diffusion(60, "n2w"), FULL, ("mixed",)),
     ("fw_61", lambda: _diffusion(61, "fw"), FULL, ("mixed",)),
+    # fab with a B per particle in FP32: from 225,000
+    ("fab_b_60", lambda: _varied(60), FULL, ("mixed",)),
+    ("fab_b_61", lambda: _varied(61), FULL, ("mixed",)),
 ]
 
 VECTORS = (("ax", "ay", "az"), ("dbx", "dby", "dbz"), ("dtdx", "dtdy", "dtdz"))
