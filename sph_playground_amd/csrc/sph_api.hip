@@ -238,7 +238,7 @@ struct sph_ctx {
   uint32_t *nb = nullptr;
   int nb_cap = 0;
   int last_maxcnt = 0;  // longest neighbour list of the last search
-  int even = -1;        // whether its lists were even (lists_even; -1: none since the load)
+  int even = -1;        // how even its lists were (lists_evenness; -1: none since the load)
   long long step_flags = 0;       // k_prep's v / B flags of this step
   bool loop2_pending = false;     // loop 2's read-back still to be taken
   bool neigh_pending = false;     // the search's read-back still to be taken (loop 1's first sync brings it)
@@ -666,7 +666,7 @@ static int finish_neighbours(sph_ctx *c, const long long *ll, int bits) {
   c->stats.n_pairs = stripe_sum(ll, 0);
   int maxcnt = (int)stripe_max(ll, 1);
   c->last_maxcnt = maxcnt;
-  c->even = lists_even(maxcnt, c->n_real, c->stats.n_pairs) ? 1 : 0;
+  c->even = lists_evenness(maxcnt, c->n_real, c->stats.n_pairs);
   c->stats.ms_k_neigh = elapsed(c, c->ev[4], c->ev[7]);
   if (bits & EB_TRUNC) return SPH_ERR_NEIGH_TRUNCATED;
   if (!(bits & EB_OVERFLOW)) return SPH_OK;
@@ -1107,99 +1107,142 @@ static bool loop2_fab(const sph_ctx *c, const Phys &P) {
 // side and every list is as long, and the loop is bound by its arithmetic.
 // Where lists differ the wave waits for its longest and its k-th neighbours
 // drift apart; several lanes of one particle read runs of its cell rows
-// instead, and few particles then still fill the chip.  Measured, one lane
-// against several, loop 2 where nothing else is said (us):
+// instead, and few particles then still fill the chip.  Short lists leave a lane
+// little more to do than what every lane repeats.  So the lines lie by the
+// particles (1D: always one lane), by the length of a list as kernel and hfac
+// give it (short: M4 at hfac 1.0, 33 in 3D; medium: M4 at 1.2, 58; long: M6, 113
+// and more; 2D: M4 13 to 18, M6 28) and by how even the lists are.  Measured,
+// one lane against several, loop 2 where nothing else is said (us):
 //   3D below 40k particles: 8 (2nw FP64 at 30^3 108 against 49).
 //   Particles that move (hydro, MHD, FLD): 8 (FP32 MHD tube of 1M 3440 against
 //     1640, sweeps 2650 against 1570; FP64 hydro tube of 300k 1118 against
-//     515), but even lists take 1 where more lanes only add work: in FP32 from
-//     170k particles (lattice, hydro: 56^3 127 and 135, 64^3 154 and 192,
-//     128^3 1207 and 1500; sweeps with grad T 64^3 69 and 92), in FP64 the
-//     sets that are not fixed at compile time from 110k (hydro with diffusion:
-//     46^3 208 and 194, 58^3 338 and 364, 100^3 1522 and 1862).
-//   General form without hydro: 4, even lists 1 from 110k in FP64 (2nw: 48^3
-//     141 and 159, 64^3 272 and 337; FLD 46^3 200 and 179, 64^3 387 and 436) and
-//     from 150k in FP32 (2nw: 52^3 124 and 114, 54^3 127 and 135, 100^3 722 and
-//     823; FLD 58^3 152 and 173; jittered, uneven: 64^3 320 and 222); the 2nw
-//     operators 1 from 300k on also where lists are uneven (FP64 80^3 616 and
-//     661).
-//   fab (and FP64 n2w, fw): 4, even lists 1 from 700k (FP32 lattice 88^3 172
-//     and 174, 100^3 236 and 254; jittered 100^3 330 and 243; FP64 lattice
-//     100^3 366 and 361, 128^3 666 and 731; jittered 128^3 1025 and 741).
-//   n2w and fw in FP32: 4 below 225k, then 1 (60^3 102 and 99, 64^3 104 and 113,
-//     100^3 393 and 431, jittered 387 and 409); fab there with velocities or a B
-//     of its own per particle 4, even lists 1 from 225k (with velocities 58^3
-//     131 and 124, 64^3 142 and 160, 80^3 315 and 356; jittered 390 and 346).
-//   Loop 1 in FP64 without hydro: 4, even lists 1 from 700k (128^3 677 and
-//     723, jittered 1015 and 733).
-//   2D, some 28 neighbours: 8 below 40k particles (64^2: sweeps 0.056 ->
-//     0.025 ms, loop 2 0.029 -> 0.011), 4 below 150k (256^2 0.051 -> 0.041 and
-//     0.032 -> 0.025), then 1 (512^2 0.078 against 0.089, 0.069 against 0.071).
+//     515).  FP32 takes 1 for even lists from 170k (lattice, hydro: 56^3 127 and
+//     135, 64^3 154 and 192, 128^3 1207 and 1500; sweeps with grad T 64^3 69 and
+//     92), medium ones from 110k (56^3 60 and 76), short ones, also disordered,
+//     from 90k (46^3 32 and 34, 56^3 jittered 45 and 57); its sweeps with grad T
+//     sooner (medium, jittered 56^3 37 and 48; short, a glass 31 and 38).  FP64
+//     loop 1: short, disordered from 90k (56^3 28 and 32, 80^3 53 and 74), medium,
+//     even from 200k (64^3 44 and 53); a fixed set's loop 2: the short ones (80^3
+//     lattice 138 and 171, jittered 166 and 175).  FP64 sets that are not fixed
+//     at compile time: even from 110k (hydro with diffusion 46^3 208 and 194, 58^3
+//     338 and 364, 100^3 1522 and 1862), a glass from 500k, medium 200k, short
+//     100k (100^3 jittered 1609 and 1738; medium 64^3 266 and 304; short 131 and
+//     187), random particles 8 (tube of 300k 1480 and 1022).
+//   General form without hydro: 4.  FP64: even 1 from 110k (2nw: 48^3 141 and
+//     159, 64^3 272 and 337; FLD 46^3 200 and 179, 64^3 387 and 436), medium and
+//     disordered too from 200k (2nw 64^3 174 and 204), short ones from 75k (46^3
+//     46 and 51).  FP32: even 1 from 150k (2nw: 52^3 124 and 114, 54^3 127 and 135,
+//     100^3 722 and 823; FLD 58^3 152 and 173; jittered 64^3 320 and 222), medium
+//     and short 120k (short, jittered 56^3 43 and 55).  The 2nw operators 1 from
+//     300k on also where lists are uneven (FP64 80^3 616 and 661).
+//   fab (and FP64 n2w, fw): 4, even 1 from 700k (FP32 lattice 88^3 172 and 174,
+//     100^3 236 and 254; jittered 100^3 330 and 243; FP64 lattice 100^3 366 and
+//     361, 128^3 666 and 731; jittered 128^3 1025 and 741), medium from 150k in
+//     FP32 and 200k in FP64 (64^3 36 and 43, 50 and 57), short and disordered ones
+//     from 100k and 150k (56^3 22 and 25; 80^3 61 and 75; FP64 n2w a glass too,
+//     80^3 122 and 135).
+//   n2w and fw in FP32: 4 below 225k (medium 200k, short 150k), then 1 (60^3 102
+//     and 99, 64^3 104 and 113, 100^3 393 and 431, jittered 387 and 409; short
+//     64^3 37 and 46); fab there with velocities or a B of its own per particle 4,
+//     even lists 1 from the same lines (with velocities 58^3 131 and 124, 64^3 142
+//     and 160, 80^3 315 and 356; jittered 390 and 346).
+//   Loop 1 in FP64 without hydro: as fab (128^3 677 and 723, jittered 1015 and
+//     733; medium 64^3 50 and 55; short 64^3 jittered 37 and 41).
+//   2D: 8 below 40k particles (M6 64^2: sweeps 0.056 -> 0.025 ms, loop 2 0.029 ->
+//     0.011), 4 below 150k (256^2 0.051 -> 0.041 and 0.032 -> 0.025), then 1 (512^2
+//     0.078 against 0.089, 0.069 against 0.071); M4 90k (387^2 30 and 35).
 // FP32: loop 1 keeps its sums in list order on 8 lanes (k_loop1), which pays
 // below 100k particles in 3D diffusion (46^3 45.8 against 43, 58^3 58 against
-// 75) and below 40k in 2D; loop 2 of 2D stays on one lane, since
+// 75; medium 50k, short 36k: 40^3 20 and 22, 15 and 18) and below 40k in 2D;
+// loop 2 of 2D stays on one lane, since
 // the accelerations of a 2D set at rest are the small remainder of large terms
 // and another order's rounding moves them by 4e-5.  The same for loop 2 of
 // particles that move where the equation set is not fixed (k_loop2).
 // `even` is of the step's own lists wherever it changes how a sum is rounded
 // (run_advanced), so that a step's bits depend on nothing before it.
-static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2, bool even) {
+static int loop_lanes(const sph_ctx *c, const Phys &P, bool loop2, int even) {
   const int64_t n = c->n;
   const bool mixed = c->opt.precision == 1;
   if (P.dim == 1 || (mixed && loop2 && P.dim == 2)) return 1;
+  const double reach = P.krad * P.hfac;
   if (P.dim == 2) {
     if (n < 40000) return 8;
-    return !mixed && n < 150000 ? 4 : 1;
+    return !mixed && n < (kPi * reach * reach < 22.0 ? 90000 : 150000) ? 4 : 1;
   }
-  const bool fixed_set = loop2_terms(c, P) >= 0;
+  const double near = 4.0 / 3.0 * kPi * reach * reach * reach;
+  const int len = near < 45.0 ? 0 : (near < 90.0 ? 1 : 2);
+  // n at or past the line of its list length (short, medium, long)
+  auto past = [&](int64_t s, int64_t m, int64_t l) { return n >= (len == 0 ? s : (len == 1 ? m : l)); };
+  const int64_t never = INT64_MAX;
+  const bool grad_t = P.diff || P.fld;
   if (P.hydro) {
-    if (mixed && loop2 && !fixed_set) return 1;
-    if (mixed) return n >= 170000 && even ? 1 : 8;
-    return loop2 && !fixed_set && n >= 110000 && even ? 1 : 8;
+    const bool fixed_set = loop2_terms(c, P) >= 0;
+    if (mixed) {
+      if (loop2 && !fixed_set) return 1;
+      if (!loop2 && grad_t && even >= (len == 0 ? kGlass : kNearEven) && past(90000, 100000, never)) return 1;
+      return even >= (len == 0 ? kNearEven : kEven) && past(90000, 110000, 170000) ? 1 : 8;
+    }
+    if (loop2 && !fixed_set)
+      return (even >= kEven && past(90000, 110000, 110000)) || (even >= kGlass && past(100000, 200000, 500000)) ? 1 : 8;
+    if (even >= kNearEven && past(90000, never, never)) return 1;
+    return !loop2 && even >= kEven && past(never, 200000, never) ? 1 : 8;
   }
-  if (mixed && !loop2) return n < 100000 ? 8 : 1;
+  if (mixed && !loop2) return past(36000, 50000, 100000) ? 1 : 8;
   if (n < 40000) return 8;
   if (loop2 && loop2_general(P)) {
-    if (n >= (mixed ? 150000 : 110000) && even) return 1;
-    return P.diff && !P.fld && (P.ddw == 403 || P.ddw == 404) && n >= 300000 ? 1 : 4;
+    if (even >= (len == 0 ? kNearEven : kEven) && (mixed ? past(120000, 120000, 150000) : past(75000, 90000, 110000)))
+      return 1;
+    if (!mixed && even >= kGlass && past(200000, 200000, never)) return 1;
+    return !P.fld && (P.ddw == 403 || P.ddw == 404) && P.diff && n >= 300000 ? 1 : 4;
   }
-  if (mixed && P.ddw != 400) return n < 225000 ? 4 : 1;
-  return n >= (mixed && !loop2_fab(c, P) ? 225000 : 700000) && even ? 1 : 4;
+  if (mixed && !loop2_fab(c, P)) return past(150000, 200000, 225000) && (P.ddw != 400 || even >= kEven) ? 1 : 4;
+  if (len == 0) {
+    const int enough = loop2 && !mixed && P.ddw != 400 ? kGlass : kNearEven;
+    return even >= enough && n >= (mixed ? 100000 : 150000) ? 1 : 4;
+  }
+  return even >= kEven && (mixed ? past(never, 150000, 700000) : past(never, 200000, 700000)) ? 1 : 4;
 }
 
-// Whether the evenness of the lists decides over lanes whose sums it rounds
-// otherwise (FP32 sums of loop 1, and of loop 2 of a fixed equation set, are in
-// the list's order on any lanes).
-static bool lanes_follow_lists(const sph_ctx *c, const Phys &P) {
-  auto differ = [&](bool loop2) { return loop_lanes(c, P, loop2, false) != loop_lanes(c, P, loop2, true); };
-  if (c->opt.precision == 1) return loop2_terms(c, P) < 0 && differ(true);
-  return differ(true) || differ(false);
+// The evennesses (a bit each) whose lanes round the sums as those of `even` do:
+// FP32 sums of loop 1, and of loop 2 of a fixed equation set, are in the list's
+// order on any lanes.
+static int same_rounding(const sph_ctx *c, const Phys &P, int even) {
+  const bool mixed = c->opt.precision == 1;
+  int same = 0;
+  for (int e = kRandom; e <= kEven; e++) {
+    bool eq = (mixed && loop2_terms(c, P) >= 0) || loop_lanes(c, P, true, e) == loop_lanes(c, P, true, even);
+    eq = eq && (mixed || loop_lanes(c, P, false, e) == loop_lanes(c, P, false, even));
+    if (eq) same |= 1 << e;
+  }
+  return same;
 }
+constexpr int kAnyLists = (1 << (kEven + 1)) - 1;
 
-// fn(constant G) for lanes = 1 (where HAS1), 4 (HAS4) or 8 (HAS8): the counts
+// fn(constant G) for lanes = 1, 4 (where HAS4) or 8 (HAS8): the counts
 // loop_lanes can give a kernel
-template <bool HAS1, bool HAS4, bool HAS8, typename Fn>
+template <bool HAS4, bool HAS8, typename Fn>
 static void with_lanes(int lanes, Fn fn) {
   if constexpr (HAS8) {
-    if (lanes == 8 || !(HAS4 || HAS1)) return fn(std::integral_constant<int, 8>{});
+    if (lanes == 8) return fn(std::integral_constant<int, 8>{});
   }
   if constexpr (HAS4) {
-    if (lanes == 4 || !HAS1) return fn(std::integral_constant<int, 4>{});
+    if (lanes == 4) return fn(std::integral_constant<int, 4>{});
   }
-  if constexpr (HAS1) fn(std::integral_constant<int, 1>{});
+  fn(std::integral_constant<int, 1>{});
 }
 
 template <int DIM, int KT>
 static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simple, Fields F) {
   bool mixed = c->opt.precision == 1;
   if (simple) {
-    // FP32 sums keep the list order: one lane.  FP64: loop 1's lanes of uneven
-    // lists (1M particles in 1D, us: one lane 32, eight 76; 1000^2 82, 122;
-    // 100^3 lattice 302, four 267, jittered 403, 279)
-    const int lanes = mixed ? 1 : loop_lanes(c, a.p, false, false);
+    // FP32 sums keep the list order: one lane.  FP64: loop 1's lanes (1M
+    // particles in 1D, us: one lane 32, eight 76; 1000^2 82, 122), of uneven lists
+    // where they are long (100^3 lattice 302, four 267, jittered 403, 279)
+    const double reach = a.p.krad * a.p.hfac;
+    const bool long_lists = 4.0 / 3.0 * kPi * reach * reach * reach >= 90.0;
+    const int lanes = mixed ? 1 : loop_lanes(c, a.p, false, long_lists ? kRandom : std::max(c->even, 0));
 #define L1S(GR, PT)                                                                                          \
-  with_lanes<DIM != 3 || std::is_same_v<PT, float>, DIM != 1 && std::is_same_v<PT, double>,                  \
-             DIM != 1 && std::is_same_v<PT, double>>(lanes, [&](auto l) {                                    \
+  with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1 && std::is_same_v<PT, double>>(lanes, [&](auto l) { \
     constexpr int G = decltype(l)::value;                                                                    \
     hipLaunchKernelGGL((k_loop1_simple<DIM, KT, GR, PT, G>), dim3(grid_for((int64_t)a.n * G)), dim3(kBlock), 0, \
                        c->stream, a, F);                                                                     \
@@ -1212,9 +1255,9 @@ static void launch_loop1(sph_ctx *c, Loop1Args<double4> &a, int grad, bool simpl
 #undef L1S
     return;
   }
-  const int lanes = loop_lanes(c, a.p, false, c->even == 1);
+  const int lanes = loop_lanes(c, a.p, false, std::max(c->even, 0));
 #define L1(GR, PT)                                                                                           \
-  with_lanes<true, DIM != 1 && std::is_same_v<PT, double>, DIM != 1>(lanes, [&](auto l) {                    \
+  with_lanes<DIM != 1 && std::is_same_v<PT, double>, DIM != 1>(lanes, [&](auto l) {                          \
     constexpr int G = decltype(l)::value;                                                                    \
     hipLaunchKernelGGL((k_loop1<DIM, KT, GR, PT, G>), dim3(grid_for((int64_t)a.n * G)), dim3(kBlock), 0, c->stream, a); \
   })
@@ -1312,8 +1355,8 @@ static void launch_sweeps(sph_ctx *c, const Phys &P, int first, int last) {
 template <int DIM, int KT, int MODE, typename PT, typename V4>
 static void launch_loop2_p(sph_ctx *c, int lanes, const Loop2Args<V4> &a) {
   constexpr bool F64 = std::is_same_v<PT, double>, MANY = DIM == 3 || (DIM == 2 && F64);
-  constexpr bool MOVING3 = DIM == 3 && MODE >= MODE_SPEC;  // eight lanes, in FP32 also one
-  with_lanes<!(MOVING3 && F64), MANY && !MOVING3, MANY>(lanes, [&](auto l) {
+  constexpr bool MOVING3 = DIM == 3 && MODE >= MODE_SPEC;  // one lane or eight
+  with_lanes<MANY && !MOVING3, MANY>(lanes, [&](auto l) {
     constexpr int G = decltype(l)::value;
     const dim3 B(grid_for(c->n * G)), T(kBlock);
     if constexpr (MODE == MODE_FAB) hipLaunchKernelGGL((k_loop2_fab<DIM, KT, PT, V4, G>), B, T, 0, c->stream, a);
@@ -1389,7 +1432,7 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
   sel.pending = pending;
   sel.lists = c->d_stripes + kSearchLL;
   sel.n_real = c->n_real;
-  sel.even = even;
+  sel.even = even == kAnyLists ? 0 : even;
   sel.go = c->d_int + kGoInt;
   hipLaunchKernelGGL(k_post1<V4>, dim3(G), dim3(kBlock), 0, c->stream, F, sel, c->real, n, P.adden ? 1 : 0,
                      c->do_eos, c->eos_iso, c1, P.gamma, q0, q1, q2, q3, q4,
@@ -1415,7 +1458,7 @@ static int run_post_and_loop2(sph_ctx *c, const Phys &P, const long long *pendin
   HIPCHK(mark(c, 5));
   const bool fab = loop2_fab(c, P);  // the loop without run-time choices
   const int terms = generic ? loop2_terms(c, P) : -1;
-  const int lanes = loop_lanes(c, P, true, c->even == 1);
+  const int lanes = loop_lanes(c, P, true, std::max(c->even, 0));
   if (terms == kSpecHydro) launch_loop2_d23<MODE_SPEC + kSpecHydro>(c, P.dim, lanes, &a);
   else if (terms == kSpecMhd) launch_loop2_d23<MODE_SPEC + kSpecMhd>(c, P.dim, lanes, &a);
   else if (terms == kSpecHydroFld) launch_loop2_d23<MODE_SPEC + kSpecHydroFld>(c, P.dim, lanes, &a);
@@ -1464,9 +1507,9 @@ static Phys call_phys(const sph_ctx *c, const double *state) {
 // The tail of a step after loop 1: Newton bookkeeping, EOS and packs
 // (k_post1), loop 2, mti gravity, and a leapfrog pass's corrector or an RKL2 stage.  pending: the
 // still-active stripes of the last sweep queued, when more could follow it;
-// even: what the loops' lanes take the lists for, while the step's own are not
-// known (-1: they are, or no matter).
-static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr, int even = -1) {
+// even: the evennesses of the step's own lists, while they are not known, for
+// which the loops' lanes are right (kAnyLists: they are known, or no matter).
+static int enqueue_tail(sph_ctx *c, const Phys &P, const long long *pending = nullptr, int even = kAnyLists) {
   HIPCHK(mark(c, 2));
   int rc = c->opt.precision == 1 ? run_post_and_loop2<float4>(c, P, pending, even)
                                    : run_post_and_loop2<double4>(c, P, pending, even);
@@ -1534,10 +1577,11 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
     const int rc2 = finish_loop2(c);
     return rc != SPH_OK ? rc : rc2;
   }
-  int even = -1;
-  if (c->neigh_pending && lanes_follow_lists(c, P)) {
-    even = c->even;
-    if (even < 0) {
+  int even = kAnyLists;
+  if (c->neigh_pending && same_rounding(c, P, kRandom) != kAnyLists) {
+    if (c->even >= 0) {
+      even = same_rounding(c, P, c->even);
+    } else {
       HIPCHK(copy_record(c, 0));
       HIPCHK(wait_stream(c));
       const int fin = take_neighbours(c);
@@ -1547,10 +1591,10 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
   }
   auto start_over = [&] {
     first = 1; sweeps = 0; pairs = 0; ms1 = 0.f;
-    even = -1;
+    even = kAnyLists;
   };
   // the step's own lists are known: were the loops queued for such?
-  auto other_lists = [&] { return even >= 0 && c->even != even; };
+  auto other_lists = [&] { return (even >> c->even & 1) == 0; };
   for (;;) {
     const int last = std::min(maxsw, first + std::max(1, c->sweep_hint) - 1);
     launch_sweeps(c, P, first, last);
@@ -1570,7 +1614,7 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
         start_over();
         continue;
       }
-      even = -1;
+      even = kAnyLists;
     }
     const int rc = enqueue_tail(c, P, last < maxsw ? c->d_sweep + (size_t)last * kSweepRegion : nullptr, even);
     // the search's read-back if still pending, error words, the tail's record
@@ -1593,7 +1637,7 @@ static int run_advanced(sph_ctx *c, const Phys &P) {
         start_over();
         continue;
       }
-      even = -1;
+      even = kAnyLists;
     }
     for (int it = first; it <= last; it++) {
       const long long *r = c->h_sweep + (size_t)it * kSweepRegion;

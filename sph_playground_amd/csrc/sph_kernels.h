@@ -241,9 +241,12 @@ struct Loop1Args {
   int sweep;
 };
 
-// Even neighbour lists: the longest within 5 % of the mean.
-__host__ __device__ inline bool lists_even(long long longest, long long n_real, long long pairs) {
-  return pairs > 0 && (double)longest * (double)n_real <= 1.05 * (double)pairs;
+// How even neighbour lists are, by the longest against the mean: a lattice's
+// whole shells, a little disorder, a glass, random particles.
+enum { kRandom = 0, kGlass = 1, kNearEven = 2, kEven = 3 };
+__host__ __device__ inline int lists_evenness(long long longest, long long n_real, long long pairs) {
+  const double most = (double)longest * (double)n_real, all = (double)pairs;
+  return pairs <= 0 || most > 2.0 * all ? kRandom : (most > 1.45 * all ? kGlass : (most > 1.05 * all ? kNearEven : kEven));
 }
 
 // Where k_post1 finds loop 1's result: st[*which] of the two sweep buffers
@@ -251,9 +254,10 @@ __host__ __device__ inline bool lists_even(long long longest, long long n_real, 
 // or loop 1 (err1) raised an error bit (the step then stops or searches again)
 // or when the last sweep queued before the tail left particles active
 // (`pending`, its still-active stripes; null: no matter): more sweeps and
-// another tail follow; nor when the lists are not as even as the loops queued
-// with it assume (`even`, -1: no matter; `lists`: the search's pair counts and
-// list lengths).  *go tells loop 2 which it was.
+// another tail follow; nor when the lists are not of the evenness the loops
+// queued with it assume (`even`, a bit for each that will do, 0: no matter;
+// `lists`: the search's pair counts and list lengths).  *go tells loop 2 which
+// it was.
 struct PostSel {
   const double4 *fin0, *fin1;
   const int *which;

@@ -1306,10 +1306,10 @@ __global__ __launch_bounds__(256) void k_post1(Fields F, PostSel sel, const uint
   if (threadIdx.x < 64) {
     const unsigned long long more = __ballot(sel.pending && sel.pending[threadIdx.x] != 0);
     bool other = false;
-    if (sel.even >= 0) {
+    if (sel.even) {
       const long long pairs = wave_sum(sel.lists[threadIdx.x]);
       const long long longest = wave_max(sel.lists[kStripes + threadIdx.x]);
-      other = lists_even(longest, sel.n_real, pairs) != (sel.even != 0);
+      other = (sel.even >> lists_evenness(longest, sel.n_real, pairs) & 1) == 0;
     }
     if (threadIdx.x == 0) {
       skip = more != 0 || other || *sel.serr != 0 || *sel.err1 != 0;
@@ -2429,10 +2429,9 @@ __global__ void k_sts_stage(double *T, const double *DT, double *y0, double *dy0
 }
 
 // ------------------------------------------------------------ instantiation
-// Lanes per particle as loop_lanes asks for them: 1, 4 and 8 in FP64 (the fixed
-// equation sets in 3D 8 alone, c1simple in 3D 4 and 8) and in loop 2 of 3D in
-// FP32 (the fixed sets 1 and 8), 1 and 8 in loop 1 of FP32, 1 alone in loop 2 of
-// 2D in FP32, in c1simple of FP32 and in 1D.
+// Lanes per particle as loop_lanes asks for them: 1, 4 and 8 in FP64 and in loop
+// 2 of 3D in FP32 (the fixed equation sets in 3D 1 and 8), 1 and 8 in loop 1 of
+// FP32, 1 alone in loop 2 of 2D in FP32, in c1simple of FP32 and in 1D.
 #define SPH_INST_L1(DIM, KT, PT, G)                                      \
   template __global__ void k_loop1<DIM, KT, 0, PT, G>(Loop1Args<double4>); \
   template __global__ void k_loop1<DIM, KT, 1, PT, G>(Loop1Args<double4>); \
@@ -2456,13 +2455,14 @@ __global__ void k_sts_stage(double *T, const double *DT, double *y0, double *dy0
 #define SPH_INST_23(DIM, KT)                                                               \
   SPH_INST_L1(DIM, KT, double, 1) SPH_INST_L1(DIM, KT, double, 4) SPH_INST_L1(DIM, KT, double, 8) \
   SPH_INST_L1(DIM, KT, float, 1) SPH_INST_L1(DIM, KT, float, 8)                            \
-  SPH_INST_L1S(DIM, KT, double, 4) SPH_INST_L1S(DIM, KT, double, 8) SPH_INST_L1S(DIM, KT, float, 1) \
+  SPH_INST_L1S(DIM, KT, double, 1) SPH_INST_L1S(DIM, KT, double, 4) SPH_INST_L1S(DIM, KT, double, 8) \
+  SPH_INST_L1S(DIM, KT, float, 1)                                                          \
   SPH_INST_L2(DIM, KT, double, double4, 1) SPH_INST_L2(DIM, KT, double, double4, 4)        \
   SPH_INST_L2(DIM, KT, double, double4, 8) SPH_INST_L2(DIM, KT, float, float4, 1)          \
-  SPH_INST_SPEC(DIM, KT, double, double4, 8) SPH_INST_SPEC(DIM, KT, float, float4, 1)
+  SPH_INST_SPEC(DIM, KT, double, double4, 1) SPH_INST_SPEC(DIM, KT, double, double4, 8)    \
+  SPH_INST_SPEC(DIM, KT, float, float4, 1)
 #define SPH_INST_2(KT)                                                                     \
-  SPH_INST_23(2, KT) SPH_INST_L1S(2, KT, double, 1)                                        \
-  SPH_INST_SPEC(2, KT, double, double4, 1) SPH_INST_SPEC(2, KT, double, double4, 4)
+  SPH_INST_23(2, KT) SPH_INST_SPEC(2, KT, double, double4, 4)
 #define SPH_INST_3(KT)                                                                     \
   SPH_INST_23(3, KT)                                                                       \
   SPH_INST_L2(3, KT, float, float4, 4) SPH_INST_L2(3, KT, float, float4, 8)                \
