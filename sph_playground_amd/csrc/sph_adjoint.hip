@@ -609,7 +609,7 @@ __global__ void k_from_sorted(const double *src, const int64_t *orig, int n, dou
 
 // These operators are bound by the latency of their gathers (a list entry,
 // then up to five records) and by FP64 divisions: 4 or 8 lanes share a
-// particle (nl_lanes), and 1/|r| is the refined reciprocal square root (a few
+// particle (the host's NL_LAUNCH), and 1/|r| is the refined reciprocal square root (a few
 // ulp, as in loop 2).  32^3 with one lane, one entry at a time and IEEE
 // divisions: grad T 97 us, the FLD operator 105, its adjoint 191; now
 // 19, 17 and 33.

@@ -2307,8 +2307,8 @@ static DiffOpArgs diff_args(sph_ctx *c, const double K[6]) {
 }
 
 // ---- operators that read grad T (frozen geometry; see sph_adjoint.hip)
-// Lanes per particle of these operators: 8 below 40k particles, else 4 (as
-// loop 2's rule for FP64 diffusion).
+// Lanes per particle of these operators: 8 below 40k particles, else 4, in
+// every dimension and whatever the lists are.
 #define COMMA ,
 #define NL_LAUNCH(KERNEL, ...)                                                                                      \
   do {                                                                                                              \
@@ -2571,7 +2571,7 @@ static int reverse_lists_radix(sph_ctx *c, int64_t npairs) {
 // The reverse lists (rent, rcnt) of the last search, capacity rcap.
 static int reverse_lists(sph_ctx *c, int64_t npairs) {
   const int n = (int)c->n, npad = (int)c->npad;
-  // room for an eighth more than the longest forward list, or what is there
+  // room for an eighth more than the longest forward list
   int cap = (c->last_maxcnt + c->last_maxcnt / 8 + 8) / 8 * 8;
   for (;;) {
     RCHK(keep(c, &c->rent, (size_t)npad * cap));

@@ -1,8 +1,8 @@
 // Device kernels of the two-loop hot path for gfx950.
 //
-// Data layout (HBM, "sorted order" = particles ordered by the Morton key of
-// their cell, so a wavefront's 64 particles and their neighbours form compact
-// 3D blobs):
+// Data layout (HBM, "sorted order" = particles ordered by the key of their
+// cell, its row and then x, so a wavefront's 64 particles lie along a row and
+// their neighbours along the rows around it):
 //   fields     32 FP64 SoA arrays, one per store row (const.f90:69-103)
 //   pm         double4 {x, y, z, m}: the 32-byte gather every pair makes
 //   st (x2)    loop-1 Newton state {h, den, om, T}, ping-pong per sweep
